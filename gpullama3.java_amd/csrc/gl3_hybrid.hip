@@ -19,6 +19,7 @@
 #include "gl3_hybrid.h"
 #include "gl3_decode_kernels.h"      // argmax_kernel
 #include "gl3_hy_kernels.h"
+#include "gl3_hy_gemm.h"
 #include "gl3_hy_heads_kernels.h"
 #include "gl3_hy_plain_kernels.h"
 
@@ -36,7 +37,7 @@ using gl3::argmax_kernel;
     } while (0)
 
 static inline int hy_cdiv(int a, int b) { return (a + b - 1) / b; }
-constexpr int HY_MOE_BM = 64;        // rows per tile of the grouped expert GEMMs
+constexpr int HY_MOE_BM = 64, HY_MOE_BM_FEW = 32;        // rows per tile of the grouped expert GEMMs; where experts have few rows each
 constexpr int HY_LATENT_DIRECT = 512;   // longest cached latent row that decode steps score in the latent's space (value columns per lane of the attention core)
 constexpr int HY_ZSPLIT = 16;        // most K-split parts of a product with very few result rows (router, token input's gate): its consumer kernel adds them
 static inline float hy_bf16_to_f32(uint16_t v) { uint32_t u = (uint32_t)v << 16; float f; memcpy(&f, &u, 4); return f; }
@@ -515,7 +516,7 @@ int32_t gl3_hy_create(const gl3_model_desc* desc, gl3_ctx** out, std::string& er
         TRY(hy_alloc(ctx, &h->wsel, P * 4));
         TRY(hy_alloc(ctx, &h->sel, P * 4));
         TRY(hy_alloc(ctx, &h->pair_row, P * 4));
-        TRY(hy_alloc(ctx, &h->tiles, 3 * (P / HY_MOE_BM + max_e + 1) * 4));
+        TRY(hy_alloc(ctx, &h->tiles, 3 * (P / HY_MOE_BM_FEW + max_e + 1) * 4));
         TRY(hy_alloc(ctx, &h->ntiles, 4));
         TRY(hy_alloc(ctx, &h->ea, P * W * es));
         TRY(hy_alloc(ctx, &h->eact, P * max_eff * es));
@@ -904,6 +905,73 @@ int32_t gl3_hy_finalize(gl3_ctx* ctx) {
 // ---- launches -----------------------------------------------------------------------------------------------------------------------
 // activation of the layer's dense feed-forward (in a mixture of experts: of the shared expert)
 static HyGlu hy_ff_glu(const HyLayer& L) { return HyGlu{L.dense_limit, L.d.ff_alpha, L.d.ff_shift, nullptr, nullptr, 0, 0, L.d.ff_act}; }
+// Tiles of hy_gemm_ring_kernel: BM x BN results, WM x WN wavefronts, rings of SA / SW stages.
+enum { HY_R256x256, HY_R256x224, HY_R256x192, HY_R256x160, HY_R256x128, HY_R128x256, HY_R128x160, HY_R128x128, HY_R64x128, HY_R64x64, HY_R_COUNT };
+static const struct { int bm, bn; } HY_RING_TILES[HY_R_COUNT] = {{256, 256}, {256, 224}, {256, 192}, {256, 160}, {256, 128}, {128, 256}, {128, 160}, {128, 128}, {64, 128}, {64, 64}};
+// Which tile and K split: the one with the least estimated time.  A stage of a BM x BN tile takes a CU its operand bytes over the rate a full
+// LDS of loads sustains plus its MFMAs (0.0012 (BM + BN) + 0.0000235 BM BN us in bfloat16; float32 MFMAs are 16 x slower for half the K);
+// 256 CUs take the workgroups in rounds of whole tiles (two workgroups of a small tile share a CU; one alone needs 0.4 us per stage for its loads'
+// way: 88 tokens, 4096 x 4096 in 64 x 64 tiles 16 us as 256 workgroups, 11 us as 512) — what decides for most shapes: 10240 x 4096 at 512 tokens is 256 tiles of 128 x 160
+// (50 us) but 320 of 128 x 128 (65 us) or 160 of 256 x 128 (53 us).  A K split writes and re-reads its part of C at ~4 TB/s.
+static void hy_ring_pick(bool f32, int M, int N, int K, bool glu, bool actmul, int max_parts, int* tile, int* ks_out) {
+    const int stages = K / (f32 ? 32 : 64);
+    double best = 1e30;
+    for (int t = 0; t < HY_R_COUNT; ++t) {
+        const int bm = HY_RING_TILES[t].bm, bn = HY_RING_TILES[t].bn;
+        if (glu ? (t != HY_R256x256 && t != HY_R128x256 && t != HY_R128x128 && t != HY_R64x128) : t == HY_R256x256) continue;
+        if (actmul && t != HY_R256x224 && t != HY_R128x128 && t != HY_R64x64) continue;
+        if (f32 && (t < HY_R256x128 || t == HY_R128x256)) continue;          // (two sets of accumulators)
+        const double stage = 0.0012 * (bm + bn) + (f32 ? 0.000105 : 0.0000235) * bm * bn;
+        const long mn = (long)hy_cdiv(M, bm) * hy_cdiv(N, bn), pair = t >= HY_R128x128 ? 2 : 1;
+        for (int ks = 1; ks <= max_parts && (ks == 1 || stages / ks >= 4); ++ks) {
+            const int per = hy_cdiv(stages, ks);
+            if (hy_cdiv(stages, per) != ks) continue;
+            const long wgs = mn * ks, rest = wgs % (256 * pair);
+            const double rounds = (double)(wgs / (256 * pair)) * pair * (per * stage + 3.0), last = rest == 0 ? 0.0 : rest <= 256 ? per * std::max(stage, 0.4) + 3.0 : 2 * (per * stage + 3.0);
+            const double us = rounds + last + (ks - 1) * (double)M * N * 8 / 4e6;
+            if (us < best) { best = us; *tile = t; *ks_out = ks; }
+        }
+    }
+}
+
+// The ring kernel for a product it can take (true), or nothing.  parts / max_parts as for hy_gemm.
+template <typename T>
+static bool hy_gemm_ring(gl3_ctx* ctx, const T* A, int lda, const HyMat& w, int M, float* C, int ldc, bool glu, T* act, int ld_act, HyGlu gp, int* parts, int max_parts) {
+    const int N = w.rows, K = w.k;
+    constexpr int PE = 16 / (int)sizeof(T), BK = 128 / (int)sizeof(T);
+    if (K % BK || lda % PE || w.ld % PE || (((uintptr_t)A | (uintptr_t)w.w) & 15)) return false;
+    if ((uint64_t)M * lda * sizeof(T) >= 0xffff0000ull || (uint64_t)N * w.ld * sizeof(T) >= 0xffff0000ull) return false;      // 32-bit offsets inside an operand
+    const bool actmul = !glu && (gp.mul_table || gp.act == 2);
+    int tile = HY_R128x128, ks = 1;
+    hy_ring_pick(sizeof(T) == 4, M, N, K, glu, actmul, parts && !glu && !actmul ? max_parts : 1, &tile, &ks);
+    const int kper = hy_cdiv(K / BK, ks) * BK, mt = hy_cdiv(M, HY_RING_TILES[tile].bm), nt = hy_cdiv(N, HY_RING_TILES[tile].bn);
+    if (parts) *parts = ks;
+    const dim3 grid((unsigned)hy_cdiv(mt * nt * ks, 8) * 8);
+#define HY_RG(BM, BN, WM, WN, SA, SW, EPI)                                                                                                              \
+    hipLaunchKernelGGL((hy_gemm_ring_kernel<T, BM, BN, WM, WN, SA, SW, EPI>), grid, dim3(WM * WN * 64), 0, ctx->stream, A, lda, (const T*)w.w, w.ld, M, N, K, C, ldc, act, \
+                       ld_act, gp, mt, nt, ks, kper)
+    if constexpr (sizeof(T) == 2) {          // tiles of the bfloat16 plans only
+        if (tile == HY_R256x256) { HY_RG(256, 256, 8, 1, 2, 3, HY_EPI_GLU); return true; }
+        if (tile == HY_R128x256) { if (glu) HY_RG(128, 256, 4, 2, 2, 3, HY_EPI_GLU); else HY_RG(128, 256, 4, 2, 2, 3, HY_EPI_STORE); return true; }
+        if (tile == HY_R256x224) { if (actmul) HY_RG(256, 224, 8, 1, 2, 3, HY_EPI_ACTMUL); else HY_RG(256, 224, 8, 1, 2, 3, HY_EPI_STORE); return true; }
+        if (tile == HY_R256x192) { HY_RG(256, 192, 4, 2, 2, 4, HY_EPI_STORE); return true; }
+        if (tile == HY_R256x160) { HY_RG(256, 160, 8, 1, 2, 4, HY_EPI_STORE); return true; }
+    }
+    if (glu) {
+        if (tile == HY_R64x128) HY_RG(64, 128, 2, 2, 2, 4, HY_EPI_GLU); else HY_RG(128, 128, 4, 2, 2, 3, HY_EPI_GLU);
+    } else if (actmul) {
+        if (tile == HY_R64x64) HY_RG(64, 64, 2, 2, 2, 6, HY_EPI_ACTMUL); else HY_RG(128, 128, 4, 2, 2, 3, HY_EPI_ACTMUL);
+    } else switch (tile) {
+        case HY_R256x128: HY_RG(256, 128, 4, 2, 3, 4, HY_EPI_STORE); break;
+        case HY_R128x160: HY_RG(128, 160, 4, 1, 3, 5, HY_EPI_STORE); break;
+        case HY_R64x128: HY_RG(64, 128, 2, 2, 2, 4, HY_EPI_STORE); break;
+        case HY_R64x64: HY_RG(64, 64, 2, 2, 2, 6, HY_EPI_STORE); break;
+        default: HY_RG(128, 128, 4, 2, 2, 3, HY_EPI_STORE);
+    }
+#undef HY_RG
+    return true;
+}
+
 // parts != null: C has room for HY_KSPLIT copies and the caller sums them (the streams kernel does); *parts = copies written
 template <typename T>
 static void hy_gemm(gl3_ctx* ctx, const T* A, int lda, const HyMat& w, int M, float* C, int ldc, bool glu, T* act, int ld_act, HyGlu gp, int* parts = nullptr, int max_parts = HY_KSPLIT) {
@@ -927,6 +995,8 @@ static void hy_gemm(gl3_ctx* ctx, const T* A, int lda, const HyMat& w, int M, fl
 #undef HY_MV
         return;
     }
+    if (hy_gemm_ring<T>(ctx, A, lda, w, M, C, ldc, glu, act, ld_act, gp, parts, max_parts)) return;
+    // shapes the ring kernel does not take: ragged K, rows that do not start on 16 bytes
     const long tiles = (long)hy_cdiv(M, 128) * hy_cdiv(N, 128);
     const bool big = tiles >= 256 || (parts && tiles >= 64);
     constexpr int BKT = HyPiece<T>::N * HyPiece<T>::PPR;
@@ -1327,9 +1397,9 @@ static void hy_ff_up(gl3_ctx* ctx, const T* hb, HyLayer& L, int n, T* act) {
 // ---- mixture of experts -------------------------------------------------------------------------------------------------------------
 // One product of every (token, choice) pair with its expert's matrix: w = ONE expert's shape (rows, k, ld) at the base of the stacked
 // matrix, wstride elements apart.  few = a few tokens (decode): pairs in their own order, one matvec per pair (blockIdx.y) with the
-// expert read from h->sel; else the pairs ordered by expert (h->tiles) and one MFMA tile per HY_MOE_BM rows of an expert.
+// expert read from h->sel; else the pairs ordered by expert (h->tiles) and one MFMA tile per bm rows of an expert.
 template <typename T>
-static void hy_gemm_grouped(gl3_ctx* ctx, const T* A, int lda, const HyMat& w, size_t wstride, int P, int max_tiles, bool few, float* C, int ldc, bool glu, T* act, int ld_act, HyGlu gp,
+static void hy_gemm_grouped(gl3_ctx* ctx, const T* A, int lda, const HyMat& w, size_t wstride, int P, int bm, int max_tiles, bool few, float* C, int ldc, bool glu, T* act, int ld_act, HyGlu gp,
                             int n_sel, int a_div = 1, const float* row_scale = nullptr) {
     gl3_hybrid_state* h = ctx->hy;
     const T* Wt = (const T*)w.w;
@@ -1351,6 +1421,15 @@ static void hy_gemm_grouped(gl3_ctx* ctx, const T* A, int lda, const HyMat& w, s
     }
     const HyGroup grp{h->tiles, h->ntiles, wstride};
     const dim3 grid(hy_cdiv(N, 128), max_tiles, 1);
+    constexpr int PE = 16 / (int)sizeof(T), BK = 128 / (int)sizeof(T);
+    if (K % BK == 0 && lda % PE == 0 && w.ld % PE == 0 && wstride % PE == 0 && (((uintptr_t)A | (uintptr_t)Wt) & 15) == 0 && (uint64_t)N * w.ld * sizeof(T) < 0xffff0000ull) {
+#define HY_RGG(BM, WM, EPI) hipLaunchKernelGGL((hy_gemm_ring_kernel<T, BM, 128, WM, 2, 2, 4, EPI, 1>), grid, dim3(WM * 128), 0, st, A, lda, Wt, w.ld, 0, N, K, C, ldc, act, ld_act, gp, 0, 0, 1, K, grp)
+#define HY_RGG_EPI(BM, WM) do { if (glu) HY_RGG(BM, WM, HY_EPI_GLU); else if (gp.act == 2) HY_RGG(BM, WM, HY_EPI_ACTMUL); else HY_RGG(BM, WM, HY_EPI_STORE); } while (0)
+        if (bm == HY_MOE_BM_FEW) HY_RGG_EPI(HY_MOE_BM_FEW, 1); else HY_RGG_EPI(HY_MOE_BM, 2);
+#undef HY_RGG_EPI
+#undef HY_RGG
+        return;
+    }
     if (glu) hipLaunchKernelGGL((hy_gemm_kernel<T, T, HY_MOE_BM, 128, HY_EPI_GLU, 1>), grid, dim3(256), 0, st, A, lda, Wt, w.ld, 0, N, K, C, ldc, act, ld_act, gp, K, grp);
     else if (gp.act == 2) hipLaunchKernelGGL((hy_gemm_kernel<T, T, HY_MOE_BM, 128, HY_EPI_ACTMUL, 1>), grid, dim3(256), 0, st, A, lda, Wt, w.ld, 0, N, K, C, ldc, act, ld_act, gp, K, grp);
     else hipLaunchKernelGGL((hy_gemm_kernel<T, T, HY_MOE_BM, 128, HY_EPI_STORE, 1>), grid, dim3(256), 0, st, A, lda, Wt, w.ld, 0, N, K, C, ldc, act, ld_act, gp, K, grp);
@@ -1368,7 +1447,10 @@ static void hy_moe(gl3_ctx* ctx, HyLayer& L, int n) {
     int zparts = 1;          // few result rows and a long K: the router's product comes in K-split parts that the route kernel adds
     hy_gemm<T>(ctx, hb, W, L.router, n, h->moe_z, RZ, false, nullptr, 0, HyGlu{}, &zparts, HY_ZSPLIT);
     const bool few = n <= 8;
-    const int max_tiles = P / HY_MOE_BM + std::min(E, P);
+    // rows per tile: an expert has P / E rows on average; with fewer than 48 half of a 64-row tile would be padding
+    // (181 tokens x 4 of 32 experts, float32, 2 x 1024 x 2048: 219 us with 64-row tiles of hy_gemm_kernel)
+    const int bm = P < 48 * E ? HY_MOE_BM_FEW : HY_MOE_BM;
+    const int max_tiles = P / bm + std::min(E, P);
     const bool on_out = d.route_on_output != 0;          // the weights multiply the experts' outputs (in the residual update) instead of their inputs
     const HyRoute rt{d.route_softmax, L.route_bias, d.route_renorm, d.route_scale != 0.f ? d.route_scale : 1.f, d.route_groups, d.route_keep, E, d.route_group_max};
 #define HY_RT(PER) hipLaunchKernelGGL((hy_route_kernel<PER>), dim3(n), dim3(64), 0, st, h->moe_z, RZ, zparts, (size_t)n * RZ, E + d.identity, top, h->sel, h->wsel,          \
@@ -1381,15 +1463,15 @@ static void hy_moe(gl3_ctx* ctx, HyLayer& L, int n) {
     const size_t gu_stride = (size_t)one_gu.rows * L.egu.ld;
     if (few) {
         // a few tokens: the pairs of a token read its normed row themselves and the score multiplies the products (W (s h) = s (W h))
-        hy_gemm_grouped<T>(ctx, hb, W, one_gu, gu_stride, P, max_tiles, true, nullptr, 0, glu, (T*)h->eact, L.eff_pad,
+        hy_gemm_grouped<T>(ctx, hb, W, one_gu, gu_stride, P, bm, max_tiles, true, nullptr, 0, glu, (T*)h->eact, L.eff_pad,
                            HyGlu{d.ff_limit, d.ff_alpha, d.ff_shift, nullptr, nullptr, 0, 0, d.ff_act}, E, top, on_out ? nullptr : h->wsel);
     } else {
-        hipLaunchKernelGGL(hy_moe_group_kernel, dim3(1), dim3(256), (size_t)2 * E * 4, st, h->sel, P, E, HY_MOE_BM, h->pair_row, h->tiles, h->ntiles);
+        hipLaunchKernelGGL(hy_moe_group_kernel, dim3(1), dim3(256), (size_t)2 * E * 4, st, h->sel, P, E, bm, h->pair_row, h->tiles, h->ntiles);
         hipLaunchKernelGGL((hy_moe_scale_kernel<T>), dim3(P), dim3(256), 0, st, hb, W, top, on_out ? (const float*)nullptr : h->wsel, h->pair_row, (T*)h->ea);
-        hy_gemm_grouped<T>(ctx, (const T*)h->ea, W, one_gu, gu_stride, P, max_tiles, false, nullptr, 0, glu, (T*)h->eact, L.eff_pad,
+        hy_gemm_grouped<T>(ctx, (const T*)h->ea, W, one_gu, gu_stride, P, bm, max_tiles, false, nullptr, 0, glu, (T*)h->eact, L.eff_pad,
                            HyGlu{d.ff_limit, d.ff_alpha, d.ff_shift, nullptr, nullptr, 0, 0, d.ff_act}, E);
     }
-    hy_gemm_grouped<T>(ctx, (const T*)h->eact, L.eff_pad, one_down, (size_t)W * L.edown.ld, P, max_tiles, few, h->eout, W, false, nullptr, 0, HyGlu{}, E);
+    hy_gemm_grouped<T>(ctx, (const T*)h->eact, L.eff_pad, one_down, (size_t)W * L.edown.ld, P, bm, max_tiles, few, h->eout, W, false, nullptr, 0, HyGlu{}, E);
     if (d.shared_ff > 0) {
         T* act = (T*)h->mixo;
         hy_ff_up<T>(ctx, hb, L, n, act);
