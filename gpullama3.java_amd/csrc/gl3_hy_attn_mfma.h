@@ -1,0 +1,175 @@
+// gl3_hy_attn_mfma.h — the attention core of the layer-list family for portions of many tokens, its products on the matrix cores
+// (v_mfma_f32_32x32x2_f32: float32 products and sums, the precision hy_attn_kernel has on the vector units).
+//
+// Workgroup = (32 rows of a key / value head, key split): rows are (token, head of the group) pairs, token-major, as in hy_attn_kernel; its four
+// wavefronts deal the key tiles of 32 out between them and join their sums in LDS at the end, so that 512 tokens x 32 heads are 512
+// workgroups and no wavefront waits for another inside the key loop.  Both products are taken transposed, keys x rows and value columns x
+// rows: a lane then holds ONE query row in all of them, the running maximum and sum are its own registers (one exchange with
+// lane ^ 32 per tile), and the scores' accumulators ARE the second product's operand (register r of a lane is key 8 (r / 4) +
+// 4 (lane / 32) + r % 4, which is the pair of keys MFMA r takes from the half-waves) — nothing is transposed through LDS.
+// Keys and values come straight from the cache (each wavefront its own tile): a lane reads its key row 16 bytes at a time (element 8 c + 4 (lane / 32)
+// + e is step e of chunk c) and DVT consecutive value columns of the keys r (value column DVT m + i is row m of tile i); the values travel under the first product
+// and the softmax, the next tile's keys under the second half of the second product (all at once do not fit 256 registers, and a second wavefront
+// per SIMD is what keeps the matrix cores busy during the softmax).  Queries (scaled) stay in LDS, rows dk + 4 floats apart.
+// Bound: 153 TFLOP/s of float32 MFMAs.  Measured against hy_attn_kernel (8 key / value heads x 4, head size 128, us):
+//   512 tokens at position 0 131 -> 45, four such portions of 2041 tokens 1795 -> 428 in all.
+#pragma once
+#include "gl3_hy_kernels.h"
+
+template <int DVT> struct HyVec;
+template <> struct HyVec<2> { typedef float2 V; };
+template <> struct HyVec<4> { typedef float4 V; };
+
+template <int DKC, int DVT>          // dk = 8 DKC, dv = 32 DVT
+static __global__ __launch_bounds__(256, DKC > 16 ? 1 : 2) void hy_attn_mfma_kernel(HyAttnArgs a) {
+    constexpr int DK = 8 * DKC, DV = 32 * DVT, QS = DK + 4, OS = DV + 4;
+    typedef typename HyVec<DVT>::V VV;
+    __shared__ __attribute__((aligned(16))) float sQ[32 * QS];
+    __shared__ __attribute__((aligned(16))) float sO[32 * OS];
+    __shared__ float sml[4][2][32];
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), r32 = lane & 31, kh = lane >> 5;
+    // the LAST row block first: late tokens see the most keys
+    const int g = blockIdx.x % a.G, rb = (int)(gridDim.x / a.G) - 1 - (int)(blockIdx.x / a.G), split = blockIdx.z, hpg = a.H / a.G;
+    const int rows = a.n * hpg, row0 = rb * 32, pos0 = a.dyn[0];
+    const int minpos = pos0 + row0 / hpg, maxpos = pos0 + min(rows - 1, row0 + 31) / hpg;
+    const int rho = row0 + r32, pr = rho < rows ? pos0 + rho / hpg : -1;          // this lane's row: position (-1: no such row), head
+    const int hr = g * hpg + (rho < rows ? rho % hpg : 0);
+    const float slope = a.slope_log2 != 0.f ? exp2f(-a.slope_log2 * (float)(hr + 1) / (float)a.H) : 0.f;
+    for (int i = tid; i < 32 * (DK / 4); i += 256) {
+        const int r = i / (DK / 4), c = i % (DK / 4), p = row0 + r;
+        float4 v = make_float4(0.f, 0.f, 0.f, 0.f);
+        if (p < rows) v = *reinterpret_cast<const float4*>(a.q + (size_t)(p / hpg) * a.ldq + (size_t)(g * hpg + p % hpg) * DK + 4 * c);
+        v.x *= a.scale; v.y *= a.scale; v.z *= a.scale; v.w *= a.scale;
+        *reinterpret_cast<float4*>(sQ + r * QS + 4 * c) = v;
+    }
+    const size_t slot = (size_t)a.dyn[1] * a.slot_stride;
+    const float *kc = a.kc + slot + (size_t)g * DK, *vc = a.vc + slot + (size_t)g * DV;
+    const int ldk = a.G * DK, ldv = a.G * DV;
+    // the list of key tiles: pooled rows, kept first keys, the window from the earliest row's to the latest row's position
+    const int win = a.window > 0 ? a.window : 0x3fffffff, P = a.pool;
+    const int lo_t = max(0, minpos - win + 1) >> 5, hi_t = maxpos >> 5, nk = min((a.keep + 31) >> 5, lo_t);
+    const int nbr = P > 0 ? max(0, pr - win + 1) / P : 0, nb_wg = P > 0 ? max(0, maxpos - win + 1) / P : 0;
+    const int np_t = (nb_wg + 31) >> 5, nv = np_t + nk + hi_t - lo_t + 1;
+    const float *pkc = P > 0 ? a.pk + slot + (size_t)g * DK : kc, *pvc = P > 0 ? a.pv + slot + (size_t)g * DV : vc;
+    auto first_key = [&](int vt) { const int w = vt - np_t; return (vt < np_t ? vt : w < nk ? w : lo_t + w - nk) << 5; };
+    float4 kr[DKC];
+    auto load_keys = [&](int vt) {          // (rows past the last one repeat it: masked)
+        const bool pooled = vt < np_t;
+        const char* p = (const char*)(pooled ? pkc : kc);          // uniform base + 32-bit byte offset
+        const uint32_t off = ((uint32_t)min(first_key(vt) + r32, pooled ? nb_wg - 1 : maxpos) * (uint32_t)ldk + 4 * kh) * 4;
+#pragma unroll
+        for (int c = 0; c < DKC; ++c) kr[c] = *reinterpret_cast<const float4*>(p + off + 32 * c);
+    };
+    hy_v16f o[DVT];
+#pragma unroll
+    for (int i = 0; i < DVT; ++i)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) o[i][r] = 0.f;
+    float m = -INFINITY, l = 0.f;
+    int vt = split * 4 + wave;
+    if (vt < nv) load_keys(vt);
+    __syncthreads();
+    for (; vt < nv; vt += 4 * a.nsplit) {
+        const bool pooled = vt < np_t;
+        const int j0 = first_key(vt), last = pooled ? nb_wg - 1 : maxpos;
+        VV vr[16];          // values of keys r, the second half under the softmax
+        const char* vb = (const char*)(pooled ? pvc : vc);
+        auto load_values = [&](int r0) {
+#pragma unroll
+            for (int r = r0; r < r0 + 8; ++r) vr[r] = *reinterpret_cast<const VV*>(vb + ((uint32_t)min(j0 + 8 * (r >> 2) + 4 * kh + (r & 3), last) * (uint32_t)ldv + DVT * r32) * 4);
+        };
+        load_values(0);
+        __builtin_amdgcn_sched_barrier(0);
+        hy_v16f s0, s1;          // two chains of sums
+#pragma unroll
+        for (int r = 0; r < 16; ++r) s0[r] = s1[r] = 0.f;
+        const float* qp = sQ + r32 * QS + 4 * kh;
+#pragma unroll
+        for (int c = 0; c < DKC; ++c) {
+            const float4 q = *reinterpret_cast<const float4*>(qp + 8 * c);
+            s0 = __builtin_amdgcn_mfma_f32_32x32x2f32(kr[c].x, q.x, s0, 0, 0, 0);
+            s1 = __builtin_amdgcn_mfma_f32_32x32x2f32(kr[c].y, q.y, s1, 0, 0, 0);
+            s0 = __builtin_amdgcn_mfma_f32_32x32x2f32(kr[c].z, q.z, s0, 0, 0, 0);
+            s1 = __builtin_amdgcn_mfma_f32_32x32x2f32(kr[c].w, q.w, s1, 0, 0, 0);
+        }
+        __builtin_amdgcn_sched_group_barrier(0x100, 2, 0);          // two query chunks ahead of their MFMAs
+#pragma unroll
+        for (int c = 0; c < DKC; ++c) { __builtin_amdgcn_sched_group_barrier(0x8, 4, 0); if (c + 2 < DKC) __builtin_amdgcn_sched_group_barrier(0x100, 1, 0); }
+        __builtin_amdgcn_sched_barrier(0);
+        load_values(8);
+        __builtin_amdgcn_sched_barrier(0);
+        float p[16], mx = m;
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+            const int j = j0 + 8 * (r >> 2) + 4 * kh + (r & 3);
+            const float s = s0[r] + s1[r];
+            if (pooled) p[r] = j < nbr ? s : -INFINITY;
+            else p[r] = (j <= pr && (pr - j < win || j < a.keep)) ? s - slope * (float)(pr - j) : -INFINITY;
+            mx = fmaxf(mx, p[r]);
+        }
+        mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
+        const bool any = mx > -INFINITY;                         // false: this row has seen no key yet
+        const float corr = any ? expf(m - mx) : 1.f;             // exp(-inf) = 0 the first time
+        float ls = 0.f;
+#pragma unroll
+        for (int r = 0; r < 16; ++r) { p[r] = any ? expf(p[r] - mx) : 0.f; ls += p[r]; }
+        l = l * corr + ls;
+        m = mx;
+#pragma unroll
+        for (int i = 0; i < DVT; ++i)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) o[i][r] *= corr;
+        auto add_values = [&](int r0) {
+#pragma unroll
+            for (int r = r0; r < r0 + 8; ++r) {
+                o[0] = __builtin_amdgcn_mfma_f32_32x32x2f32(vr[r].x, p[r], o[0], 0, 0, 0);
+                o[1] = __builtin_amdgcn_mfma_f32_32x32x2f32(vr[r].y, p[r], o[1], 0, 0, 0);
+                if constexpr (DVT == 4) {
+                    o[2] = __builtin_amdgcn_mfma_f32_32x32x2f32(vr[r].z, p[r], o[2], 0, 0, 0);
+                    o[3] = __builtin_amdgcn_mfma_f32_32x32x2f32(vr[r].w, p[r], o[3], 0, 0, 0);
+                }
+            }
+        };
+        add_values(0);
+        __builtin_amdgcn_sched_barrier(0);
+        if (vt + 4 * a.nsplit < nv) load_keys(vt + 4 * a.nsplit);
+        __builtin_amdgcn_sched_barrier(0);
+        add_values(8);
+        __builtin_amdgcn_sched_barrier(0);
+    }
+    // join the wavefronts: every lane scales by e^(m - M), the wavefronts add up in LDS one after the other
+    l += __shfl_xor(l, 32, 64);
+    if (kh == 0) { sml[wave][0][r32] = m; sml[wave][1][r32] = l; }
+    __syncthreads();
+    const float M = fmaxf(fmaxf(sml[0][0][r32], sml[1][0][r32]), fmaxf(sml[2][0][r32], sml[3][0][r32]));
+    const float sc = m > -INFINITY ? expf(m - M) : 0.f;
+    for (int w = 0; w < 4; ++w) {
+        if (wave == w) {
+#pragma unroll
+            for (int r = 0; r < 16; ++r) {
+                VV* d = reinterpret_cast<VV*>(sO + r32 * OS + DVT * (8 * (r >> 2) + 4 * kh + (r & 3)));
+                VV v;
+                if (w > 0) v = *d;
+                v.x = (w > 0 ? v.x : 0.f) + sc * o[0][r];
+                v.y = (w > 0 ? v.y : 0.f) + sc * o[1][r];
+                if constexpr (DVT == 4) { v.z = (w > 0 ? v.z : 0.f) + sc * o[2][r]; v.w = (w > 0 ? v.w : 0.f) + sc * o[3][r]; }
+                *d = v;
+            }
+        }
+        __syncthreads();
+    }
+    for (int i = tid; i < 32 * (DV / 4); i += 256) {
+        const int r = i / (DV / 4), c = i % (DV / 4), q = row0 + r;
+        if (q >= rows) continue;
+        const size_t ob = ((size_t)(q / hpg) * a.H + g * hpg + q % hpg) * a.nsplit + split;
+        *reinterpret_cast<float4*>(a.part_acc + ob * DV + 4 * c) = *reinterpret_cast<const float4*>(sO + r * OS + 4 * c);
+    }
+    if (tid < 32 && pr >= 0) {
+        float L = 0.f;
+#pragma unroll
+        for (int w = 0; w < 4; ++w) if (sml[w][0][r32] > -INFINITY) L += expf(sml[w][0][r32] - M) * sml[w][1][r32];
+        const size_t ob = ((size_t)(rho / hpg) * a.H + hr) * a.nsplit + split;
+        a.part_ml[2 * ob] = M;
+        a.part_ml[2 * ob + 1] = L;
+    }
+}

@@ -20,6 +20,7 @@
 #include "gl3_decode_kernels.h"      // argmax_kernel
 #include "gl3_hy_kernels.h"
 #include "gl3_hy_gemm.h"
+#include "gl3_hy_attn_mfma.h"
 #include "gl3_hy_heads_kernels.h"
 #include "gl3_hy_plain_kernels.h"
 
@@ -39,6 +40,7 @@ using gl3::argmax_kernel;
 static inline int hy_cdiv(int a, int b) { return (a + b - 1) / b; }
 constexpr int HY_MOE_BM = 64, HY_MOE_BM_FEW = 32;        // rows per tile of the grouped expert GEMMs; where experts have few rows each
 constexpr int HY_LATENT_DIRECT = 512;   // longest cached latent row that decode steps score in the latent's space (value columns per lane of the attention core)
+constexpr int HY_MFMA_SPLITS = 8;    // most key splits of the attention core on the matrix cores
 constexpr int HY_ZSPLIT = 16;        // most K-split parts of a product with very few result rows (router, token input's gate): its consumer kernel adds them
 static inline float hy_bf16_to_f32(uint16_t v) { uint32_t u = (uint32_t)v << 16; float f; memcpy(&f, &u, 4); return f; }
 static inline uint16_t hy_f32_to_bf16(float f) {
@@ -1053,6 +1055,29 @@ static int32_t hy_attention(gl3_ctx* ctx, const float* q, int ldq, const float* 
                             int n, int pos0, int* nsplit_out, bool in_slot = true, int window = 0, int keep = 0, const float* pk = nullptr, const float* pv = nullptr, int pool = 0) {
     gl3_hybrid_state* h = ctx->hy;
     const bool shared_kv = kc == vc && dk == dv;
+    HyAttnArgs a;
+    a.q = q; a.ldq = ldq; a.kc = kc; a.vc = vc; a.slot_stride = in_slot ? h->slot_floats : 0; a.H = H; a.G = G; a.dk = dk; a.dv = dv; a.scale = scale; a.slope_log2 = slope_log2;
+    a.dyn = h->dyn; a.n = n; a.part_acc = h->part_acc; a.part_ml = h->part_ml; a.shared_kv = shared_kv ? 1 : 0; a.window = window; a.keep = keep;
+    a.pk = pk; a.pv = pv; a.pool = pool;
+    // Matrix cores from 17 tokens on (up to 16 the keys are split over many workgroups, below), for the head sizes the kernel is built for.
+    const bool aligned = ((ldq | H * dk | a.slot_stride) & 3) == 0 && (((uintptr_t)q | (uintptr_t)kc | (uintptr_t)vc | (uintptr_t)pk | (uintptr_t)pv) & 15) == 0;
+    if (n > 16 && !shared_kv && aligned && (uint64_t)(pos0 + n) * G * std::max(dk, dv) < 0x3fff0000ull) {          // (32-bit byte offsets inside a cache)
+        // few row blocks (a short portion): more workgroups per block while each wavefront keeps four key tiles or more
+        const int blocks = hy_cdiv(n * (H / G), 32) * G;
+        int nsplit = std::max(1, std::min({512 / blocks, HY_MFMA_SPLITS, hy_cdiv(pos0 + n, 512)}));
+        if ((size_t)n * nsplit > h->part_rows) nsplit = std::max<size_t>(1, h->part_rows / n);
+        a.nsplit = nsplit; a.kt = 32;
+        const dim3 grid(blocks, 1, nsplit);
+        bool done = true;
+#define HY_AM(DKC, DVT) hipLaunchKernelGGL((hy_attn_mfma_kernel<DKC, DVT>), grid, dim3(256), 0, ctx->stream, a)
+        if (dk == 128 && dv == 128) HY_AM(16, 4);
+        else if (dk == 64 && dv == 64) HY_AM(8, 2);
+        else if (dk == 192 && dv == 128) HY_AM(24, 4);
+        else if (dk == 96 && dv == 64) HY_AM(12, 2);
+        else done = false;
+#undef HY_AM
+        if (done) { *nsplit_out = nsplit; return GL3_OK; }
+    }
     HyAttnPlan p = hy_attn_plan(n * (H / G), dk, dv, shared_kv);
     if (p.smem > 150 * 1024) GL3_FAIL(GL3_E_UNSUPPORTED, "attention: key + value row too large for the LDS tile");
     int nsplit = 1;                                          // few tokens: one key tile per split while that gives <= 128 splits
@@ -1063,10 +1088,7 @@ static int32_t hy_attention(gl3_ctx* ctx, const float* q, int ldq, const float* 
         nsplit = std::min(HY_MAX_SPLITS, std::max(1, tiles));
     }
     if ((size_t)n * nsplit > h->part_rows) nsplit = std::max<size_t>(1, h->part_rows / n);
-    HyAttnArgs a;
-    a.q = q; a.ldq = ldq; a.kc = kc; a.vc = vc; a.slot_stride = in_slot ? h->slot_floats : 0; a.H = H; a.G = G; a.dk = dk; a.dv = dv; a.scale = scale; a.slope_log2 = slope_log2;
-    a.dyn = h->dyn; a.n = n; a.nsplit = nsplit; a.part_acc = h->part_acc; a.part_ml = h->part_ml; a.kt = p.kt; a.shared_kv = shared_kv ? 1 : 0; a.window = window; a.keep = keep;
-    a.pk = pk; a.pv = pv; a.pool = pool;
+    a.nsplit = nsplit; a.kt = p.kt;
     const dim3 grid((unsigned)hy_cdiv(n * (H / G), 4 * p.rw) * G, 1, nsplit);
 #define HY_AT(RW, DVL) hipLaunchKernelGGL((hy_attn_kernel<RW, DVL>), grid, dim3(256), p.smem, ctx->stream, a)
 #define HY_AT_RW(RW) do { if (p.dvl == 1) HY_AT(RW, 1); else if (p.dvl == 2) HY_AT(RW, 2); else if (p.dvl == 4) HY_AT(RW, 4); else HY_AT(RW, 8); } while (0)

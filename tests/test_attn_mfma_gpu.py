@@ -1,0 +1,49 @@
+"""The attention core on the matrix cores (csrc/gl3_hy_attn_mfma.h): the head sizes it is built for, whole prompts and portions behind earlier
+positions, row blocks and key tiles of 32 with remainders, groups of 1, 3 and 4 query heads, windows with kept first keys and with pooled
+blocks, latent attention's expanded keys with and without a rotated part, a distance penalty with the extra unit; the short portions at
+the end of a cut prompt go through the key-split kernel.
+
+Yardstick: the designs' float64 restatements.  Bound: float32 scores of up to 192 terms, a softmax and sums over the keys err by some 1e-6 of the
+logits' root mean square (queries and keys of size one); a lost or extra key of a few hundred is an error of 1e-3 and more."""
+import numpy as np
+import pytest
+
+import __graft_entry__ as ge
+import test_kosusun_gpu as K
+import test_kugadra_gpu as U
+import test_noditar_gpu as N
+import test_vonulix_gpu as V
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def hy():
+    from importlib import import_module
+    ge.load_package()
+    return import_module(ge.PKG_NAME + ".hybrid")
+
+
+LAYERS = {
+    "64_gqa2": (N, N.att(heads=4, kv_heads=2, dim=64, vdim=64, ff=0)), "128_gqa3": (N, N.att(heads=6, kv_heads=2, dim=128, vdim=128, ff=0, scale=0.1)),
+    "128_mha": (N, N.att(heads=3, kv_heads=3, dim=128, vdim=128, ff=0, scale=0.1)), "latent64": (N, N.lat(heads=4, dim=64, vdim=64, kv_rank=96, ff=0)),
+    "window_pool64": (K, K.par(left=K.attn(heads=4, kv_heads=1, dim=64, vdim=64, size=37, pool=5), ff=0)),
+    "window_pool128": (K, K.par(left=K.attn(heads=4, kv_heads=2, dim=128, vdim=128, size=100, pool=16, scale=0.1), ff=0)),
+    "window_keep64": (V, V.layer(size=29, keep=3, experts=0, heads=4, kv_heads=2, dim=64, vdim=64)),
+    "latent96": (U, U.lat(heads=4, dim=64, rot_dim=32, vdim=64, kv_rank=60, mlp=None)), "latent192": (U, U.lat(heads=2, dim=128, rot_dim=64, vdim=128, kv_rank=60, mlp=None, scale=0.1)),
+}
+
+
+@pytest.mark.parametrize("n,batch", [(17, 64), (33, 64), (200, 256), (333, 128), (300, 97)])
+@pytest.mark.parametrize("name", list(LAYERS))
+def test_portions_and_tiles(hy, tmp_path, name, n, batch):
+    mod, layer = LAYERS[name]
+    cfg = mod.config([layer])
+    m = mod.Model(hy, tmp_path, cfg, seed=n)
+    toks = np.random.default_rng(n).integers(0, cfg["vocab"], n).astype(np.int32)
+    p = m.plan("float32", ctx=n + 8, max_batch=batch)
+    s = p.acquire()
+    got = p.step(s, toks, 0, list(range(n)))
+    p.close()
+    want = m.ref(toks)
+    assert N.err(got, want) < 2e-5, N.err(got, want)
