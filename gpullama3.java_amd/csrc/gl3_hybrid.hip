@@ -21,6 +21,7 @@
 #include "gl3_hy_kernels.h"
 #include "gl3_hy_gemm.h"
 #include "gl3_hy_attn_mfma.h"
+#include "gl3_hy_scan_chunk.h"
 #include "gl3_hy_heads_kernels.h"
 #include "gl3_hy_plain_kernels.h"
 
@@ -1164,12 +1165,32 @@ static void hy_delta_scan(gl3_ctx* ctx, const HyDeltaScan& a) {
 #undef HY_DS
 }
 
+// Whether a recurrence goes 32 tokens at a time (hy_scan_chunk_kernel): one decay per head and token, keys of 64 / 128 / 256 entries in rows of
+// whole 16-byte pieces, and more than 16 tokens (a chunk takes ~3 us whatever it holds, the token-by-token walk 0.35 - 0.5 us a token).
+static bool hy_scan_chunks(const HyScanArgs& a) {
+    return a.n > 16 && a.mode != 3 && (a.N == 64 || a.N == 128 || a.N == 256) && ((a.ldk | a.k_off | a.k_hstride | a.ldq | a.q_off | a.q_hstride) & 3) == 0 &&
+           (((uintptr_t)a.ksrc | (uintptr_t)a.qsrc) & 15) == 0;
+}
+static void hy_scan_chunk_launch(gl3_ctx* ctx, const HyScanArgs& a) {
+    // 16 value columns per workgroup while that is one round of 256 CUs, else 32 (q . k is made once per workgroup): 16 heads x 256 columns 52 us
+    // with 16 and 61 with 32, 8 x 513 (264 or 136 workgroups) 112 and 96, 128 x 64 (512 or 256) 80 and 71
+    const int pc = (long)a.heads * hy_cdiv(a.P, 16) <= 256 ? 16 : 32;
+    const size_t smem = (size_t)(2 * 32 * (a.N + 4) + 32 * (pc + 4) + 32 * 36 + 32 * 33 + 64) * 4;
+    const dim3 grid(hy_cdiv(a.P, pc), a.heads);
+#define HY_SC(NT, PC) hipLaunchKernelGGL((hy_scan_chunk_kernel<NT, PC>), grid, dim3(256), smem, ctx->stream, a)
+#define HY_SC_N(PC) do { if (a.N == 64) HY_SC(1, PC); else if (a.N == 128) HY_SC(2, PC); else HY_SC(4, PC); } while (0)
+    if (pc == 32) HY_SC_N(32); else HY_SC_N(16);
+#undef HY_SC_N
+#undef HY_SC
+}
+
 // The recurrence kernel: a column's states over NG lanes x NL registers: NL = 16 (32 for more than 1024 states, 8 / 4 for very small
 // ones), NG a power of two; tokens staged per round: what fits 48 KB of LDS, at most 32.  Fills in a.NG and a.TB.
 // With few workgroups (few heads, narrow values) NL = 16 is halved once so that more of them share the columns; below 8 every workgroup
 // stages the same key / query rows for too few columns and the traffic from L2 eats the gain (measured: 16 and 8 within 2 %, 4 slower).
 // GL3_HY_SCAN_NL forces a value.
 static void hy_scan(gl3_ctx* ctx, HyScanArgs& a) {
+    if (hy_scan_chunks(a)) { hy_scan_chunk_launch(ctx, a); return; }
     int NL = a.N > 1024 ? 32 : a.N > 8 ? 16 : a.N > 4 ? 8 : 4;
     auto wgs = [&](int nl) { int ng = 1; while (ng * nl < a.N) ng *= 2; return (long)hy_cdiv(a.P, 4 * (64 / ng)) * a.heads; };
     if (NL == 16 && 8 * 64 >= a.N && wgs(16) < 512) NL = 8;
@@ -1292,6 +1313,11 @@ static int32_t hy_mixer_core(gl3_ctx* ctx, HyLayer& L, int np, int ldo, int n, i
         a.ga = ga; a.gb = gb; a.decay = L.decay; a.ones_col = eg ? 1 : 0;
         a.heads = d.heads; a.P = P; a.N = d.dim; a.G = d.heads;
         a.state = h->slots + L.off_state; a.slot_stride = h->slot_floats; a.dyn = h->dyn; a.n = n; a.y = h->ssm_y; a.ldy = ldy;
+        if (hy_scan_chunks(a) && ((a.act & 3) || a.rot.dims > 0 || a.k_mul != 1.f || a.q_mul != 1.f)) {
+            // keys and queries are finished once, in place (the chunks' workgroups would each make them again for their few columns)
+            hipLaunchKernelGGL(hy_scan_prep_kernel, dim3(n), dim3(256), (size_t)std::max(1, d.rot_dims) * 4, st, h->proj, np, L.q_off, L.k_off, d.heads, d.dim, a.q_mul, a.k_mul, a.act, a.rot, h->dyn);
+            a.act &= 4; a.k_mul = a.q_mul = 1.f; a.rot = HyScanRot{};
+        }
         if (cg && n > 32) {
             hipLaunchKernelGGL(hy_mem_prep_kernel, dim3(n, hy_cdiv(d.heads * d.dim, 1024)), dim3(256), 0, st, h->proj, np, L.q_off, L.f_off, d.heads * d.dim, a.act & 2, a.fbias, a.lower);
             a.act &= ~2; a.fbias = nullptr;

@@ -1,0 +1,58 @@
+"""The recurrences 32 tokens at a time (csrc/gl3_hy_scan_chunk.h): every kind that takes them (state-space layers, exponential gates with their
+normaliser column, retention with turned keys, a fixed decay behind silu) at the key sizes 64 / 128 / 256, value columns that do not fill a column
+block, portions whose last chunk is full, holds one token or is cut behind an earlier portion, decays near one and decays that underflow.
+
+Yardstick: the designs' float64 restatements, which walk token by token.  Bound: float32 products and sums of a few hundred terms err by some
+1e-6 of the logits' root mean square (heads are normed to size one behind the memory); a lost token or a wrong decay is an error of order one."""
+import numpy as np
+import pytest
+
+import __graft_entry__ as ge
+import test_kosusun_gpu as K
+import test_kugadra_gpu as U
+import test_noditar_gpu as N
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def hy():
+    from importlib import import_module
+    ge.load_package()
+    return import_module(ge.PKG_NAME + ".hybrid")
+
+
+def decays(lo, hi):
+    def tweak(w):
+        for k in w:
+            if k.endswith("A_log"):
+                w[k][:] = np.linspace(lo, hi, w[k].size)
+    return tweak
+
+
+LAYERS = {
+    "ssm128": (N, N.ssm(heads=6, vdim=64, state=128, groups=2, norm_groups=3, conv=4), None),
+    "ssm64_odd_columns": (N, N.ssm(heads=4, vdim=25, state=64, groups=4, norm_groups=2), None),
+    "ssm128_underflow": (N, N.ssm(heads=8, vdim=32, state=128), decays(-9.0, 6.0)),
+    "mlstm64": (K, K.mls(heads=4, dim=64, vdim=40, ff=0), None), "mlstm256": (K, K.mls(heads=2, dim=256, vdim=64, ff=0), None),
+    "retention128": (K, K.par(right=K.ret(heads=4, dim=128, vdim=34, rot_dims=128), ff=0), None),
+    "retention64_part": (K, K.par(right=K.ret(heads=6, dim=64, vdim=50, rot_dims=24), ff=0), None),
+    "lightning64": (U, U.lig(heads=4, dim=64, vdim=56, mlp=None), None), "lightning128": (U, U.lig(heads=2, dim=128, vdim=16, mlp=None), None),
+}
+
+
+@pytest.mark.parametrize("n,batch", [(17, 64), (32, 64), (65, 128), (160, 160), (230, 97)])
+@pytest.mark.parametrize("name", list(LAYERS))
+def test_chunks_and_portions(hy, tmp_path, name, n, batch):
+    mod, layer, tweak = LAYERS[name]
+    cfg = mod.config([layer])
+    m = mod.Model(hy, tmp_path, cfg, n, tweak) if tweak else mod.Model(hy, tmp_path, cfg, n)
+    toks = np.random.default_rng(n).integers(0, cfg["vocab"], n + 3).astype(np.int32)
+    p = m.plan("float32", ctx=n + 8, max_batch=batch)
+    s = p.acquire()
+    got = [p.step(s, toks[:n], 0, list(range(n)))]
+    for i in range(3):                        # the state goes on token by token
+        got.append(p.step(s, toks[n + i:n + i + 1], n + i, [0]))
+    p.close()
+    got, want = np.concatenate(got), m.ref(toks)
+    assert N.err(got, want) < 3e-5, N.err(got, want)
