@@ -37,28 +37,6 @@ struct HyResid {
 };
 // V = 4: rows are read and written 16 bytes at a time (W a multiple of 4); every load of a chunk is issued before the first use, so one
 // round trip to memory covers them all.  The first HY_RC chunks of a thread stay in registers for the norm's second pass.
-template <int V> __device__ __forceinline__ void hy_ldv(const float* __restrict__ p, float* v) {
-    if constexpr (V == 4) { const float4 t = *reinterpret_cast<const float4*>(p); v[0] = t.x; v[1] = t.y; v[2] = t.z; v[3] = t.w; }
-    else v[0] = *p;
-}
-template <int V> __device__ __forceinline__ void hy_ldv(const bf16_t* __restrict__ p, float* v) {
-    if constexpr (V == 4) {
-        const uint2 t = *reinterpret_cast<const uint2*>(p);
-        v[0] = __uint_as_float(t.x << 16); v[1] = __uint_as_float(t.x & 0xffff0000u); v[2] = __uint_as_float(t.y << 16); v[3] = __uint_as_float(t.y & 0xffff0000u);
-    } else v[0] = hy_bf2f(*p);
-}
-template <int V> __device__ __forceinline__ void hy_stv(float* __restrict__ p, const float* v) {
-    if constexpr (V == 4) *reinterpret_cast<float4*>(p) = make_float4(v[0], v[1], v[2], v[3]);
-    else *p = v[0];
-}
-template <int V> __device__ __forceinline__ void hy_stv(bf16_t* __restrict__ p, const float* v) {
-    if constexpr (V == 4) {
-        uint2 t;
-        t.x = (uint32_t)hy_f2bf(v[0]) | ((uint32_t)hy_f2bf(v[1]) << 16);
-        t.y = (uint32_t)hy_f2bf(v[2]) | ((uint32_t)hy_f2bf(v[3]) << 16);
-        *reinterpret_cast<uint2*>(p) = t;
-    } else *p = hy_f2bf(v[0]);
-}
 constexpr int HY_RC = 2, HY_MAX_PARTS = 4, HY_MIX_UNROLL = 4;
 template <typename TO, int NT, int V, bool BR>
 static __global__ __launch_bounds__(NT) void hy_resid_kernel(HyResid a, TO* __restrict__ xt, TO* h_out) {

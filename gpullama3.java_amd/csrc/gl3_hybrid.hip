@@ -1023,6 +1023,14 @@ static void hy_gemm(gl3_ctx* ctx, const T* A, int lda, const HyMat& w, int M, fl
 template <typename T>
 static void hy_streams(gl3_ctx* ctx, int blocks, float* X, int W, int S, size_t sstride, const float* y, int yparts, size_t ystride, const float* post_mix, const float* post_out, const float* pre_in,
                        const float* norm_w, float eps, T* h_out, float* sum_out, const int* rows) {
+#define HY_ST4(NT, NS) hipLaunchKernelGGL((hy_streams4_kernel<T, NT, NS>), dim3(blocks), dim3(NT), 0, ctx->stream, X, W, sstride, y, yparts, ystride, post_mix, post_out, pre_in, norm_w, eps, h_out, sum_out, rows)
+#define HY_ST4_S(NT) do { if (S == 1) HY_ST4(NT, 1); else if (S == 2) HY_ST4(NT, 2); else HY_ST4(NT, 4); } while (0)
+    if (W % 4 == 0 && (S == 1 || S == 2 || S == 4)) {          // (every row then starts on 16 bytes: the plan's buffers do)
+        if (blocks <= 32) HY_ST4_S(1024); else HY_ST4_S(256);
+        return;
+    }
+#undef HY_ST4_S
+#undef HY_ST4
     if (blocks <= 32)
         hipLaunchKernelGGL((hy_streams_kernel<T, 1024>), dim3(blocks), dim3(1024), 0, ctx->stream, X, W, S, sstride, y, yparts, ystride, post_mix, post_out, pre_in, norm_w, eps, h_out, sum_out, rows);
     else
