@@ -16,6 +16,7 @@
 #pragma once
 #include "gl3_hy_kernels.h"
 
+typedef float hy_acc4 __attribute__((ext_vector_type(4)));
 template <int DVT> struct HyVec;
 template <> struct HyVec<2> { typedef float2 V; };
 template <> struct HyVec<4> { typedef float4 V; };
@@ -172,4 +173,131 @@ static __global__ __launch_bounds__(256, DKC > 16 ? 1 : 2) void hy_attn_mfma_ker
         a.part_ml[2 * ob] = M;
         a.part_ml[2 * ob + 1] = L;
     }
+}
+
+// A few tokens (decode): workgroup = (32 rows of a key / value head, key split) with one tile of 32 keys at a time for all its wavefronts (four; eight for long rows): each multiplies
+// its share of the entries (queries and keys straight from memory), the shares of the scores meet in LDS, every wavefront makes its share of the
+// softmax and the weighted sum of its own value columns.  Same layouts as above; rows that are not there cost MFMAs nobody waits for.  Latent attention's
+// cached rows (keys = values) come as kc = vc.  A tile is one round trip to memory and (DK + DV) / 2 MFMAs over the wavefronts, and the tiles of a
+// token up to 32 x HY_MAX_SPLITS positions run side by side, where hy_attn_kernel walked tiles of 64 keys with four rows per wavefront (us):
+// 32 heads on 512-entry latents 29 - 33 -> 11.8, 8 x 4 heads of 64 7.3 -> 5.7, of 128 behind 2041 positions 13.5 -> 8.2 us.
+template <int DK, int DV, int NW = 4>          // NW wavefronts
+static __global__ __launch_bounds__(64 * NW, 1) void hy_attn_few_kernel(HyAttnArgs a) {
+    constexpr int RQ = DK / NW, KC = RQ / 8, CW = DV >= 32 * NW ? DV / NW : 32, NE = 16 / NW, DVT = CW / 32;
+    __shared__ float sS[NW][16][64], sP[16][64], sM[NW][64];
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), r32 = lane & 31, kh = lane >> 5;
+    const int g = blockIdx.x % a.G, rb = blockIdx.x / a.G, split = blockIdx.z, hpg = a.H / a.G, rows = a.n * hpg, row0 = rb * 32, pos0 = a.dyn[0];
+    const int minpos = pos0 + row0 / hpg, maxpos = pos0 + min(rows - 1, row0 + 31) / hpg;
+    const int rho = row0 + r32, pr = rho < rows ? pos0 + rho / hpg : -1, hr = g * hpg + (rho < rows ? rho % hpg : 0);
+    const float slope = a.slope_log2 != 0.f ? exp2f(-a.slope_log2 * (float)(hr + 1) / (float)a.H) : 0.f;
+    const size_t slot = (size_t)a.dyn[1] * a.slot_stride;
+    const int ldk = a.G * DK, ldv = a.G * DV, col0 = wave * CW;
+    const bool live = col0 < DV;          // (64 value columns are two wavefronts' work)
+    const float *kc = a.kc + slot + (size_t)g * DK, *vc = a.vc + slot + (size_t)g * DV;
+    const int win = a.window > 0 ? a.window : 0x3fffffff, P = a.pool;
+    const int lo_t = max(0, minpos - win + 1) >> 5, hi_t = maxpos >> 5, nk = min((a.keep + 31) >> 5, lo_t);
+    const int nbr = P > 0 ? max(0, pr - win + 1) / P : 0, nb_wg = P > 0 ? max(0, maxpos - win + 1) / P : 0;
+    const int np_t = (nb_wg + 31) >> 5, nv = np_t + nk + hi_t - lo_t + 1;
+    const float *pkc = P > 0 ? a.pk + slot + (size_t)g * DK : kc, *pvc = P > 0 ? a.pv + slot + (size_t)g * DV : vc;
+    hy_acc4 qr[KC];
+    {
+        const int q = min(rho, rows - 1);
+        const float* p = a.q + (size_t)(q / hpg) * a.ldq + (size_t)(g * hpg + q % hpg) * DK + wave * RQ + 4 * kh;
+#pragma unroll
+        for (int c = 0; c < KC; ++c) qr[c] = *reinterpret_cast<const hy_acc4*>(p + 8 * c);
+    }
+    hy_v16f o[DVT];
+#pragma unroll
+    for (int i = 0; i < DVT; ++i)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) o[i][r] = 0.f;
+    float m = -INFINITY, l = 0.f;
+    for (int vt = split; vt < nv; vt += a.nsplit) {          // (uniform over the workgroup)
+        const bool pooled = vt < np_t;
+        const int w_ = vt - np_t, j0 = (pooled ? vt : w_ < nk ? w_ : lo_t + w_ - nk) << 5, last = pooled ? nb_wg - 1 : maxpos;
+        hy_acc4 kr[KC];
+        const float* kp = (pooled ? pkc : kc) + (size_t)min(j0 + r32, last) * ldk + wave * RQ + 4 * kh;
+#pragma unroll
+        for (int c = 0; c < KC; ++c) kr[c] = *reinterpret_cast<const hy_acc4*>(kp + 8 * c);
+        float vr[16][DVT];
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+            const float* vp = (pooled ? pvc : vc) + (size_t)min(j0 + 8 * (r >> 2) + 4 * kh + (r & 3), last) * ldv + (live ? col0 : 0) + DVT * r32;
+#pragma unroll
+            for (int i = 0; i < DVT; ++i) vr[r][i] = vp[i];
+        }
+        hy_v16f s0, s1;
+#pragma unroll
+        for (int r = 0; r < 16; ++r) s0[r] = s1[r] = 0.f;
+#pragma unroll
+        for (int c = 0; c < KC; ++c) {
+            s0 = __builtin_amdgcn_mfma_f32_32x32x2f32(kr[c][0], qr[c][0], s0, 0, 0, 0);
+            s1 = __builtin_amdgcn_mfma_f32_32x32x2f32(kr[c][1], qr[c][1], s1, 0, 0, 0);
+            s0 = __builtin_amdgcn_mfma_f32_32x32x2f32(kr[c][2], qr[c][2], s0, 0, 0, 0);
+            s1 = __builtin_amdgcn_mfma_f32_32x32x2f32(kr[c][3], qr[c][3], s1, 0, 0, 0);
+        }
+        if (vt != split) __syncthreads();
+#pragma unroll
+        for (int r = 0; r < 16; ++r) sS[wave][r][lane] = s0[r] + s1[r];
+        __syncthreads();
+        // scores NE wave .. of every lane: a share of the softmax per wavefront (all sixteen in each would be four or eight times the exponentials)
+        float p[NE], mx = -INFINITY;
+#pragma unroll
+        for (int e = 0; e < NE; ++e) {
+            const int r = NE * wave + e, j = j0 + 8 * (r >> 2) + 4 * kh + (r & 3);
+            float s = 0.f;
+#pragma unroll
+            for (int w = 0; w < NW; w += 2) s += sS[w][r][lane] + sS[w + 1][r][lane];
+            s *= a.scale;
+            if (pooled) p[e] = j < nbr ? s : -INFINITY;
+            else p[e] = (j <= pr && (pr - j < win || j < a.keep)) ? s - slope * (float)(pr - j) : -INFINITY;
+            mx = fmaxf(mx, p[e]);
+        }
+        mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
+        sM[wave][lane] = mx;
+        __syncthreads();
+        mx = m;
+#pragma unroll
+        for (int w = 0; w < NW; ++w) mx = fmaxf(mx, sM[w][lane]);
+        const bool any = mx > -INFINITY;                         // false: this row has seen no key yet
+        const float corr = any ? expf(m - mx) : 1.f;
+        float ls = 0.f;
+#pragma unroll
+        for (int e = 0; e < NE; ++e) {
+            p[e] = any ? expf(p[e] - mx) : 0.f;
+            ls += p[e];
+            sP[NE * wave + e][lane] = p[e];
+        }
+        l = l * corr + ls;                                       // (this wavefront's share)
+        m = mx;
+        __syncthreads();
+#pragma unroll
+        for (int i = 0; i < DVT; ++i)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) o[i][r] *= corr;
+        if (live) {
+#pragma unroll
+            for (int r = 0; r < 16; ++r) {
+                const float pr_ = sP[r][lane];
+#pragma unroll
+                for (int i = 0; i < DVT; ++i) o[i] = __builtin_amdgcn_mfma_f32_32x32x2f32(vr[r][i], pr_, o[i], 0, 0, 0);
+            }
+        }
+    }
+    l += __shfl_xor(l, 32, 64);
+    __syncthreads();
+    sM[wave][lane] = l;
+    __syncthreads();
+    l = 0.f;
+#pragma unroll
+    for (int w = 0; w < NW; ++w) l += sM[w][lane];
+    if (pr < 0) return;
+    const size_t ob = ((size_t)(rho / hpg) * a.H + hr) * a.nsplit + split;
+    if (wave == 0 && kh == 0) { a.part_ml[2 * ob] = m; a.part_ml[2 * ob + 1] = l; }
+    if (!live) return;
+    float* dst = a.part_acc + ob * DV + col0;
+#pragma unroll
+    for (int r = 0; r < 16; ++r)
+#pragma unroll
+        for (int i = 0; i < DVT; ++i) dst[DVT * (8 * (r >> 2) + 4 * kh + (r & 3)) + i] = o[i][r];
 }

@@ -1128,8 +1128,8 @@ static __global__ __launch_bounds__(256) void hy_attn_kernel(HyAttnArgs a) {
 // z = sink_w ? sink_w[h] : 0 (a learned logit per head, or one plain unit).
 // gate_mode 1: gate[t][h dv + c], 2: gate[t][h] (one per head).  v_freq != null: the head's output is turned back by the token's
 // position over all dv entries (pairs c, c + dv / 2, angle -pos v_freq[c]) before the gate.
-template <typename TO>
-static __global__ __launch_bounds__(64) void hy_attn_merge_kernel(const float* __restrict__ part_acc, const float* __restrict__ part_ml, int H, int dv, int nsplit,
+template <typename TO, int NT = 64>          // threads per (token, head)
+static __global__ __launch_bounds__(NT) void hy_attn_merge_kernel(const float* __restrict__ part_acc, const float* __restrict__ part_ml, int H, int dv, int nsplit,
                                                                   int sink, const float* __restrict__ gate, int ldg, int gate_mode, TO* __restrict__ out, int ldo,
                                                                   const float* __restrict__ v_freq, const int* __restrict__ dyn,
                                                                   const float* __restrict__ sink_w = nullptr, float out_mul = 1.f) {
@@ -1159,7 +1159,7 @@ static __global__ __launch_bounds__(64) void hy_attn_merge_kernel(const float* _
     if (v_freq) {
         const int half = dv >> 1;
         const float pos = (float)(dyn[0] + t);
-        for (int c = lane; c < half; c += 64) {
+        for (int c = lane; c < half; c += NT) {
             float sn, cs;
             sincosf(pos * v_freq[c], &sn, &cs);
             const float u = column(c), v = column(c + half);
@@ -1167,7 +1167,7 @@ static __global__ __launch_bounds__(64) void hy_attn_merge_kernel(const float* _
             put(c + half, v * cs - u * sn);
         }
     } else {
-        for (int c = lane; c < dv; c += 64) put(c, column(c));
+        for (int c = lane; c < dv; c += NT) put(c, column(c));
     }
 }
 

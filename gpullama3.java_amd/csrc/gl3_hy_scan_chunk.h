@@ -13,9 +13,8 @@
 // Keys and queries come finished (hy_scan_prep_kernel); x passes through silu on the way into LDS where the layer asks for it (act & 4).
 // Measured for 512 tokens (us), hy_ssm_scan_kernel -> this: 128 heads x (128 x 64) 278 -> 73, 16 x (128 x 256) 310 -> 52, 8 x (256 x 513) 430 -> 97.
 #pragma once
-#include "gl3_hy_kernels.h"
+#include "gl3_hy_attn_mfma.h"
 
-typedef float hy_acc4 __attribute__((ext_vector_type(4)));
 // workgroup barrier for LDS alone (__syncthreads() also waits for every global load in flight: the next chunk's rows)
 __device__ __forceinline__ void hy_lds_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
 __device__ __forceinline__ hy_acc4 hy_mma4(float a, float b, hy_acc4 c) { return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0); }

@@ -1070,6 +1070,25 @@ static int32_t hy_attention(gl3_ctx* ctx, const float* q, int ldq, const float* 
     a.pk = pk; a.pv = pv; a.pool = pool;
     // Matrix cores from 17 tokens on (up to 16 the keys are split over many workgroups, below), for the head sizes the kernel is built for.
     const bool aligned = ((ldq | H * dk | a.slot_stride) & 3) == 0 && (((uintptr_t)q | (uintptr_t)kc | (uintptr_t)vc | (uintptr_t)pk | (uintptr_t)pv) & 15) == 0;
+    // a few tokens: one tile of 32 keys per split
+    if (n <= 16 && aligned) {
+        int tiles = hy_cdiv(pos0 + n, 32);
+        if (window > 0) tiles = std::min<long>(tiles, hy_cdiv(keep, 32) + ((long)window + n) / 32 + 2);      // kept first keys + the window's tiles
+        if (pool > 0) tiles += hy_cdiv(std::max(0, pos0 + n - window) / pool, 32);                           // + the tiles of pooled rows
+        int nsplit = std::min(HY_MAX_SPLITS, std::max(1, tiles));
+        if ((size_t)n * nsplit > h->part_rows) nsplit = std::max<size_t>(1, h->part_rows / n);
+        a.nsplit = nsplit; a.kt = 32;
+        const dim3 grid(hy_cdiv(n * (H / G), 32) * G, 1, nsplit);
+        bool done = true;
+#define HY_AF(DK, DV, NW) hipLaunchKernelGGL((hy_attn_few_kernel<DK, DV, NW>), grid, dim3(64 * NW), 0, ctx->stream, a)
+        if (dk == 128 && dv == 128) HY_AF(128, 128, 4);
+        else if (dk == 64 && dv == 64) HY_AF(64, 64, 4);
+        else if (dk == 512 && dv == 512) HY_AF(512, 512, 8);
+        else if (dk == 256 && dv == 256) HY_AF(256, 256, 8);
+        else done = false;
+#undef HY_AF
+        if (done) { *nsplit_out = nsplit; return GL3_OK; }
+    }
     if (n > 16 && !shared_kv && aligned && (uint64_t)(pos0 + n) * G * std::max(dk, dv) < 0x3fff0000ull) {          // (32-bit byte offsets inside a cache)
         // few row blocks (a short portion): more workgroups per block while each wavefront keeps four key tiles or more
         const int blocks = hy_cdiv(n * (H / G), 32) * G;
@@ -1118,9 +1137,12 @@ static void hy_merge(gl3_ctx* ctx, const HyLayer& L, int n, int dv, int nsplit, 
     if (nsplit > 2 && nsplit <= HY_MAX_SPLITS && n <= 16)
         hipLaunchKernelGGL((hy_attn_merge_few_kernel<TO>), dim3(n, d.heads), dim3(256), 0, ctx->stream, h->part_acc, h->part_ml, d.heads, dv, nsplit, d.softmax_sink, gate, ldg, gate_mode, out, ldo,
                            v_freq, h->dyn, sink_w, out_mul);
-    else
-        hipLaunchKernelGGL((hy_attn_merge_kernel<TO>), dim3(n, d.heads), dim3(64), 0, ctx->stream, h->part_acc, h->part_ml, d.heads, dv, nsplit, d.softmax_sink, gate, ldg, gate_mode, out, ldo,
-                           v_freq, h->dyn, sink_w, out_mul);
+    else {
+        // (one or two splits of 512 columns: 5.8 us on one wavefront)
+#define HY_MG(NT) hipLaunchKernelGGL((hy_attn_merge_kernel<TO, NT>), dim3(n, d.heads), dim3(NT), 0, ctx->stream, h->part_acc, h->part_ml, d.heads, dv, nsplit, d.softmax_sink, gate, ldg, gate_mode, out, ldo, v_freq, h->dyn, sink_w, out_mul)
+        if (dv > 128) HY_MG(256); else HY_MG(64);
+#undef HY_MG
+    }
 }
 
 // Attention over all heads at once (hy_heads_attn_kernel): temperatures, capped and mixed scores, chunks.

@@ -47,3 +47,29 @@ def test_portions_and_tiles(hy, tmp_path, name, n, batch):
     p.close()
     want = m.ref(toks)
     assert N.err(got, want) < 2e-5, N.err(got, want)
+
+
+# a few tokens at a time (hy_attn_few_kernel): the head sizes above and latents of 128 / 256 / 512 cached entries scored in the latent's space
+FEW = {k: LAYERS[k] for k in ("64_gqa2", "128_gqa3", "128_mha", "window_pool64", "window_pool128", "window_keep64")}
+FEW.update({"latent_direct128": (U, U.lat(heads=5, dim=24, rot_dim=32, vdim=20, kv_rank=96, mlp=None)), "latent_direct256": (N, N.lat(heads=3, dim=16, vdim=24, kv_rank=256, ff=0)),
+            "latent_direct512": (N, N.lat(heads=40, dim=16, vdim=16, kv_rank=512, ff=0))})
+
+
+@pytest.mark.parametrize("n", [0, 31, 130])
+@pytest.mark.parametrize("name", list(FEW))
+def test_a_few_tokens(hy, tmp_path, name, n):
+    mod, layer = FEW[name]
+    cfg = mod.config([layer])
+    m = mod.Model(hy, tmp_path, cfg, seed=n)
+    steps = [1, 1, 3, 8, 16, 1, 5]
+    toks = np.random.default_rng(n).integers(0, cfg["vocab"], n + sum(steps)).astype(np.int32)
+    p = m.plan("float32", ctx=len(toks) + 8, max_batch=64)
+    s, got, pos = p.acquire(), [], n
+    if n:
+        got.append(p.step(s, toks[:n], 0, list(range(n))))
+    for k in steps:
+        got.append(p.step(s, toks[pos:pos + k], pos, list(range(k))))
+        pos += k
+    p.close()
+    want = m.ref(toks)
+    assert N.err(np.concatenate(got), want) < 2e-5
