@@ -916,7 +916,7 @@ static const struct { int bm, bn; } HY_RING_TILES[HY_R_COUNT] = {{256, 256}, {25
 // 256 CUs take the workgroups in rounds of whole tiles (two workgroups of a small tile share a CU; one alone needs 0.4 us per stage for its loads'
 // way: 88 tokens, 4096 x 4096 in 64 x 64 tiles 16 us as 256 workgroups, 11 us as 512) — what decides for most shapes: 10240 x 4096 at 512 tokens is 256 tiles of 128 x 160
 // (50 us) but 320 of 128 x 128 (65 us) or 160 of 256 x 128 (53 us).  A K split writes and re-reads its part of C at ~4 TB/s.
-static void hy_ring_pick(bool f32, int M, int N, int K, bool glu, bool actmul, int max_parts, int* tile, int* ks_out) {
+static double hy_ring_pick(bool f32, int M, int N, int K, bool glu, bool actmul, int max_parts, int* tile, int* ks_out) {
     const int stages = K / (f32 ? 32 : 64);
     double best = 1e30;
     for (int t = 0; t < HY_R_COUNT; ++t) {
@@ -935,18 +935,19 @@ static void hy_ring_pick(bool f32, int M, int N, int K, bool glu, bool actmul, i
             if (us < best) { best = us; *tile = t; *ks_out = ks; }
         }
     }
+    return std::max(best, (double)N * K * (f32 ? 4 : 2) / 4.4e6 + 3.0);          // the weights leave HBM at 4.4 TB/s
 }
 
-// The ring kernel for a product it can take (true), or nothing.  parts / max_parts as for hy_gemm.
+// The ring kernel for a product it can take in less than limit_us (true), or nothing.  parts / max_parts as for hy_gemm.
 template <typename T>
-static bool hy_gemm_ring(gl3_ctx* ctx, const T* A, int lda, const HyMat& w, int M, float* C, int ldc, bool glu, T* act, int ld_act, HyGlu gp, int* parts, int max_parts) {
+static bool hy_gemm_ring(gl3_ctx* ctx, const T* A, int lda, const HyMat& w, int M, float* C, int ldc, bool glu, T* act, int ld_act, HyGlu gp, int* parts, int max_parts, double limit_us = 1e30) {
     const int N = w.rows, K = w.k;
     constexpr int PE = 16 / (int)sizeof(T), BK = 128 / (int)sizeof(T);
     if (K % BK || lda % PE || w.ld % PE || (((uintptr_t)A | (uintptr_t)w.w) & 15)) return false;
     if ((uint64_t)M * lda * sizeof(T) >= 0xffff0000ull || (uint64_t)N * w.ld * sizeof(T) >= 0xffff0000ull) return false;      // 32-bit offsets inside an operand
     const bool actmul = !glu && (gp.mul_table || gp.act == 2);
     int tile = HY_R128x128, ks = 1;
-    hy_ring_pick(sizeof(T) == 4, M, N, K, glu, actmul, parts && !glu && !actmul ? max_parts : 1, &tile, &ks);
+    if (hy_ring_pick(sizeof(T) == 4, M, N, K, glu, actmul, parts && !glu && !actmul ? max_parts : 1, &tile, &ks) >= limit_us) return false;
     const int kper = hy_cdiv(K / BK, ks) * BK, mt = hy_cdiv(M, HY_RING_TILES[tile].bm), nt = hy_cdiv(N, HY_RING_TILES[tile].bn);
     if (parts) *parts = ks;
     const dim3 grid((unsigned)hy_cdiv(mt * nt * ks, 8) * 8);
@@ -982,6 +983,9 @@ static void hy_gemm(gl3_ctx* ctx, const T* A, int lda, const HyMat& w, int M, fl
     const T* Wt = (const T*)w.w;
     const int N = w.rows, K = w.k;
     hipStream_t st = ctx->stream;
+    // Five to eight tokens cost the matvec 1.8 - 2.5 times one token's time (its vector units), the matrix cores no more than one: 28672 x 4096 100 and 55 us,
+    // 12000 x 2048 33 and 20, but 2048 x 2048 9.4 and 11.5.
+    if (M > 4 && M <= 8 && sizeof(T) == 2 && hy_gemm_ring<T>(ctx, A, lda, w, M, C, ldc, glu, act, ld_act, gp, parts, max_parts, 2.1 * N * K * 2 / 5.6e6 + 3.0)) return;
     if (M <= 8) {
         const int pairs = hy_cdiv(N, 2);
         const bool ksplit = pairs < 8192 && K >= 1024;       // few rows: a workgroup's four wavefronts share one pair's K

@@ -25,7 +25,8 @@ def hy():
 
 # (tokens, width, vocabulary, feed-forward): tiles of the head's product bf16 / f32 behind each
 CASES = [(9, 64, 211, 96), (33, 192, 1003, 160), (64, 128, 20001, 64), (65, 128, 20003, 288), (129, 128, 20005, 416), (130, 64, 29999, 96),
-         (257, 128, 20007, 7008), (300, 64, 30001, 15008), (255, 704, 451, 608), (191, 1024, 333, 1056), (256, 128, 33001, 64), (70, 104, 515, 72)]
+         (257, 128, 20007, 7008), (300, 64, 30001, 15008), (255, 704, 451, 608), (191, 1024, 333, 1056), (256, 128, 33001, 64), (70, 104, 515, 72),
+         (5, 1024, 333, 9024), (8, 704, 12001, 608), (6, 1024, 12003, 9056)]          # 5 to 8 tokens: where the tiles cost less than the dot products
 
 
 @pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
