@@ -809,12 +809,18 @@ static __global__ __launch_bounds__(64) void hy_latent_norm_kernel(const float* 
                                                                    float* __restrict__ cc, size_t slot_stride, const int* __restrict__ dyn) {
     const int t = blockIdx.x, lane = threadIdx.x;
     const float* src = proj + (size_t)t * ld + c_off;
-    float ss = 0.f;
-    for (int r = lane; r < R; r += 64) ss += src[r] * src[r];
+    float* dst = cc + (size_t)dyn[1] * slot_stride + (size_t)(dyn[0] + t) * R;
+    float v[8], w[8], ss = 0.f;          // the first 512 entries and their weights: one round trip (a load per loop round: 6.8 us for one token)
+#pragma unroll
+    for (int i = 0; i < 8; ++i) { const int r = min(lane + 64 * i, R - 1); v[i] = src[r]; w[i] = cnorm[r]; }
+#pragma unroll
+    for (int i = 0; i < 8; ++i) if (lane + 64 * i < R) ss += v[i] * v[i];
+    for (int r = lane + 512; r < R; r += 64) ss += src[r] * src[r];
     ss = hy_wave_sum(ss);
     const float s = 1.f / sqrtf(ss / (float)R + eps);
-    float* dst = cc + (size_t)dyn[1] * slot_stride + (size_t)(dyn[0] + t) * R;
-    for (int r = lane; r < R; r += 64) dst[r] = src[r] * s * cnorm[r];
+#pragma unroll
+    for (int i = 0; i < 8; ++i) if (lane + 64 * i < R) dst[lane + 64 * i] = v[i] * s * w[i];
+    for (int r = lane + 512; r < R; r += 64) dst[r] = src[r] * s * cnorm[r];
 }
 
 // Latent attention with a rotated part (D unrotated + P rotated entries per query head, one rotated key part of P entries for all heads,
@@ -895,11 +901,11 @@ static __global__ __launch_bounds__(256) void hy_softcap_kernel(float* __restric
 // sigmoid(gate[t][h]), one gate per head), for portions of a
 // few tokens (decode).  Two uses: the query carried into the latent's space, qa = Wk^T q (scores are then plain dot products with the
 // cached latents: q . (Wk c) = (Wk^T q) . c), and the value expansion applied after the weighted sum of latents.  Workgroup = (TT tokens, head, 64 columns): lane =
-// column, the four wavefronts split k and meet in LDS, a weight is read once for TT tokens.
-template <typename TO, int TT>
-static __global__ __launch_bounds__(256) void hy_headmm_kernel(const float* __restrict__ in, int ld_in, int K, int C, const float* __restrict__ Wt,
+// column, the NW wavefronts split k and meet in LDS, a weight is read once for TT tokens.
+template <typename TO, int TT, int NW = 4>
+static __global__ __launch_bounds__(64 * NW) void hy_headmm_kernel(const float* __restrict__ in, int ld_in, int K, int C, const float* __restrict__ Wt,
                                                                const float* __restrict__ gate, int ldg, TO* __restrict__ out, int ldo, int n, int gate_mode = 1) {
-    __shared__ float red[3][TT][64];
+    __shared__ float red[NW - 1][TT][64];
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, h = blockIdx.y, c = blockIdx.z * 64 + lane, t0 = blockIdx.x * TT;
     const bool livec = c < C;
     float acc[TT];
@@ -911,7 +917,7 @@ static __global__ __launch_bounds__(256) void hy_headmm_kernel(const float* __re
     const float* xr[TT];
 #pragma unroll
     for (int i = 0; i < TT; ++i) xr[i] = x + (size_t)(t0 + i < n ? i : 0) * ld_in;
-    for (int k0 = wave * 8; k0 < K; k0 += 32) {
+    for (int k0 = wave * 8; k0 < K; k0 += 8 * NW) {
         float wv[8], xv[TT][8];
 #pragma unroll
         for (int u = 0; u < 8; ++u) {
@@ -934,7 +940,9 @@ static __global__ __launch_bounds__(256) void hy_headmm_kernel(const float* __re
 #pragma unroll
     for (int i = 0; i < TT; ++i) {
         if (t0 + i >= n) break;
-        float v = (acc[i] + red[0][i][lane]) + (red[1][i][lane] + red[2][i][lane]);
+        float v = acc[i] + red[0][i][lane];
+#pragma unroll
+        for (int w = 1; w < NW - 1; w += 2) v += red[w][i][lane] + red[w + 1][i][lane];
         if (gate) v *= hy_sigmoid(gate[(size_t)(t0 + i) * ldg + (gate_mode == 2 ? h : h * C + c)]);
         hy_st(out + (size_t)(t0 + i) * ldo + h * C + c, v);
     }
@@ -1252,20 +1260,41 @@ static __global__ __launch_bounds__(256) void hy_attn_merge_few_kernel(const flo
 // ---- state-space mixer ------------------------------------------------------------------------------------------------------------
 // Causal depthwise convolution over the step's tokens; inputs before the step come from the slot's tail (the last taps - 1 inputs of
 // the sequence), zeros before position 0.  out = silu(bias + sum_k w[c][k] in(t - (taps - 1 - k))).
+// One thread per channel and HY_CONV_T tokens: every input is loaded once (one token per thread loads it taps times: 28 -> 14 us for 512 tokens x
+// 10240 channels).  A portion that fits one thread's tokens moves the tail on as well; longer ones leave that to hy_conv_tail_kernel.
+constexpr int HY_CONV_T = 8;
 static __global__ __launch_bounds__(256) void hy_conv_kernel(const float* __restrict__ proj, int ld, int x_off, int ch, int taps, const float* __restrict__ w,
-                                                             const float* __restrict__ bias, const float* __restrict__ tail, size_t slot_stride,
+                                                             const float* __restrict__ bias, float* __restrict__ tail, size_t slot_stride,
                                                              const int* __restrict__ dyn, int n, float* __restrict__ out) {
-    const int c = blockIdx.x * 256 + threadIdx.x, t = blockIdx.y;
+    const int c = blockIdx.x * 256 + threadIdx.x, t0 = blockIdx.y * HY_CONV_T;
     if (c >= ch) return;
     const bool fresh = dyn[0] == 0;
-    const float* tl = tail + (size_t)dyn[1] * slot_stride;
-    float a = bias[c];
-    for (int k = 0; k < taps; ++k) {
-        const int tau = t - (taps - 1 - k);
-        const float v = tau >= 0 ? proj[(size_t)tau * ld + x_off + c] : (fresh ? 0.f : tl[(size_t)(taps - 1 + tau) * ch + c]);
-        a = fmaf(w[(size_t)c * taps + k], v, a);
-    }
-    out[(size_t)t * ch + c] = hy_silu(a);
+    float* tl = tail + (size_t)dyn[1] * slot_stride;
+    const float* src = proj + x_off + c;
+    auto at = [&](int tau) { return tau >= 0 ? src[(size_t)min(tau, n - 1) * ld] : (fresh || taps - 1 + tau < 0) ? 0.f : tl[(size_t)(taps - 1 + tau) * ch + c]; };
+    const float b = bias[c];
+    if (taps <= 4) {
+        float v[HY_CONV_T + 3], wt[4];
+#pragma unroll
+        for (int i = 0; i < HY_CONV_T + 3; ++i) v[i] = at(t0 + i - 3);
+#pragma unroll
+        for (int k = 0; k < 4; ++k) wt[k] = w[(size_t)c * taps + max(0, k - (4 - taps))];          // taps 4 - taps .. 3 of four
+#pragma unroll
+        for (int i = 0; i < HY_CONV_T; ++i) {
+            float a = b;
+#pragma unroll
+            for (int k = 0; k < 4; ++k)
+                if (k >= 4 - taps) a = fmaf(wt[k], v[i + k], a);
+            if (t0 + i < n) out[(size_t)(t0 + i) * ch + c] = hy_silu(a);
+        }
+    } else
+        for (int t = t0; t < min(t0 + HY_CONV_T, n); ++t) {
+            float a = b;
+            for (int k = 0; k < taps; ++k) a = fmaf(w[(size_t)c * taps + k], at(t - (taps - 1 - k)), a);
+            out[(size_t)t * ch + c] = hy_silu(a);
+        }
+    if (gridDim.y == 1)
+        for (int i = 0; i < taps - 1; ++i) tl[(size_t)i * ch + c] = at(n + i - (taps - 1));          // ascending: reads only rows not yet rewritten
 }
 // new tail[i] = input at step-relative time n + i - (taps - 1); one thread per channel, ascending i (reads only rows not yet rewritten)
 static __global__ __launch_bounds__(256) void hy_conv_tail_kernel(const float* __restrict__ proj, int ld, int x_off, int ch, int taps, float* __restrict__ tail,
@@ -1462,6 +1491,78 @@ static __global__ __launch_bounds__(256) void hy_ssm_scan_kernel(HyScanArgs a) {
         const int nn = ng * NL + i;
         if (livep && nn < N) S[(size_t)nn * P + p] = s[i];
     }
+}
+
+// One token: S <- a S + b k x^T (mode 3: S += g (x - S)), y = S^T q + D x with every state element read and written once, where hy_ssm_scan_kernel stages, walks and
+// joins as for a block of tokens (64 heads x 128 x 64: 10 -> 5.4 us).  Workgroup = one head x 64 columns; its sixteen wavefronts share the states, sixteen
+// rows of 64 columns each on the way at once (256 states: one round trip); keys and queries of the head are made in LDS meanwhile.
+static __global__ __launch_bounds__(1024) void hy_scan_one_kernel(HyScanArgs a) {
+    extern __shared__ float smem[];
+    const int N = a.N, P = a.P, Px = P - (a.ones_col ? 1 : 0), head = blockIdx.y, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, p = blockIdx.x * 64 + lane;
+    const int gr = head / (a.heads / a.G), pos = a.dyn[0];
+    const bool fresh = pos == 0, cg = a.mode == 3;
+    float *sK = smem, *sQ = smem + N, *red = smem + 2 * N;          // red: [16][64]
+    const float *kb = a.ksrc + a.k_off + (size_t)gr * a.k_hstride, *qb = a.qsrc + a.q_off + (size_t)gr * a.q_hstride;
+    float* S = a.state + (size_t)a.dyn[1] * a.slot_stride + (size_t)head * N * P;
+    const int half = a.rot.dims >> 1;
+    const int nq = (N + 15) / 16, n0 = wave * nq, n1 = min(N, n0 + nq), pc = min(p, P - 1);
+    float s[16], y = 0.f;
+    auto load = [&](int n) {
+#pragma unroll
+        for (int u = 0; u < 16; ++u) s[u] = S[(size_t)min(n + u, N - 1) * P + pc];
+    };
+    load(n0);
+    for (int i = tid; i < 2 * N; i += 1024) {
+        const bool q = i >= N;
+        const int n = q ? i - N : i;
+        float v;
+        if (cg && !q && a.fbias) v = (1.f - a.lower[(size_t)head * N + n]) * hy_sigmoid(-(kb[n] + a.fbias[(size_t)head * N + n]));
+        else {
+            const bool si = a.act & (q ? 2 : 1);
+            const float mul = q ? a.q_mul : a.k_mul;
+            const float* src = q ? qb : kb;
+            v = (si ? hy_silu(src[n]) : src[n]) * mul;
+            if (n < a.rot.dims) {          // the other entry of the pair, and which of the two this is
+                const int j = a.rot.interleaved ? n >> 1 : n < half ? n : n - half, o = a.rot.interleaved ? n ^ 1 : n < half ? n + half : n - half;
+                const bool first = a.rot.interleaved ? !(n & 1) : n < half;
+                const float w = (si ? hy_silu(src[o]) : src[o]) * mul;
+                float sn, cs;
+                sincosf((float)pos * a.rot.freq[j], &sn, &cs);
+                v = first ? v * cs - w * sn : v * cs + w * sn;
+            }
+        }
+        (q ? sQ : sK)[n] = v;
+    }
+    float av = 1.f, bv = 1.f, dd = 0.f;
+    if (a.mode == 0) {
+        bv = hy_softplus(a.dtsrc[a.dt_off + head] + a.dt_bias[head]);
+        av = expf(-expf(a.A_log[head]) * bv);
+        if (a.Dp) dd = a.Dp[head];
+    } else if (a.mode == 1) { av = a.ga[head]; bv = a.gb[head]; }
+    else if (a.mode == 2) av = a.decay[head];
+    float x = 0.f;
+    if (p < Px) { x = a.xsrc[a.x_off + (size_t)head * Px + p]; if (a.act & 4) x = hy_silu(x); }
+    else if (p < P) x = 1.f;
+    const float bx = bv * x;
+    __syncthreads();
+    for (int n = n0; n < n1; n += 16) {
+        if (n > n0) load(n);
+#pragma unroll
+        for (int u = 0; u < 16; ++u) {
+            if (n + u >= n1) break;
+            const float k = sK[n + u], old = fresh ? 0.f : s[u];
+            const float v = cg ? fmaf(k, x - old, old) : fmaf(av, old, k * bx);
+            y = fmaf(v, sQ[n + u], y);
+            if (p < P) S[(size_t)(n + u) * P + p] = v;
+        }
+    }
+    red[wave * 64 + lane] = y;
+    __syncthreads();
+    if (wave > 0 || p >= P) return;
+    float v = 0.f;
+#pragma unroll
+    for (int w = 0; w < 16; ++w) v += red[w * 64 + lane];
+    a.y[head * P + p] = fmaf(dd, x, v);
 }
 
 // Gates of a matrix memory with exponential gating, per (token, head), from the raw gate projections z_i, z_f (+ biases):

@@ -1224,6 +1224,10 @@ static void hy_scan_chunk_launch(gl3_ctx* ctx, const HyScanArgs& a) {
 // stages the same key / query rows for too few columns and the traffic from L2 eats the gain (measured: 16 and 8 within 2 %, 4 slower).
 // GL3_HY_SCAN_NL forces a value.
 static void hy_scan(gl3_ctx* ctx, HyScanArgs& a) {
+    if (a.n == 1 && a.N <= 4096) {
+        hipLaunchKernelGGL(hy_scan_one_kernel, dim3(hy_cdiv(a.P, 64), a.heads), dim3(1024), (size_t)(2 * a.N + 1024) * 4, ctx->stream, a);
+        return;
+    }
     if (hy_scan_chunks(a)) { hy_scan_chunk_launch(ctx, a); return; }
     int NL = a.N > 1024 ? 32 : a.N > 8 ? 16 : a.N > 4 ? 8 : 4;
     auto wgs = [&](int nl) { int ng = 1; while (ng * nl < a.N) ng *= 2; return (long)hy_cdiv(a.P, 4 * (64 / ng)) * a.heads; };
@@ -1400,7 +1404,10 @@ static int32_t hy_mixer_core(gl3_ctx* ctx, HyLayer& L, int np, int ldo, int n, i
             int32_t r = hy_attention(ctx, h->qa, d.heads * R, cc, cc, d.heads, 1, R, R, d.scale, 0.f, n, pos0, &nsplit);
             if (r != GL3_OK) return r;
             hy_merge<float>(ctx, L, n, R, nsplit, nullptr, 0, 0, h->oc, d.heads * R);
-            if (n == 1)
+            if (n == 1 && R >= 256)          // a long sum per output: sixteen wavefronts share it (512 entries: 14 us with four)
+                hipLaunchKernelGGL((hy_headmm_kernel<T, 1, 16>), dim3(1, d.heads, hy_cdiv(d.vdim, 64)), dim3(1024), 0, st, h->oc, d.heads * R, R, d.vdim, L.wvT,
+                                   d.out_gate ? h->proj + L.g_off : nullptr, np, mixo, ldo, n, d.out_gate == 2 ? 2 : 1);
+            else if (n == 1)
                 hipLaunchKernelGGL((hy_headmm_kernel<T, 1>), dim3(1, d.heads, hy_cdiv(d.vdim, 64)), dim3(256), 0, st, h->oc, d.heads * R, R, d.vdim, L.wvT,
                                    d.out_gate ? h->proj + L.g_off : nullptr, np, mixo, ldo, n, d.out_gate == 2 ? 2 : 1);
             else
@@ -1411,9 +1418,9 @@ static int32_t hy_mixer_core(gl3_ctx* ctx, HyLayer& L, int np, int ldo, int n, i
         const int inner = d.heads * d.vdim, ch = hy_conv_ch(d), dt_off = 2 * inner + 2 * d.groups * d.state;
         float* state = h->slots + L.off_state;
         float* tail = h->slots + L.off_tail;
-        hipLaunchKernelGGL(hy_conv_kernel, dim3(hy_cdiv(ch, 256), n), dim3(256), 0, st, h->proj, np, inner, ch, d.conv, L.conv_w, L.conv_b, tail, h->slot_floats, h->dyn,
+        hipLaunchKernelGGL(hy_conv_kernel, dim3(hy_cdiv(ch, 256), hy_cdiv(n, HY_CONV_T)), dim3(256), 0, st, h->proj, np, inner, ch, d.conv, L.conv_w, L.conv_b, tail, h->slot_floats, h->dyn,
                            n, h->conv);
-        if (d.conv > 1)
+        if (d.conv > 1 && n > HY_CONV_T)
             hipLaunchKernelGGL(hy_conv_tail_kernel, dim3(hy_cdiv(ch, 256)), dim3(256), 0, st, h->proj, np, inner, ch, d.conv, tail, h->slot_floats, h->dyn, n);
         HyScanArgs a{};
         a.ksrc = h->conv; a.ldk = ch; a.k_off = inner; a.k_hstride = d.state;
