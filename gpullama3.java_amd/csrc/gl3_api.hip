@@ -1082,6 +1082,7 @@ int32_t gl3_forward_decode(gl3_ctx* ctx, int32_t token, int32_t pos, float* logi
         for (const auto& pr : ctx->pinned)
             if ((uint8_t*)logits_out >= (uint8_t*)pr.first && (uint8_t*)logits_out + (size_t)ctx->d.vocab * 4 <= (uint8_t*)pr.first + pr.second) direct = true;
     if (logits_out) GL3_HIP(hipMemcpyAsync(direct ? logits_out : ctx->h_logits, ctx->logits, (size_t)ctx->d.vocab * 4, hipMemcpyDeviceToHost, ctx->stream));
+    if (logits_out && !direct) gl3_touch_pages(logits_out, (size_t)ctx->d.vocab * 4);
     GL3_HIP(hipStreamSynchronize(ctx->stream));
     if ((r = gl3_tp_check(ctx)) != GL3_OK) return r;
     if (logits_out && !direct) memcpy(logits_out, ctx->h_logits, (size_t)ctx->d.vocab * 4);

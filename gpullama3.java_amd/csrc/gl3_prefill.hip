@@ -10,6 +10,7 @@
 // (Q8_0FloatTensor.java:90-123), and that is what the GEMM below does on CDNA4's int8 matrix cores:
 //   one v_mfma_i32_32x32x32_i8 = the int32 dot of one Q8_0 block for a 32-row x 32-token tile (exact), then
 //   acc = acc + float(isum) * (wScale * aScale) on the VALU, blocks ascending — the reference's f32 order.
+#include <cstring>
 #include <cstdio>
 #include <cstdlib>
 #include <vector>
@@ -31,6 +32,9 @@ void gl3_gemm3_launch(int epi, const GemmArgs& a, int rows, int ntok, hipStream_
 bool gl3_gemm3_swiglu_quantises(int rows, int ntok);
 hipError_t gl3_gemm3_allow_lds();
 
+constexpr int PF_LOG_SLOTS = 3;                         // pinned pieces of logits in flight (static-batched decode)
+constexpr size_t PF_LOG_PIECE = (size_t)4 << 20;
+
 struct gl3_prefill_state {
     int max_batch = 0;
     int32_t* tokens = nullptr;          // [M]
@@ -50,7 +54,10 @@ struct gl3_prefill_state {
     float* TMX = nullptr;               // [M][n_heads][tmx_tiles] per-64-timestep-tile maxima of the score rows (pf_scores_tiled_kernel -> pf_softmax_rows_kernel)
     float* SUMS = nullptr;              // [M][n_heads] softmax denominators (pf_softmax_rows_kernel -> pf_pv_tiled_kernel)
     int tmx_tiles = 0;
-    int32_t* seqpos = nullptr;          // [2][M]: sequence id, position of every token of the step
+    int32_t* seqpos = nullptr;          // [2][M] behind tokens: sequence id, position of every token of the step
+    int32_t* h_io = nullptr;            // pinned [4][M]: tokens, sequence ids, positions of the step on their way in, greedy ids on their way out
+    uint8_t* h_log[PF_LOG_SLOTS] = {};  // pinned pieces of logits on their way to the caller (static-batched decode), made at its first use
+    hipEvent_t log_ev[PF_LOG_SLOTS] = {};
     float* LOGITS = nullptr;            // [rows][vocab], grown on demand (batched decode)
     int logits_rows = 0;
     std::vector<hipGraphExec_t> step_graphs;   // static-batched decode: one captured step per batch size (positions < AF_MAXN)
@@ -2185,7 +2192,9 @@ int32_t gl3_prefill_alloc(gl3_ctx* ctx) {
     const size_t M = d.max_batch;
     p->vl = ctx->emb.vl;
     if (p->vl) {       // f32-activation weight types: f32 buffers; the gathered ones (X, AO, HB, LOGITS) in the arena under tensor parallelism
-        GL3_HIP(hipMalloc((void**)&p->tokens, M * sizeof(int32_t)));
+        GL3_HIP(hipMalloc((void**)&p->tokens, 3 * M * sizeof(int32_t)));
+        p->seqpos = p->tokens + M;
+        GL3_HIP(hipHostMalloc((void**)&p->h_io, 4 * M * sizeof(int32_t)));
         if (ctx->arena.base && ctx->arena.off[GB_PF_X]) {
             uint8_t* b = ctx->arena.base;
             p->X = (float*)(b + ctx->arena.off[GB_PF_X]); p->AO = (float*)(b + ctx->arena.off[GB_PF_AO]); p->HB = (float*)(b + ctx->arena.off[GB_PF_HB]);
@@ -2205,7 +2214,6 @@ int32_t gl3_prefill_alloc(gl3_ctx* ctx) {
         p->tmx_tiles = (d.ctx + 63) / 64;
         GL3_HIP(hipMalloc((void**)&p->TMX, M * d.n_heads * (size_t)p->tmx_tiles * 4));
         GL3_HIP(hipMalloc((void**)&p->SUMS, M * d.n_heads * 4));
-        GL3_HIP(hipMalloc((void**)&p->seqpos, 2 * M * sizeof(int32_t)));
         GL3_HIP(hipMalloc((void**)&p->amax, M * sizeof(int32_t)));
         GL3_HIP(hipMalloc((void**)&p->amx_v, M * AMX_SPLIT * sizeof(float)));
         GL3_HIP(hipMalloc((void**)&p->amx_i, M * AMX_SPLIT * sizeof(int)));
@@ -2230,7 +2238,9 @@ int32_t gl3_prefill_alloc(gl3_ctx* ctx) {
     p->maxk = d.hidden > ctx->q_dim ? d.hidden : ctx->q_dim;
     if (d.dim > p->maxk) p->maxk = d.dim;
     p->maxk = (p->maxk + 127) & ~127;
-    GL3_HIP(hipMalloc((void**)&p->tokens, M * sizeof(int32_t)));
+    GL3_HIP(hipMalloc((void**)&p->tokens, 3 * M * sizeof(int32_t)));
+    p->seqpos = p->tokens + M;
+    GL3_HIP(hipHostMalloc((void**)&p->h_io, 4 * M * sizeof(int32_t)));
     if (ctx->arena.base && ctx->arena.off[GB_PF_X]) {      // tensor parallel: the gathered activations live in the arena the peers map
         uint8_t* b = ctx->arena.base;
         p->X = (float*)(b + ctx->arena.off[GB_PF_X]); p->AO = (float*)(b + ctx->arena.off[GB_PF_AO]); p->HB = (float*)(b + ctx->arena.off[GB_PF_HB]);
@@ -2265,7 +2275,6 @@ int32_t gl3_prefill_alloc(gl3_ctx* ctx) {
     p->tmx_tiles = (d.ctx + 63) / 64;
     GL3_HIP(hipMalloc((void**)&p->TMX, M * d.n_heads * (size_t)p->tmx_tiles * 4));
     GL3_HIP(hipMalloc((void**)&p->SUMS, M * d.n_heads * 4));
-    GL3_HIP(hipMalloc((void**)&p->seqpos, 2 * M * sizeof(int32_t)));
     GL3_HIP(hipMalloc((void**)&p->amax, M * sizeof(int32_t)));
     GL3_HIP(hipMalloc((void**)&p->amx_v, M * AMX_SPLIT * sizeof(float)));
     GL3_HIP(hipMalloc((void**)&p->amx_i, M * AMX_SPLIT * sizeof(int)));
@@ -2297,8 +2306,11 @@ void gl3_prefill_free(gl3_ctx* ctx) {
     if (!p) return;
     for (auto ge : p->step_graphs) if (ge) hipGraphExecDestroy(ge);
     auto f = [](void* q) { if (q) hipFree(q); };
-    f(p->tokens); f(p->XQ); f(p->XS); f(p->XP); f(p->XQh); f(p->XPh); f(p->XQb); f(p->XSb); f(p->QKV); f(p->ATT); f(p->TMX); f(p->SUMS); f(p->seqpos); f(p->amax); f(p->amx_v); f(p->amx_i); f(p->XN); f(p->HB2);
+    f(p->tokens); f(p->XQ); f(p->XS); f(p->XP); f(p->XQh); f(p->XPh); f(p->XQb); f(p->XSb); f(p->QKV); f(p->ATT); f(p->TMX); f(p->SUMS); f(p->amax); f(p->amx_v); f(p->amx_i); f(p->XN); f(p->HB2);
     if (!p->in_arena) { f(p->X); f(p->AO); f(p->HB); f(p->LOGITS); }
+    if (p->h_io) hipHostFree(p->h_io);
+    for (auto q : p->h_log) if (q) hipHostFree(q);
+    for (auto e : p->log_ev) if (e) hipEventDestroy(e);
     delete p;
     ctx->pf = nullptr;
 }
@@ -2728,11 +2740,40 @@ static __global__ void pf_unchunk_row_kernel(const float* __restrict__ X, int b,
     for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < dim; i += gridDim.x * blockDim.x) out[i] = X[chunked(b, i, cc, ntok)];
 }
 
-static int32_t pf_stage_tokens(gl3_ctx* ctx, const int32_t* tokens, const int32_t* seqs, const int32_t* poss, int n) {
+// The step's (token, sequence, position) triples: one copy from pinned memory.  Every run that used h_io has been waited for.
+static int32_t pf_stage_tokens(gl3_ctx* ctx, int n) {
     gl3_prefill_state* p = ctx->pf;
-    GL3_HIP(hipMemcpyAsync(p->tokens, tokens, (size_t)n * sizeof(int32_t), hipMemcpyHostToDevice, ctx->stream));
-    GL3_HIP(hipMemcpyAsync(p->seqpos, seqs, (size_t)n * sizeof(int32_t), hipMemcpyHostToDevice, ctx->stream));
-    GL3_HIP(hipMemcpyAsync(p->seqpos + p->max_batch, poss, (size_t)n * sizeof(int32_t), hipMemcpyHostToDevice, ctx->stream));
+    GL3_HIP(hipMemcpyAsync(p->tokens, p->h_io, ((size_t)2 * p->max_batch + n) * sizeof(int32_t), hipMemcpyHostToDevice, ctx->stream));
+    return GL3_OK;
+}
+
+// n rows of logits to the caller: through pinned pieces of at most PF_LOG_PIECE bytes, a piece on its way while the one before it is copied on.  (A copy to
+// pageable memory goes row by row through the runtime's own staging: 32 rows x 16896 570 - 740 us, this way 45 on the link + 30 - 70 on the host; x 151936
+// 1041 and 767.)  False: no pinned memory for the pieces.
+static bool pf_logits_slots(gl3_prefill_state* p) {
+    for (int i = 0; i < PF_LOG_SLOTS; ++i) {
+        if (!p->h_log[i] && hipHostMalloc((void**)&p->h_log[i], PF_LOG_PIECE) != hipSuccess) { p->h_log[i] = nullptr; (void)hipGetLastError(); return false; }
+        if (!p->log_ev[i] && hipEventCreateWithFlags(&p->log_ev[i], hipEventDisableTiming) != hipSuccess) { p->log_ev[i] = nullptr; (void)hipGetLastError(); return false; }
+    }
+    return true;
+}
+static int32_t pf_logits_out(gl3_ctx* ctx, float* out, size_t bytes) {
+    gl3_prefill_state* p = ctx->pf;
+    const size_t pieces = (bytes + PF_LOG_PIECE - 1) / PF_LOG_PIECE, per = ((bytes + pieces - 1) / pieces + 4095) & ~(size_t)4095;
+    auto send = [&](size_t i) -> int32_t {
+        if (i * per >= bytes) return GL3_OK;
+        GL3_HIP(hipMemcpyAsync(p->h_log[i % PF_LOG_SLOTS], (const uint8_t*)p->LOGITS + i * per, std::min(per, bytes - i * per), hipMemcpyDeviceToHost, ctx->stream));
+        GL3_HIP(hipEventRecord(p->log_ev[i % PF_LOG_SLOTS], ctx->stream));
+        return GL3_OK;
+    };
+    int32_t r;
+    for (size_t i = 0; i < PF_LOG_SLOTS; ++i) if ((r = send(i)) != GL3_OK) return r;
+    gl3_touch_pages(out, bytes);
+    for (size_t i = 0; i * per < bytes; ++i) {
+        GL3_HIP(hipEventSynchronize(p->log_ev[i % PF_LOG_SLOTS]));
+        memcpy((uint8_t*)out + i * per, p->h_log[i % PF_LOG_SLOTS], std::min(per, bytes - i * per));
+        if ((r = send(i + PF_LOG_SLOTS)) != GL3_OK) return r;
+    }
     return GL3_OK;
 }
 
@@ -2742,9 +2783,8 @@ int32_t gl3_prefill_run(gl3_ctx* ctx, int32_t seq, const int32_t* tokens, int32_
     for (int i = 0; i < n; ++i)
         if (tokens[i] < 0 || tokens[i] >= d.vocab) GL3_FAIL(GL3_E_ARG, "token id out of range");
     GL3_HIP(hipSetDevice(d.device));
-    std::vector<int32_t> seqs(n, seq), poss(n);
-    for (int i = 0; i < n; ++i) poss[i] = start_pos + i;
-    int32_t r = pf_stage_tokens(ctx, tokens, seqs.data(), poss.data(), n);
+    for (int i = 0; i < n; ++i) { p->h_io[i] = tokens[i]; p->h_io[p->max_batch + i] = seq; p->h_io[2 * p->max_batch + i] = start_pos + i; }
+    int32_t r = pf_stage_tokens(ctx, n);
     if (r != GL3_OK) return r;
     if ((r = pf_layers(ctx, n, start_pos + n - 1, seq)) != GL3_OK) return r;
     // keep the decode path's x in step with the last prefilled token (parity tap gl3_get_x)
@@ -2770,7 +2810,8 @@ int32_t gl3_decode_batch_run(gl3_ctx* ctx, const int32_t* tokens, const int32_t*
     }
     int max_pos = 0;
     for (int i = 0; i < n; ++i) max_pos = positions[i] > max_pos ? positions[i] : max_pos;
-    int32_t r = pf_stage_tokens(ctx, tokens, seq_ids, positions, n);
+    for (int i = 0; i < n; ++i) { p->h_io[i] = tokens[i]; p->h_io[p->max_batch + i] = seq_ids[i]; p->h_io[2 * p->max_batch + i] = positions[i]; }
+    int32_t r = pf_stage_tokens(ctx, n);
     if (r != GL3_OK) return r;
     hipStream_t s = ctx->stream;
     const int vl = ctx->vocab_l;
@@ -2810,14 +2851,17 @@ int32_t gl3_decode_batch_run(gl3_ctx* ctx, const int32_t* tokens, const int32_t*
         }
         GL3_HIP(hipGraphLaunch(p->step_graphs[n], s));
     } else if ((r = enqueue_step(max_pos)) != GL3_OK) return r;
-    if (argmax_out) GL3_HIP(hipMemcpyAsync(argmax_out, p->amax, (size_t)n * sizeof(int32_t), hipMemcpyDeviceToHost, s));
-    if (logits_out) {      // un-chunk on the way out: [tp][n][vl] -> [n][vocab]
+    if (argmax_out) GL3_HIP(hipMemcpyAsync(p->h_io + 3 * p->max_batch, p->amax, (size_t)n * sizeof(int32_t), hipMemcpyDeviceToHost, s));
+    if (logits_out && d.tp_size == 1 && pf_logits_slots(p)) {
+        if ((r = pf_logits_out(ctx, logits_out, (size_t)n * d.vocab * 4)) != GL3_OK) return r;
+    } else if (logits_out) {      // un-chunk on the way out: [tp][n][vl] -> [n][vocab]
         for (int c = 0; c < d.tp_size; ++c)
             GL3_HIP(hipMemcpy2DAsync(logits_out + (size_t)c * vl, (size_t)d.vocab * 4, p->LOGITS + (size_t)c * n * vl, (size_t)vl * 4, (size_t)vl * 4, n,
                                      hipMemcpyDeviceToHost, s));
     }
     GL3_HIP(hipGetLastError());
     GL3_HIP(hipStreamSynchronize(s));
+    if (argmax_out) memcpy(argmax_out, p->h_io + 3 * p->max_batch, (size_t)n * sizeof(int32_t));
     return gl3_tp_check(ctx);
 }
 

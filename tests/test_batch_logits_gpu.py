@@ -1,0 +1,30 @@
+"""Logits of a static-batched decode step on their way to the caller: in one pinned piece, in several, in more than are in flight at once, with a last
+piece of odd length, into memory that was never touched and into memory that was.  Every row is the single-sequence step's, bit for bit
+(position 0: a row depends on its token alone)."""
+import dataclasses
+
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("vocab,n", [(512, 1), (33008, 31), (33008, 32), (50000, 43), (70000, 64)])
+def test_every_row_arrives(vocab, n):
+    from importlib import import_module
+    import __graft_entry__ as ge
+    pkg = ge.load_package()
+    plans = import_module(ge.PKG_NAME + ".plan")
+    cfg = dataclasses.replace(pkg.synth.CONFIGS["tiny-llama"], vocab=vocab)
+    plan = plans.HipMasterPlan.initializeTornadoVMPlan(pkg.synth.make_numpy(cfg, seed=3), prefill_batch_size=64, n_seqs=64)
+    rng = np.random.default_rng(n)
+    for _ in range(2):
+        toks = rng.integers(0, vocab, n)
+        logits, ids = plan.forward_decode_batch(toks, np.arange(n), np.zeros(n))
+        only, ids2 = plan.forward_decode_batch(toks, np.arange(n), np.zeros(n), want_logits=False)
+        assert only is None and np.array_equal(ids, ids2)
+        for i in (range(n) if n < 5 else (0, 1, n // 3, n // 2, n - 2, n - 1)):
+            row = plan.forward_decode(int(toks[i]), 0)
+            assert np.array_equal(logits[i], row) and ids[i] == row.argmax(), i
+        assert np.array_equal(logits.argmax(axis=1), ids)
+    plan.freeTornadoExecutionPlan()
