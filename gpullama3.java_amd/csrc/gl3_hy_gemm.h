@@ -4,7 +4,8 @@
 // What bounds it.  A workgroup fills at most 160 KB of LDS, so at most that much can travel to a CU; behind HBM misses (1.3 - 1.7 us
 // under load) that is 60 - 75 GB/s per CU, while 256 x 256 results need 60 GB/s to keep the matrix cores busy and 128 x 128 twice that.  So:
 //   * operands go straight to LDS (global_load_lds, 16 bytes per lane: no staging registers, no store pass) into two rings, SA stages of A
-//     (re-read by every workgroup: L2 hits) and SW > SA stages of W (each row read once: HBM misses, hence the longer lead);
+//     (re-read by every workgroup: L2 hits, 0.4 us under load — a ring of two leaves it one stage's time, less than that in the small tiles) and SW > SA stages of
+//     W (each row read once: HBM misses, hence the longer lead);
 //   * the barrier of a stage sits a quarter of a stage before its end: the last quarter's MFMAs run behind it while the next stage's first
 //     fragments are read, and it waits with a counted vmcnt for everything but the loads that have a whole stage left to travel;
 //   * the loads are spread between the MFMAs (issued in one go they hold the wavefront for ~1000 cycles: the address unit takes 16 cycles each);
@@ -12,8 +13,8 @@
 //     (SQ_LDS_BANK_CONFLICT 0; with r % 8 half of the cycles were conflicts);
 //   * XCD-aware order: the row tiles of A that share a tile of W run on one XCD, so W leaves HBM once.
 // The tile is picked per shape (hy_ring_pick in gl3_hybrid.hip).  Measured against hy_gemm_kernel, 512 tokens, W cold in HBM (us):
-//   28672 x 4096 220 -> 126, 18560 x 4096 200 -> 83, 10240 x 4096 98 -> 50, 4096 x 4096 (K split in 2) 50 -> 24, 4096 x 14336 157 -> 65 - 75;
-//   24 tokens, 28672 x 4096: 89 -> 52 (4.5 TB/s of weights).
+//   28672 x 4096 220 -> 107 - 125, 18560 x 4096 200 -> 75 - 83, 10240 x 4096 98 -> 49, 4096 x 4096 50 -> 31 (K split in 2: 24), 4096 x 14336 157 -> 65 - 75;
+//   88 tokens, 4096 x 14336: 56; 24 tokens, 28672 x 4096: 89 -> 52 (4.5 TB/s of weights).
 // float32 matrices (v_mfma_f32_32x32x2_f32): a lane's 16-byte chunk holds 4 k of its row, so one read feeds four MFMAs (the half-wave's
 // chunks pair up; k enters in the order 0, 4, 1, 5, ...); the accumulators are added to a second set every HY_FLUSH stages (128 k), so that the
 // rounding of a long K grows with the number of blocks and not with K.

@@ -911,11 +911,10 @@ static HyGlu hy_ff_glu(const HyLayer& L) { return HyGlu{L.dense_limit, L.d.ff_al
 // Tiles of hy_gemm_ring_kernel: BM x BN results, WM x WN wavefronts, rings of SA / SW stages.
 enum { HY_R256x256, HY_R256x224, HY_R256x192, HY_R256x160, HY_R256x128, HY_R128x256, HY_R128x160, HY_R128x128, HY_R64x128, HY_R64x64, HY_R_COUNT };
 static const struct { int bm, bn; } HY_RING_TILES[HY_R_COUNT] = {{256, 256}, {256, 224}, {256, 192}, {256, 160}, {256, 128}, {128, 256}, {128, 160}, {128, 128}, {64, 128}, {64, 64}};
-// Which tile and K split: the one with the least estimated time.  A stage of a BM x BN tile takes a CU its operand bytes over the rate a full
-// LDS of loads sustains plus its MFMAs (0.0012 (BM + BN) + 0.0000235 BM BN us in bfloat16; float32 MFMAs are 16 x slower for half the K);
-// 256 CUs take the workgroups in rounds of whole tiles (two workgroups of a small tile share a CU; one alone needs 0.4 us per stage for its loads'
-// way: 88 tokens, 4096 x 4096 in 64 x 64 tiles 16 us as 256 workgroups, 11 us as 512) — what decides for most shapes: 10240 x 4096 at 512 tokens is 256 tiles of 128 x 160
-// (50 us) but 320 of 128 x 128 (65 us) or 160 of 256 x 128 (53 us).  A K split writes and re-reads its part of C at ~4 TB/s.
+// Which tile and K split: the one with the least estimated time.  A stage of a BM x BN tile takes a CU 0.00154 (BM + BN) us for its operand bytes (83 GB/s per CU,
+// what the loads of all 256 sustain) + 0.0000128 BM BN us that its MFMAs add (fits 64 x 64 ... 256 x 256 within 8 %; float32 MFMAs are 16 x slower for half the
+// K); 256 CUs take the workgroups in rounds of whole tiles (two workgroups of a small tile share a CU, and its loads) — what decides for most shapes: 10240 x 4096 at
+// 512 tokens is 256 tiles of 128 x 160 (49 us) but 320 of 128 x 128 (65 us) or 160 of 256 x 128 (53 us).  A K split writes and re-reads its part of C at ~4 TB/s.
 static double hy_ring_pick(bool f32, int M, int N, int K, bool glu, bool actmul, int max_parts, int* tile, int* ks_out) {
     const int stages = K / (f32 ? 32 : 64);
     double best = 1e30;
@@ -924,13 +923,13 @@ static double hy_ring_pick(bool f32, int M, int N, int K, bool glu, bool actmul,
         if (glu ? (t != HY_R256x256 && t != HY_R128x256 && t != HY_R128x128 && t != HY_R64x128) : t == HY_R256x256) continue;
         if (actmul && t != HY_R256x224 && t != HY_R128x128 && t != HY_R64x64) continue;
         if (f32 && (t < HY_R256x128 || t == HY_R128x256)) continue;          // (two sets of accumulators)
-        const double stage = 0.0012 * (bm + bn) + (f32 ? 0.000105 : 0.0000235) * bm * bn;
+        const double stage = 0.00154 * (bm + bn) + (f32 ? 0.000105 : 0.0000128) * bm * bn;
         const long mn = (long)hy_cdiv(M, bm) * hy_cdiv(N, bn), pair = t >= HY_R128x128 ? 2 : 1;
         for (int ks = 1; ks <= max_parts && (ks == 1 || stages / ks >= 4); ++ks) {
             const int per = hy_cdiv(stages, ks);
             if (hy_cdiv(stages, per) != ks) continue;
             const long wgs = mn * ks, rest = wgs % (256 * pair);
-            const double rounds = (double)(wgs / (256 * pair)) * pair * (per * stage + 3.0), last = rest == 0 ? 0.0 : rest <= 256 ? per * std::max(stage, 0.4) + 3.0 : 2 * (per * stage + 3.0);
+            const double rounds = (double)(wgs / (256 * pair)) * pair * (per * stage + 3.0), last = rest == 0 ? 0.0 : (rest <= 256 ? 1 : 2) * (per * stage + 3.0);
             const double us = rounds + last + (ks - 1) * (double)M * N * 8 / 4e6;
             if (us < best) { best = us; *tile = t; *ks_out = ks; }
         }
@@ -954,24 +953,32 @@ static bool hy_gemm_ring(gl3_ctx* ctx, const T* A, int lda, const HyMat& w, int 
 #define HY_RG(BM, BN, WM, WN, SA, SW, EPI)                                                                                                              \
     hipLaunchKernelGGL((hy_gemm_ring_kernel<T, BM, BN, WM, WN, SA, SW, EPI>), grid, dim3(WM * WN * 64), 0, ctx->stream, A, lda, (const T*)w.w, w.ld, M, N, K, C, ldc, act, \
                        ld_act, gp, mt, nt, ks, kper)
+    // The rings: A has to be on its way for more than one stage as well (L2's answer takes 0.4 us; 64 x 64 with a ring of 2 + 6 took that long per stage and 0.25 with
+    // 4 + 5: 88 tokens, 4096 x 14336 90 -> 56 us; 512 tokens, 2048 x 8192 51 -> 37).  What two workgroups of a CU cannot have one alone takes (64 x 128: 4096 x 4096 at 512
+    // tokens 35 -> 31 us; 128 x 128: 6144 x 4096 41 -> 39).
+    const bool lone = mt * nt * ks <= 256;
     if constexpr (sizeof(T) == 2) {          // tiles of the bfloat16 plans only
-        if (tile == HY_R256x256) { HY_RG(256, 256, 8, 1, 2, 3, HY_EPI_GLU); return true; }
+        if (tile == HY_R256x256) { HY_RG(256, 256, 4, 2, 2, 3, HY_EPI_GLU); return true; }
         if (tile == HY_R128x256) { if (glu) HY_RG(128, 256, 4, 2, 2, 3, HY_EPI_GLU); else HY_RG(128, 256, 4, 2, 2, 3, HY_EPI_STORE); return true; }
         if (tile == HY_R256x224) { if (actmul) HY_RG(256, 224, 8, 1, 2, 3, HY_EPI_ACTMUL); else HY_RG(256, 224, 8, 1, 2, 3, HY_EPI_STORE); return true; }
         if (tile == HY_R256x192) { HY_RG(256, 192, 4, 2, 2, 4, HY_EPI_STORE); return true; }
         if (tile == HY_R256x160) { HY_RG(256, 160, 8, 1, 2, 4, HY_EPI_STORE); return true; }
     }
+#define HY_RG_64x128(EPI) do { if (lone) HY_RG(64, 128, 2, 2, 3, 4, EPI); else HY_RG(64, 128, 2, 2, 2, 4, EPI); } while (0)
+#define HY_RG_128x128(EPI) do { if (lone) HY_RG(128, 128, 4, 2, 3, 4, EPI); else HY_RG(128, 128, 4, 2, 2, 3, EPI); } while (0)
     if (glu) {
-        if (tile == HY_R64x128) HY_RG(64, 128, 2, 2, 2, 4, HY_EPI_GLU); else HY_RG(128, 128, 4, 2, 2, 3, HY_EPI_GLU);
+        if (tile == HY_R64x128) HY_RG_64x128(HY_EPI_GLU); else HY_RG_128x128(HY_EPI_GLU);
     } else if (actmul) {
-        if (tile == HY_R64x64) HY_RG(64, 64, 2, 2, 2, 6, HY_EPI_ACTMUL); else HY_RG(128, 128, 4, 2, 2, 3, HY_EPI_ACTMUL);
+        if (tile == HY_R64x64) HY_RG(64, 64, 2, 2, 4, 5, HY_EPI_ACTMUL); else HY_RG_128x128(HY_EPI_ACTMUL);
     } else switch (tile) {
         case HY_R256x128: HY_RG(256, 128, 4, 2, 3, 4, HY_EPI_STORE); break;
         case HY_R128x160: HY_RG(128, 160, 4, 1, 3, 5, HY_EPI_STORE); break;
-        case HY_R64x128: HY_RG(64, 128, 2, 2, 2, 4, HY_EPI_STORE); break;
-        case HY_R64x64: HY_RG(64, 64, 2, 2, 2, 6, HY_EPI_STORE); break;
-        default: HY_RG(128, 128, 4, 2, 2, 3, HY_EPI_STORE);
+        case HY_R64x128: HY_RG_64x128(HY_EPI_STORE); break;
+        case HY_R64x64: HY_RG(64, 64, 2, 2, 4, 5, HY_EPI_STORE); break;
+        default: HY_RG_128x128(HY_EPI_STORE);
     }
+#undef HY_RG_64x128
+#undef HY_RG_128x128
 #undef HY_RG
     return true;
 }
@@ -1512,7 +1519,7 @@ static void hy_gemm_grouped(gl3_ctx* ctx, const T* A, int lda, const HyMat& w, s
     const dim3 grid(hy_cdiv(N, 128), max_tiles, 1);
     constexpr int PE = 16 / (int)sizeof(T), BK = 128 / (int)sizeof(T);
     if (K % BK == 0 && lda % PE == 0 && w.ld % PE == 0 && wstride % PE == 0 && (((uintptr_t)A | (uintptr_t)Wt) & 15) == 0 && (uint64_t)N * w.ld * sizeof(T) < 0xffff0000ull) {
-#define HY_RGG(BM, WM, EPI) hipLaunchKernelGGL((hy_gemm_ring_kernel<T, BM, 128, WM, 2, 2, 4, EPI, 1>), grid, dim3(WM * 128), 0, st, A, lda, Wt, w.ld, 0, N, K, C, ldc, act, ld_act, gp, 0, 0, 1, K, grp)
+#define HY_RGG(BM, WM, EPI) hipLaunchKernelGGL((hy_gemm_ring_kernel<T, BM, 128, WM, 2, BM == 32 ? 3 : 2, 4, EPI, 1>), grid, dim3(WM * 128), 0, st, A, lda, Wt, w.ld, 0, N, K, C, ldc, act, ld_act, gp, 0, 0, 1, K, grp)
 #define HY_RGG_EPI(BM, WM) do { if (glu) HY_RGG(BM, WM, HY_EPI_GLU); else if (gp.act == 2) HY_RGG(BM, WM, HY_EPI_ACTMUL); else HY_RGG(BM, WM, HY_EPI_STORE); } while (0)
         if (bm == HY_MOE_BM_FEW) HY_RGG_EPI(HY_MOE_BM_FEW, 1); else HY_RGG_EPI(HY_MOE_BM, 2);
 #undef HY_RGG_EPI
