@@ -770,7 +770,7 @@ int32_t gl3_create(const gl3_model_desc* desc, gl3_ctx** out) {
     TRYHIP(hipMemset(ctx->argmax, 0, (2 + 2 * AMX_WGS) * sizeof(int)));
     if (d.flags & GL3_FLAG_LAYER_TAPS) TRY(dmalloc(ctx, &ctx->taps, (size_t)d.n_layers * d.dim));
     TRYHIP(hipHostMalloc((void**)&ctx->h_dyn, 4 * sizeof(int)));
-    TRYHIP(hipHostMalloc((void**)&ctx->h_logits, (size_t)d.vocab * 4));
+    TRYHIP(hipHostMalloc((void**)&ctx->h_logits, ((size_t)d.vocab + 4 * (size_t)(d.max_batch > 1 ? d.max_batch : 0)) * 4));      // + the batched steps' inputs and ids (gl3_prefill.hip: h_io)
     TRYHIP(hipHostMalloc((void**)&ctx->h_argmax, sizeof(int)));
     // batched prefill / static-batched decode: int8 MFMA GEMMs for Q8_0 (any tensor-parallel degree); f32-MFMA / VALU GEMMs in the
     // Vector-API order for F16, Q4_0 and Q8_0 with the f32 activation (gl3_prefill_vl.h).  The scalar dot order
@@ -1082,7 +1082,6 @@ int32_t gl3_forward_decode(gl3_ctx* ctx, int32_t token, int32_t pos, float* logi
         for (const auto& pr : ctx->pinned)
             if ((uint8_t*)logits_out >= (uint8_t*)pr.first && (uint8_t*)logits_out + (size_t)ctx->d.vocab * 4 <= (uint8_t*)pr.first + pr.second) direct = true;
     if (logits_out) GL3_HIP(hipMemcpyAsync(direct ? logits_out : ctx->h_logits, ctx->logits, (size_t)ctx->d.vocab * 4, hipMemcpyDeviceToHost, ctx->stream));
-    if (logits_out && !direct) gl3_touch_pages(logits_out, (size_t)ctx->d.vocab * 4);
     GL3_HIP(hipStreamSynchronize(ctx->stream));
     if ((r = gl3_tp_check(ctx)) != GL3_OK) return r;
     if (logits_out && !direct) memcpy(logits_out, ctx->h_logits, (size_t)ctx->d.vocab * 4);

@@ -251,14 +251,6 @@ int32_t gl3_sample_run(gl3_ctx* ctx, const float* logits_dev, float temperature,
 int32_t gl3_sample_probs(gl3_ctx* ctx, float* out);
 void gl3_sample_free(gl3_ctx* ctx);
 
-// Result memory the caller has just got from the system has no pages yet, and taking them one fault at a time costs more than the copy that follows
-// (2 MB: 430 us, 30 with pages).  The pages are touched while the device still works on the step.
-static inline void gl3_touch_pages(void* mem, size_t bytes) {
-    volatile uint8_t* q = (volatile uint8_t*)mem;
-    for (size_t i = 0; i < bytes; i += 4096) q[i] = q[i];
-    if (bytes) q[bytes - 1] = q[bytes - 1];
-}
-
 // gl3_prefill.hip
 float* gl3_prefill_buf(gl3_ctx* ctx, int which);
 int32_t gl3_prefill_alloc(gl3_ctx* ctx);

@@ -1801,7 +1801,6 @@ int32_t gl3_hy_step(gl3_ctx* ctx, int32_t seq, const int32_t* tokens, int32_t n,
             if (r != GL3_OK) return r;
             h->last_tok[seq] = tokens[off + pn - 1];
             if (g > 0 && logits_out) HY_HIP(hipMemcpyAsync(h->h_logits, h->logits, (size_t)g * V * 4, hipMemcpyDeviceToHost, ctx->stream));
-            if (g > 0 && logits_out) gl3_touch_pages(logits_out + (size_t)done * V, (size_t)g * V * 4);
             HY_HIP(hipStreamSynchronize(ctx->stream));
             if (g > 0 && logits_out) memcpy(logits_out + (size_t)done * V, h->h_logits, (size_t)g * V * 4);
             done += g;

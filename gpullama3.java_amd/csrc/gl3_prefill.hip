@@ -55,7 +55,7 @@ struct gl3_prefill_state {
     float* SUMS = nullptr;              // [M][n_heads] softmax denominators (pf_softmax_rows_kernel -> pf_pv_tiled_kernel)
     int tmx_tiles = 0;
     int32_t* seqpos = nullptr;          // [2][M] behind tokens: sequence id, position of every token of the step
-    int32_t* h_io = nullptr;            // pinned [4][M]: tokens, sequence ids, positions of the step on their way in, greedy ids on their way out
+    int32_t* h_io = nullptr;            // pinned [4][M], behind ctx->h_logits: tokens, sequence ids, positions of the step on their way in, greedy ids on their way out
     uint8_t* h_log[PF_LOG_SLOTS] = {};  // pinned pieces of logits on their way to the caller (static-batched decode), made at its first use
     hipEvent_t log_ev[PF_LOG_SLOTS] = {};
     float* LOGITS = nullptr;            // [rows][vocab], grown on demand (batched decode)
@@ -2194,7 +2194,7 @@ int32_t gl3_prefill_alloc(gl3_ctx* ctx) {
     if (p->vl) {       // f32-activation weight types: f32 buffers; the gathered ones (X, AO, HB, LOGITS) in the arena under tensor parallelism
         GL3_HIP(hipMalloc((void**)&p->tokens, 3 * M * sizeof(int32_t)));
         p->seqpos = p->tokens + M;
-        GL3_HIP(hipHostMalloc((void**)&p->h_io, 4 * M * sizeof(int32_t)));
+        p->h_io = (int32_t*)(ctx->h_logits + d.vocab);
         if (ctx->arena.base && ctx->arena.off[GB_PF_X]) {
             uint8_t* b = ctx->arena.base;
             p->X = (float*)(b + ctx->arena.off[GB_PF_X]); p->AO = (float*)(b + ctx->arena.off[GB_PF_AO]); p->HB = (float*)(b + ctx->arena.off[GB_PF_HB]);
@@ -2240,7 +2240,7 @@ int32_t gl3_prefill_alloc(gl3_ctx* ctx) {
     p->maxk = (p->maxk + 127) & ~127;
     GL3_HIP(hipMalloc((void**)&p->tokens, 3 * M * sizeof(int32_t)));
     p->seqpos = p->tokens + M;
-    GL3_HIP(hipHostMalloc((void**)&p->h_io, 4 * M * sizeof(int32_t)));
+    p->h_io = (int32_t*)(ctx->h_logits + d.vocab);
     if (ctx->arena.base && ctx->arena.off[GB_PF_X]) {      // tensor parallel: the gathered activations live in the arena the peers map
         uint8_t* b = ctx->arena.base;
         p->X = (float*)(b + ctx->arena.off[GB_PF_X]); p->AO = (float*)(b + ctx->arena.off[GB_PF_AO]); p->HB = (float*)(b + ctx->arena.off[GB_PF_HB]);
@@ -2308,7 +2308,6 @@ void gl3_prefill_free(gl3_ctx* ctx) {
     auto f = [](void* q) { if (q) hipFree(q); };
     f(p->tokens); f(p->XQ); f(p->XS); f(p->XP); f(p->XQh); f(p->XPh); f(p->XQb); f(p->XSb); f(p->QKV); f(p->ATT); f(p->TMX); f(p->SUMS); f(p->amax); f(p->amx_v); f(p->amx_i); f(p->XN); f(p->HB2);
     if (!p->in_arena) { f(p->X); f(p->AO); f(p->HB); f(p->LOGITS); }
-    if (p->h_io) hipHostFree(p->h_io);
     for (auto q : p->h_log) if (q) hipHostFree(q);
     for (auto e : p->log_ev) if (e) hipEventDestroy(e);
     delete p;
@@ -2747,6 +2746,13 @@ static int32_t pf_stage_tokens(gl3_ctx* ctx, int n) {
     return GL3_OK;
 }
 
+// Result memory the caller has just got from the system has no pages yet, and taking them one fault at a time costs more than the copy that follows
+// (2 MB: 430 us, 30 with pages).  The pages are touched while the device still works on the step.
+static inline void pf_touch_pages(void* mem, size_t bytes) {
+    volatile uint8_t* q = (volatile uint8_t*)mem;
+    for (size_t i = 0; i < bytes; i += 4096) q[i] = q[i];
+    if (bytes) q[bytes - 1] = q[bytes - 1];
+}
 // n rows of logits to the caller: through pinned pieces of at most PF_LOG_PIECE bytes, a piece on its way while the one before it is copied on.  (A copy to
 // pageable memory goes row by row through the runtime's own staging: 32 rows x 16896 570 - 740 us, this way 45 on the link + 30 - 70 on the host; x 151936
 // 1041 and 767.)  False: no pinned memory for the pieces.
@@ -2768,7 +2774,7 @@ static int32_t pf_logits_out(gl3_ctx* ctx, float* out, size_t bytes) {
     };
     int32_t r;
     for (size_t i = 0; i < PF_LOG_SLOTS; ++i) if ((r = send(i)) != GL3_OK) return r;
-    gl3_touch_pages(out, bytes);
+    pf_touch_pages(out, bytes);
     for (size_t i = 0; i * per < bytes; ++i) {
         GL3_HIP(hipEventSynchronize(p->log_ev[i % PF_LOG_SLOTS]));
         memcpy((uint8_t*)out + i * per, p->h_log[i % PF_LOG_SLOTS], std::min(per, bytes - i * per));
