@@ -49,6 +49,7 @@ static __global__ __launch_bounds__(256) void hy_scan_prep_kernel(float* __restr
 template <int NT, int PC>          // N = 64 NT states per column, PC value columns
 static __global__ __launch_bounds__(256, 2) void hy_scan_chunk_kernel(HyScanArgs a) {
     constexpr int C = 32, N = 64 * NT, QS = N + 4, XS = PC + 4, JC = PC / 16, NV = C * N / 4 / 256, XV = C * PC / 256;
+    static_assert(4 * C * PC <= C * QS, "the shares of y end where the query rows do: x and the masked product behind them are still read while the shares are written");
     extern __shared__ __attribute__((aligned(16))) float smem[];
     float* sK = smem;                    // [C][QS]
     float* sQ = sK + C * QS;             // [C][QS]

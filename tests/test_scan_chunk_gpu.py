@@ -1,6 +1,7 @@
 """The recurrences 32 tokens at a time (csrc/gl3_hy_scan_chunk.h): every kind that takes them (state-space layers, exponential gates with their
 normaliser column, retention with turned keys, a fixed decay behind silu) at the key sizes 64 / 128 / 256, value columns that do not fill a column
-block, portions whose last chunk is full, holds one token or is cut behind an earlier portion, decays near one and decays that underflow.
+block, portions whose last chunk is full, holds one token or is cut behind an earlier portion, decays near one and decays that underflow; the same kinds with
+so many heads or values that there are more than 256 blocks of 16 value columns (128 and 256 states then go 32 columns at a time, 64 stay with 16).
 
 Yardstick: the designs' float64 restatements, which walk token by token.  Bound: float32 products and sums of a few hundred terms err by some
 1e-6 of the logits' root mean square (heads are normed to size one behind the memory); a lost token or a wrong decay is an error of order one."""
@@ -52,6 +53,38 @@ def test_chunks_and_portions(hy, tmp_path, name, n, batch):
     s = p.acquire()
     got = [p.step(s, toks[:n], 0, list(range(n)))]
     for i in range(3):                        # the state goes on token by token
+        got.append(p.step(s, toks[n + i:n + i + 1], n + i, [0]))
+    p.close()
+    got, want = np.concatenate(got), m.ref(toks)
+    assert N.err(got, want) < 3e-5, N.err(got, want)
+
+
+SLOW = [1.0 - 2.0 ** (-1.0 - 0.4 * i) for i in range(24)]
+
+
+# more than 256 blocks of 16 value columns; 56, 72, 209 (208 and the normaliser) and 170 columns leave 24, 8, 17 and 10 in the last block of 32
+WIDE = {
+    "ssm64": (N, N.ssm(heads=64, vdim=80, state=64, groups=4, norm_groups=4)), "ssm128": (N, N.ssm(heads=70, vdim=56, state=128, groups=2, norm_groups=2)),
+    "ssm256": (N, N.ssm(heads=52, vdim=72, state=256)),
+    "mlstm64": (K, K.mls(heads=32, dim=64, vdim=128, ff=0)), "mlstm256": (K, K.mls(heads=20, dim=256, vdim=208, ff=0)),
+    "retention64": (K, K.par(right=K.ret(heads=24, dim=64, vdim=170, rot_dims=24, decay=SLOW), ff=0)), "lightning64": (U, U.lig(heads=24, dim=64, vdim=170, decay=SLOW, mlp=None)),
+    "lightning128": (U, U.lig(heads=24, dim=128, vdim=170, decay=SLOW, mlp=None)),
+}
+
+
+@pytest.mark.parametrize("n,batch", [(17, 64), (33, 64), (65, 128), (130, 97)])
+@pytest.mark.parametrize("name", list(WIDE))
+def test_many_column_blocks(hy, tmp_path, name, n, batch):
+    mod, layer = WIDE[name]
+    mix = layer["mixer"].get("right") or layer["mixer"]
+    assert mix["heads"] * ((mix["vdim"] + (layer["type"] == "mlstm") + 15) // 16) > 256
+    cfg = mod.config([layer])
+    m = mod.Model(hy, tmp_path, cfg, n)
+    toks = np.random.default_rng(n).integers(0, cfg["vocab"], n + 2).astype(np.int32)
+    p = m.plan("float32", ctx=n + 8, max_batch=batch)
+    s = p.acquire()
+    got = [p.step(s, toks[:n], 0, list(range(n)))]
+    for i in range(2):
         got.append(p.step(s, toks[n + i:n + i + 1], n + i, [0]))
     p.close()
     got, want = np.concatenate(got), m.ref(toks)
