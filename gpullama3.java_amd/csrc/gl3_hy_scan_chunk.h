@@ -10,6 +10,8 @@
 // register r of a lane is row 4 (lane / 16) + r of its tile, they are the second operand of Q S as they stand.  Per chunk: q . k in three 16 x 16
 // tiles by wavefronts 0 - 2 while the fourth makes L; then every wavefront adds its rows' share of Q S and its eight tokens' share of the masked
 // product to y (joined in LDS) and updates its rows.  The next chunk's rows travel in registers meanwhile.
+// A token whose x is not finite must not reach the tokens in front of it, and a product with its zero place in the masked matrix would carry it there:
+// the matrix cores take zero in its stead, and a chunk that holds one (looked for on the way into LDS) adds its products entry by entry as y is written.
 // Keys and queries come finished (hy_scan_prep_kernel); x passes through silu on the way into LDS where the layer asks for it (act & 4).
 // Measured for 512 tokens (us), hy_ssm_scan_kernel -> this: 128 heads x (128 x 64) 278 -> 73, 16 x (128 x 256) 310 -> 52, 8 x (256 x 513) 430 -> 97.
 #pragma once
@@ -57,6 +59,7 @@ static __global__ __launch_bounds__(256, 2) void hy_scan_chunk_kernel(HyScanArgs
     float* sM = sX + C * XS;             // [C][36] masked, weighted q . k
     float* sL = sM + C * 36;             // [C][33]
     float* sA = sL + C * 33;             // [C] a, [C] b
+    int* sF = (int*)(sA + 2 * C);        // [4] whether a wavefront staged an x that is not finite
     float* sY = sQ;                      // [4][C][PC] the wavefronts' shares of y, when the query rows have been read
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), l16 = lane & 15, g = lane >> 4;
     const int P = a.P, n = a.n, Px = P - (a.ones_col ? 1 : 0), head = blockIdx.y, col0 = blockIdx.x * PC, gr = head / (a.heads / a.G);
@@ -111,13 +114,17 @@ static __global__ __launch_bounds__(256, 2) void hy_scan_chunk_kernel(HyScanArgs
             *reinterpret_cast<hy_acc4*>(sQ + t * QS + c) = qv;
         }
         float xs[XV];
+        bool odd = false;
 #pragma unroll
         for (int u = 0; u < XV; ++u) {
             const int i = tid + u * 256, p = col0 + i % PC;
             const float x = (a.act & 4) ? hy_silu(rx[u]) : rx[u];
             xs[u] = t0 + i / PC >= n ? 0.f : p < Px ? x : p < P ? 1.f : 0.f;
             sX[(i / PC) * XS + i % PC] = xs[u];
+            odd |= !(fabsf(xs[u]) < INFINITY);
         }
+        const bool wodd = __any(odd);
+        if (lane == 0) sF[wave] = wodd;
         if (tid < C) {
             float av = 1.f, bv = 0.f;
             if (t0 + tid < n) {
@@ -158,11 +165,12 @@ static __global__ __launch_bounds__(256, 2) void hy_scan_chunk_kernel(HyScanArgs
 #pragma unroll
             for (int r = 0; r < 4; ++r) {
                 const int t = tt + 4 * g + r;
-                sM[t * 36 + ss + l16] = (g0[r] + g1[r]) * (sL[t * 33 + ss + l16] * bs);
+                sM[t * 36 + ss + l16] = t >= ss + l16 ? (g0[r] + g1[r]) * (sL[t * 33 + ss + l16] * bs) : 0.f;          // (chosen: a later key may be infinite)
             }
         }
         hy_acc4 y[2][JC];
         const float a0 = sA[0];
+        const int entries = __builtin_amdgcn_readfirstlane((sF[0] | sF[1]) | (sF[2] | sF[3]));
 #pragma unroll
         for (int u = 0; u < 2; ++u) {
 #pragma unroll
@@ -192,7 +200,8 @@ static __global__ __launch_bounds__(256, 2) void hy_scan_chunk_kernel(HyScanArgs
             const float m0 = sM[l16 * 36 + s], m1 = sM[(16 + l16) * 36 + s];
 #pragma unroll
             for (int j = 0; j < JC; ++j) {
-                const float x = sX[s * XS + 16 * j + l16];
+                float x = sX[s * XS + 16 * j + l16];
+                x = fabsf(x) < INFINITY ? x : 0.f;
                 y[0][j] = hy_mma4(m0, x, y[0][j]);
                 y[1][j] = hy_mma4(m1, x, y[1][j]);
             }
@@ -225,11 +234,26 @@ static __global__ __launch_bounds__(256, 2) void hy_scan_chunk_kernel(HyScanArgs
 #pragma unroll
                 for (int r = 0; r < 4; ++r) sY[(wave * C + 16 * u + 4 * g + r) * PC + 16 * j + l16] = y[u][j][r];
         hy_lds_barrier();
+        float v[XV];
+#pragma unroll
+        for (int u = 0; u < XV; ++u) {
+            const int i = tid + u * 256;
+            v[u] = (sY[i] + sY[C * PC + i]) + (sY[2 * C * PC + i] + sY[3 * C * PC + i]);
+        }
+        if (entries)
+#pragma unroll
+            for (int u = 0; u < XV; ++u) {
+                const int t = (tid + u * 256) / PC, c = (tid + u * 256) % PC;
+#pragma unroll 1
+                for (int s = 0; s <= t; ++s) {
+                    const float x = sX[s * XS + c];
+                    if (!(fabsf(x) < INFINITY)) v[u] = fmaf(sM[t * 36 + s], x, v[u]);
+                }
+            }
 #pragma unroll
         for (int u = 0; u < XV; ++u) {
             const int i = tid + u * 256, t = t0 + i / PC, p = col0 + i % PC;
-            const float v = (sY[i] + sY[C * PC + i]) + (sY[2 * C * PC + i] + sY[3 * C * PC + i]);
-            if (t < n && p < P) a.y[(size_t)t * a.ldy + head * P + p] = fmaf(dd, xs[u], v);
+            if (t < n && p < P) a.y[(size_t)t * a.ldy + head * P + p] = fmaf(dd, xs[u], v[u]);
         }
         hy_lds_barrier();
     }

@@ -1217,7 +1217,7 @@ static void hy_scan_chunk_launch(gl3_ctx* ctx, const HyScanArgs& a) {
     // with 16 and 61 with 32, 8 x 513 (264 or 136 workgroups) 112 and 96, 128 x 64 (512 or 256) 80 and 71.  64 states: always 16 (four layers of 64 heads x 80, 96 x 64,
     // 128 x 64, 32 x 129, 32 x 257, whole steps of 33 - 512 tokens: 32 columns take 0 - 6 % longer, with LDS of their own for the shares of y)
     const int pc = a.N == 64 || (long)a.heads * hy_cdiv(a.P, 16) <= 256 ? 16 : 32;
-    const size_t smem = (size_t)(2 * 32 * (a.N + 4) + 32 * (pc + 4) + 32 * 36 + 32 * 33 + 64) * 4;
+    const size_t smem = (size_t)(2 * 32 * (a.N + 4) + 32 * (pc + 4) + 32 * 36 + 32 * 33 + 68) * 4;
     const dim3 grid(hy_cdiv(a.P, pc), a.heads);
 #define HY_SC(NT, PC) hipLaunchKernelGGL((hy_scan_chunk_kernel<NT, PC>), grid, dim3(256), smem, ctx->stream, a)
     if (a.N == 64) HY_SC(1, 16);

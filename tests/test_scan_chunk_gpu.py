@@ -89,3 +89,24 @@ def test_many_column_blocks(hy, tmp_path, name, n, batch):
     p.close()
     got, want = np.concatenate(got), m.ref(toks)
     assert N.err(got, want) < 3e-5, N.err(got, want)
+
+
+@pytest.mark.parametrize("bad", [5, 40, 79])
+@pytest.mark.parametrize("name", ["ssm128", "ssm64_odd_columns", "mlstm64", "mlstm256", "lightning64", "lightning128"])
+def test_a_token_that_is_not_finite(hy, tmp_path, name, bad):
+    """It is its own row's and the later ones' concern: the rows in front of it are the restatement's of the tokens in front of it."""
+    mod, layer, _ = LAYERS[name]
+    cfg = mod.config([layer])
+    odd = cfg["vocab"] - 1
+
+    def tweak(*a):
+        a[-1]["embed"][odd] = np.nan
+    m = mod.Model(hy, tmp_path, cfg, bad, tweak)
+    toks = np.random.default_rng(bad).integers(0, odd, 80).astype(np.int32)
+    toks[bad] = odd
+    p = m.plan("float32", ctx=88, max_batch=128)
+    got = p.step(p.acquire(), toks, 0, list(range(80)))[:, :odd]          # (a tied head has a column of the odd token)
+    p.close()
+    want = m.ref(toks[:bad])[:, :odd]
+    assert N.err(got[:bad], want) < 3e-5
+    assert np.isnan(got[bad:]).all()
