@@ -11,6 +11,10 @@
 // + e is step e of chunk c) and DVT consecutive value columns of the keys r (value column DVT m + i is row m of tile i); the values travel under the first product
 // and the softmax, the next tile's keys under the second half of the second product (all at once do not fit 256 registers, and a second wavefront
 // per SIMD is what keeps the matrix cores busy during the softmax).  Queries (scaled) stay in LDS, rows dk + 4 floats apart.
+// A value that is not finite must stay with the rows that see its key, and the second product carries it to every row of the tile (p = 0 times infinity).  Nothing in the
+// loops below looks for one (values cleaned in the tiles with unseen keys cost 1 and 5 % of the two kernels, right in front of every MFMA 6 - 12 %): sums that hold a
+// not-a-number at the end are made once more, key by key on the vector units (hy_attn_again), which costs other inputs the look at the sums: 0.5 % and 1 - 3 %.  It
+// stands behind the last exchange in LDS, which the loop's last MFMAs run under.
 // Bound: 153 TFLOP/s of float32 MFMAs.  Measured against hy_attn_kernel (8 key / value heads x 4, head size 128, us):
 //   512 tokens at position 0 131 -> 45, four such portions of 2041 tokens 1795 -> 428 in all.
 #pragma once
@@ -20,6 +24,49 @@ typedef float hy_acc4 __attribute__((ext_vector_type(4)));
 template <int DVT> struct HyVec;
 template <> struct HyVec<2> { typedef float2 V; };
 template <> struct HyVec<4> { typedef float4 V; };
+
+// The weighted sums of a lane's row over the keys it sees, vt0, vt0 + step ... of the tile list (key(vt): first key, last one, pooled or not): register r of tile i is
+// value column DVT (8 (r / 4) + 4 (lane / 32) + r % 4) + i behind col0.  q: the row's query; m: its maximum.
+template <int DVT> __device__ __forceinline__ bool hy_attn_nan(const hy_v16f* o) {
+    bool nan = false;
+#pragma unroll
+    for (int i = 0; i < DVT; ++i)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) nan |= o[i][r] != o[i][r];
+    return nan;
+}
+template <int DK, int DVT, typename Key>
+__device__ __forceinline__ void hy_attn_again(hy_v16f* o, const HyAttnArgs& a, const float* q, float scale, float m, float slope, int pr, int nbr, int win, const float* kc, const float* vc,
+                                              const float* pkc, const float* pvc, int col0, int kh, int vt0, int step, int nv, Key key) {
+#pragma unroll
+    for (int i = 0; i < DVT; ++i)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) o[i][r] = 0.f;
+    const int ldk = a.G * DK, ldv = a.G * a.dv;
+#pragma unroll 1
+    for (int vt = vt0; vt < nv; vt += step) {
+        int j, last;
+        bool pooled;
+        key(vt, j, last, pooled);
+        last = min(j + 31, last);
+#pragma unroll 1
+        for (; j <= last; ++j) {
+            if (!(pooled ? j < nbr : (j <= pr && (pr - j < win || j < a.keep)))) continue;
+            const float *k = (pooled ? pkc : kc) + (size_t)j * ldk, *v = (pooled ? pvc : vc) + (size_t)j * ldv + col0 + DVT * 4 * kh;
+            float s = 0.f;
+#pragma unroll 4
+            for (int d = 0; d < DK; ++d) s = fmaf(k[d], q[d], s);
+            s *= scale;
+            const float p = expf((pooled ? s : s - slope * (float)(pr - j)) - m);
+#pragma unroll
+            for (int r = 0; r < 16; ++r) {
+#pragma unroll
+                for (int i = 0; i < DVT; ++i) o[i][r] = fmaf(p, v[DVT * (8 * (r >> 2) + (r & 3)) + i], o[i][r]);
+                __builtin_amdgcn_sched_barrier(0);          // (rarely run: a few loads at a time rather than registers for sixty-four)
+            }
+        }
+    }
+}
 
 template <int DKC, int DVT>          // dk = 8 DKC, dv = 32 DVT
 static __global__ __launch_bounds__(256, DKC > 16 ? 1 : 2) void hy_attn_mfma_kernel(HyAttnArgs a) {
@@ -144,6 +191,9 @@ static __global__ __launch_bounds__(256, DKC > 16 ? 1 : 2) void hy_attn_mfma_ker
     __syncthreads();
     const float M = fmaxf(fmaxf(sml[0][0][r32], sml[1][0][r32]), fmaxf(sml[2][0][r32], sml[3][0][r32]));
     const float sc = m > -INFINITY ? expf(m - M) : 0.f;
+    if (__any(hy_attn_nan<DVT>(o) && pr >= 0))
+        hy_attn_again<DK, DVT>(o, a, sQ + r32 * QS, 1.f, m, slope, pr, nbr, win, kc, vc, pkc, pvc, 0, kh, split * 4 + wave, 4 * a.nsplit, nv,
+                               [&](int t, int& j, int& last, bool& pooled) { pooled = t < np_t; j = first_key(t); last = pooled ? nb_wg - 1 : maxpos; });
     for (int w = 0; w < 4; ++w) {
         if (wave == w) {
 #pragma unroll
@@ -296,8 +346,16 @@ static __global__ __launch_bounds__(64 * NW, 1) void hy_attn_few_kernel(HyAttnAr
     if (wave == 0 && kh == 0) { a.part_ml[2 * ob] = m; a.part_ml[2 * ob + 1] = l; }
     if (!live) return;
     float* dst = a.part_acc + ob * DV + col0;
+    auto store = [&](const hy_v16f* v) {
 #pragma unroll
-    for (int r = 0; r < 16; ++r)
+        for (int r = 0; r < 16; ++r)
 #pragma unroll
-        for (int i = 0; i < DVT; ++i) dst[DVT * (8 * (r >> 2) + 4 * kh + (r & 3)) + i] = o[i][r];
+            for (int i = 0; i < DVT; ++i) dst[DVT * (8 * (r >> 2) + 4 * kh + (r & 3)) + i] = v[i][r];
+    };
+    if (hy_attn_nan<DVT>(o)) {
+        hy_v16f again[DVT];
+        hy_attn_again<DK, DVT>(again, a, a.q + (size_t)(rho / hpg) * a.ldq + (size_t)hr * DK, a.scale, m, slope, pr, nbr, win, kc, vc, pkc, pvc, col0, kh, split, a.nsplit, nv,
+                               [&](int t, int& j, int& last, bool& pooled) { const int w = t - np_t; pooled = t < np_t; j = (pooled ? t : w < nk ? w : lo_t + w - nk) << 5; last = pooled ? nb_wg - 1 : maxpos; });
+        store(again);
+    } else store(o);
 }

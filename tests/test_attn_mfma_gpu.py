@@ -73,3 +73,54 @@ def test_a_few_tokens(hy, tmp_path, name, n):
     p.close()
     want = m.ref(toks)
     assert N.err(np.concatenate(got), want) < 2e-5
+
+
+def odd_model(hy, tmp_path, mod, layer, seed):
+    """A model whose last token embeds as not-a-number: its key and its value are none."""
+    cfg = mod.config([layer])
+    odd = cfg["vocab"] - 1
+
+    def tweak(*a):
+        a[-1]["embed"][odd] = np.nan
+    return mod.Model(hy, tmp_path, cfg, seed, tweak), odd
+
+
+@pytest.mark.parametrize("bad", [3, 50, 99])
+@pytest.mark.parametrize("name", list(LAYERS))
+def test_rows_that_do_not_see_a_bad_key(hy, tmp_path, name, bad):
+    """Rows in front of a key and value that are not numbers, and rows whose window has left them behind, are the restatement's."""
+    mod, layer = LAYERS[name]
+    m, odd = odd_model(hy, tmp_path, mod, layer, bad)
+    toks = np.random.default_rng(bad).integers(0, odd, 100).astype(np.int32)
+    good = toks.copy()
+    toks[bad] = odd
+    p = m.plan("float32", ctx=108, max_batch=128)
+    got = p.step(p.acquire(), toks, 0, list(range(100)))[:, :odd]
+    p.close()
+    want = m.ref(good)[:, :odd]
+    assert N.err(got[:bad], want[:bad]) < 2e-5
+    assert np.isnan(got[bad]).all()
+    if name == "window_keep64" and bad >= 3:          # 29 keys and the first three
+        assert N.err(got[bad + 29:], want[bad + 29:]) < 2e-5 if bad + 29 < 100 else True
+        assert np.isnan(got[bad:bad + 29]).all()
+
+
+@pytest.mark.parametrize("name", list(FEW))
+def test_few_rows_that_do_not_see_a_bad_key(hy, tmp_path, name):
+    mod, layer = FEW[name]
+    m, odd = odd_model(hy, tmp_path, mod, layer, 7)
+    toks = np.random.default_rng(7).integers(0, odd, 61).astype(np.int32)
+    good = toks.copy()
+    p = m.plan("float32", ctx=80, max_batch=64)
+    s = p.acquire()
+    first = 10 if name == "window_keep64" else 35          # (out of the window by the next step, or inside it)
+    toks[first] = odd
+    p.step(s, toks[:31], 0, [])
+    got = [p.step(s, toks[31:39], 31, list(range(8))), p.step(s, toks[39:55], 39, list(range(16)))]
+    got += [p.step(s, toks[i:i + 1], i, [0]) for i in range(55, 61)]
+    p.close()
+    got, want = np.concatenate(got)[:, :odd], m.ref(good)[31:, :odd]
+    if name == "window_keep64":
+        assert np.isnan(got[:8]).all() and N.err(got[8:], want[8:]) < 2e-5
+    else:
+        assert N.err(got[:4], want[:4]) < 2e-5 and np.isnan(got[4]).all()
