@@ -2739,7 +2739,13 @@ static __global__ void pf_unchunk_row_kernel(const float* __restrict__ X, int b,
     for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < dim; i += gridDim.x * blockDim.x) out[i] = X[chunked(b, i, cc, ntok)];
 }
 
-// The step's (token, sequence, position) triples: one copy from pinned memory.  Every run that used h_io has been waited for.
+// Pinned memory of the plan (h_io, h_log) belongs to a call until the stream has passed it: a call that fails behind its first copy waits as well.
+struct PfDrain {
+    hipStream_t stream;
+    bool passed = false;
+    ~PfDrain() { if (!passed) (void)hipStreamSynchronize(stream); }
+};
+// The step's (token, sequence, position) triples: one copy from pinned memory.  Every call that used h_io has been waited for (PfDrain).
 static int32_t pf_stage_tokens(gl3_ctx* ctx, int n) {
     gl3_prefill_state* p = ctx->pf;
     GL3_HIP(hipMemcpyAsync(p->tokens, p->h_io, ((size_t)2 * p->max_batch + n) * sizeof(int32_t), hipMemcpyHostToDevice, ctx->stream));
@@ -2790,12 +2796,14 @@ int32_t gl3_prefill_run(gl3_ctx* ctx, int32_t seq, const int32_t* tokens, int32_
         if (tokens[i] < 0 || tokens[i] >= d.vocab) GL3_FAIL(GL3_E_ARG, "token id out of range");
     GL3_HIP(hipSetDevice(d.device));
     for (int i = 0; i < n; ++i) { p->h_io[i] = tokens[i]; p->h_io[p->max_batch + i] = seq; p->h_io[2 * p->max_batch + i] = start_pos + i; }
+    PfDrain drain{ctx->stream};
     int32_t r = pf_stage_tokens(ctx, n);
     if (r != GL3_OK) return r;
     if ((r = pf_layers(ctx, n, start_pos + n - 1, seq)) != GL3_OK) return r;
     // keep the decode path's x in step with the last prefilled token (parity tap gl3_get_x)
     hipLaunchKernelGGL(pf_unchunk_row_kernel, dim3(4), dim3(256), 0, ctx->stream, p->X, n - 1, d.dim, ctx->dim_l, n, ctx->x);
     GL3_HIP(hipStreamSynchronize(ctx->stream));
+    drain.passed = true;
     return gl3_tp_check(ctx);
 }
 
@@ -2817,6 +2825,7 @@ int32_t gl3_decode_batch_run(gl3_ctx* ctx, const int32_t* tokens, const int32_t*
     int max_pos = 0;
     for (int i = 0; i < n; ++i) max_pos = positions[i] > max_pos ? positions[i] : max_pos;
     for (int i = 0; i < n; ++i) { p->h_io[i] = tokens[i]; p->h_io[p->max_batch + i] = seq_ids[i]; p->h_io[2 * p->max_batch + i] = positions[i]; }
+    PfDrain drain{ctx->stream};
     int32_t r = pf_stage_tokens(ctx, n);
     if (r != GL3_OK) return r;
     hipStream_t s = ctx->stream;
@@ -2867,6 +2876,7 @@ int32_t gl3_decode_batch_run(gl3_ctx* ctx, const int32_t* tokens, const int32_t*
     }
     GL3_HIP(hipGetLastError());
     GL3_HIP(hipStreamSynchronize(s));
+    drain.passed = true;
     if (argmax_out) memcpy(argmax_out, p->h_io + 3 * p->max_batch, (size_t)n * sizeof(int32_t));
     return gl3_tp_check(ctx);
 }
