@@ -33,7 +33,7 @@ bool gl3_gemm3_swiglu_quantises(int rows, int ntok);
 hipError_t gl3_gemm3_allow_lds();
 
 constexpr int PF_LOG_SLOTS = 3;                         // pinned pieces of logits in flight (static-batched decode)
-constexpr size_t PF_LOG_PIECE = (size_t)4 << 20;
+constexpr size_t PF_LOG_PIECE = (size_t)1 << 20;
 
 struct gl3_prefill_state {
     int max_batch = 0;
@@ -56,7 +56,7 @@ struct gl3_prefill_state {
     int tmx_tiles = 0;
     int32_t* seqpos = nullptr;          // [2][M] behind tokens: sequence id, position of every token of the step
     int32_t* h_io = nullptr;            // pinned [4][M], behind ctx->h_logits: tokens, sequence ids, positions of the step on their way in, greedy ids on their way out
-    uint8_t* h_log[PF_LOG_SLOTS] = {};  // pinned pieces of logits on their way to the caller (static-batched decode), made at its first use
+    uint8_t* h_log[PF_LOG_SLOTS] = {};  // pinned pieces of logits on their way to the caller (static-batched decode), made when first needed
     hipEvent_t log_ev[PF_LOG_SLOTS] = {};
     float* LOGITS = nullptr;            // [rows][vocab], grown on demand (batched decode)
     int logits_rows = 0;
@@ -2760,10 +2760,13 @@ static inline void pf_touch_pages(void* mem, size_t bytes) {
     if (bytes) q[bytes - 1] = q[bytes - 1];
 }
 // n rows of logits to the caller: through pinned pieces of at most PF_LOG_PIECE bytes, a piece on its way while the one before it is copied on.  (A copy to
-// pageable memory goes row by row through the runtime's own staging: 32 rows x 16896 570 - 740 us, this way 45 on the link + 30 - 70 on the host; x 151936
-// 1041 and 767.)  False: no pinned memory for the pieces.
-static bool pf_logits_slots(gl3_prefill_state* p) {
-    for (int i = 0; i < PF_LOG_SLOTS; ++i) {
+// pageable memory goes row by row through the runtime's own staging.)  Pieces are made when a step first needs them, and their first use costs a page fault per
+// 4 KB: 1 MB each, no more of them than the step has.  A step of 32 rows, a plan's first / later ones (us): x 16896 1090 - 1960 / 780 by the runtime's staging,
+// 840 - 1880 / 560 with pieces of 4 MB, 790 - 1880 / 535 with 1 MB, 900 - 1210 / 622 with 256 KB; x 151936 2130 - 3160 / 1620, 1630 - 6170 / 1340,
+// 1590 - 4000 / 1215, 2300 - 2710 / 2000.  False: no pinned memory for the pieces.
+static size_t pf_logits_pieces(size_t bytes) { return (bytes + PF_LOG_PIECE - 1) / PF_LOG_PIECE; }
+static bool pf_logits_slots(gl3_prefill_state* p, size_t bytes) {
+    for (size_t i = 0; i < PF_LOG_SLOTS && i < pf_logits_pieces(bytes); ++i) {
         if (!p->h_log[i] && hipHostMalloc((void**)&p->h_log[i], PF_LOG_PIECE) != hipSuccess) { p->h_log[i] = nullptr; (void)hipGetLastError(); return false; }
         if (!p->log_ev[i] && hipEventCreateWithFlags(&p->log_ev[i], hipEventDisableTiming) != hipSuccess) { p->log_ev[i] = nullptr; (void)hipGetLastError(); return false; }
     }
@@ -2771,7 +2774,7 @@ static bool pf_logits_slots(gl3_prefill_state* p) {
 }
 static int32_t pf_logits_out(gl3_ctx* ctx, float* out, size_t bytes) {
     gl3_prefill_state* p = ctx->pf;
-    const size_t pieces = (bytes + PF_LOG_PIECE - 1) / PF_LOG_PIECE, per = ((bytes + pieces - 1) / pieces + 4095) & ~(size_t)4095;
+    const size_t pieces = pf_logits_pieces(bytes), per = ((bytes + pieces - 1) / pieces + 4095) & ~(size_t)4095;
     auto send = [&](size_t i) -> int32_t {
         if (i * per >= bytes) return GL3_OK;
         GL3_HIP(hipMemcpyAsync(p->h_log[i % PF_LOG_SLOTS], (const uint8_t*)p->LOGITS + i * per, std::min(per, bytes - i * per), hipMemcpyDeviceToHost, ctx->stream));
@@ -2867,8 +2870,9 @@ int32_t gl3_decode_batch_run(gl3_ctx* ctx, const int32_t* tokens, const int32_t*
         GL3_HIP(hipGraphLaunch(p->step_graphs[n], s));
     } else if ((r = enqueue_step(max_pos)) != GL3_OK) return r;
     if (argmax_out) GL3_HIP(hipMemcpyAsync(p->h_io + 3 * p->max_batch, p->amax, (size_t)n * sizeof(int32_t), hipMemcpyDeviceToHost, s));
-    if (logits_out && d.tp_size == 1 && pf_logits_slots(p)) {
-        if ((r = pf_logits_out(ctx, logits_out, (size_t)n * d.vocab * 4)) != GL3_OK) return r;
+    const size_t logit_bytes = (size_t)n * d.vocab * 4;
+    if (logits_out && d.tp_size == 1 && pf_logits_slots(p, logit_bytes)) {
+        if ((r = pf_logits_out(ctx, logits_out, logit_bytes)) != GL3_OK) return r;
     } else if (logits_out) {      // un-chunk on the way out: [tp][n][vl] -> [n][vocab]
         for (int c = 0; c < d.tp_size; ++c)
             GL3_HIP(hipMemcpy2DAsync(logits_out + (size_t)c * vl, (size_t)d.vocab * 4, p->LOGITS + (size_t)c * n * vl, (size_t)vl * 4, (size_t)vl * 4, n,

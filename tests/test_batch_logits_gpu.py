@@ -28,3 +28,24 @@ def test_every_row_arrives(vocab, n):
             assert np.array_equal(logits[i], row) and ids[i] == row.argmax(), i
         assert np.array_equal(logits.argmax(axis=1), ids)
     plan.freeTornadoExecutionPlan()
+
+
+@pytest.mark.parametrize("vocab,n", [(4096, 64), (4112, 64), (4096, 33), (8192, 63), (8224, 64), (12288, 64), (12304, 64)])
+def test_around_whole_pieces(vocab, n):
+    """Steps whose logits end at, in front of or behind one, two and three pieces of 1 MB; destinations that do not start on a page."""
+    from importlib import import_module
+    import __graft_entry__ as ge
+    pkg = ge.load_package()
+    plans, hip = import_module(ge.PKG_NAME + ".plan"), import_module(ge.PKG_NAME + ".hip")
+    cfg = dataclasses.replace(pkg.synth.CONFIGS["tiny-llama"], vocab=vocab)
+    plan = plans.HipMasterPlan.initializeTornadoVMPlan(pkg.synth.make_numpy(cfg, seed=3), prefill_batch_size=64, n_seqs=64)
+    rng = np.random.default_rng(n)
+    t, s, p, ids = rng.integers(0, vocab, n).astype(np.int32), np.arange(n, dtype=np.int32), np.zeros(n, np.int32), np.empty(n, np.int32)
+    want = np.stack([plan.forward_decode(int(x), 0) for x in t])
+    for off in (0, 1, 1023):
+        mem = np.full(n * vocab + 2048, 7.0, np.float32)
+        out = mem[off:off + n * vocab]
+        hip.check(hip.lib().gl3_forward_decode_batch(plan._ctx, plans._p(t), plans._p(s), plans._p(p), n, plans._p(out), plans._p(ids)), plan._ctx)
+        assert np.array_equal(out.reshape(n, vocab), want) and np.array_equal(ids, want.argmax(axis=1))
+        assert (mem[:off] == 7).all() and (mem[off + n * vocab:] == 7).all()
+    plan.freeTornadoExecutionPlan()
