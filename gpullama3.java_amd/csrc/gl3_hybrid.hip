@@ -1206,10 +1206,16 @@ static void hy_delta_scan(gl3_ctx* ctx, const HyDeltaScan& a) {
 #undef HY_DS
 }
 
+// States per lane that GL3_HY_SCAN_NL (4, 8, 16 or 32) asks of the token-by-token walk, which then takes every recurrence that fits it; 0: unset, or too few for N states.
+static int hy_scan_forced(int N) {
+    static const int nl = getenv("GL3_HY_SCAN_NL") ? atoi(getenv("GL3_HY_SCAN_NL")) : 0;
+    return (nl == 4 || nl == 8 || nl == 16 || nl == 32) && nl * 64 >= N ? nl : 0;
+}
+
 // Whether a recurrence goes 32 tokens at a time (hy_scan_chunk_kernel): one decay per head and token, keys of 64 / 128 / 256 entries in rows of
 // whole 16-byte pieces, and more than 16 tokens (a chunk takes ~3 us whatever it holds, the token-by-token walk 0.35 - 0.5 us a token).
 static bool hy_scan_chunks(const HyScanArgs& a) {
-    return a.n > 16 && a.mode != 3 && (a.N == 64 || a.N == 128 || a.N == 256) && ((a.ldk | a.k_off | a.k_hstride | a.ldq | a.q_off | a.q_hstride) & 3) == 0 &&
+    return a.n > 16 && a.mode != 3 && !hy_scan_forced(a.N) && (a.N == 64 || a.N == 128 || a.N == 256) && ((a.ldk | a.k_off | a.k_hstride | a.ldq | a.q_off | a.q_hstride) & 3) == 0 &&
            (((uintptr_t)a.ksrc | (uintptr_t)a.qsrc) & 15) == 0;
 }
 static void hy_scan_chunk_launch(gl3_ctx* ctx, const HyScanArgs& a) {
@@ -1230,9 +1236,10 @@ static void hy_scan_chunk_launch(gl3_ctx* ctx, const HyScanArgs& a) {
 // ones), NG a power of two; tokens staged per round: what fits 48 KB of LDS, at most 32.  Fills in a.NG and a.TB.
 // With few workgroups (few heads, narrow values) NL = 16 is halved once so that more of them share the columns; below 8 every workgroup
 // stages the same key / query rows for too few columns and the traffic from L2 eats the gain (measured: 16 and 8 within 2 %, 4 slower).
-// GL3_HY_SCAN_NL forces a value.
+// GL3_HY_SCAN_NL forces a value, and the walk.
 static void hy_scan(gl3_ctx* ctx, HyScanArgs& a) {
-    if (a.n == 1 && a.N <= 4096) {
+    const int forced = hy_scan_forced(a.N);
+    if (a.n == 1 && a.N <= 4096 && !forced) {
         hipLaunchKernelGGL(hy_scan_one_kernel, dim3(hy_cdiv(a.P, 64), a.heads), dim3(1024), (size_t)(2 * a.N + 1024) * 4, ctx->stream, a);
         return;
     }
@@ -1240,8 +1247,7 @@ static void hy_scan(gl3_ctx* ctx, HyScanArgs& a) {
     int NL = a.N > 1024 ? 32 : a.N > 8 ? 16 : a.N > 4 ? 8 : 4;
     auto wgs = [&](int nl) { int ng = 1; while (ng * nl < a.N) ng *= 2; return (long)hy_cdiv(a.P, 4 * (64 / ng)) * a.heads; };
     if (NL == 16 && 8 * 64 >= a.N && wgs(16) < 512) NL = 8;
-    static const int env_nl = getenv("GL3_HY_SCAN_NL") ? atoi(getenv("GL3_HY_SCAN_NL")) : 0;
-    if ((env_nl == 4 || env_nl == 8 || env_nl == 16 || env_nl == 32) && env_nl * 64 >= a.N) NL = env_nl;
+    if (forced) NL = forced;
     int NG = 1;
     while (NG * NL < a.N) NG *= 2;
     const int cols = 4 * (64 / NG), Ns = NG * NL;

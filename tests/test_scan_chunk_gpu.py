@@ -110,3 +110,27 @@ def test_a_token_that_is_not_finite(hy, tmp_path, name, bad):
     want = m.ref(toks[:bad])[:, :odd]
     assert N.err(got[:bad], want) < 3e-5
     assert np.isnan(got[bad:]).all()
+
+
+def test_forced_walk(hy, tmp_path):
+    """GL3_HY_SCAN_NL: the token-by-token walk with that many states per lane, for a portion and for single tokens.  Its sums are added in another order for each value
+    (so the bits differ), and every one is the restatement's."""
+    import os
+    import subprocess
+    import sys
+    cfg = N.config([N.ssm(heads=4, vdim=64, state=128)])
+    m = N.Model(hy, tmp_path, cfg, 3)
+    toks = np.random.default_rng(3).integers(0, cfg["vocab"], 43).astype(np.int32)
+    code = ("import sys, numpy as np; from importlib import import_module; import __graft_entry__ as ge; ge.load_package(); hy = import_module(ge.PKG_NAME + '.hybrid')\n"
+            "toks = np.array(%r, np.int32); p = hy.HybridPlan.from_dir(%r, dtype='float32', ctx=64, max_batch=64); s = p.acquire()\n"
+            "out = [p.step(s, toks[:40], 0, list(range(40)))] + [p.step(s, toks[i:i + 1], i, [0]) for i in range(40, 43)]\n"
+            "np.save(sys.argv[1], np.concatenate(out)); p.close()" % (toks.tolist(), m.dir))
+    got = {}
+    for nl in ("", "8", "32"):
+        path = str(tmp_path / ("out%s.npy" % nl))
+        env = {k: v for k, v in os.environ.items() if k != "GL3_HY_SCAN_NL"}
+        subprocess.run([sys.executable, "-c", code, path], env=dict(env, GL3_HY_SCAN_NL=nl) if nl else env, cwd=ge.ROOT, check=True, timeout=100)
+        got[nl] = np.load(path)
+        assert N.err(got[nl], m.ref(toks)) < 3e-5
+    for a, b in (("", "8"), ("", "32"), ("8", "32")):
+        assert not np.array_equal(got[a][:40], got[b][:40]), (a, b)
