@@ -1,5 +1,5 @@
 """The attention core on the matrix cores (csrc/gl3_hy_attn_mfma.h): the head sizes it is built for, whole prompts and portions behind earlier
-positions, row blocks and key tiles of 32 with remainders, groups of 1, 3 and 4 query heads, windows with kept first keys and with pooled
+positions, key splits of short portions and single tokens far from the start, row blocks and key tiles of 32 with remainders, groups of 1, 3 and 4 query heads, windows with kept first keys and with pooled
 blocks, latent attention's expanded keys with and without a rotated part, a distance penalty with the extra unit; the short portions at
 the end of a cut prompt go through the key-split kernel.
 
@@ -124,3 +124,36 @@ def test_few_rows_that_do_not_see_a_bad_key(hy, tmp_path, name):
         assert np.isnan(got[:8]).all() and N.err(got[8:], want[8:]) < 2e-5
     else:
         assert N.err(got[:4], want[:4]) < 2e-5 and np.isnan(got[4]).all()
+
+
+# Key splits: a short portion behind more than 512 positions is dealt out to up to eight workgroups per row block, single tokens to up to 128 (more tiles than
+# splits from 4097 positions on).  A split without a key, and rows that see none of a split's keys, leave partial sums that the merge must pass over.
+@pytest.mark.parametrize("fill,n", [(600, 17), (1100, 40), (1500, 33), (2100, 18)])
+@pytest.mark.parametrize("name", ["64_gqa2", "128_gqa3", "window_pool64", "window_pool128", "window_keep64", "latent64", "latent192"])
+def test_key_splits(hy, tmp_path, name, fill, n):
+    mod, layer = LAYERS[name]
+    cfg = mod.config([layer])
+    m = mod.Model(hy, tmp_path, cfg, seed=n)
+    toks = np.random.default_rng(n).integers(0, cfg["vocab"], fill + n).astype(np.int32)
+    p = m.plan("float32", ctx=fill + n + 8, max_batch=512)
+    s = p.acquire()
+    p.step(s, toks[:fill], 0, [])
+    got = p.step(s, toks[fill:], fill, list(range(n)))
+    p.close()
+    assert N.err(got, m.ref(toks)[fill:]) < 2e-5
+
+
+@pytest.mark.parametrize("dim", [64, 128])
+def test_more_tiles_than_splits(hy, tmp_path, dim):
+    cfg = N.config([N.att(heads=2, kv_heads=1, dim=dim, vdim=dim, ff=0)])
+    m = N.Model(hy, tmp_path, cfg, seed=dim)
+    fill, steps = 4180, [1, 5, 1]
+    toks = np.random.default_rng(dim).integers(0, cfg["vocab"], fill + sum(steps)).astype(np.int32)
+    p = m.plan("float32", ctx=len(toks) + 8, max_batch=512)
+    s, got, pos = p.acquire(), [], fill
+    p.step(s, toks[:fill], 0, [])
+    for k in steps:
+        got.append(p.step(s, toks[pos:pos + k], pos, list(range(k))))
+        pos += k
+    p.close()
+    assert N.err(np.concatenate(got), m.ref(toks)[fill:]) < 2e-5
