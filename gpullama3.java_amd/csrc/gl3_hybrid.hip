@@ -1081,11 +1081,15 @@ static int32_t hy_attention(gl3_ctx* ctx, const float* q, int ldq, const float* 
     a.pk = pk; a.pv = pv; a.pool = pool;
     // Matrix cores from 17 tokens on (up to 16 the keys are split over many workgroups, below), for the head sizes the kernel is built for.
     const bool aligned = ((ldq | H * dk | a.slot_stride) & 3) == 0 && (((uintptr_t)q | (uintptr_t)kc | (uintptr_t)vc | (uintptr_t)pk | (uintptr_t)pv) & 15) == 0;
-    // a few tokens: one tile of 32 keys per split
-    if (n <= 16 && aligned) {
-        int tiles = hy_cdiv(pos0 + n, 32);
-        if (window > 0) tiles = std::min<long>(tiles, hy_cdiv(keep, 32) + ((long)window + n) / 32 + 2);      // kept first keys + the window's tiles
-        if (pool > 0) tiles += hy_cdiv(std::max(0, pos0 + n - window) / pool, 32);                           // + the tiles of pooled rows
+    // A few tokens: one tile of 32 keys per split.  Heads of 64 with up to 8 rows a key / value head go to the vector kernel below once their tiles do not run side by side
+    // any more (three workgroups a CU): then the MFMAs of the rows that are not there are waited for.  One token, two layers, whole steps (us, few / vector): 16 heads
+    // 1000 positions 75 / 75, 2000 87 / 79, 8000 119 / 103; 32 heads 700 80 / 83, 1000 89 / 83, 4000 128 / 104; 8 heads 3000 78 / 79, 4000 87 / 80, 32000 172 / 122;
+    // 8 x 4 heads 3000 82 / 84, 3500 89 / 84, 32000 177 / 141; eight tokens of 8 heads 32000 192 / 173.  Heads of 128: the few-token kernel is ahead everywhere.
+    int tiles = hy_cdiv(pos0 + n, 32);
+    if (window > 0) tiles = std::min<long>(tiles, hy_cdiv(keep, 32) + ((long)window + n) / 32 + 2);      // kept first keys + the window's tiles
+    if (pool > 0) tiles += hy_cdiv(std::max(0, pos0 + n - window) / pool, 32);                           // + the tiles of pooled rows
+    const bool rounds = dk == 64 && n * (H / G) <= 8 && (long)G * tiles > 3 * 256;
+    if (n <= 16 && aligned && !rounds) {
         int nsplit = std::min(HY_MAX_SPLITS, std::max(1, tiles));
         if ((size_t)n * nsplit > h->part_rows) nsplit = std::max<size_t>(1, h->part_rows / n);
         a.nsplit = nsplit; a.kt = 32;

@@ -157,3 +157,20 @@ def test_more_tiles_than_splits(hy, tmp_path, dim):
         pos += k
     p.close()
     assert N.err(np.concatenate(got), m.ref(toks)[fill:]) < 2e-5
+
+
+@pytest.mark.parametrize("heads,kv_heads", [(16, 16), (32, 16)])
+def test_few_rows_of_many_tiles(hy, tmp_path, heads, kv_heads):
+    """Heads of 64 whose tiles are more than run side by side: up to 8 rows a key / value head through the vector kernel, more through the few-token kernel."""
+    cfg = N.config([N.att(heads=heads, kv_heads=kv_heads, dim=64, vdim=64, ff=0)])
+    m = N.Model(hy, tmp_path, cfg, seed=heads)
+    fill, steps = 1530, [1, 1, 4, 5, 1, 8, 9, 2]          # 768 tiles end at position 1536
+    toks = np.random.default_rng(heads).integers(0, cfg["vocab"], fill + sum(steps)).astype(np.int32)
+    p = m.plan("float32", ctx=len(toks) + 8, max_batch=512)
+    s, got, pos = p.acquire(), [], fill
+    p.step(s, toks[:fill], 0, [])
+    for k in steps:
+        got.append(p.step(s, toks[pos:pos + k], pos, list(range(k))))
+        pos += k
+    p.close()
+    assert N.err(np.concatenate(got), m.ref(toks)[fill:]) < 2e-5
