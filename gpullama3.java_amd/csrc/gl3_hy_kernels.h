@@ -1261,12 +1261,15 @@ static __global__ __launch_bounds__(256) void hy_attn_merge_few_kernel(const flo
 // Causal depthwise convolution over the step's tokens; inputs before the step come from the slot's tail (the last taps - 1 inputs of
 // the sequence), zeros before position 0.  out = silu(bias + sum_k w[c][k] in(t - (taps - 1 - k))).
 // One thread per channel and HY_CONV_T tokens: every input is loaded once (one token per thread loads it taps times: 28 -> 14 us for 512 tokens x
-// 10240 channels).  A portion that fits one thread's tokens moves the tail on as well; longer ones leave that to hy_conv_tail_kernel.
+// 10240 channels).  More than four taps do not stay in registers: a thread walks taps x tokens one load after the other, so it has one token (32 taps,
+// 2304 channels, two layers' steps of eight tokens: 200 us with eight tokens per thread, 143 with one; of 512: 657 and 581).  A portion that
+// fits one thread's tokens moves the tail on as well; longer ones leave that to hy_conv_tail_kernel.
 constexpr int HY_CONV_T = 8;
+__host__ __device__ __forceinline__ int hy_conv_tokens(int taps) { return taps <= 4 ? HY_CONV_T : 1; }
 static __global__ __launch_bounds__(256) void hy_conv_kernel(const float* __restrict__ proj, int ld, int x_off, int ch, int taps, const float* __restrict__ w,
                                                              const float* __restrict__ bias, float* __restrict__ tail, size_t slot_stride,
                                                              const int* __restrict__ dyn, int n, float* __restrict__ out) {
-    const int c = blockIdx.x * 256 + threadIdx.x, t0 = blockIdx.y * HY_CONV_T;
+    const int c = blockIdx.x * 256 + threadIdx.x, t0 = blockIdx.y * hy_conv_tokens(taps);
     if (c >= ch) return;
     const bool fresh = dyn[0] == 0;
     float* tl = tail + (size_t)dyn[1] * slot_stride;
@@ -1287,12 +1290,11 @@ static __global__ __launch_bounds__(256) void hy_conv_kernel(const float* __rest
                 if (k >= 4 - taps) a = fmaf(wt[k], v[i + k], a);
             if (t0 + i < n) out[(size_t)(t0 + i) * ch + c] = hy_silu(a);
         }
-    } else
-        for (int t = t0; t < min(t0 + HY_CONV_T, n); ++t) {
-            float a = b;
-            for (int k = 0; k < taps; ++k) a = fmaf(w[(size_t)c * taps + k], at(t - (taps - 1 - k)), a);
-            out[(size_t)t * ch + c] = hy_silu(a);
-        }
+    } else {
+        float a = b;
+        for (int k = 0; k < taps; ++k) a = fmaf(w[(size_t)c * taps + k], at(t0 - (taps - 1 - k)), a);
+        out[(size_t)t0 * ch + c] = hy_silu(a);
+    }
     if (gridDim.y == 1)
         for (int i = 0; i < taps - 1; ++i) tl[(size_t)i * ch + c] = at(n + i - (taps - 1));          // ascending: reads only rows not yet rewritten
 }

@@ -1436,9 +1436,9 @@ static int32_t hy_mixer_core(gl3_ctx* ctx, HyLayer& L, int np, int ldo, int n, i
         const int inner = d.heads * d.vdim, ch = hy_conv_ch(d), dt_off = 2 * inner + 2 * d.groups * d.state;
         float* state = h->slots + L.off_state;
         float* tail = h->slots + L.off_tail;
-        hipLaunchKernelGGL(hy_conv_kernel, dim3(hy_cdiv(ch, 256), hy_cdiv(n, HY_CONV_T)), dim3(256), 0, st, h->proj, np, inner, ch, d.conv, L.conv_w, L.conv_b, tail, h->slot_floats, h->dyn,
+        hipLaunchKernelGGL(hy_conv_kernel, dim3(hy_cdiv(ch, 256), hy_cdiv(n, hy_conv_tokens(d.conv))), dim3(256), 0, st, h->proj, np, inner, ch, d.conv, L.conv_w, L.conv_b, tail, h->slot_floats, h->dyn,
                            n, h->conv);
-        if (d.conv > 1 && n > HY_CONV_T)
+        if (d.conv > 1 && n > hy_conv_tokens(d.conv))
             hipLaunchKernelGGL(hy_conv_tail_kernel, dim3(hy_cdiv(ch, 256)), dim3(256), 0, st, h->proj, np, inner, ch, d.conv, tail, h->slot_floats, h->dyn, n);
         HyScanArgs a{};
         a.ksrc = h->conv; a.ldk = ch; a.k_off = inner; a.k_hstride = d.state;

@@ -28,6 +28,7 @@ def hy():
 LAYERS = {
     "ssm_one_state": (N, N.ssm(heads=3, vdim=63, state=1, conv=1)), "ssm_17_states": (N, N.ssm(heads=4, vdim=65, state=17, groups=2, norm_groups=2, conv=2)),
     "ssm_300_states": (N, N.ssm(heads=2, vdim=130, state=300, conv=4)), "ssm_taps_5": (N, N.ssm(heads=6, vdim=64, state=64, groups=3, conv=5)),
+    "ssm_taps_23": (N, N.ssm(heads=4, vdim=64, state=24, conv=23)),
     "mlstm_normaliser_column_64": (K, K.mls(heads=3, dim=20, vdim=63, ff=0)), "mlstm_normaliser_column_65": (K, K.mls(heads=2, dim=260, vdim=64, ff=0)),
     "retention_turned": (K, K.par(right=K.ret(heads=4, dim=64, vdim=66, rot_dims=32), ff=0)), "lightning": (U, U.lig(heads=3, dim=15, vdim=70, mlp=None)),
     "hgrn_odd": (T, T.hgrn(heads=3, dim=19, vdim=65)), "hgrn_272": (T, T.hgrn(heads=2, dim=272, vdim=24)),
@@ -52,3 +53,20 @@ def test_single_steps_and_short_portions(hy, tmp_path, name):
     p.close()
     for i in range(2):
         assert N.err(np.concatenate(got[i]), m.ref(toks[i])) < 3e-5
+
+
+def test_many_taps_do_not_queue(hy, tmp_path):
+    """Eight tokens of a convolution with 64 taps: a thread that walks them one after the other takes 512 loads in a row, three times the step with 4 taps."""
+    import time
+    best = {}
+    for conv in (4, 64):
+        cfg = N.config([N.ssm(heads=32, vdim=64, state=128, conv=conv)] * 3)
+        p = N.Model(hy, tmp_path, cfg, conv).plan("float32", ctx=40, max_batch=32)
+        s, toks, times = p.acquire(), np.arange(8, dtype=np.int32), []
+        for _ in range(30):
+            a = time.perf_counter()
+            p.step(s, toks, 0, [7])
+            times.append(time.perf_counter() - a)
+        p.close()
+        best[conv] = min(times)
+    assert best[64] < 2.0 * best[4], best
