@@ -13,8 +13,8 @@
 // per SIMD is what keeps the matrix cores busy during the softmax).  Queries (scaled) stay in LDS, rows dk + 4 floats apart.
 // A value that is not finite must stay with the rows that see its key, and the second product carries it to every row of the tile (p = 0 times infinity).  Nothing in the
 // loops below looks for one (values cleaned in the tiles with unseen keys cost 1 and 5 % of the two kernels, right in front of every MFMA 6 - 12 %): sums that hold a
-// not-a-number at the end are made once more, key by key on the vector units (hy_attn_again), which costs other inputs the look at the sums: 0.5 % and 1 - 3 %.  It
-// stands behind the last exchange in LDS, which the loop's last MFMAs run under.
+// not-a-number at the end are made once more, key by key on the vector units (hy_attn_again), which costs other inputs the look at the sums: 1 % of the kernel of
+// many tokens, of that of few 2 % with 64 and 256 entries and 7 % with 512.  It stands behind the last exchange in LDS, which the loop's last MFMAs run under.
 // Bound: 153 TFLOP/s of float32 MFMAs.  Measured against hy_attn_kernel (8 key / value heads x 4, head size 128, us):
 //   512 tokens at position 0 131 -> 45, four such portions of 2041 tokens 1795 -> 428 in all.
 #pragma once
@@ -191,7 +191,7 @@ static __global__ __launch_bounds__(256, DKC > 16 ? 1 : 2) void hy_attn_mfma_ker
     __syncthreads();
     const float M = fmaxf(fmaxf(sml[0][0][r32], sml[1][0][r32]), fmaxf(sml[2][0][r32], sml[3][0][r32]));
     const float sc = m > -INFINITY ? expf(m - M) : 0.f;
-    if (__any(hy_attn_nan<DVT>(o) && pr >= 0))
+    if (__builtin_expect(__any(hy_attn_nan<DVT>(o) && pr >= 0), 0))
         hy_attn_again<DK, DVT>(o, a, sQ + r32 * QS, 1.f, m, slope, pr, nbr, win, kc, vc, pkc, pvc, 0, kh, split * 4 + wave, 4 * a.nsplit, nv,
                                [&](int t, int& j, int& last, bool& pooled) { pooled = t < np_t; j = first_key(t); last = pooled ? nb_wg - 1 : maxpos; });
     for (int w = 0; w < 4; ++w) {
@@ -230,7 +230,7 @@ static __global__ __launch_bounds__(256, DKC > 16 ? 1 : 2) void hy_attn_mfma_ker
 // softmax and the weighted sum of its own value columns.  Same layouts as above; rows that are not there cost MFMAs nobody waits for.  Latent attention's
 // cached rows (keys = values) come as kc = vc.  A tile is one round trip to memory and (DK + DV) / 2 MFMAs over the wavefronts, and the tiles of a
 // token up to 32 x HY_MAX_SPLITS positions run side by side, where hy_attn_kernel walked tiles of 64 keys with four rows per wavefront (us):
-// 32 heads on 512-entry latents 29 - 33 -> 11.8, 8 x 4 heads of 64 7.3 -> 5.7, of 128 behind 2041 positions 13.5 -> 8.2 us.
+// 32 heads on 512-entry latents 29 - 33 -> 12.4, 8 x 4 heads of 64 7.3 -> 5.8, of 128 behind 2041 positions 13.5 -> 8.2 us.
 template <int DK, int DV, int NW = 4>          // NW wavefronts
 static __global__ __launch_bounds__(64 * NW, 1) void hy_attn_few_kernel(HyAttnArgs a) {
     constexpr int RQ = DK / NW, KC = RQ / 8, CW = DV >= 32 * NW ? DV / NW : 32, NE = 16 / NW, DVT = CW / 32;
@@ -352,7 +352,9 @@ static __global__ __launch_bounds__(64 * NW, 1) void hy_attn_few_kernel(HyAttnAr
 #pragma unroll
             for (int i = 0; i < DVT; ++i) dst[DVT * (8 * (r >> 2) + 4 * kh + (r & 3)) + i] = v[i][r];
     };
-    if (hy_attn_nan<DVT>(o)) {
+    const bool nan = hy_attn_nan<DVT>(o);
+    if (__builtin_expect(!__any(nan), 1)) store(o);          // (the rare way out of line: 256 entries 9.2 -> 8.6 us, 64 6.1 -> 6.0)
+    else if (nan) {
         hy_v16f again[DVT];
         hy_attn_again<DK, DVT>(again, a, a.q + (size_t)(rho / hpg) * a.ldq + (size_t)hr * DK, a.scale, m, slope, pr, nbr, win, kc, vc, pkc, pvc, col0, kh, split, a.nsplit, nv,
                                [&](int t, int& j, int& last, bool& pooled) { const int w = t - np_t; pooled = t < np_t; j = (pooled ? t : w < nk ? w : lo_t + w - nk) << 5; last = pooled ? nb_wg - 1 : maxpos; });

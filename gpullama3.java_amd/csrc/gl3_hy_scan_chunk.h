@@ -13,7 +13,8 @@
 // A token whose x is not finite must not reach the tokens in front of it, and a product with its zero place in the masked matrix would carry it there:
 // the matrix cores take zero in its stead, and a chunk that holds one (looked for on the way into LDS) adds its products entry by entry as y is written.
 // Keys and queries come finished (hy_scan_prep_kernel); x passes through silu on the way into LDS where the layer asks for it (act & 4).
-// Measured for 512 tokens (us), hy_ssm_scan_kernel -> this: 128 heads x (128 x 64) 278 -> 73, 16 x (128 x 256) 310 -> 52, 8 x (256 x 513) 430 -> 97.
+// Measured for 512 tokens (us), hy_ssm_scan_kernel -> this: 128 heads x (128 x 64) 278 -> 75, 16 x (128 x 256) 310 -> 55, 8 x (256 x 513) 430 -> 100 (the look for an x that is
+// not finite is 1, 3 and 2 us of them).
 #pragma once
 #include "gl3_hy_attn_mfma.h"
 
