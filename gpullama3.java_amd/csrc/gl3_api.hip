@@ -450,15 +450,17 @@ static int32_t enqueue_decode(gl3_ctx* ctx, bool want_logits, gl3_kernel_times* 
     pr.begin(GL3_K_OTHER, (uint64_t)d.dim / 32 * 34);
     const int fold = ctx->tp_fold, fmask = fold ? ctx->tp_fold_mask : 0, L_ = d.n_layers;
     uint32_t* vl_step = fold ? reinterpret_cast<uint32_t*>(ctx->arena.base + GL3_ARENA_STEP) : (uint32_t*)nullptr;
+    const int* host = ctx->dyn_cur == ctx->dyn ? ctx->h_dyn : nullptr;          // (a token-by-token prefill's pairs are on the device)
+    const dim3 eg(vl_step ? 1 : (d.dim + 1023) / 1024);                         // (folded gathers: one workgroup opens the step)
     if (ctx->emb.fmt == GL3_TYPE_Q8_0)
-        hipLaunchKernelGGL(embed_q8t_kernel, dim3(1), dim3(256), 0, s, ctx->emb.w, ctx->emb.ng, d.dim, ctx->dyn_cur, ctx->x, ctx->emb_scale,
+        hipLaunchKernelGGL(embed_q8t_kernel, eg, dim3(256), 0, s, ctx->emb.w, ctx->emb.ng, d.dim, ctx->dyn_cur, host, ctx->x, ctx->emb_scale,
                            (fmask & TF_EMBED) ? tp_rec(ctx, L_, 0) : (const TpRec*)nullptr,
                            fold ? reinterpret_cast<uint32_t*>(ctx->arena.base + GL3_ARENA_STEP) : (uint32_t*)nullptr);
-    else if (ctx->emb.vl && ctx->emb.fmt == GL3_TYPE_F16) hipLaunchKernelGGL((embed_vl_kernel<WT_F16>), dim3(1), dim3(256), 0, s, ctx->emb.w, d.dim, ctx->dyn_cur, ctx->x, ctx->emb_scale, vl_step);
-    else if (ctx->emb.vl && ctx->emb.fmt == GL3_FMT_Q8V) hipLaunchKernelGGL((embed_vl_kernel<WT_Q8_0>), dim3(1), dim3(256), 0, s, ctx->emb.w, d.dim, ctx->dyn_cur, ctx->x, ctx->emb_scale, vl_step);
-    else if (ctx->emb.vl) hipLaunchKernelGGL((embed_vl_kernel<WT_Q4_0>), dim3(1), dim3(256), 0, s, ctx->emb.w, d.dim, ctx->dyn_cur, ctx->x, ctx->emb_scale, vl_step);
-    else if (ctx->emb.fmt == GL3_TYPE_F16) hipLaunchKernelGGL((embed_rl_kernel<WT_F16>), dim3(1), dim3(256), 0, s, ctx->emb.w, d.dim, ctx->dyn_cur, ctx->x, ctx->emb_scale);
-    else hipLaunchKernelGGL((embed_rl_kernel<WT_Q4_0>), dim3(1), dim3(256), 0, s, ctx->emb.w, d.dim, ctx->dyn_cur, ctx->x, ctx->emb_scale);
+    else if (ctx->emb.vl && ctx->emb.fmt == GL3_TYPE_F16) hipLaunchKernelGGL((embed_vl_kernel<WT_F16>), eg, dim3(256), 0, s, ctx->emb.w, d.dim, ctx->dyn_cur, host, ctx->x, ctx->emb_scale, vl_step);
+    else if (ctx->emb.vl && ctx->emb.fmt == GL3_FMT_Q8V) hipLaunchKernelGGL((embed_vl_kernel<WT_Q8_0>), eg, dim3(256), 0, s, ctx->emb.w, d.dim, ctx->dyn_cur, host, ctx->x, ctx->emb_scale, vl_step);
+    else if (ctx->emb.vl) hipLaunchKernelGGL((embed_vl_kernel<WT_Q4_0>), eg, dim3(256), 0, s, ctx->emb.w, d.dim, ctx->dyn_cur, host, ctx->x, ctx->emb_scale, vl_step);
+    else if (ctx->emb.fmt == GL3_TYPE_F16) hipLaunchKernelGGL((embed_rl_kernel<WT_F16>), eg, dim3(256), 0, s, ctx->emb.w, d.dim, ctx->dyn_cur, host, ctx->x, ctx->emb_scale);
+    else hipLaunchKernelGGL((embed_rl_kernel<WT_Q4_0>), eg, dim3(256), 0, s, ctx->emb.w, d.dim, ctx->dyn_cur, host, ctx->x, ctx->emb_scale);
     pr.end();
 
     for (int l = 0; l < d.n_layers; ++l) {
@@ -769,8 +771,8 @@ int32_t gl3_create(const gl3_model_desc* desc, gl3_ctx** out) {
     TRY(dmalloc(ctx, &ctx->argmax, 2 + 2 * AMX_WGS));          // result, ticket, (value, index) pairs of argmax_kernel
     TRYHIP(hipMemset(ctx->argmax, 0, (2 + 2 * AMX_WGS) * sizeof(int)));
     if (d.flags & GL3_FLAG_LAYER_TAPS) TRY(dmalloc(ctx, &ctx->taps, (size_t)d.n_layers * d.dim));
-    TRYHIP(hipHostMalloc((void**)&ctx->h_dyn, 4 * sizeof(int)));
-    TRYHIP(hipHostMalloc((void**)&ctx->h_logits, ((size_t)d.vocab + 4 * (size_t)(d.max_batch > 1 ? d.max_batch : 0)) * 4));      // + the batched steps' inputs and ids (gl3_prefill.hip: h_io)
+    TRYHIP(hipHostMalloc((void**)&ctx->h_dyn, 4 * sizeof(int), hipHostMallocCoherent));          // (kernels read it: embed_q8t_kernel)
+    TRYHIP(hipHostMalloc((void**)&ctx->h_logits, ((size_t)d.vocab + 4 * (size_t)(d.max_batch > 1 ? d.max_batch : 0)) * 4, hipHostMallocCoherent));      // + the batched steps' inputs and ids (gl3_prefill.hip: h_io)
     TRYHIP(hipHostMalloc((void**)&ctx->h_argmax, sizeof(int)));
     // batched prefill / static-batched decode: int8 MFMA GEMMs for Q8_0 (any tensor-parallel degree); f32-MFMA / VALU GEMMs in the
     // Vector-API order for F16, Q4_0 and Q8_0 with the f32 activation (gl3_prefill_vl.h).  The scalar dot order
@@ -1051,8 +1053,7 @@ static int32_t set_dyn(gl3_ctx* ctx, int32_t token, int32_t pos) {
     if (token < 0 || token >= ctx->d.vocab) GL3_FAIL(GL3_E_ARG, "token id out of range");
     if (pos < 0 || pos >= ctx->d.ctx) GL3_FAIL(GL3_E_ARG, "position outside the KV cache (context length)");
     GL3_HIP(hipSetDevice(ctx->d.device));
-    ctx->h_dyn[0] = token; ctx->h_dyn[1] = pos;
-    GL3_HIP(hipMemcpyAsync(ctx->dyn, ctx->h_dyn, 2 * sizeof(int), hipMemcpyHostToDevice, ctx->stream));
+    ctx->h_dyn[0] = token; ctx->h_dyn[1] = pos;          // (every step that read the pair has been waited for)
     return GL3_OK;
 }
 
@@ -1067,13 +1068,14 @@ int32_t gl3_forward_decode(gl3_ctx* ctx, int32_t token, int32_t pos, float* logi
     if (ctx->hy) return hy_forward_decode(ctx, 0, token, pos, logits_out, argmax_out);
     int32_t r = set_dyn(ctx, token, pos);
     if (r != GL3_OK) return r;
+    gl3_drain drain{ctx->stream};
     const bool want_logits = logits_out || argmax_out;
     const int amode = attn_mode(ctx, pos);
     if (ctx->graph_exec && want_logits) GL3_HIP(hipGraphLaunch(step_graph(ctx, amode), ctx->stream));
     else if ((r = enqueue_decode(ctx, want_logits, nullptr, amode)) != GL3_OK) return r;
     if (argmax_out) {
-        hipLaunchKernelGGL(argmax_kernel, dim3(AMX_WGS), dim3(256), 0, ctx->stream, ctx->logits, ctx->d.vocab, ctx->argmax);
-        GL3_HIP(hipMemcpyAsync(ctx->h_argmax, ctx->argmax, sizeof(int), hipMemcpyDeviceToHost, ctx->stream));
+        hipLaunchKernelGGL(argmax_kernel, dim3(AMX_WGS), dim3(256), 0, ctx->stream, ctx->logits, ctx->d.vocab, ctx->argmax, ctx->h_argmax);
+        GL3_HIP(hipGetLastError());
     }
     // logits D2H: straight into the caller's buffer when it is page-locked (gl3_pin_host_buffer), else through the plan's pinned
     // staging buffer + one host memcpy (513 KB for a 128 k vocabulary: ~40 us per token on the host)
@@ -1081,8 +1083,10 @@ int32_t gl3_forward_decode(gl3_ctx* ctx, int32_t token, int32_t pos, float* logi
     if (logits_out)
         for (const auto& pr : ctx->pinned)
             if ((uint8_t*)logits_out >= (uint8_t*)pr.first && (uint8_t*)logits_out + (size_t)ctx->d.vocab * 4 <= (uint8_t*)pr.first + pr.second) direct = true;
-    if (logits_out) GL3_HIP(hipMemcpyAsync(direct ? logits_out : ctx->h_logits, ctx->logits, (size_t)ctx->d.vocab * 4, hipMemcpyDeviceToHost, ctx->stream));
+    if (logits_out && direct) GL3_HIP(hipMemcpyAsync(logits_out, ctx->logits, (size_t)ctx->d.vocab * 4, hipMemcpyDeviceToHost, ctx->stream));
+    else if (logits_out) { launch_to_host(ctx->logits, ctx->h_logits, ctx->d.vocab, ctx->stream); GL3_HIP(hipGetLastError()); }
     GL3_HIP(hipStreamSynchronize(ctx->stream));
+    drain.passed = true;
     if ((r = gl3_tp_check(ctx)) != GL3_OK) return r;
     if (logits_out && !direct) memcpy(logits_out, ctx->h_logits, (size_t)ctx->d.vocab * 4);
     if (argmax_out) *argmax_out = *ctx->h_argmax;
@@ -1098,10 +1102,12 @@ int32_t gl3_forward_decode_sample(gl3_ctx* ctx, int32_t token, int32_t pos, floa
     if (!(coin >= 0.f && coin < 1.f)) GL3_FAIL(GL3_E_ARG, "coin must be rng.nextFloat(1f): in [0, 1)");
     int32_t r = set_dyn(ctx, token, pos);
     if (r != GL3_OK) return r;
+    gl3_drain drain{ctx->stream};
     const int amode = attn_mode(ctx, pos);
     if (ctx->graph_exec) GL3_HIP(hipGraphLaunch(step_graph(ctx, amode), ctx->stream));
     else if ((r = enqueue_decode(ctx, true, nullptr, amode)) != GL3_OK) return r;
     if ((r = gl3_sample_run(ctx, ctx->logits, temperature, topp, coin, token_out)) != GL3_OK) return r;
+    drain.passed = true;          // (the sampler has waited)
     return gl3_tp_check(ctx);
 }
 

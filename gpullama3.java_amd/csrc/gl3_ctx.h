@@ -127,6 +127,13 @@ constexpr size_t GL3_ARENA_HDR = 1024, GL3_ARENA_SEQ = 64, GL3_ARENA_ARRIVE = 68
 // rank p has completed into this arena), u32 ticket[3] (finished producer wavefronts of the running launch), u32 step (decode steps)
 constexpr size_t GL3_ARENA_FOLD = 512, GL3_ARENA_FOLD_TICKET = 704, GL3_ARENA_STEP = 720;
 
+// Page-locked memory of a plan (h_dyn, h_io, h_logits, h_log) belongs to a call until the stream has passed it: a call that fails behind its first launch waits as well.
+struct gl3_drain {
+    hipStream_t stream;
+    bool passed = false;
+    ~gl3_drain() { if (!passed) (void)hipStreamSynchronize(stream); }
+};
+
 struct gl3_ctx {
     gl3_model_desc d{};
     // derived (local = this tensor-parallel rank's share)
@@ -164,7 +171,7 @@ struct gl3_ctx {
     void* moe_slots = nullptr;                    // MoeSlots[n_layers][3]: gate/up with the shared expert merged, gate/up alone, down
     int *dyn = nullptr, *argmax = nullptr;        // dyn[0] = token, dyn[1] = position
     int* h_dyn = nullptr;                         // pinned
-    const int* dyn_cur = nullptr;                 // (token, position) pair the next launches read: dyn, or an entry of dyn_seq
+    int* dyn_cur = nullptr;                       // (token, position) pair the next launches read: dyn, or an entry of dyn_seq
     int* dyn_seq = nullptr;                       // [2 * dyn_seq_cap] pairs of a sequential (token-by-token) prefill chunk
     int dyn_seq_cap = 0;
     float* h_logits = nullptr;                    // pinned f32[vocab]

@@ -543,12 +543,39 @@ __global__ __launch_bounds__(mv_threads(NPW), NPW == 4 ? 4 : 2) void matvec_q8t_
 }
 
 // ---------------------------------------------------------------------------------------------------
+// What crosses the link to the host goes in kernels of the step's own: a copy of the runtime's takes 2 - 4 us and stands 6 us (in front of a captured step) and
+// 11 - 19 us (behind the last kernel) apart from its neighbours.
+// Tokens of a step whose ids the embedding reads over the link itself; more take one copy in front of it, for the link answers a read every ~35 ns (whole steps, us,
+// copy / own reads: batched prompt of 2 tokens 137 / 132, 4 137 / 135, 8 142 / 141; layer-list steps, whose embedding has 8 - 16 workgroups a token: 1 token 112 / 109,
+// 4 152 / 152, 16 143 / 152, 32 146 / 164).
+constexpr int GL3_HOST_TOKENS = 4;
+__device__ __forceinline__ int host_int(const int* p) { return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM); }
+__device__ __forceinline__ int step_token(int* dyn, const int* host) {
+    if (!host) return dyn[0];
+    __shared__ int sh[2];          // (one read over the link per workgroup)
+    if (threadIdx.x < 2) sh[threadIdx.x] = host_int(host + threadIdx.x);
+    __syncthreads();
+    if (blockIdx.x == 0 && threadIdx.x < 2) dyn[threadIdx.x] = sh[threadIdx.x];
+    return sh[0];
+}
+// n floats to page-locked host memory; both ends start on 16 bytes
+static __global__ __launch_bounds__(256) void to_host_kernel(const float* __restrict__ src, float* __restrict__ dst, size_t n) {
+    for (size_t i = (size_t)blockIdx.x * 256 + threadIdx.x; i < n / 4; i += (size_t)256 * gridDim.x) reinterpret_cast<float4*>(dst)[i] = reinterpret_cast<const float4*>(src)[i];
+    if (blockIdx.x == 0 && threadIdx.x < n % 4) dst[n / 4 * 4 + threadIdx.x] = src[n / 4 * 4 + threadIdx.x];
+}
+static inline void launch_to_host(const float* src, float* dst, size_t n, hipStream_t s) {
+    const size_t wgs = (n / 4 + 255) / 256;
+    hipLaunchKernelGGL(to_host_kernel, dim3((unsigned)(wgs < 1 ? 1 : wgs > 256 ? 256 : wgs)), dim3(256), 0, s, src, dst, n);
+}
+
+// ---------------------------------------------------------------------------------------------------
 // Embedding row gather + dequant: x[i] = q * d  (token_embedding_table.copyTo, InferenceCore.java:61;
 // replaces the host row copy of forwardTornadoVM :956-980 + convertQ8_0toFP32).
+// host: the step's token and position in page-locked host memory (null: in dyn already); the kernel leaves a copy in dyn for the kernels behind it.
 // tp (folded gathers): the kernel opens decode step number *step + 1 of the plan — it first waits until the peers' last pushes of
 // the previous step into x have landed (a later arrival would overwrite this step's embedding), then bumps the step word.
 static __global__ __launch_bounds__(256) void embed_q8t_kernel(const uint8_t* __restrict__ emb, int ng, int dim,
-                                                         const int* __restrict__ dyn, float* __restrict__ x, float emb_scale,
+                                                         int* dyn, const int* host, float* __restrict__ x, float emb_scale,
                                                          const TpRec* tp = nullptr, uint32_t* step = nullptr) {
     if (step) {
         const uint32_t s = *step;
@@ -568,10 +595,10 @@ static __global__ __launch_bounds__(256) void embed_q8t_kernel(const uint8_t* __
             }
         }
     }
-    const int token = dyn[0];
+    const int token = step_token(dyn, host);
     const uint8_t* strip = emb + (size_t)(token >> 4) * ng * TILE_BYTES;
     const int i16 = token & 15;
-    for (int i = threadIdx.x; i < dim; i += 256) {
+    for (int i = blockIdx.x * 256 + threadIdx.x; i < dim; i += 256 * gridDim.x) {
         const int b = i >> 5, j = i & 31;
         const uint8_t* p = strip + (size_t)(b >> 2) * TILE_BYTES;
         const int l = i16 + 16 * (b & 3);
@@ -1686,7 +1713,7 @@ constexpr int AMX_WGS = 64;
 __device__ __forceinline__ void amx_take(float& best, int& idx, float f, int i) {
     if (f > best || (f == best && i < idx)) { best = f; idx = i; }
 }
-static __global__ __launch_bounds__(256) void argmax_kernel(const float* __restrict__ v, int n, int* __restrict__ ws) {
+static __global__ __launch_bounds__(256) void argmax_kernel(const float* __restrict__ v, int n, int* __restrict__ ws, int* __restrict__ host) {
     __shared__ float bv[4];
     __shared__ int bi[4];
     __shared__ int last;
@@ -1733,7 +1760,7 @@ static __global__ __launch_bounds__(256) void argmax_kernel(const float* __restr
             amx_take(best, idx, ob, oi);
         }
         if (t == 0) {
-            ws[0] = idx == 0x7FFFFFFF ? 0 : idx;
+            ws[0] = *host = idx == 0x7FFFFFFF ? 0 : idx;          // (host: page-locked)
             __hip_atomic_store(ws + 1, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         }
     }

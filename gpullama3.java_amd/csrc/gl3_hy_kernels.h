@@ -90,20 +90,31 @@ template <int V> __device__ __forceinline__ void hy_stv(bf16_t* __restrict__ p, 
 // dyn[0] = position of the step's first token, dyn[1] = sequence slot, dyn[2] = the sequence's token before the step's first one
 constexpr int HY_MAX_STREAMS = 8;
 
-// ---- embedding: every stream starts as the token's row times `scale`, plus (bg.table) a row picked by the token pair,
+// ---- embedding, the first kernel of a portion: it reads the record [dyn 4 | want | tokens from entry tok0 on] in page-locked host memory and leaves a copy
+// (nw wanted rows) in rec for the kernels behind it (host null: the record is there already).  Every stream starts as the token's row times `scale`, plus (bg.table) a row picked by the token pair,
 // (previous mul_prev + token mul_cur) mod buckets, or row `buckets` for a sequence's first token; copy != null keeps the embedding output
 // for the depth average ----
 struct HyBigram { const void* table; int buckets, mul_prev, mul_cur; };
 template <typename T>
-static __global__ __launch_bounds__(256) void hy_embed_kernel(const int* __restrict__ tokens, const T* __restrict__ emb, float* __restrict__ X,
-                                                              int W, int S, size_t sstride, float scale, float* __restrict__ copy, HyBigram bg = HyBigram{},
-                                                              const int* __restrict__ dyn = nullptr) {
-    const int t = blockIdx.x, tok = tokens[t];
+static __global__ __launch_bounds__(256) void hy_embed_kernel(const int* host, int* __restrict__ rec, int tok0, int nw, const T* __restrict__ emb, float* __restrict__ X,
+                                                              int W, int S, size_t sstride, float scale, float* __restrict__ copy, HyBigram bg = HyBigram{}) {
+    __shared__ int sh[4];          // token, the one before it, position of the portion's first
+    const int t = blockIdx.x;
+    if (threadIdx.x < 3) {
+        const int at = threadIdx.x == 0 ? tok0 + t : threadIdx.x == 2 ? 0 : t > 0 ? tok0 + t - 1 : 2;
+        if (threadIdx.x == 0 || bg.table) sh[threadIdx.x] = host ? gl3::host_int(host + at) : rec[at];
+    }
+    if (host && blockIdx.y == 0) {
+        if (t == 0) for (int i = threadIdx.x; i < 4 + nw; i += 256) rec[i] = gl3::host_int(host + i);
+        if (threadIdx.x == 0) rec[tok0 + t] = sh[0];
+    }
+    __syncthreads();
+    const int tok = sh[0];
     const T* row = emb + (size_t)tok * W;
     const T* pair = nullptr;
     if (bg.table) {
-        const int prev = t > 0 ? tokens[t - 1] : dyn[2];
-        const int b = (t == 0 && dyn[0] == 0) ? bg.buckets : (int)(((long long)prev * bg.mul_prev + (long long)tok * bg.mul_cur) % bg.buckets);
+        const int prev = sh[1];
+        const int b = (t == 0 && sh[2] == 0) ? bg.buckets : (int)(((long long)prev * bg.mul_prev + (long long)tok * bg.mul_cur) % bg.buckets);
         pair = (const T*)bg.table + (size_t)b * W;
     }
     for (int w = blockIdx.y * 256 + threadIdx.x; w < W; w += 256 * gridDim.y) {

@@ -27,6 +27,8 @@
 
 using gl3::AMX_WGS;
 using gl3::argmax_kernel;
+using gl3::launch_to_host;
+using gl3::GL3_HOST_TOKENS;
 
 #define HY_BIT(id) (HyHave().set(id))
 #define HY_HIP(call)                                                                                   \
@@ -535,10 +537,10 @@ int32_t gl3_hy_create(const gl3_model_desc* desc, gl3_ctx** out, std::string& er
         for (float& v : one) v = 1.f;
         TRYHIP(hipMemcpy(h->ones, one, sizeof one, hipMemcpyHostToDevice));
     }
-    // step record, wanted rows and token ids travel in one copy: [dyn 4 | want want_cap | tokens mb]
+    // step record, wanted rows and token ids: [dyn 4 | want want_cap | tokens mb], copied to the device by the embedding
     TRY(hy_alloc(ctx, &h->dyn, (size_t)(4 + h->want_cap + mb) * 4));
     h->want = h->dyn + 4; h->tokens = h->want + h->want_cap;
-    TRYHIP(hipHostMalloc((void**)&h->h_dyn, (size_t)(4 + h->want_cap + mb) * 4));
+    TRYHIP(hipHostMalloc((void**)&h->h_dyn, (size_t)(4 + h->want_cap + mb) * 4, hipHostMallocCoherent));
     h->h_want = h->h_dyn + 4; h->h_tokens = h->h_want + h->want_cap;
     TRYHIP(hipHostMalloc((void**)&h->h_logits, (size_t)h->want_cap * V * 4));
     TRYHIP(hipMalloc((void**)&ctx->argmax, (2 + 2 * AMX_WGS) * sizeof(int)));
@@ -1625,9 +1627,10 @@ static int32_t hy_portion_plain(gl3_ctx* ctx, int seq, const int32_t* tokens, in
     memcpy(h->h_tokens, tokens, (size_t)n * 4);
     if (nw > 0) memcpy(h->h_want, want, (size_t)nw * 4);
     h->h_dyn[0] = pos0; h->h_dyn[1] = seq; h->h_dyn[2] = h->last_tok[seq];
-    HY_HIP(hipMemcpyAsync(h->dyn, h->h_dyn, (size_t)(4 + h->want_cap + n) * 4, hipMemcpyHostToDevice, st));
-    hipLaunchKernelGGL((hy_embed_kernel<T>), dim3(n, hy_cdiv(W, n <= 32 ? 256 : 1024)), dim3(256), 0, st, h->tokens, (const T*)h->emb.w, h->X, W, 1, lstride, h->emb_scale, h->depth ? h->hist : nullptr,
-                       HyBigram{h->bigram.w, h->bg_buckets, h->bg_prev, h->bg_cur}, h->dyn);
+    const int* host = n <= GL3_HOST_TOKENS ? h->h_dyn : nullptr;
+    if (!host) HY_HIP(hipMemcpyAsync(h->dyn, h->h_dyn, (size_t)(4 + h->want_cap + n) * 4, hipMemcpyHostToDevice, st));
+    hipLaunchKernelGGL((hy_embed_kernel<T>), dim3(n, hy_cdiv(W, n <= 32 ? 256 : 1024)), dim3(256), 0, st, host, h->dyn, 4 + h->want_cap, nw, (const T*)h->emb.w, h->X, W, 1, lstride, h->emb_scale, h->depth ? h->hist : nullptr,
+                       HyBigram{h->bigram.w, h->bg_buckets, h->bg_prev, h->bg_cur});
     T* hb = (T*)h->h;
     HyResid base{};
     base.x = h->X; base.W = W; base.eps = eps; base.ya_parts = 1; base.ya_mul = 1.f;
@@ -1736,8 +1739,9 @@ static int32_t hy_portion(gl3_ctx* ctx, int seq, const int32_t* tokens, int n, i
     memcpy(h->h_tokens, tokens, (size_t)n * 4);
     if (nw > 0) memcpy(h->h_want, want, (size_t)nw * 4);
     h->h_dyn[0] = pos0; h->h_dyn[1] = seq;
-    HY_HIP(hipMemcpyAsync(h->dyn, h->h_dyn, (size_t)(4 + h->want_cap + n) * 4, hipMemcpyHostToDevice, st));
-    hipLaunchKernelGGL((hy_embed_kernel<T>), dim3(n, hy_cdiv(W, n <= 32 ? 256 : 1024)), dim3(256), 0, st, h->tokens, (const T*)h->emb.w, h->X, W, S, sstride, h->emb_scale, (float*)nullptr);
+    const int* host = n <= GL3_HOST_TOKENS ? h->h_dyn : nullptr;
+    if (!host) HY_HIP(hipMemcpyAsync(h->dyn, h->h_dyn, (size_t)(4 + h->want_cap + n) * 4, hipMemcpyHostToDevice, st));
+    hipLaunchKernelGGL((hy_embed_kernel<T>), dim3(n, hy_cdiv(W, n <= 32 ? 256 : 1024)), dim3(256), 0, st, host, h->dyn, 4 + h->want_cap, nw, (const T*)h->emb.w, h->X, W, S, sstride, h->emb_scale, (float*)nullptr);
     T* hb = (T*)h->h;
     const int nl = (int)h->L.size();
     hy_streams<T>(ctx, n, h->X, W, S, sstride, (const float*)nullptr, 1, 0, (const float*)nullptr, (const float*)nullptr,
@@ -1781,6 +1785,7 @@ int32_t gl3_hy_step(gl3_ctx* ctx, int32_t seq, const int32_t* tokens, int32_t n,
     for (int i = 0; i < n_want; ++i)
         if (want[i] < 0 || want[i] >= n || (i && want[i] <= want[i - 1])) GL3_FAIL(GL3_E_ARG, "want must be ascending indices into the step's tokens");
     HY_HIP(hipSetDevice(ctx->d.device));
+    gl3_drain drain{ctx->stream};
     const size_t V = ctx->d.vocab;
     int wi = 0;
     for (int off = 0; off < n; off += h->mb) {
@@ -1811,7 +1816,7 @@ int32_t gl3_hy_step(gl3_ctx* ctx, int32_t seq, const int32_t* tokens, int32_t n,
             }
             if (r != GL3_OK) return r;
             h->last_tok[seq] = tokens[off + pn - 1];
-            if (g > 0 && logits_out) HY_HIP(hipMemcpyAsync(h->h_logits, h->logits, (size_t)g * V * 4, hipMemcpyDeviceToHost, ctx->stream));
+            if (g > 0 && logits_out) { launch_to_host(h->logits, h->h_logits, (size_t)g * V, ctx->stream); HY_HIP(hipGetLastError()); }
             HY_HIP(hipStreamSynchronize(ctx->stream));
             if (g > 0 && logits_out) memcpy(logits_out + (size_t)done * V, h->h_logits, (size_t)g * V * 4);
             done += g;
@@ -1819,13 +1824,14 @@ int32_t gl3_hy_step(gl3_ctx* ctx, int32_t seq, const int32_t* tokens, int32_t n,
         wi = we;
         h->last_n = pn;
     }
+    drain.passed = true;
     h->len[seq] = start_pos + n;
     return GL3_OK;
 }
 
 int32_t gl3_hy_argmax(gl3_ctx* ctx, int32_t* out) {
-    hipLaunchKernelGGL(argmax_kernel, dim3(AMX_WGS), dim3(256), 0, ctx->stream, ctx->hy->logits, ctx->d.vocab, ctx->argmax);
-    HY_HIP(hipMemcpyAsync(ctx->h_argmax, ctx->argmax, sizeof(int), hipMemcpyDeviceToHost, ctx->stream));
+    hipLaunchKernelGGL(argmax_kernel, dim3(AMX_WGS), dim3(256), 0, ctx->stream, ctx->hy->logits, ctx->d.vocab, ctx->argmax, ctx->h_argmax);
+    HY_HIP(hipGetLastError());
     HY_HIP(hipStreamSynchronize(ctx->stream));
     *out = *ctx->h_argmax;
     return GL3_OK;

@@ -62,7 +62,6 @@ struct gl3_prefill_state {
     int logits_rows = 0;
     std::vector<hipGraphExec_t> step_graphs;   // static-batched decode: one captured step per batch size (positions < AF_MAXN)
     bool in_arena = false;              // X / AO / HB / LOGITS are slices of the tensor-parallel arena (not freed here)
-    int32_t* amax = nullptr;            // [M]
     float* amx_v = nullptr;             // [M][AMX_SPLIT] partial maxima of the greedy scan
     int* amx_i = nullptr;
     int maxk = 0;
@@ -81,8 +80,8 @@ struct gl3_prefill_state {
 __device__ __forceinline__ size_t chunked(int b, int j, int cc, int ntok) { return ((size_t)(j / cc) * ntok + b) * cc + (j % cc); }
 
 __global__ __launch_bounds__(256) void pf_embed_kernel(const uint8_t* __restrict__ emb, int ng, int dim,
-                                                        const int32_t* __restrict__ tokens, float* __restrict__ X, int cc, float emb_scale) {
-    const int token = tokens[blockIdx.x];
+                                                        const int32_t* host, int32_t* __restrict__ rec, int M, float* __restrict__ X, int cc, float emb_scale) {
+    const int token = pf_step_token(host, rec, M);
     const uint8_t* strip = emb + (size_t)(token >> 4) * ng * TILE_BYTES;
     const int i16 = token & 15;
     const int bt = blockIdx.x, nt = gridDim.x;
@@ -1698,12 +1697,12 @@ __global__ __launch_bounds__(256) void pf_argmax_part_kernel(const float* __rest
         pv[row * AMX_SPLIT + seg] = best; pi[row * AMX_SPLIT + seg] = idx;
     }
 }
-__global__ __launch_bounds__(64) void pf_argmax_fold_kernel(const float* __restrict__ pv, const int* __restrict__ pi, int32_t* __restrict__ out) {
+__global__ __launch_bounds__(64) void pf_argmax_fold_kernel(const float* __restrict__ pv, const int* __restrict__ pi, int32_t* __restrict__ host) {
     const int row = blockIdx.x, t = threadIdx.x;
     float best = t < AMX_SPLIT ? pv[row * AMX_SPLIT + t] : -INFINITY;
     int idx = t < AMX_SPLIT ? pi[row * AMX_SPLIT + t] : 0x7FFFFFFF;
     for (int m = 32; m >= 1; m >>= 1) amx_fold(best, idx, __shfl_xor(best, m, 64), __shfl_xor(idx, m, 64));
-    if (t == 0) out[row] = idx == 0x7FFFFFFF ? 0 : idx;
+    if (t == 0) host[row] = idx == 0x7FFFFFFF ? 0 : idx;
 }
 
 // ------------------------------------------------------------------------------------------------ host side
@@ -2214,12 +2213,11 @@ int32_t gl3_prefill_alloc(gl3_ctx* ctx) {
         p->tmx_tiles = (d.ctx + 63) / 64;
         GL3_HIP(hipMalloc((void**)&p->TMX, M * d.n_heads * (size_t)p->tmx_tiles * 4));
         GL3_HIP(hipMalloc((void**)&p->SUMS, M * d.n_heads * 4));
-        GL3_HIP(hipMalloc((void**)&p->amax, M * sizeof(int32_t)));
         GL3_HIP(hipMalloc((void**)&p->amx_v, M * AMX_SPLIT * sizeof(float)));
         GL3_HIP(hipMalloc((void**)&p->amx_i, M * AMX_SPLIT * sizeof(int)));
         if (getenv("GL3_DEBUG_ALLOC"))
-            fprintf(stderr, "[gl3 alloc vl] M %zu tokens %p X %p XN %p AO %p HB %p HB2 %p QKV %p ATT %p seqpos %p amax %p (dim %d hidden %d qdim %d ctx %d)\n", M, (void*)p->tokens,
-                    (void*)p->X, (void*)p->XN, (void*)p->AO, (void*)p->HB, (void*)p->HB2, (void*)p->QKV, (void*)p->ATT, (void*)p->seqpos, (void*)p->amax, d.dim, d.hidden, ctx->q_dim, d.ctx);
+            fprintf(stderr, "[gl3 alloc vl] M %zu tokens %p X %p XN %p AO %p HB %p HB2 %p QKV %p ATT %p seqpos %p (dim %d hidden %d qdim %d ctx %d)\n", M, (void*)p->tokens,
+                    (void*)p->X, (void*)p->XN, (void*)p->AO, (void*)p->HB, (void*)p->HB2, (void*)p->QKV, (void*)p->ATT, (void*)p->seqpos, d.dim, d.hidden, ctx->q_dim, d.ctx);
         GL3_HIP(hipFuncSetAttribute((const void*)gemm_f16_mfma_kernel<EPI_STORE>, hipFuncAttributeMaxDynamicSharedMemorySize, 2 * F16G_STAGE));
         GL3_HIP(hipFuncSetAttribute((const void*)gemm_f16_mfma_kernel<EPI_RESID>, hipFuncAttributeMaxDynamicSharedMemorySize, 2 * F16G_STAGE));
         GL3_HIP(hipFuncSetAttribute((const void*)gemm_vlq_kernel<WT_Q4_0, EPI_STORE>, hipFuncAttributeMaxDynamicSharedMemorySize, 2 * vlq_stage_floats<WT_Q4_0>() * 4));
@@ -2275,7 +2273,6 @@ int32_t gl3_prefill_alloc(gl3_ctx* ctx) {
     p->tmx_tiles = (d.ctx + 63) / 64;
     GL3_HIP(hipMalloc((void**)&p->TMX, M * d.n_heads * (size_t)p->tmx_tiles * 4));
     GL3_HIP(hipMalloc((void**)&p->SUMS, M * d.n_heads * 4));
-    GL3_HIP(hipMalloc((void**)&p->amax, M * sizeof(int32_t)));
     GL3_HIP(hipMalloc((void**)&p->amx_v, M * AMX_SPLIT * sizeof(float)));
     GL3_HIP(hipMalloc((void**)&p->amx_i, M * AMX_SPLIT * sizeof(int)));
 #define GL3_GEMM_LDS(...) GL3_HIP(hipFuncSetAttribute((const void*)pf_gemm_kernel<__VA_ARGS__>, hipFuncAttributeMaxDynamicSharedMemorySize, 2 * gm_stage_bytes(128)))
@@ -2306,7 +2303,7 @@ void gl3_prefill_free(gl3_ctx* ctx) {
     if (!p) return;
     for (auto ge : p->step_graphs) if (ge) hipGraphExecDestroy(ge);
     auto f = [](void* q) { if (q) hipFree(q); };
-    f(p->tokens); f(p->XQ); f(p->XS); f(p->XP); f(p->XQh); f(p->XPh); f(p->XQb); f(p->XSb); f(p->QKV); f(p->ATT); f(p->TMX); f(p->SUMS); f(p->amax); f(p->amx_v); f(p->amx_i); f(p->XN); f(p->HB2);
+    f(p->tokens); f(p->XQ); f(p->XS); f(p->XP); f(p->XQh); f(p->XPh); f(p->XQb); f(p->XSb); f(p->QKV); f(p->ATT); f(p->TMX); f(p->SUMS); f(p->amx_v); f(p->amx_i); f(p->XN); f(p->HB2);
     if (!p->in_arena) { f(p->X); f(p->AO); f(p->HB); f(p->LOGITS); }
     for (auto q : p->h_log) if (q) hipHostFree(q);
     for (auto e : p->log_ev) if (e) hipEventDestroy(e);
@@ -2604,6 +2601,14 @@ static void launch_gemm_vl(gl3_ctx* ctx, const Q8Mat& w, int ntok, const float* 
     }
 }
 
+// The step's (token, sequence, position) triples: a few are read over the link by the embedding (*host), many take one copy.
+static int32_t pf_stage_tokens(gl3_ctx* ctx, int n, int32_t** host) {
+    gl3_prefill_state* p = ctx->pf;
+    *host = n <= GL3_HOST_TOKENS ? p->h_io : nullptr;
+    if (!*host) GL3_HIP(hipMemcpyAsync(p->tokens, p->h_io, ((size_t)2 * p->max_batch + n) * sizeof(int32_t), hipMemcpyHostToDevice, ctx->stream));
+    return GL3_OK;
+}
+
 // The same layers for F16 / Q4_0 / Q8_0-with-f32-activation matrices: RMSNorm to f32 (exact sum of squares), GEMMs on the f32
 // activations, gate and up as two GEMMs + an element-wise SwiGLU.  Tensor parallel (r4): the row-split matrices write this rank's
 // chunk of the rank-chunked X / AO / HB (as the int8 path does), the gathers are in place, and the next GEMM's operand is the
@@ -2619,10 +2624,12 @@ static int32_t pf_layers_vl(gl3_ctx* ctx, int n, int max_pos, int one_seq) {
     float* AOr = p->AO + (size_t)rank * n * qd;
     float* HBr = p->HB + (size_t)rank * n * hid;
     int32_t r;
+    int32_t* host;
+    if ((r = pf_stage_tokens(ctx, n, &host)) != GL3_OK) return r;
     // every rank holds the whole embedding table: the full X, written in the rank-chunked layout
-    if (ctx->emb.fmt == GL3_TYPE_F16) hipLaunchKernelGGL((pf_embed_vl_kernel<WT_F16>), dim3(n), dim3(256), 0, s, ctx->emb.w, d.dim, p->tokens, p->X, ctx->emb_scale, dml);
-    else if (ctx->emb.fmt == GL3_TYPE_Q4_0) hipLaunchKernelGGL((pf_embed_vl_kernel<WT_Q4_0>), dim3(n), dim3(256), 0, s, ctx->emb.w, d.dim, p->tokens, p->X, ctx->emb_scale, dml);
-    else hipLaunchKernelGGL((pf_embed_vl_kernel<WT_Q8_0>), dim3(n), dim3(256), 0, s, ctx->emb.w, d.dim, p->tokens, p->X, ctx->emb_scale, dml);
+    if (ctx->emb.fmt == GL3_TYPE_F16) hipLaunchKernelGGL((pf_embed_vl_kernel<WT_F16>), dim3(n), dim3(256), 0, s, ctx->emb.w, d.dim, host, p->tokens, p->max_batch, p->X, ctx->emb_scale, dml);
+    else if (ctx->emb.fmt == GL3_TYPE_Q4_0) hipLaunchKernelGGL((pf_embed_vl_kernel<WT_Q4_0>), dim3(n), dim3(256), 0, s, ctx->emb.w, d.dim, host, p->tokens, p->max_batch, p->X, ctx->emb_scale, dml);
+    else hipLaunchKernelGGL((pf_embed_vl_kernel<WT_Q8_0>), dim3(n), dim3(256), 0, s, ctx->emb.w, d.dim, host, p->tokens, p->max_batch, p->X, ctx->emb_scale, dml);
     const size_t nq = (size_t)(d.dim + 32) * 4 + ss_scratch_bytes(d.dim) + 64;
     auto unchunk = [&](const float* src, int k, int cc) {          // rank-chunked [tp][n][cc] -> plain XN[n][k] (tp = 1: a copy the GEMM could skip, kept for one code path)
         hipLaunchKernelGGL((pf_norm_quant_kernel<PQ_PLAIN_F32>), dim3(n, (k / 4 + 255) / 256), dim3(256), 0, s, src, k, cc, (const float*)nullptr, 0.f, (uint8_t*)nullptr, p->XN, 0, 0);
@@ -2663,7 +2670,7 @@ static int32_t pf_layers_vl(gl3_ctx* ctx, int n, int max_pos, int one_seq) {
     return GL3_OK;
 }
 
-// All layers for n tokens whose (token, sequence, position) are already on the device.  max_pos = largest position.
+// All layers for n tokens whose (token, sequence, position) stand in h_io (every call that used it has been waited for: gl3_drain).  max_pos = largest position.
 // one_seq >= 0: all n tokens belong to that sequence at consecutive positions ending at max_pos (prefill).
 static int32_t pf_layers(gl3_ctx* ctx, int n, int max_pos, int one_seq) {
     Gl3Range chunk_range("gl3 batched step, tokens", n);
@@ -2684,7 +2691,9 @@ static int32_t pf_layers(gl3_ctx* ctx, int n, int max_pos, int one_seq) {
     float* AOr = p->AO + (size_t)rank * n * qd;
     float* HBr = p->HB + (size_t)rank * n * hid;
     int32_t r;
-    hipLaunchKernelGGL(pf_embed_kernel, dim3(n), dim3(256), 0, s, ctx->emb.w, ctx->emb.ng, d.dim, p->tokens, p->X, dml, ctx->emb_scale);
+    int32_t* host;
+    if ((r = pf_stage_tokens(ctx, n, &host)) != GL3_OK) return r;
+    hipLaunchKernelGGL(pf_embed_kernel, dim3(n), dim3(256), 0, s, ctx->emb.w, ctx->emb.ng, d.dim, host, p->tokens, p->max_batch, p->X, dml, ctx->emb_scale);
     auto nq_smem = [&](int k) { return (size_t)(k + 32) * 4 + ss_scratch_bytes(k) + 64; };
     for (int l = 0; l < d.n_layers; ++l) {
         gl3_layer& L = ctx->layers[l];
@@ -2739,19 +2748,6 @@ static __global__ void pf_unchunk_row_kernel(const float* __restrict__ X, int b,
     for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < dim; i += gridDim.x * blockDim.x) out[i] = X[chunked(b, i, cc, ntok)];
 }
 
-// Pinned memory of the plan (h_io, h_log) belongs to a call until the stream has passed it: a call that fails behind its first copy waits as well.
-struct PfDrain {
-    hipStream_t stream;
-    bool passed = false;
-    ~PfDrain() { if (!passed) (void)hipStreamSynchronize(stream); }
-};
-// The step's (token, sequence, position) triples: one copy from pinned memory.  Every call that used h_io has been waited for (PfDrain).
-static int32_t pf_stage_tokens(gl3_ctx* ctx, int n) {
-    gl3_prefill_state* p = ctx->pf;
-    GL3_HIP(hipMemcpyAsync(p->tokens, p->h_io, ((size_t)2 * p->max_batch + n) * sizeof(int32_t), hipMemcpyHostToDevice, ctx->stream));
-    return GL3_OK;
-}
-
 // Result memory the caller has just got from the system has no pages yet, and taking them one fault at a time costs more than the copy that follows
 // (2 MB: 430 us, 30 with pages).  The pages are touched while the device still works on the step.
 static inline void pf_touch_pages(void* mem, size_t bytes) {
@@ -2783,7 +2779,8 @@ static int32_t pf_logits_out(gl3_ctx* ctx, float* out, size_t bytes) {
     const size_t pieces = pf_logits_pieces(bytes), per = ((bytes + pieces - 1) / pieces + 4095) & ~(size_t)4095;
     auto send = [&](size_t i) -> int32_t {
         if (i * per >= bytes) return GL3_OK;
-        GL3_HIP(hipMemcpyAsync(p->h_log[i % PF_LOG_SLOTS], (const uint8_t*)p->LOGITS + i * per, std::min(per, bytes - i * per), hipMemcpyDeviceToHost, ctx->stream));
+        launch_to_host(p->LOGITS + i * per / 4, (float*)p->h_log[i % PF_LOG_SLOTS], std::min(per, bytes - i * per) / 4, ctx->stream);
+        GL3_HIP(hipGetLastError());
         GL3_HIP(hipEventRecord(p->log_ev[i % PF_LOG_SLOTS], ctx->stream));
         return GL3_OK;
     };
@@ -2805,10 +2802,9 @@ int32_t gl3_prefill_run(gl3_ctx* ctx, int32_t seq, const int32_t* tokens, int32_
         if (tokens[i] < 0 || tokens[i] >= d.vocab) GL3_FAIL(GL3_E_ARG, "token id out of range");
     GL3_HIP(hipSetDevice(d.device));
     for (int i = 0; i < n; ++i) { p->h_io[i] = tokens[i]; p->h_io[p->max_batch + i] = seq; p->h_io[2 * p->max_batch + i] = start_pos + i; }
-    PfDrain drain{ctx->stream};
-    int32_t r = pf_stage_tokens(ctx, n);
+    gl3_drain drain{ctx->stream};
+    int32_t r = pf_layers(ctx, n, start_pos + n - 1, seq);
     if (r != GL3_OK) return r;
-    if ((r = pf_layers(ctx, n, start_pos + n - 1, seq)) != GL3_OK) return r;
     // keep the decode path's x in step with the last prefilled token (parity tap gl3_get_x)
     hipLaunchKernelGGL(pf_unchunk_row_kernel, dim3(4), dim3(256), 0, ctx->stream, p->X, n - 1, d.dim, ctx->dim_l, n, ctx->x);
     GL3_HIP(hipStreamSynchronize(ctx->stream));
@@ -2834,9 +2830,8 @@ int32_t gl3_decode_batch_run(gl3_ctx* ctx, const int32_t* tokens, const int32_t*
     int max_pos = 0;
     for (int i = 0; i < n; ++i) max_pos = positions[i] > max_pos ? positions[i] : max_pos;
     for (int i = 0; i < n; ++i) { p->h_io[i] = tokens[i]; p->h_io[p->max_batch + i] = seq_ids[i]; p->h_io[2 * p->max_batch + i] = positions[i]; }
-    PfDrain drain{ctx->stream};
-    int32_t r = pf_stage_tokens(ctx, n);
-    if (r != GL3_OK) return r;
+    gl3_drain drain{ctx->stream};
+    int32_t r;
     hipStream_t s = ctx->stream;
     const int vl = ctx->vocab_l;
     // the whole step: layers, final RMSNorm + vocabulary projection of every row, greedy ids
@@ -2854,7 +2849,7 @@ int32_t gl3_decode_batch_run(gl3_ctx* ctx, const int32_t* tokens, const int32_t*
         }
         if ((rr = gl3_all_gather(ctx, GB_PF_LOGITS, (size_t)n * vl)) != GL3_OK) return rr;
         hipLaunchKernelGGL(pf_argmax_part_kernel, dim3(AMX_SPLIT, n), dim3(256), 0, s, p->LOGITS, d.vocab, vl, p->amx_v, p->amx_i);
-        hipLaunchKernelGGL(pf_argmax_fold_kernel, dim3(n), dim3(64), 0, s, p->amx_v, p->amx_i, p->amax);
+        hipLaunchKernelGGL(pf_argmax_fold_kernel, dim3(n), dim3(64), 0, s, p->amx_v, p->amx_i, p->h_io + 3 * p->max_batch);
         return GL3_OK;
     };
     // ~400 launches per step: replay them as one hipGraph per batch size.  Nothing position-dependent is baked in when every
@@ -2875,7 +2870,6 @@ int32_t gl3_decode_batch_run(gl3_ctx* ctx, const int32_t* tokens, const int32_t*
         }
         GL3_HIP(hipGraphLaunch(p->step_graphs[n], s));
     } else if ((r = enqueue_step(max_pos)) != GL3_OK) return r;
-    if (argmax_out) GL3_HIP(hipMemcpyAsync(p->h_io + 3 * p->max_batch, p->amax, (size_t)n * sizeof(int32_t), hipMemcpyDeviceToHost, s));
     const size_t logit_bytes = (size_t)n * d.vocab * 4;
     if (logits_out && d.tp_size == 1 && !pf_page_locked(logits_out) && pf_logits_slots(p, logit_bytes)) {
         if ((r = pf_logits_out(ctx, logits_out, logit_bytes)) != GL3_OK) return r;

@@ -479,11 +479,24 @@ static __global__ __launch_bounds__(256) void pf_swiglu_kernel(float* __restrict
 }
 
 // token_embedding_table.copyTo per token of the batch (batchForwardJavaPrefill :96), VL layouts
+// The first kernel of a batched step reads its (token, sequence, position) triples ([3][M]) in page-locked host memory and leaves a copy in rec (host null: they are there).
+__device__ __forceinline__ int pf_step_token(const int32_t* host, int32_t* rec, int M) {
+    const int b = blockIdx.x;
+    if (!host) return rec[b];
+    __shared__ int token;
+    if (threadIdx.x < 3) {
+        const int v = host_int(host + threadIdx.x * M + b);
+        rec[threadIdx.x * M + b] = v;
+        if (threadIdx.x == 0) token = v;
+    }
+    __syncthreads();
+    return token;
+}
 template <int WT>
-static __global__ __launch_bounds__(256) void pf_embed_vl_kernel(const uint8_t* __restrict__ emb, int dim, const int32_t* __restrict__ tokens,
+static __global__ __launch_bounds__(256) void pf_embed_vl_kernel(const uint8_t* __restrict__ emb, int dim, const int32_t* host, int32_t* __restrict__ rec, int M,
                                                                  float* __restrict__ X, float emb_scale, int cc) {
     // X is rank-chunked [dim / cc][ntok][cc] (cc = dim: the plain [ntok][dim]); element i of token b at ((i / cc) ntok + b) cc + i % cc
-    const int token = tokens[blockIdx.x], g = token >> 3, rr = token & 7;
+    const int token = pf_step_token(host, rec, M), g = token >> 3, rr = token & 7;
     const uint8_t* gb = emb + (size_t)g * vl_group_bytes(WT, dim);
     const int bt = blockIdx.x, nt = gridDim.x;
 #define x(I_) X[((size_t)((I_) / cc) * nt + bt) * cc + (I_) % cc]

@@ -52,11 +52,11 @@ static __global__ __launch_bounds__(256) void repack_rl_kernel(const uint8_t* __
 
 // token_embedding_table.copyTo -> getFloat per element (InferenceCore.java:61)
 template <int WT>
-static __global__ __launch_bounds__(256) void embed_rl_kernel(const uint8_t* __restrict__ emb, int dim, const int* __restrict__ dyn,
+static __global__ __launch_bounds__(256) void embed_rl_kernel(const uint8_t* __restrict__ emb, int dim, int* dyn, const int* host,
                                                               float* __restrict__ x, float emb_scale) {
-    const int token = dyn[0], g = token >> 6, lane = token & 63;
+    const int token = step_token(dyn, host), g = token >> 6, lane = token & 63;
     const uint8_t* gb = emb + (size_t)g * rl_group_bytes(WT, dim);
-    for (int i = threadIdx.x; i < dim; i += 256) {
+    for (int i = blockIdx.x * 256 + threadIdx.x; i < dim; i += 256 * gridDim.x) {
         if (WT == WT_F16) {
             x[i] = h2f(*reinterpret_cast<const uint16_t*>(gb + (size_t)(i >> 3) * 1024 + lane * 16 + 2 * (i & 7))) * emb_scale;
         } else {

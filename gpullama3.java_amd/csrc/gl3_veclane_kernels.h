@@ -73,16 +73,16 @@ static __global__ __launch_bounds__(256) void repack_vl_kernel(const uint8_t* __
 
 // token_embedding_table.copyTo -> getFloat per element (InferenceCore.java:61): SCALAR semantics (IEEE f16 -> f32)
 template <int WT>
-static __global__ __launch_bounds__(256) void embed_vl_kernel(const uint8_t* __restrict__ emb, int dim, const int* __restrict__ dyn,
+static __global__ __launch_bounds__(256) void embed_vl_kernel(const uint8_t* __restrict__ emb, int dim, int* dyn, const int* host,
                                                               float* __restrict__ x, float emb_scale, uint32_t* step = nullptr) {
     if (step) {                              // folded gathers: the kernel opens decode step *step + 1 of the plan (as embed_q8t_kernel; the wait for the
         const uint32_t s0 = *step;           // previous step's last pushes into x is the wait launch behind the last down projection)
         __syncthreads();
         if (threadIdx.x == 0) *step = s0 + 1;
     }
-    const int token = dyn[0], g = token >> 3, rr = token & 7;
+    const int token = step_token(dyn, host), g = token >> 3, rr = token & 7;
     const uint8_t* gb = emb + (size_t)g * vl_group_bytes(WT, dim);
-    for (int i = threadIdx.x; i < dim; i += 256) {
+    for (int i = blockIdx.x * 256 + threadIdx.x; i < dim; i += 256 * gridDim.x) {
         if (WT == WT_F16) {
             const int c = i >> 6, e = i & 63, l = e & 7, kk = e >> 3;
             x[i] = h2f(reinterpret_cast<const uint16_t*>(gb + (size_t)c * 1024 + (rr * 8 + l) * 16)[kk]) * emb_scale;
