@@ -731,12 +731,12 @@ __global__ __launch_bounds__(256) void pf_scores_tiled_kernel(const float* __res
     }
 }
 
-// r6 — pf_scores_tiled_kernel on packed f32: two tokens' chains advance in ONE register pair, {s_a, s_b} = {s_a, s_b} + {q_a[j], q_b[j]} * k[j]
-// (v_pk_mul_f32 + v_pk_add_f32: every product and every sum rounded as before, j ascending), two pairs side by side per wavefront.  The query
+// pf_scores_tiled_kernel with the query rows through LDS: four tokens' chains advance side by side in a wavefront, s_b = s_b + q_b[j] * k[j]
+// (v_mul_f32 + v_add_f32: every product and every sum rounded as the reference does, j ascending; packed f32 is off, see the Makefile).  The query
 // rows of the tile's 16 tokens reach LDS once per workgroup, interleaved by token pairs ([head][pair][j][2]), so a 16-byte broadcast read is
-// two steps of a pair; the reads of the next group of 8 steps are pinned under the current group's 32 packed instructions.  (The scalar-load
+// two steps of a pair; the reads of the next group of 8 steps are pinned under the current group's instructions.  (The scalar-load
 // form feeds q through SGPRs: its lead is bounded by the SGPR file — one group of 16 steps — and the scalar cache misses to L2 at 32 KB of
-// query rows per workgroup.)  K rows in registers as before, lane = timestep.  Two wavefronts per SIMD (~210 VGPRs, 65 KB of LDS).
+// query rows per workgroup.)  K rows in registers as before, lane = timestep.  Two wavefronts per SIMD (~240 VGPRs, 65 KB of LDS).
 typedef float v2f_native __attribute__((ext_vector_type(2)));
 typedef float v4f_native_s __attribute__((ext_vector_type(4)));
 template <int HS, int KVM>
@@ -793,20 +793,20 @@ __global__ __launch_bounds__(64 * KVM) __attribute__((amdgpu_waves_per_eu(2, 2))
     for (int pp = 0; 4 * pp < nb; ++pp) {
         const float* q01 = qs + (size_t)(hq * (PA_TB / 2) + 2 * pp) * HS * 2;      // pairs (4 pp, 4 pp + 1) and (4 pp + 2, 4 pp + 3)
         const float* q23 = q01 + HS * 2;
-        v2f_native c0 = {0.f, 0.f}, c1 = {0.f, 0.f};
+        float sv[4] = {0.f, 0.f, 0.f, 0.f};                            // tokens 4 pp .. 4 pp + 3
         v4f_native_s qa[8], qb[8];                                     // two groups of 8 steps: [0..3] pair 0, [4..7] pair 1
 #define SPK_LD(G_, R_) do { _Pragma("unroll") for (int i_ = 0; i_ < 4; ++i_) { \
             R_[i_] = *reinterpret_cast<const v4f_native_s*>(q01 + 16 * (G_) + 4 * i_); R_[4 + i_] = *reinterpret_cast<const v4f_native_s*>(q23 + 16 * (G_) + 4 * i_); } } while (0)
-        // two steps of both pairs in one block: the K value is broadcast out of its register pair by op_sel (the compiler materialises {k, k}
-        // pairs instead: twice the K registers), and every dependent instruction has an independent one in front of it (packed f32 needs a wait
-        // state between a result and its use)
-#define SPK_STEP2(QA_, QB_, K_) do { v2f_native p0_, p1_; \
-            asm("v_pk_mul_f32 %[p0], %[qa0], %[k] op_sel_hi:[1,0]\n\tv_pk_mul_f32 %[p1], %[qb0], %[k] op_sel_hi:[1,0]\n\t" \
-                "v_pk_add_f32 %[c0], %[c0], %[p0]\n\tv_pk_add_f32 %[c1], %[c1], %[p1]\n\t" \
-                "v_pk_mul_f32 %[p0], %[qa1], %[k] op_sel:[0,1]\n\tv_pk_mul_f32 %[p1], %[qb1], %[k] op_sel:[0,1]\n\t" \
-                "v_pk_add_f32 %[c0], %[c0], %[p0]\n\tv_pk_add_f32 %[c1], %[c1], %[p1]" \
-                : [c0] "+v"(c0), [c1] "+v"(c1), [p0] "=&v"(p0_), [p1] "=&v"(p1_) \
-                : [qa0] "v"(QA_.xy), [qa1] "v"(QA_.zw), [qb0] "v"(QB_.xy), [qb1] "v"(QB_.zw), [k] "v"(K_)); } while (0)
+        // two steps of four tokens in one block: left to itself the compiler reads the K row from LDS again for every token (15 x slower), and every dependent
+        // instruction has three independent ones in front of it
+#define SPK_STEP2(QA_, QB_, K_) do { float p0_, p1_, p2_, p3_; \
+            asm("v_mul_f32 %[p0], %[a0], %[k0]\n\tv_mul_f32 %[p1], %[a1], %[k0]\n\tv_mul_f32 %[p2], %[b0], %[k0]\n\tv_mul_f32 %[p3], %[b1], %[k0]\n\t" \
+                "v_add_f32 %[c0], %[c0], %[p0]\n\tv_add_f32 %[c1], %[c1], %[p1]\n\tv_add_f32 %[c2], %[c2], %[p2]\n\tv_add_f32 %[c3], %[c3], %[p3]\n\t" \
+                "v_mul_f32 %[p0], %[a2], %[k1]\n\tv_mul_f32 %[p1], %[a3], %[k1]\n\tv_mul_f32 %[p2], %[b2], %[k1]\n\tv_mul_f32 %[p3], %[b3], %[k1]\n\t" \
+                "v_add_f32 %[c0], %[c0], %[p0]\n\tv_add_f32 %[c1], %[c1], %[p1]\n\tv_add_f32 %[c2], %[c2], %[p2]\n\tv_add_f32 %[c3], %[c3], %[p3]" \
+                : [c0] "+v"(sv[0]), [c1] "+v"(sv[1]), [c2] "+v"(sv[2]), [c3] "+v"(sv[3]), [p0] "=&v"(p0_), [p1] "=&v"(p1_), [p2] "=&v"(p2_), [p3] "=&v"(p3_) \
+                : [a0] "v"(QA_.x), [a1] "v"(QA_.y), [a2] "v"(QA_.z), [a3] "v"(QA_.w), [b0] "v"(QB_.x), [b1] "v"(QB_.y), [b2] "v"(QB_.z), [b3] "v"(QB_.w), \
+                  [k0] "v"(K_.x), [k1] "v"(K_.y)); } while (0)
 #define SPK_ACC(G_, R_) do { SPK_STEP2(R_[0], R_[4], kr[4 * (G_)]); SPK_STEP2(R_[1], R_[5], kr[4 * (G_) + 1]); \
             SPK_STEP2(R_[2], R_[6], kr[4 * (G_) + 2]); SPK_STEP2(R_[3], R_[7], kr[4 * (G_) + 3]); } while (0)
         SPK_LD(0, qa); SPK_LD(1, qb); __builtin_amdgcn_sched_barrier(0);
@@ -817,7 +817,6 @@ __global__ __launch_bounds__(64 * KVM) __attribute__((amdgpu_waves_per_eu(2, 2))
             SPK_ACC(g + 1, qb);
             SPK_LD((g + 3 < NGR ? g + 3 : NGR - 1), qb); __builtin_amdgcn_sched_barrier(0);
         });
-        const float sv[4] = {c0.x, c0.y, c1.x, c1.y};
 #pragma unroll
         for (int u = 0; u < 4; ++u) {
             const int tb = 4 * pp + u, b = b0 + tb;
@@ -1494,10 +1493,10 @@ __global__ __launch_bounds__(512) void pf_attn_fused2_kernel(const float* __rest
                 const v4f_native_s x = *reinterpret_cast<const v4f_native_s*>(ktg + min(lane, t1 - t0 - 1) * PITCH + 4 * c);
                 kr[2 * c] = x.xy; kr[2 * c + 1] = x.zw;
             }
-            for (int pp = 0; 4 * pp < nb; ++pp) {                    // four tokens = two packed chains per pass (pf_scores_pk_kernel's inner loop)
+            for (int pp = 0; 4 * pp < nb; ++pp) {                    // four tokens' chains per pass (pf_scores_pk_kernel's inner loop)
                 const float* q01 = qs + (size_t)(hq * (FA_TB / 2) + 2 * pp) * HS * 2;
                 const float* q23 = q01 + HS * 2;
-                v2f_native c0 = {0.f, 0.f}, c1 = {0.f, 0.f};
+                float sv[4] = {0.f, 0.f, 0.f, 0.f};
                 v4f_native_s qa[8], qb[8];
                 SPK_LD(0, qa); SPK_LD(1, qb); __builtin_amdgcn_sched_barrier(0);
                 static_for<0, HS / 8, 2>([&](auto gc) {
@@ -1507,7 +1506,6 @@ __global__ __launch_bounds__(512) void pf_attn_fused2_kernel(const float* __rest
                     SPK_ACC(g + 1, qb);
                     SPK_LD((g + 3 < HS / 8 ? g + 3 : HS / 8 - 1), qb); __builtin_amdgcn_sched_barrier(0);
                 });
-                const float sv[4] = {c0.x, c0.y, c1.x, c1.y};
                 const int ts = t0 + lane;
 #pragma unroll
                 for (int u = 0; u < 4; ++u) {

@@ -288,9 +288,8 @@ __global__ __launch_bounds__(256, 2) void gemm_vlq_kernel(const VlGemmArgs a) {
 //   "f32-input MFMA"; a zero product of either sign plus +0 leaves the sums' and the fma's values unchanged).  With block q = the
 //   four elements 8 q + l of a weight block, A = x of 16 tokens and B = the dequantised quants of 16 rows, ONE instruction delivers
 //   the four product tiles P0..P3 of (16 tokens x 16 rows, block, accumulator lane l); the VALU then does the reference's three
-//   adds and the fma with the row's scale on the 4 registers of the tile (v_pk_add_f32 / v_pk_fma_f32): 2 packed VALU
-//   instructions per MFMA-delivered product quad instead of 4, and the matrix pipe (64 FLOP/clk/SIMD, the f32 VALU's own rate)
-//   runs beside them.  Both pipes are ~balanced: 8 packed VALU instructions per 32-cycle MFMA.
+//   adds and the fma with the row's scale on the 4 registers of the tile, and the matrix pipe (64 FLOP/clk/SIMD, the f32 VALU's own rate)
+//   runs beside them.  16 VALU instructions per 32-cycle MFMA.
 // Workgroup = 8 wavefronts = 64 rows x 64 tokens; wavefront (rt, th) = 16 rows x 32 tokens (two tiles) for all 8 accumulator
 // lanes (64 accumulator registers).  K advances 64 elements (two blocks) per stage through double-buffered LDS:
 //   XF[64 tokens][68]                 x, natural order (A operand of lane (q, token): 8 consecutive floats = l 0..7)
@@ -387,12 +386,13 @@ __global__ __launch_bounds__(512, OCC) void gemm_vlq_mfma_kernel(const VlGemmArg
         } \
     } while (0)
 
-    typedef float v2f_q __attribute__((ext_vector_type(2)));
-    v2f_q val[2][8][2];                              // [token tile][accumulator lane][register pair]: tokens 4 (lane >> 4) + 0..3, row lane & 15
+    float val[2][8][4];                              // [token tile][accumulator lane][register]: tokens 4 (lane >> 4) + 0..3, row lane & 15
 #pragma unroll
     for (int tt = 0; tt < 2; ++tt)
 #pragma unroll
-        for (int ll = 0; ll < 8; ++ll) { val[tt][ll][0] = (v2f_q){0.f, 0.f}; val[tt][ll][1] = (v2f_q){0.f, 0.f}; }
+        for (int ll = 0; ll < 8; ++ll)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) val[tt][ll][r] = 0.f;
     const bool live = tok0 + th * 32 < a.ntok;       // a token half past the end only helps staging (static-batched decode, B <= 32)
     const int mq = lane >> 4, mi = lane & 15;        // MFMA operand slot: block q, token / row index
     VQM_WLOAD(0);
@@ -410,38 +410,29 @@ __global__ __launch_bounds__(512, OCC) void gemm_vlq_mfma_kernel(const VlGemmArg
             const float* WS = QF + 2 * VQM_SB;
 #pragma unroll
             for (int b = 0; b < 2; ++b) {
-                float av[2][8], bv[8];
+                float bv[8];
+#pragma unroll
+                for (int ll = 0; ll < 8; ++ll) bv[ll] = QF[b * VQM_SB + ll * VQM_SL + mq * VQM_SQ + rt * 16 + mi];
+                const float ws = WS[b * VQM_ROWS + rt * 16 + mi];
+                // One MFMA, then its 16 VALU instructions, tile after tile.  Issuing the MFMAs ahead of the VALU chain (two or three P buffers) bought nothing — 1380 vs 1290 us for the 8B gate GEMM:
+                // on gfx950 an MFMA (f32 or bf16) and f32 VALU work of the same SIMD do not overlap, not even between two
+                // wavefronts (scripts/probes/mfma_overlap_probe.hip), so the matrix core only REPLACES the product instructions of a tile — the gain
+                // over gemm_vlq_kernel comes from the operand traffic, not from a second pipe.
 #pragma unroll
                 for (int tt = 0; tt < 2; ++tt) {
                     const float* xa = XF + (th * 32 + tt * 16 + mi) * VQM_XP + 32 * b + 8 * mq;
                     const float4 lo = *reinterpret_cast<const float4*>(xa), hi = *reinterpret_cast<const float4*>(xa + 4);
-                    av[tt][0] = lo.x; av[tt][1] = lo.y; av[tt][2] = lo.z; av[tt][3] = lo.w;
-                    av[tt][4] = hi.x; av[tt][5] = hi.y; av[tt][6] = hi.z; av[tt][7] = hi.w;
-                }
+                    const float av[8] = {lo.x, lo.y, lo.z, lo.w, hi.x, hi.y, hi.z, hi.w};
 #pragma unroll
-                for (int ll = 0; ll < 8; ++ll) bv[ll] = QF[b * VQM_SB + ll * VQM_SL + mq * VQM_SQ + rt * 16 + mi];
-                const float ws = WS[b * VQM_ROWS + rt * 16 + mi];
-                const v2f_q ws2 = {ws, ws};
-                // One MFMA, then its 8 packed VALU instructions, tile after tile.  Issuing the MFMAs ahead of the VALU chain (two or
-                // three P buffers, VALU chain pinned in inline assembly) bought nothing — 1380 vs 1290 us for the 8B gate GEMM:
-                // on gfx950 an MFMA (f32 or bf16) and f32 VALU work of the same SIMD do not overlap, not even between two
-                // wavefronts (scripts/probes/mfma_overlap_probe.hip: 4 MFMA 123 ns + 32 v_pk_fma_f32 153 ns = 258 ns together), so
-                // the matrix core only REPLACES the 8 product instructions of a tile at the same cost (32 cycles) — the gain
-                // over gemm_vlq_kernel comes from the operand traffic and the packed adds, not from a second pipe.
-#pragma unroll
-                for (int ll = 0; ll < 8; ++ll)
-#pragma unroll
-                    for (int tt = 0; tt < 2; ++tt) {
+                    for (int ll = 0; ll < 8; ++ll) {
                         const v16f_vl z = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-                        const v16f_vl P = __builtin_amdgcn_mfma_f32_16x16x1f32(av[tt][ll], bv[ll], z, 0, 0, 0);
+                        const v16f_vl P = __builtin_amdgcn_mfma_f32_16x16x1f32(av[ll], bv[ll], z, 0, 0, 0);
 #pragma unroll
-                        for (int h = 0; h < 2; ++h) {
-                            const v2f_q p0 = {P[2 * h], P[2 * h + 1]}, p1 = {P[4 + 2 * h], P[5 + 2 * h]};
-                            const v2f_q p2 = {P[8 + 2 * h], P[9 + 2 * h]}, p3 = {P[12 + 2 * h], P[13 + 2 * h]};
-                            const v2f_q sm2 = ((p0 + p1) + p2) + p3;                                   // sum0.add(sum1).add(sum2).add(sum3)
-                            val[tt][ll][h] = __builtin_elementwise_fma(sm2, ws2, val[tt][ll][h]);     // .fma(wScale, val)
-                        }
+                        for (int r = 0; r < 4; ++r)                                                    // sum0.add(sum1).add(sum2).add(sum3), .fma(wScale, val)
+                            val[tt][ll][r] = __builtin_fmaf(((P[r] + P[4 + r]) + P[8 + r]) + P[12 + r], ws, val[tt][ll][r]);
                     }
+                    __builtin_amdgcn_sched_barrier(0);          // one token tile's operands at a time: 128 registers are two workgroups a CU
+                }
             }
         }
         if ((sn % SPC) == 0) { cq = wq; cs = wsc; }
@@ -462,7 +453,7 @@ __global__ __launch_bounds__(512, OCC) void gemm_vlq_mfma_kernel(const VlGemmArg
             if (b >= a.ntok) continue;
             float v = 0.f;
 #pragma unroll
-            for (int ll = 0; ll < 8; ++ll) v = v + val[tt][ll][r >> 1][r & 1];
+            for (int ll = 0; ll < 8; ++ll) v = v + val[tt][ll][r];
             float* o = a.out + (size_t)b * a.out_stride + row;
             if (EPI == EPI_RESID) *o = *o + v * a.out_scale;
             else *o = v * a.out_scale;
