@@ -23,6 +23,7 @@
 #include "gl3_hy_attn_mfma.h"
 #include "gl3_hy_scan_chunk.h"
 #include "gl3_hy_heads_kernels.h"
+#include "gl3_hy_one_kernels.h"
 #include "gl3_hy_plain_kernels.h"
 
 using gl3::AMX_WGS;
@@ -1292,6 +1293,53 @@ static void hy_mem_out(gl3_ctx* ctx, const HyLayer& L, int n, int ldy, int P, co
 #undef HY_MO
 }
 
+// ---- one token behind few positions: a mixer's kernels in one launch (gl3_hy_one_kernels.h); false: the form or the position is not theirs ----
+template <typename T>
+static bool hy_attn_one(gl3_ctx* ctx, const HyLayer& L, int pos0, const HyRot& rot, const HyPrepX& px, T* out) {
+    gl3_hybrid_state* h = ctx->hy;
+    const gl3_layer_desc& d = L.d;
+    float *kc = h->slots + L.off_k, *vc = h->slots + L.off_v;
+    const int big = std::max(d.dim, d.vdim);
+    if (hy_by_heads(d) || d.qk_conv > 0 || big > 256 || ((d.dim | d.vdim | (int)(h->slot_floats & 3)) & 3) || (((uintptr_t)kc | (uintptr_t)vc) & 15) || (d.window > 0 && pos0 >= d.window)) return false;
+    if ((long)(pos0 + 1) * (d.dim + d.vdim) * 4 > HY_ATTN_ONE) return false;
+    HyAttnOne a{};
+    a.proj = h->proj; a.q_off = L.q_off; a.k_off = L.k_off; a.v_off = L.v_off; a.H = d.heads; a.G = d.kv_heads; a.D = d.dim; a.V = d.vdim; a.unit_norm = d.qk_unit_norm; a.eps = ctx->d.rms_eps;
+    a.kc = kc; a.vc = vc; a.slot_stride = h->slot_floats; a.dyn = h->dyn; a.rot = rot; a.bias = px.bias; a.qn = L.qn; a.kn = L.kn; a.v_from_k = d.v_from_k; a.scale = d.scale; a.slope_log2 = d.slope_log2;
+    a.sink = d.softmax_sink; a.sink_w = d.softmax_sink == 2 ? L.sink : nullptr;
+    a.gate = d.out_gate ? h->proj + L.g_off : nullptr; a.gate_mode = d.out_gate; a.v_freq = d.v_rot ? L.vrot_freq : nullptr; a.out_mul = d.out_norm ? 1.f : L.out_mul;
+#define HY_A1(NI) hipLaunchKernelGGL((hy_attn_one_kernel<T, NI>), dim3(d.heads), dim3(1024), 0, ctx->stream, a, out)
+    if (big <= 64) HY_A1(1); else if (big <= 128) HY_A1(2); else HY_A1(4);
+#undef HY_A1
+    return true;
+}
+template <typename T>
+static bool hy_latent_one(gl3_ctx* ctx, const HyLayer& L, int pos0, const float* q, T* out) {
+    gl3_hybrid_state* h = ctx->hy;
+    const gl3_layer_desc& d = L.d;
+    float* cc = h->slots + L.off_k;
+    if (L.Re > HY_LATENT_ONE || ((L.Re | d.vdim | (int)(h->slot_floats & 3)) & 3) || ((uintptr_t)cc & 15) || pos0 >= HY_LATENT_ONE_POS) return false;
+    HyLatentOne a{};
+    a.q = q; a.D = d.dim; a.P = d.rot_dim; a.src = d.kv_share > 0 ? nullptr : h->proj + L.c_off; a.R0 = d.kv_rank; a.lat_norm = L.lat_norm; a.eps = ctx->d.rms_eps;
+    a.cc = cc; a.slot_stride = h->slot_floats; a.dyn = h->dyn; a.freq = L.lat_freq; a.mscale = L.rot_mscale; a.wk = L.wk; a.wvT = L.wvT; a.R = L.Re; a.V = d.vdim; a.scale = d.scale;
+    a.sink = d.softmax_sink; a.sink_w = d.softmax_sink == 2 ? L.sink : nullptr; a.gate = d.out_gate ? h->proj + L.g_off : nullptr; a.gate_mode = d.out_gate == 2 ? 2 : 1;
+    hipLaunchKernelGGL((hy_latent_one_kernel<T>), dim3(d.heads), dim3(1024), 0, ctx->stream, a, out);
+    return true;
+}
+template <typename T>
+static bool hy_scan_out(gl3_ctx* ctx, const HyLayer& L, const HyScanArgs& s, T* out) {
+    gl3_hybrid_state* h = ctx->hy;
+    const gl3_layer_desc& d = L.d;
+    if (s.mode == 3 || d.mem_norm_whole || s.N > 256 || s.P > HY_SCAN_OUT_P || s.N * s.P > HY_SCAN_OUT || hy_scan_forced(s.N)) return false;
+    HyScanOut b{};
+    b.s = s; b.i_off = L.i_off; b.f_off = L.f_off; b.gbias = L.pbias; b.cap = d.mem_gate_cap; b.m = h->slots + L.off_m;
+    b.gate = d.mem_gate_act == 2 ? nullptr : h->proj + L.g_off; b.gate_act = d.mem_gate_act; b.w = d.mem_norm_weight ? L.ssm_norm : nullptr; b.w_stride = d.mem_norm_weight == 2 ? 0 : d.vdim;
+    b.eps = ctx->d.rms_eps; b.out_mul = d.out_norm ? 1.f : L.out_mul;
+#define HY_SO(QN) hipLaunchKernelGGL((hy_scan_out_kernel<T, QN>), dim3(s.heads), dim3(1024), 0, ctx->stream, b, out)
+    if (s.N <= 64) HY_SO(4); else if (s.N <= 128) HY_SO(8); else HY_SO(16);
+#undef HY_SO
+    return true;
+}
+
 // One mixer of a layer on the n rows of the fused projection in h->proj (row stride np): its heads land in mixo (row stride ldo) from
 // column L.o0 on, multiplied by L.out_mul.
 template <typename T>
@@ -1315,21 +1363,25 @@ static int32_t hy_mixer_core(gl3_ctx* ctx, HyLayer& L, int np, int ldo, int n, i
             px.conv_w = L.qk_conv_w; px.taps = d.qk_conv; px.tail = h->slots + L.off_tail; px.qout = h->conv; px.ldq = d.heads * d.dim; px.n = n;
             q = h->conv; ldq = px.ldq;
         }
-        if (d.qk_unit_norm == 2) {
-            if (n <= 32) hipLaunchKernelGGL((hy_rowrms_kernel<1024>), dim3(n, 2), dim3(1024), 0, st, h->proj, np, L.q_off, d.heads * d.dim, L.k_off, d.kv_heads * d.dim, px.bias, eps, h->rowr);
-            else hipLaunchKernelGGL((hy_rowrms_kernel<256>), dim3(n, 2), dim3(256), 0, st, h->proj, np, L.q_off, d.heads * d.dim, L.k_off, d.kv_heads * d.dim, px.bias, eps, h->rowr);
+        const bool one = n == 1 && hy_attn_one<T>(ctx, L, pos0, rot, px, mixo);          // (pooled blocks that this token completes follow it: no window is passed yet)
+        if (!one) {
+            if (d.qk_unit_norm == 2) {
+                if (n <= 32) hipLaunchKernelGGL((hy_rowrms_kernel<1024>), dim3(n, 2), dim3(1024), 0, st, h->proj, np, L.q_off, d.heads * d.dim, L.k_off, d.kv_heads * d.dim, px.bias, eps, h->rowr);
+                else hipLaunchKernelGGL((hy_rowrms_kernel<256>), dim3(n, 2), dim3(256), 0, st, h->proj, np, L.q_off, d.heads * d.dim, L.k_off, d.kv_heads * d.dim, px.bias, eps, h->rowr);
+            }
+            hipLaunchKernelGGL(hy_attn_prep_kernel, dim3(n, d.heads + (d.v_from_k ? 1 : 2) * d.kv_heads), dim3(64), 0, st, h->proj, np, L.q_off, L.k_off, L.v_off, d.heads, d.kv_heads, d.dim,
+                               d.vdim, d.qk_unit_norm, eps, kc, vc, h->slot_floats, h->dyn, rot, px);
+            if (d.qk_conv > 1 && n > 1)          // (q and k stand side by side in the projection row; a single token's tail moved on above)
+                hipLaunchKernelGGL(hy_conv_tail_kernel, dim3(hy_cdiv(hy_qk_ch(d), 256)), dim3(256), 0, st, h->proj, np, L.q_off, hy_qk_ch(d), d.qk_conv, h->slots + L.off_tail,
+                                   h->slot_floats, h->dyn, n);
         }
-        hipLaunchKernelGGL(hy_attn_prep_kernel, dim3(n, d.heads + (d.v_from_k ? 1 : 2) * d.kv_heads), dim3(64), 0, st, h->proj, np, L.q_off, L.k_off, L.v_off, d.heads, d.kv_heads, d.dim,
-                           d.vdim, d.qk_unit_norm, eps, kc, vc, h->slot_floats, h->dyn, rot, px);
-        if (d.qk_conv > 1 && n > 1)          // (q and k stand side by side in the projection row; a single token's tail moved on above)
-            hipLaunchKernelGGL(hy_conv_tail_kernel, dim3(hy_cdiv(hy_qk_ch(d), 256)), dim3(256), 0, st, h->proj, np, L.q_off, hy_qk_ch(d), d.qk_conv, h->slots + L.off_tail,
-                               h->slot_floats, h->dyn, n);
         if (d.pool > 0) {
             const int done = (pos0 + n) / d.pool - pos0 / d.pool;          // blocks whose last position lies in this portion
             if (done > 0)
                 hipLaunchKernelGGL(hy_pool_kernel, dim3(done, 2, done <= 8 ? std::min(16, hy_cdiv(d.kv_heads * std::max(d.dim, d.vdim), 256)) : 1), dim3(256), 0, st, kc, vc, pk, pv,
                                    d.kv_heads * d.dim, d.kv_heads * d.vdim, d.pool, h->slot_floats, h->dyn, n);
         }
+        if (one) return GL3_OK;
         int32_t r = hy_by_heads(d) ? hy_attention_heads(ctx, L, q, ldq, kc, vc, n, pos0, &nsplit)
                                    : hy_attention(ctx, q, ldq, kc, vc, d.heads, d.kv_heads, d.dim, d.vdim, d.scale, d.slope_log2, n, pos0, &nsplit, true, d.window, d.keep_first,
                                                   pk, pv, d.pool);
@@ -1357,9 +1409,6 @@ static int32_t hy_mixer_core(gl3_ctx* ctx, HyLayer& L, int np, int ldo, int n, i
         const bool eg = d.mem_gates == GL3_MEM_EXP_GATES, cg = d.mem_gates == GL3_MEM_CHANNEL_GATES;
         const int P = d.vdim + (eg ? 1 : 0), ldy = d.heads * P;
         float *ga = h->gates, *gb = ga + (size_t)h->mb * h->max_heads, *ge = gb + (size_t)h->mb * h->max_heads;
-        if (eg)
-            hipLaunchKernelGGL(hy_mem_gates_kernel, dim3(d.heads), dim3(256), 0, st, h->proj, np, L.i_off, L.f_off, L.pbias, d.mem_gate_cap, d.heads, h->slots + L.off_m,
-                               h->slot_floats, h->dyn, n, ga, gb, ge);
         HyScanArgs a{};
         a.ksrc = h->proj; a.ldk = np; a.k_off = L.k_off; a.k_hstride = d.dim;
         a.qsrc = h->proj; a.ldq = np; a.q_off = L.q_off; a.q_hstride = d.dim;
@@ -1371,6 +1420,10 @@ static int32_t hy_mixer_core(gl3_ctx* ctx, HyLayer& L, int np, int ldo, int n, i
         a.ga = ga; a.gb = gb; a.decay = L.decay; a.ones_col = eg ? 1 : 0;
         a.heads = d.heads; a.P = P; a.N = d.dim; a.G = d.heads;
         a.state = h->slots + L.off_state; a.slot_stride = h->slot_floats; a.dyn = h->dyn; a.n = n; a.y = h->ssm_y; a.ldy = ldy;
+        if (n == 1 && hy_scan_out<T>(ctx, L, a, mixo)) return GL3_OK;
+        if (eg)
+            hipLaunchKernelGGL(hy_mem_gates_kernel, dim3(d.heads), dim3(256), 0, st, h->proj, np, L.i_off, L.f_off, L.pbias, d.mem_gate_cap, d.heads, h->slots + L.off_m,
+                               h->slot_floats, h->dyn, n, ga, gb, ge);
         if (hy_scan_chunks(a) && ((a.act & 3) || a.rot.dims > 0 || a.k_mul != 1.f || a.q_mul != 1.f)) {
             // keys and queries are finished once, in place (the chunks' workgroups would each make them again for their few columns)
             hipLaunchKernelGGL(hy_scan_prep_kernel, dim3(n), dim3(256), (size_t)std::max(1, d.rot_dims) * 4, st, h->proj, np, L.q_off, L.k_off, d.heads, d.dim, a.q_mul, a.k_mul, a.act, a.rot, h->dyn);
@@ -1393,6 +1446,7 @@ static int32_t hy_mixer_core(gl3_ctx* ctx, HyLayer& L, int np, int ldo, int n, i
             q = h->qfull; ldq = d.heads * De;
             hy_gemm<T>(ctx, (const T*)h->cq, d.q_rank, L.uq, n, q, ldq, false, nullptr, 0, HyGlu{});
         }
+        if (n == 1 && hy_latent_one<T>(ctx, L, pos0, q, mixo)) return GL3_OK;
         if (d.rot_dim > 0)
             hipLaunchKernelGGL(hy_latent_prep_kernel, dim3(n, 1 + d.heads), dim3(64), 0, st, q, ldq, d.dim, d.rot_dim, h->proj, np, L.c_off, d.kv_rank, L.lat_norm, eps,
                                d.kv_share > 0 ? (float*)nullptr : cc, h->slot_floats, h->dyn, L.lat_freq, L.rot_mscale);
