@@ -125,6 +125,61 @@ static __global__ __launch_bounds__(256) void hy_embed_kernel(const int* host, i
     }
 }
 
+// The same for a step of a few tokens together with the norm in front of the first sublayer (pre_in: the streams' weights, null = one stream; norm_w null: the row itself in
+// the matrix type, if h_out is there at all): one workgroup per token, its first HY_EN entries per thread in registers.  One launch, and no second trip to memory, for
+// what took 4.2 + 3.7 us.
+constexpr int HY_EN = 8;
+template <typename T>
+static __global__ __launch_bounds__(1024) void hy_embed_norm_kernel(const int* host, int* __restrict__ rec, int tok0, int nw, const T* __restrict__ emb, float* __restrict__ X,
+                                                                    int W, int S, size_t sstride, float scale, float* __restrict__ copy, HyBigram bg, const float* __restrict__ pre_in,
+                                                                    const float* __restrict__ norm_w, float eps, T* __restrict__ h_out) {
+    __shared__ int sh[4];          // token, the one before it, position of the portion's first
+    __shared__ float red[16];
+    const int t = blockIdx.x, tid = threadIdx.x;
+    if (tid < 3) {
+        const int at = tid == 0 ? tok0 + t : tid == 2 ? 0 : t > 0 ? tok0 + t - 1 : 2;
+        if (tid == 0 || bg.table) sh[tid] = gl3::host_int(host + at);
+    }
+    if (t == 0) for (int i = tid - 64; i >= 0 && i < 4 + nw; i += 960) rec[i] = gl3::host_int(host + i);          // (wavefronts that do not wait for the token)
+    if (tid == 0) rec[tok0 + t] = sh[0];
+    float ps = 1.f;
+    if (pre_in) { ps = 0.f; for (int s = 0; s < S; ++s) ps += pre_in[s]; }
+    __syncthreads();
+    const int tok = sh[0];
+    const T* row = emb + (size_t)tok * W;
+    const T* pair = nullptr;
+    if (bg.table) {
+        const int prev = sh[1];
+        const int b = (t == 0 && sh[2] == 0) ? bg.buckets : (int)(((long long)prev * bg.mul_prev + (long long)tok * bg.mul_cur) % bg.buckets);
+        pair = (const T*)bg.table + (size_t)b * W;
+    }
+    float keep[HY_EN], wt[HY_EN], ss = 0.f;
+#pragma unroll
+    for (int u = 0; u < HY_EN; ++u) {
+        const int w = tid + u * 1024;
+        keep[u] = w < W ? hy_ld(row + w) * scale + (pair ? hy_ld(pair + w) : 0.f) : 0.f;
+        wt[u] = w < W && norm_w ? norm_w[w] : 1.f;
+    }
+    auto put = [&](int w, float v) {
+        for (int s = 0; s < S; ++s) X[s * sstride + (size_t)t * W + w] = v;
+        if (copy) copy[(size_t)t * W + w] = v;
+        ss += v * ps * (v * ps);
+    };
+#pragma unroll
+    for (int u = 0; u < HY_EN; ++u)
+        if (tid + u * 1024 < W) put(tid + u * 1024, keep[u]);
+    for (int w = tid + HY_EN * 1024; w < W; w += 1024) put(w, hy_ld(row + w) * scale + (pair ? hy_ld(pair + w) : 0.f));
+    if (!h_out) return;
+    ss = hy_block_sum<1024>(ss, red);
+    const float r = norm_w ? ps / sqrtf(ss / (float)W + eps) : 1.f;
+#pragma unroll
+    for (int u = 0; u < HY_EN; ++u) {
+        const int w = tid + u * 1024;
+        if (w < W) hy_st(h_out + (size_t)t * W + w, keep[u] * r * wt[u]);
+    }
+    for (int w = tid + HY_EN * 1024; w < W; w += 1024) hy_st(h_out + (size_t)t * W + w, X[(size_t)t * W + w] * r * (norm_w ? norm_w[w] : 1.f));          // (a thread re-reads what it wrote)
+}
+
 // ---- stream tables + norm -----------------------------------------------------------------------------------------------------
 // One workgroup per token.  "post" (y != null): x_t <- sum_s mix[s][t] x_s + out[t] y for all streams at once.  "pre" (pre_in != null):
 // u = sum_s in[s] x_s, h = u / sqrt(mean(u^2) + eps) * norm_w, written as TO.  sum_out (taps): the plain sum of the streams.
@@ -330,7 +385,7 @@ typedef float hy_v16f __attribute__((ext_vector_type(16)));
 // type: gelu_tanh(product) times an entry of a per-token table row (mul_table[mul_rows[m]][mul_col0 + feature], the per-layer token
 // input), or relu(product)^2 alone (act = 2, mul_table = null: a feed-forward without a gate).
 enum { HY_EPI_STORE = 0, HY_EPI_GLU = 1, HY_EPI_ACTMUL = 2 };
-struct HyGlu { float limit, alpha, shift; const void* mul_table; const int* mul_rows; int mul_ld, mul_col0; int act; };      // act 1: gelu_tanh(g) u; 2: relu(u)^2, no gate
+struct HyGlu { float limit, alpha, shift; const void* mul_table; const int* mul_rows; int mul_ld, mul_col0; int act; float cap; };      // act 1: gelu_tanh(g) u; 2: relu(u)^2, no gate; cap: plain products of a few tokens become cap tanh(. / cap)
 __device__ __forceinline__ float hy_gelu_tanh(float z) { return 0.5f * z * (1.f + tanhf(0.7978845608028654f * (z + 0.044715f * z * z * z))); }
 template <typename T>
 __device__ __forceinline__ float hy_actmul(float a, int m, int feature, const HyGlu& p) {
@@ -617,8 +672,8 @@ static __global__ __launch_bounds__(256) void hy_matvec_kernel(const T* __restri
                 hy_st(act + (size_t)m * ld_act + r0, hy_actmul<T>(a0[m], m, r0, glu));
                 if (has1) hy_st(act + (size_t)m * ld_act + r1, hy_actmul<T>(a1[m], m, r1, glu));
             } else {
-                C[(size_t)m * ldc + r0] = a0[m];
-                if (has1) C[(size_t)m * ldc + r1] = a1[m];
+                C[(size_t)m * ldc + r0] = glu.cap > 0.f ? glu.cap * tanhf(a0[m] / glu.cap) : a0[m];
+                if (has1) C[(size_t)m * ldc + r1] = glu.cap > 0.f ? glu.cap * tanhf(a1[m] / glu.cap) : a1[m];
             }
         }
     }
@@ -1509,7 +1564,37 @@ static __global__ __launch_bounds__(256) void hy_ssm_scan_kernel(HyScanArgs a) {
 // One token: S <- a S + b k x^T (mode 3: S += g (x - S)), y = S^T q + D x with every state element read and written once, where hy_ssm_scan_kernel stages, walks and
 // joins as for a block of tokens (64 heads x 128 x 64: 10 -> 5.4 us).  Workgroup = one head x 64 columns; its sixteen wavefronts share the states, sixteen
 // rows of 64 columns each on the way at once (256 states: one round trip); keys and queries of the head are made in LDS meanwhile.
-static __global__ __launch_bounds__(1024) void hy_scan_one_kernel(HyScanArgs a) {
+// With cv.w (a state-space layer with up to four taps) the sources are the raw projections: every workgroup makes the convolution of the channels it reads (one channel a
+// thread; the kernel behind this one moves the tail on, hy_conv_move), a launch of 5 us less.
+struct HyConvOne { const float* x; const float* w; const float* bias; float* tail; int ch, taps; };          // x: the token's raw channels
+struct HyConvTaps { float v[4], w[4], b; };
+__device__ __forceinline__ void hy_conv_load(HyConvTaps& q, const HyConvOne& cv, const float* tl, bool fresh, int c) {
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {          // taps 4 - taps .. 3 of four
+        const int j = k - (4 - cv.taps);
+        q.w[k] = j >= 0 ? cv.w[(size_t)c * cv.taps + j] : 0.f;
+        q.v[k] = k == 3 ? cv.x[c] : j >= 0 && !fresh ? tl[(size_t)j * cv.ch + c] : 0.f;
+    }
+    q.b = cv.bias[c];
+}
+__device__ __forceinline__ float hy_conv_sum(const HyConvTaps& q, int taps) {
+    float s = q.b;
+#pragma unroll
+    for (int k = 0; k < 4; ++k)
+        if (k >= 4 - taps) s = fmaf(q.w[k], q.v[k], s);
+    return hy_silu(s);
+}
+__device__ __forceinline__ void hy_conv_move(const HyConvOne& cv, const int* dyn, size_t slot_stride, int c) {
+    if (c >= cv.ch) return;
+    float *tl = cv.tail + (size_t)dyn[1] * slot_stride, v[3];
+    const bool fresh = dyn[0] == 0;
+#pragma unroll
+    for (int i = 0; i < 3; ++i) v[i] = i + 2 == cv.taps ? cv.x[c] : i + 2 < cv.taps && !fresh ? tl[(size_t)(i + 1) * cv.ch + c] : 0.f;
+#pragma unroll
+    for (int i = 0; i < 3; ++i)
+        if (i + 1 < cv.taps) tl[(size_t)i * cv.ch + c] = v[i];
+}
+static __global__ __launch_bounds__(1024) void hy_scan_one_kernel(HyScanArgs a, HyConvOne cv) {
     extern __shared__ float smem[];
     const int N = a.N, P = a.P, Px = P - (a.ones_col ? 1 : 0), head = blockIdx.y, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, p = blockIdx.x * 64 + lane;
     const int gr = head / (a.heads / a.G), pos = a.dyn[0];
@@ -1525,11 +1610,21 @@ static __global__ __launch_bounds__(1024) void hy_scan_one_kernel(HyScanArgs a) 
         for (int u = 0; u < 16; ++u) s[u] = S[(size_t)min(n + u, N - 1) * P + pc];
     };
     load(n0);
+    HyConvTaps ck, cx;          // this thread's first key or query entry and its x, on the way together
+    const float* tl = cv.w ? cv.tail + (size_t)a.dyn[1] * a.slot_stride : nullptr;
+    auto entry = [&](int i) { return (i >= N ? a.q_off + gr * a.q_hstride + i - N : a.k_off + gr * a.k_hstride + i); };
+    if (cv.w) {
+        hy_conv_load(ck, cv, tl, fresh, entry(min(tid, 2 * N - 1)));
+        hy_conv_load(cx, cv, tl, fresh, a.x_off + head * Px + min(p, Px - 1));
+    }
     for (int i = tid; i < 2 * N; i += 1024) {
         const bool q = i >= N;
         const int n = q ? i - N : i;
         float v;
-        if (cg && !q && a.fbias) v = (1.f - a.lower[(size_t)head * N + n]) * hy_sigmoid(-(kb[n] + a.fbias[(size_t)head * N + n]));
+        if (cv.w) {
+            if (i > tid) hy_conv_load(ck, cv, tl, fresh, entry(i));
+            v = hy_conv_sum(ck, cv.taps);
+        } else if (cg && !q && a.fbias) v = (1.f - a.lower[(size_t)head * N + n]) * hy_sigmoid(-(kb[n] + a.fbias[(size_t)head * N + n]));
         else {
             const bool si = a.act & (q ? 2 : 1);
             const float mul = q ? a.q_mul : a.k_mul;
@@ -1554,7 +1649,8 @@ static __global__ __launch_bounds__(1024) void hy_scan_one_kernel(HyScanArgs a) 
     } else if (a.mode == 1) { av = a.ga[head]; bv = a.gb[head]; }
     else if (a.mode == 2) av = a.decay[head];
     float x = 0.f;
-    if (p < Px) { x = a.xsrc[a.x_off + (size_t)head * Px + p]; if (a.act & 4) x = hy_silu(x); }
+    if (p < Px && cv.w) x = hy_conv_sum(cx, cv.taps);
+    else if (p < Px) { x = a.xsrc[a.x_off + (size_t)head * Px + p]; if (a.act & 4) x = hy_silu(x); }
     else if (p < P) x = 1.f;
     const float bx = bv * x;
     __syncthreads();
@@ -1659,21 +1755,45 @@ static __global__ __launch_bounds__(NT) void hy_mem_out_kernel(const float* __re
     }
 }
 
-// y * silu(z), unit root mean square per part (ngroups equal parts of inner), times the weight
+// y * silu(z), unit root mean square per part (ngroups equal parts of inner), times the weight; the first HY_GN entries of a thread stay in registers between the
+// two passes.  Workgroups behind the parts move the tail of a single token on
+// whose convolution hy_scan_one_kernel made (cv).
+constexpr int HY_GN = 4;
 template <typename TO>
 static __global__ __launch_bounds__(256) void hy_gated_norm_kernel(const float* __restrict__ y, const float* __restrict__ proj, int ld, int z_off, int inner,
-                                                                   int ngroups, const float* __restrict__ w, float eps, TO* __restrict__ out, int ldo) {
+                                                                   int ngroups, const float* __restrict__ w, float eps, TO* __restrict__ out, int ldo, HyConvOne cv, const int* __restrict__ dyn,
+                                                                   size_t slot_stride) {
     __shared__ float red[4];
+    if ((int)blockIdx.y >= ngroups) { hy_conv_move(cv, dyn, slot_stride, (blockIdx.y - ngroups) * 256 + threadIdx.x); return; }
     const int t = blockIdx.x, grp = blockIdx.y, len = inner / ngroups, c0 = grp * len;
-    float ss = 0.f;
-    for (int i = threadIdx.x; i < len; i += 256) {
-        const float v = y[(size_t)t * inner + c0 + i] * hy_silu(proj[(size_t)t * ld + z_off + c0 + i]);
+    const float *yr = y + (size_t)t * inner + c0, *zr = proj + (size_t)t * ld + z_off + c0;
+    float keep[HY_GN], wt[HY_GN], ss = 0.f;
+    {
+        float a[HY_GN], z[HY_GN];
+#pragma unroll
+        for (int u = 0; u < HY_GN; ++u) {
+            const int i = min((int)threadIdx.x + 256 * u, len - 1);
+            a[u] = yr[i]; z[u] = zr[i]; wt[u] = w[c0 + i];
+        }
+#pragma unroll
+        for (int u = 0; u < HY_GN; ++u) {
+            keep[u] = a[u] * hy_silu(z[u]);
+            if ((int)threadIdx.x + 256 * u < len) ss += keep[u] * keep[u];
+        }
+    }
+    for (int i = threadIdx.x + 256 * HY_GN; i < len; i += 256) {
+        const float v = yr[i] * hy_silu(zr[i]);
         ss += v * v;
     }
     ss = hy_block_sum<256>(ss, red);
     const float r = 1.f / sqrtf(ss / (float)len + eps);
-    for (int i = threadIdx.x; i < len; i += 256) {
-        const float v = y[(size_t)t * inner + c0 + i] * hy_silu(proj[(size_t)t * ld + z_off + c0 + i]);
+#pragma unroll
+    for (int u = 0; u < HY_GN; ++u) {
+        const int i = threadIdx.x + 256 * u;
+        if (i < len) hy_st(out + (size_t)t * ldo + c0 + i, keep[u] * r * wt[u]);
+    }
+    for (int i = threadIdx.x + 256 * HY_GN; i < len; i += 256) {
+        const float v = yr[i] * hy_silu(zr[i]);
         hy_st(out + (size_t)t * ldo + c0 + i, v * r * w[c0 + i]);
     }
 }

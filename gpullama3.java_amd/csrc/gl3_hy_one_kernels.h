@@ -54,12 +54,12 @@ struct HyAttnOne {
 };
 constexpr long HY_ATTN_ONE = 384 * 1024;
 template <typename TO, int NI>          // head sizes up to 64 NI
-static __global__ __launch_bounds__(1024) void hy_attn_one_kernel(HyAttnOne a, TO* __restrict__ out) {
+__device__ __forceinline__ void hy_attn_one(const HyAttnOne& a, TO* __restrict__ out, const int h) {
     constexpr int U = 4 / NI, NW = 16, MD = 64 * NI;
     __shared__ __attribute__((aligned(16))) float sQ[MD], sK[MD], sV[MD], sO[NW][MD];
     __shared__ float sML[NW][2], sW[NW], sR[2 * NW];
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), l16 = lane & 15, grp = lane >> 4;
-    const int h = blockIdx.x, g = h / (a.H / a.G), D = a.D, V = a.V, pos = a.dyn[0];
+    const int g = h / (a.H / a.G), D = a.D, V = a.V, pos = a.dyn[0];
     const size_t slot = (size_t)a.dyn[1] * a.slot_stride;
     float *kc = a.kc + slot + (size_t)g * D, *vc = a.vc + slot + (size_t)g * V;
     const int ldk = a.G * D, ldv = a.G * V;
@@ -205,6 +205,9 @@ static __global__ __launch_bounds__(1024) void hy_attn_one_kernel(HyAttnOne a, T
         }
     } else if (tid < V) put(tid, column(tid));
 }
+
+template <typename TO, int NI>
+static __global__ __launch_bounds__(1024) void hy_attn_one_kernel(HyAttnOne a, TO* __restrict__ out) { hy_attn_one<TO, NI>(a, out, blockIdx.x); }
 
 // ---- latent attention -------------------------------------------------------------------------------------------------------------------
 // Workgroup = one head, sixteen wavefronts: the token's cached row (norm, weight, turned part), the query carried into the latent's space (the head's rows of the
@@ -390,7 +393,7 @@ static __global__ __launch_bounds__(1024) void hy_latent_one_kernel(HyLatentOne 
 
 // ---- matrix memories ----------------------------------------------------------------------------------------------------------------------
 // Workgroup = one head: the gates of a memory with exponential gating (hy_mem_gates_kernel's arithmetic for one token), the step of the state (hy_scan_one_kernel's:
-// every element read and written once, QN rows of 64 CB columns a wavefront, the next columns' rows on their way under this one's products) and what leaves the
+// every element read and written once, QN rows of 64 CB NB columns a wavefront on their way at once) and what leaves the
 // head (hy_mem_out_kernel's norm and gate).  It replaces two launches, three with exponential gates.  Bound: one CU reads and writes the head's state,
 // so it is taken while that is small (HY_SCAN_OUT); one norm over the heads side by side needs them all and stays apart.  Whole steps, us, with and without: retention of 16 x
 // 64 x 128 and mLSTM 8 x 128 x 257 144 / 149; retention 16 x 128 x 256 equal; with mLSTM 8 x 256 x 513 too 313 / 291.
@@ -403,23 +406,26 @@ struct HyScanOut {
 constexpr int HY_SCAN_OUT = 40 * 1024;                       // state elements a head
 constexpr int HY_SCAN_OUT_P = 1024;                          // value columns a head
 template <typename TO, int QN>
-static __global__ __launch_bounds__(1024) void hy_scan_out_kernel(HyScanOut b, TO* __restrict__ out) {
-    constexpr int CB = 16 / QN, NW = 16;
-    __shared__ float sK[16 * QN], sQ[16 * QN], sY[NW][64 * CB], sP[HY_SCAN_OUT_P], red[NW];
+__device__ __forceinline__ void hy_scan_out(const HyScanOut& b, TO* __restrict__ out, const int head) {
+    constexpr int CB = 16 / QN, NB = QN == 4 ? 1 : 3, NW = 16;          // NB times 64 CB columns at once
+    __shared__ float sK[16 * QN], sQ[16 * QN], sY[NW][64 * CB * NB], sP[HY_SCAN_OUT_P], red[NW];
     const HyScanArgs& a = b.s;
-    const int N = a.N, P = a.P, V = P - (a.ones_col ? 1 : 0), head = blockIdx.x, tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), pos = a.dyn[0];
+    const int N = a.N, P = a.P, V = P - (a.ones_col ? 1 : 0), tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), pos = a.dyn[0];
     const bool fresh = pos == 0;
     const float *kb = a.ksrc + a.k_off + (size_t)head * a.k_hstride, *qb = a.qsrc + a.q_off + (size_t)head * a.q_hstride;
     float* S = a.state + (size_t)a.dyn[1] * a.slot_stride + (size_t)head * N * P;
     const int half = a.rot.dims >> 1, n0 = wave * QN;
-    float s[CB][QN], nx[CB][QN];
-    auto load = [&](float (*d)[QN], int p0) {
+    float s[NB][CB][QN];
+    auto load = [&](int p0) {
 #pragma unroll
-        for (int c = 0; c < CB; ++c)
+        for (int k = 0; k < NB; ++k)
+            if (k == 0 || p0 + 64 * CB * k < P)
 #pragma unroll
-            for (int u = 0; u < QN; ++u) d[c][u] = S[(size_t)min(n0 + u, N - 1) * P + min(p0 + 64 * c + lane, P - 1)];
+                for (int c = 0; c < CB; ++c)
+#pragma unroll
+                    for (int u = 0; u < QN; ++u) s[k][c][u] = S[(size_t)min(n0 + u, N - 1) * P + min(p0 + 64 * (CB * k + c) + lane, P - 1)];
     };
-    load(s, 0);
+    load(0);
     for (int i = tid; i < 2 * N; i += 1024) {
         const bool q = i >= N;
         const int n = q ? i - N : i;
@@ -449,36 +455,36 @@ static __global__ __launch_bounds__(1024) void hy_scan_out_kernel(HyScanOut b, T
         if (tid == 0) *mp = mt;
     } else av = a.decay[head];
     __syncthreads();
-    for (int p0 = 0; p0 < P; p0 += 64 * CB) {
-        if (p0 + 64 * CB < P) load(nx, p0 + 64 * CB);
+    for (int p0 = 0; p0 < P; p0 += 64 * CB * NB) {
+        if (p0 > 0) load(p0);
 #pragma unroll
-        for (int c = 0; c < CB; ++c) {
-            const int p = p0 + 64 * c + lane;
-            float x = 0.f, y = 0.f;
-            if (p < V) { x = a.xsrc[a.x_off + (size_t)head * V + p]; if (a.act & 4) x = hy_silu(x); }
-            else if (p < P) x = 1.f;
-            const float bx = bv * x;
+        for (int k = 0; k < NB; ++k) {
+            if (k > 0 && p0 + 64 * CB * k >= P) break;
 #pragma unroll
-            for (int u = 0; u < QN; ++u) {
-                if (n0 + u >= N) break;
-                const float v = fmaf(av, fresh ? 0.f : s[c][u], sK[n0 + u] * bx);
-                y = fmaf(v, sQ[n0 + u], y);
-                if (p < P) S[(size_t)(n0 + u) * P + p] = v;
+            for (int c = 0; c < CB; ++c) {
+                const int p = p0 + 64 * (CB * k + c) + lane;
+                float x = 0.f, y = 0.f;
+                if (p < V) { x = a.xsrc[a.x_off + (size_t)head * V + p]; if (a.act & 4) x = hy_silu(x); }
+                else if (p < P) x = 1.f;
+                const float bx = bv * x;
+#pragma unroll
+                for (int u = 0; u < QN; ++u) {
+                    if (n0 + u >= N) break;
+                    const float v = fmaf(av, fresh ? 0.f : s[k][c][u], sK[n0 + u] * bx);
+                    y = fmaf(v, sQ[n0 + u], y);
+                    if (p < P) S[(size_t)(n0 + u) * P + p] = v;
+                }
+                sY[wave][64 * (CB * k + c) + lane] = y;
             }
-            sY[wave][64 * c + lane] = y;
         }
         __syncthreads();
-        for (int c = tid; c < 64 * CB && p0 + c < P; c += 1024) {
+        for (int c = tid; c < 64 * CB * NB && p0 + c < P; c += 1024) {
             float v = 0.f;
 #pragma unroll
             for (int w = 0; w < NW; ++w) v += sY[w][c];
             sP[p0 + c] = v;
         }
         __syncthreads();
-#pragma unroll
-        for (int c = 0; c < CB; ++c)
-#pragma unroll
-            for (int u = 0; u < QN; ++u) s[c][u] = nx[c][u];
     }
     // P <= 1024: a column per thread
     const float inv = a.mode == 1 ? 1.f / (fmaxf(fabsf(sP[V]), ge) + 1e-6f) : 1.f;
@@ -487,4 +493,14 @@ static __global__ __launch_bounds__(1024) void hy_scan_out_kernel(HyScanOut b, T
     const float r = 1.f / sqrtf(hy_block_sum<1024>(o * o, red) / (float)V + b.eps);
     const float act = !b.gate ? 1.f : b.gate_act == 1 ? hy_sigmoid(gz) : hy_silu(gz);
     if (tid < V) hy_st(out + head * V + tid, o * r * w * act * b.out_mul);
+}
+template <typename TO, int QN>
+static __global__ __launch_bounds__(1024) void hy_scan_out_kernel(HyScanOut b, TO* __restrict__ out) { hy_scan_out<TO, QN>(b, out, blockIdx.x); }
+
+// Attention and a matrix memory side by side on one input: the heads of both are workgroups of one launch (one after the other the second waits for the first's
+// last head and for a launch, on a chip that is idle but for some dozens of CUs).
+template <typename TO, int NI, int QN>
+static __global__ __launch_bounds__(1024) void hy_pair_one_kernel(HyAttnOne a, TO* __restrict__ out_a, HyScanOut b, TO* __restrict__ out_b) {
+    if ((int)blockIdx.x < a.H) hy_attn_one<TO, NI>(a, out_a, blockIdx.x);
+    else hy_scan_out<TO, QN>(b, out_b, (int)blockIdx.x - a.H);
 }

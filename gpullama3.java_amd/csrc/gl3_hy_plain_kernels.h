@@ -249,6 +249,12 @@ static __global__ __launch_bounds__(NT) void hy_resid_kernel(HyResid a, TO* __re
                 for (int i = 0; i < V; ++i) keep[q][i] = x[i];
     }
     if (!a.norm_w) return;
+    float nk[HY_RC][V];          // the norm's weights travel while the sum is made
+#pragma unroll
+    for (int q = 0; q < HY_RC; ++q) {
+        const int w = (threadIdx.x + q * NT) * V;
+        if (w < W) hy_ldv<V>(a.norm_w + w, nk[q]);
+    }
     ss = hy_block_sum<NT>(ss, red);
     const float r = 1.f / sqrtf(ss / (float)W + a.eps);
     float* prev = a.shift_mu ? a.shift_prev + (size_t)a.dyn[1] * a.slot_stride : nullptr;
@@ -261,9 +267,11 @@ static __global__ __launch_bounds__(NT) void hy_resid_kernel(HyResid a, TO* __re
             for (int q = 0; q < HY_RC; ++q)
                 if (q == it)
 #pragma unroll
-                    for (int i = 0; i < V; ++i) x[i] = keep[q][i];
-        } else hy_ldv<V>(a.x + row + w, x);          // a thread re-reads what it wrote
-        hy_ldv<V>(a.norm_w + w, nw);
+                    for (int i = 0; i < V; ++i) { x[i] = keep[q][i]; nw[i] = nk[q][i]; }
+        } else {
+            hy_ldv<V>(a.x + row + w, x);          // a thread re-reads what it wrote
+            hy_ldv<V>(a.norm_w + w, nw);
+        }
 #pragma unroll
         for (int i = 0; i < V; ++i) x[i] = x[i] * r * nw[i];
         if (a.shift_mu) {

@@ -1244,10 +1244,10 @@ static void hy_scan_chunk_launch(gl3_ctx* ctx, const HyScanArgs& a) {
 // With few workgroups (few heads, narrow values) NL = 16 is halved once so that more of them share the columns; below 8 every workgroup
 // stages the same key / query rows for too few columns and the traffic from L2 eats the gain (measured: 16 and 8 within 2 %, 4 slower).
 // GL3_HY_SCAN_NL forces a value, and the walk.
-static void hy_scan(gl3_ctx* ctx, HyScanArgs& a) {
+static void hy_scan(gl3_ctx* ctx, HyScanArgs& a, const HyConvOne& cv = HyConvOne{}) {
     const int forced = hy_scan_forced(a.N);
     if (a.n == 1 && a.N <= 4096 && !forced) {
-        hipLaunchKernelGGL(hy_scan_one_kernel, dim3(hy_cdiv(a.P, 64), a.heads), dim3(1024), (size_t)(2 * a.N + 1024) * 4, ctx->stream, a);
+        hipLaunchKernelGGL(hy_scan_one_kernel, dim3(hy_cdiv(a.P, 64), a.heads), dim3(1024), (size_t)(2 * a.N + 1024) * 4, ctx->stream, a, cv);
         return;
     }
     if (hy_scan_chunks(a)) { hy_scan_chunk_launch(ctx, a); return; }
@@ -1294,20 +1294,25 @@ static void hy_mem_out(gl3_ctx* ctx, const HyLayer& L, int n, int ldy, int P, co
 }
 
 // ---- one token behind few positions: a mixer's kernels in one launch (gl3_hy_one_kernels.h); false: the form or the position is not theirs ----
-template <typename T>
-static bool hy_attn_one(gl3_ctx* ctx, const HyLayer& L, int pos0, const HyRot& rot, const HyPrepX& px, T* out) {
+static HyRot hy_attn_rot(const HyLayer& L) { return HyRot{L.d.rot_dims, L.rot_freq64, L.d.v_unit_norm, L.d.v_rot ? L.vrot_freq : nullptr, L.d.rot_interleaved}; }
+static bool hy_attn_one_args(gl3_ctx* ctx, const HyLayer& L, int pos0, HyAttnOne& a) {
     gl3_hybrid_state* h = ctx->hy;
     const gl3_layer_desc& d = L.d;
     float *kc = h->slots + L.off_k, *vc = h->slots + L.off_v;
-    const int big = std::max(d.dim, d.vdim);
-    if (hy_by_heads(d) || d.qk_conv > 0 || big > 256 || ((d.dim | d.vdim | (int)(h->slot_floats & 3)) & 3) || (((uintptr_t)kc | (uintptr_t)vc) & 15) || (d.window > 0 && pos0 >= d.window)) return false;
-    if ((long)(pos0 + 1) * (d.dim + d.vdim) * 4 > HY_ATTN_ONE) return false;
-    HyAttnOne a{};
+    if (d.mixer != GL3_MIX_ATTENTION || hy_by_heads(d) || d.qk_conv > 0 || std::max(d.dim, d.vdim) > 256 || ((d.dim | d.vdim | (int)(h->slot_floats & 3)) & 3) || (((uintptr_t)kc | (uintptr_t)vc) & 15)) return false;
+    if ((d.window > 0 && pos0 >= d.window) || (long)(pos0 + 1) * (d.dim + d.vdim) * 4 > HY_ATTN_ONE) return false;
     a.proj = h->proj; a.q_off = L.q_off; a.k_off = L.k_off; a.v_off = L.v_off; a.H = d.heads; a.G = d.kv_heads; a.D = d.dim; a.V = d.vdim; a.unit_norm = d.qk_unit_norm; a.eps = ctx->d.rms_eps;
-    a.kc = kc; a.vc = vc; a.slot_stride = h->slot_floats; a.dyn = h->dyn; a.rot = rot; a.bias = px.bias; a.qn = L.qn; a.kn = L.kn; a.v_from_k = d.v_from_k; a.scale = d.scale; a.slope_log2 = d.slope_log2;
-    a.sink = d.softmax_sink; a.sink_w = d.softmax_sink == 2 ? L.sink : nullptr;
+    a.kc = kc; a.vc = vc; a.slot_stride = h->slot_floats; a.dyn = h->dyn; a.rot = hy_attn_rot(L); a.bias = d.qk_bias ? L.pbias : nullptr; a.qn = L.qn; a.kn = L.kn; a.v_from_k = d.v_from_k;
+    a.scale = d.scale; a.slope_log2 = d.slope_log2; a.sink = d.softmax_sink; a.sink_w = d.softmax_sink == 2 ? L.sink : nullptr;
     a.gate = d.out_gate ? h->proj + L.g_off : nullptr; a.gate_mode = d.out_gate; a.v_freq = d.v_rot ? L.vrot_freq : nullptr; a.out_mul = d.out_norm ? 1.f : L.out_mul;
-#define HY_A1(NI) hipLaunchKernelGGL((hy_attn_one_kernel<T, NI>), dim3(d.heads), dim3(1024), 0, ctx->stream, a, out)
+    return true;
+}
+template <typename T>
+static bool hy_attn_one(gl3_ctx* ctx, const HyLayer& L, int pos0, T* out) {
+    HyAttnOne a{};
+    if (!hy_attn_one_args(ctx, L, pos0, a)) return false;
+    const int big = std::max(a.D, a.V);
+#define HY_A1(NI) hipLaunchKernelGGL((hy_attn_one_kernel<T, NI>), dim3(a.H), dim3(1024), 0, ctx->stream, a, out)
     if (big <= 64) HY_A1(1); else if (big <= 128) HY_A1(2); else HY_A1(4);
 #undef HY_A1
     return true;
@@ -1325,19 +1330,67 @@ static bool hy_latent_one(gl3_ctx* ctx, const HyLayer& L, int pos0, const float*
     hipLaunchKernelGGL((hy_latent_one_kernel<T>), dim3(d.heads), dim3(1024), 0, ctx->stream, a, out);
     return true;
 }
-template <typename T>
-static bool hy_scan_out(gl3_ctx* ctx, const HyLayer& L, const HyScanArgs& s, T* out) {
+// The recurrence of a matrix memory on the n rows in h->proj (row stride np), its gates and result in plan scratch.
+static HyScanArgs hy_mem_scan_args(gl3_ctx* ctx, const HyLayer& L, int np, int n) {
     gl3_hybrid_state* h = ctx->hy;
     const gl3_layer_desc& d = L.d;
-    if (s.mode == 3 || d.mem_norm_whole || s.N > 256 || s.P > HY_SCAN_OUT_P || s.N * s.P > HY_SCAN_OUT || hy_scan_forced(s.N)) return false;
-    HyScanOut b{};
-    b.s = s; b.i_off = L.i_off; b.f_off = L.f_off; b.gbias = L.pbias; b.cap = d.mem_gate_cap; b.m = h->slots + L.off_m;
+    const bool eg = d.mem_gates == GL3_MEM_EXP_GATES, cg = d.mem_gates == GL3_MEM_CHANNEL_GATES;
+    HyScanArgs a{};
+    a.ksrc = h->proj; a.ldk = np; a.k_off = L.k_off; a.k_hstride = d.dim;
+    a.qsrc = h->proj; a.ldq = np; a.q_off = L.q_off; a.q_hstride = d.dim;
+    a.xsrc = h->proj; a.ldx = np; a.x_off = L.v_off;
+    a.k_mul = d.mem_k_mul != 0.f ? d.mem_k_mul : 1.f; a.q_mul = d.mem_q_mul != 0.f ? d.mem_q_mul : 1.f;
+    a.act = d.mem_qkv_act == 1 ? 7 : d.mem_qkv_act == 2 ? 2 : 0;
+    a.rot = HyScanRot{d.rot_dims, L.rot_freq, d.rot_interleaved};
+    a.mode = eg ? 1 : cg ? 3 : 2; if (cg) { a.fbias = L.pbias + L.f_off; a.lower = L.mem_lower; }
+    a.ga = h->gates; a.gb = h->gates + (size_t)h->mb * h->max_heads; a.decay = L.decay; a.ones_col = eg ? 1 : 0;
+    a.heads = d.heads; a.P = d.vdim + (eg ? 1 : 0); a.N = d.dim; a.G = d.heads;
+    a.state = h->slots + L.off_state; a.slot_stride = h->slot_floats; a.dyn = h->dyn; a.n = n; a.y = h->ssm_y; a.ldy = a.heads * a.P;
+    return a;
+}
+static bool hy_scan_out_args(gl3_ctx* ctx, const HyLayer& L, int np, HyScanOut& b) {
+    gl3_hybrid_state* h = ctx->hy;
+    const gl3_layer_desc& d = L.d;
+    if (d.mixer != GL3_MIX_MEMORY || d.mem_gates == GL3_MEM_DELTA || d.mem_gates == GL3_MEM_CHANNEL_GATES || d.mem_norm_whole) return false;
+    b.s = hy_mem_scan_args(ctx, L, np, 1);
+    if (b.s.N > 256 || b.s.P > HY_SCAN_OUT_P || b.s.N * b.s.P > HY_SCAN_OUT || hy_scan_forced(b.s.N)) return false;
+    b.i_off = L.i_off; b.f_off = L.f_off; b.gbias = L.pbias; b.cap = d.mem_gate_cap; b.m = h->slots + L.off_m;
     b.gate = d.mem_gate_act == 2 ? nullptr : h->proj + L.g_off; b.gate_act = d.mem_gate_act; b.w = d.mem_norm_weight ? L.ssm_norm : nullptr; b.w_stride = d.mem_norm_weight == 2 ? 0 : d.vdim;
     b.eps = ctx->d.rms_eps; b.out_mul = d.out_norm ? 1.f : L.out_mul;
-#define HY_SO(QN) hipLaunchKernelGGL((hy_scan_out_kernel<T, QN>), dim3(s.heads), dim3(1024), 0, ctx->stream, b, out)
-    if (s.N <= 64) HY_SO(4); else if (s.N <= 128) HY_SO(8); else HY_SO(16);
+    return true;
+}
+template <typename T>
+static bool hy_scan_out(gl3_ctx* ctx, const HyLayer& L, int np, T* out) {
+    HyScanOut b{};
+    if (!hy_scan_out_args(ctx, L, np, b)) return false;
+#define HY_SO(QN) hipLaunchKernelGGL((hy_scan_out_kernel<T, QN>), dim3(b.s.heads), dim3(1024), 0, ctx->stream, b, out)
+    if (b.s.N <= 64) HY_SO(4); else if (b.s.N <= 128) HY_SO(8); else HY_SO(16);
 #undef HY_SO
     return true;
+}
+// Attention and a matrix memory side by side in one launch (head sizes up to 128 and 128 states: what their kernels are built for together).
+template <typename T>
+static bool hy_pair_one(gl3_ctx* ctx, const HyLayer& L, const HyLayer& R, int np, int pos0) {
+    gl3_hybrid_state* h = ctx->hy;
+    HyAttnOne a{};
+    HyScanOut b{};
+    if (!hy_attn_one_args(ctx, L, pos0, a) || !hy_scan_out_args(ctx, R, np, b) || std::max(a.D, a.V) > 128 || b.s.N > 128) return false;
+    T *oa = (T*)h->mixo + L.o0, *ob = (T*)h->mixo + R.o0;
+#define HY_P1(NI, QN) hipLaunchKernelGGL((hy_pair_one_kernel<T, NI, QN>), dim3(a.H + b.s.heads), dim3(1024), 0, ctx->stream, a, oa, b, ob)
+    if (std::max(a.D, a.V) <= 64) { if (b.s.N <= 64) HY_P1(1, 4); else HY_P1(1, 8); }
+    else { if (b.s.N <= 64) HY_P1(2, 4); else HY_P1(2, 8); }
+#undef HY_P1
+    return true;
+}
+
+// Pooled rows of the blocks whose last position lies in this portion.
+static void hy_pool(gl3_ctx* ctx, const HyLayer& L, int n, int pos0) {
+    gl3_hybrid_state* h = ctx->hy;
+    const gl3_layer_desc& d = L.d;
+    const int done = d.pool > 0 ? (pos0 + n) / d.pool - pos0 / d.pool : 0;
+    if (done > 0)
+        hipLaunchKernelGGL(hy_pool_kernel, dim3(done, 2, done <= 8 ? std::min(16, hy_cdiv(d.kv_heads * std::max(d.dim, d.vdim), 256)) : 1), dim3(256), 0, ctx->stream, h->slots + L.off_k,
+                           h->slots + L.off_v, h->slots + L.off_pk, h->slots + L.off_pv, d.kv_heads * d.dim, d.kv_heads * d.vdim, d.pool, h->slot_floats, h->dyn, n);
 }
 
 // One mixer of a layer on the n rows of the fused projection in h->proj (row stride np): its heads land in mixo (row stride ldo) from
@@ -1355,7 +1408,7 @@ static int32_t hy_mixer_core(gl3_ctx* ctx, HyLayer& L, int np, int ldo, int n, i
         float* vc = h->slots + L.off_v;
         float* pk = d.pool > 0 ? h->slots + L.off_pk : nullptr;
         float* pv = d.pool > 0 ? h->slots + L.off_pv : nullptr;
-        const HyRot rot{d.rot_dims, L.rot_freq64, d.v_unit_norm, d.v_rot ? L.vrot_freq : nullptr, d.rot_interleaved};
+        const HyRot rot = hy_attn_rot(L);
         HyPrepX px{d.qk_bias ? L.pbias : nullptr, L.qn, L.kn, h->rowr, d.v_from_k};
         const float* q = h->proj + L.q_off;
         int ldq = np;
@@ -1363,25 +1416,17 @@ static int32_t hy_mixer_core(gl3_ctx* ctx, HyLayer& L, int np, int ldo, int n, i
             px.conv_w = L.qk_conv_w; px.taps = d.qk_conv; px.tail = h->slots + L.off_tail; px.qout = h->conv; px.ldq = d.heads * d.dim; px.n = n;
             q = h->conv; ldq = px.ldq;
         }
-        const bool one = n == 1 && hy_attn_one<T>(ctx, L, pos0, rot, px, mixo);          // (pooled blocks that this token completes follow it: no window is passed yet)
-        if (!one) {
-            if (d.qk_unit_norm == 2) {
-                if (n <= 32) hipLaunchKernelGGL((hy_rowrms_kernel<1024>), dim3(n, 2), dim3(1024), 0, st, h->proj, np, L.q_off, d.heads * d.dim, L.k_off, d.kv_heads * d.dim, px.bias, eps, h->rowr);
-                else hipLaunchKernelGGL((hy_rowrms_kernel<256>), dim3(n, 2), dim3(256), 0, st, h->proj, np, L.q_off, d.heads * d.dim, L.k_off, d.kv_heads * d.dim, px.bias, eps, h->rowr);
-            }
-            hipLaunchKernelGGL(hy_attn_prep_kernel, dim3(n, d.heads + (d.v_from_k ? 1 : 2) * d.kv_heads), dim3(64), 0, st, h->proj, np, L.q_off, L.k_off, L.v_off, d.heads, d.kv_heads, d.dim,
-                               d.vdim, d.qk_unit_norm, eps, kc, vc, h->slot_floats, h->dyn, rot, px);
-            if (d.qk_conv > 1 && n > 1)          // (q and k stand side by side in the projection row; a single token's tail moved on above)
-                hipLaunchKernelGGL(hy_conv_tail_kernel, dim3(hy_cdiv(hy_qk_ch(d), 256)), dim3(256), 0, st, h->proj, np, L.q_off, hy_qk_ch(d), d.qk_conv, h->slots + L.off_tail,
-                                   h->slot_floats, h->dyn, n);
+        if (n == 1 && hy_attn_one<T>(ctx, L, pos0, mixo)) { hy_pool(ctx, L, n, pos0); return GL3_OK; }          // (pooled blocks that this token completes: no window is passed yet)
+        if (d.qk_unit_norm == 2) {
+            if (n <= 32) hipLaunchKernelGGL((hy_rowrms_kernel<1024>), dim3(n, 2), dim3(1024), 0, st, h->proj, np, L.q_off, d.heads * d.dim, L.k_off, d.kv_heads * d.dim, px.bias, eps, h->rowr);
+            else hipLaunchKernelGGL((hy_rowrms_kernel<256>), dim3(n, 2), dim3(256), 0, st, h->proj, np, L.q_off, d.heads * d.dim, L.k_off, d.kv_heads * d.dim, px.bias, eps, h->rowr);
         }
-        if (d.pool > 0) {
-            const int done = (pos0 + n) / d.pool - pos0 / d.pool;          // blocks whose last position lies in this portion
-            if (done > 0)
-                hipLaunchKernelGGL(hy_pool_kernel, dim3(done, 2, done <= 8 ? std::min(16, hy_cdiv(d.kv_heads * std::max(d.dim, d.vdim), 256)) : 1), dim3(256), 0, st, kc, vc, pk, pv,
-                                   d.kv_heads * d.dim, d.kv_heads * d.vdim, d.pool, h->slot_floats, h->dyn, n);
-        }
-        if (one) return GL3_OK;
+        hipLaunchKernelGGL(hy_attn_prep_kernel, dim3(n, d.heads + (d.v_from_k ? 1 : 2) * d.kv_heads), dim3(64), 0, st, h->proj, np, L.q_off, L.k_off, L.v_off, d.heads, d.kv_heads, d.dim,
+                           d.vdim, d.qk_unit_norm, eps, kc, vc, h->slot_floats, h->dyn, rot, px);
+        if (d.qk_conv > 1 && n > 1)          // (q and k stand side by side in the projection row; a single token's tail moved on above)
+            hipLaunchKernelGGL(hy_conv_tail_kernel, dim3(hy_cdiv(hy_qk_ch(d), 256)), dim3(256), 0, st, h->proj, np, L.q_off, hy_qk_ch(d), d.qk_conv, h->slots + L.off_tail,
+                               h->slot_floats, h->dyn, n);
+        hy_pool(ctx, L, n, pos0);
         int32_t r = hy_by_heads(d) ? hy_attention_heads(ctx, L, q, ldq, kc, vc, n, pos0, &nsplit)
                                    : hy_attention(ctx, q, ldq, kc, vc, d.heads, d.kv_heads, d.dim, d.vdim, d.scale, d.slope_log2, n, pos0, &nsplit, true, d.window, d.keep_first,
                                                   pk, pv, d.pool);
@@ -1409,18 +1454,8 @@ static int32_t hy_mixer_core(gl3_ctx* ctx, HyLayer& L, int np, int ldo, int n, i
         const bool eg = d.mem_gates == GL3_MEM_EXP_GATES, cg = d.mem_gates == GL3_MEM_CHANNEL_GATES;
         const int P = d.vdim + (eg ? 1 : 0), ldy = d.heads * P;
         float *ga = h->gates, *gb = ga + (size_t)h->mb * h->max_heads, *ge = gb + (size_t)h->mb * h->max_heads;
-        HyScanArgs a{};
-        a.ksrc = h->proj; a.ldk = np; a.k_off = L.k_off; a.k_hstride = d.dim;
-        a.qsrc = h->proj; a.ldq = np; a.q_off = L.q_off; a.q_hstride = d.dim;
-        a.xsrc = h->proj; a.ldx = np; a.x_off = L.v_off;
-        a.k_mul = d.mem_k_mul != 0.f ? d.mem_k_mul : 1.f; a.q_mul = d.mem_q_mul != 0.f ? d.mem_q_mul : 1.f;
-        a.act = d.mem_qkv_act == 1 ? 7 : d.mem_qkv_act == 2 ? 2 : 0;
-        a.rot = HyScanRot{d.rot_dims, L.rot_freq, d.rot_interleaved};
-        a.mode = eg ? 1 : cg ? 3 : 2; if (cg) { a.fbias = L.pbias + L.f_off; a.lower = L.mem_lower; }
-        a.ga = ga; a.gb = gb; a.decay = L.decay; a.ones_col = eg ? 1 : 0;
-        a.heads = d.heads; a.P = P; a.N = d.dim; a.G = d.heads;
-        a.state = h->slots + L.off_state; a.slot_stride = h->slot_floats; a.dyn = h->dyn; a.n = n; a.y = h->ssm_y; a.ldy = ldy;
-        if (n == 1 && hy_scan_out<T>(ctx, L, a, mixo)) return GL3_OK;
+        if (n == 1 && hy_scan_out<T>(ctx, L, np, mixo)) return GL3_OK;
+        HyScanArgs a = hy_mem_scan_args(ctx, L, np, n);
         if (eg)
             hipLaunchKernelGGL(hy_mem_gates_kernel, dim3(d.heads), dim3(256), 0, st, h->proj, np, L.i_off, L.f_off, L.pbias, d.mem_gate_cap, d.heads, h->slots + L.off_m,
                                h->slot_floats, h->dyn, n, ga, gb, ge);
@@ -1492,10 +1527,14 @@ static int32_t hy_mixer_core(gl3_ctx* ctx, HyLayer& L, int np, int ldo, int n, i
         const int inner = d.heads * d.vdim, ch = hy_conv_ch(d), dt_off = 2 * inner + 2 * d.groups * d.state;
         float* state = h->slots + L.off_state;
         float* tail = h->slots + L.off_tail;
-        hipLaunchKernelGGL(hy_conv_kernel, dim3(hy_cdiv(ch, 256), hy_cdiv(n, hy_conv_tokens(d.conv))), dim3(256), 0, st, h->proj, np, inner, ch, d.conv, L.conv_w, L.conv_b, tail, h->slot_floats, h->dyn,
-                           n, h->conv);
-        if (d.conv > 1 && n > hy_conv_tokens(d.conv))
-            hipLaunchKernelGGL(hy_conv_tail_kernel, dim3(hy_cdiv(ch, 256)), dim3(256), 0, st, h->proj, np, inner, ch, d.conv, tail, h->slot_floats, h->dyn, n);
+        HyConvOne cv{};          // one token: the recurrence makes the convolution itself
+        if (n == 1 && d.conv <= 4 && d.state <= 4096 && !hy_scan_forced(d.state)) { cv.x = h->proj + inner; cv.w = L.conv_w; cv.bias = L.conv_b; cv.tail = tail; cv.ch = ch; cv.taps = d.conv; }
+        else {
+            hipLaunchKernelGGL(hy_conv_kernel, dim3(hy_cdiv(ch, 256), hy_cdiv(n, hy_conv_tokens(d.conv))), dim3(256), 0, st, h->proj, np, inner, ch, d.conv, L.conv_w, L.conv_b, tail, h->slot_floats, h->dyn,
+                               n, h->conv);
+            if (d.conv > 1 && n > hy_conv_tokens(d.conv))
+                hipLaunchKernelGGL(hy_conv_tail_kernel, dim3(hy_cdiv(ch, 256)), dim3(256), 0, st, h->proj, np, inner, ch, d.conv, tail, h->slot_floats, h->dyn, n);
+        }
         HyScanArgs a{};
         a.ksrc = h->conv; a.ldk = ch; a.k_off = inner; a.k_hstride = d.state;
         a.qsrc = h->conv; a.ldq = ch; a.q_off = inner + d.groups * d.state; a.q_hstride = d.state;
@@ -1504,8 +1543,8 @@ static int32_t hy_mixer_core(gl3_ctx* ctx, HyLayer& L, int np, int ldo, int n, i
         a.mode = 0; a.dtsrc = h->proj; a.ld_dt = np; a.dt_off = dt_off; a.dt_bias = L.dt_bias; a.A_log = L.a_log; a.Dp = L.dskip;
         a.heads = d.heads; a.P = d.vdim; a.N = d.state; a.G = d.groups;
         a.state = state; a.slot_stride = h->slot_floats; a.dyn = h->dyn; a.n = n; a.y = h->ssm_y; a.ldy = inner;
-        hy_scan(ctx, a);
-        hipLaunchKernelGGL((hy_gated_norm_kernel<T>), dim3(n, d.norm_groups), dim3(256), 0, st, h->ssm_y, h->proj, np, 0, inner, d.norm_groups, L.ssm_norm, eps, mixo, ldo);
+        hy_scan(ctx, a, cv);
+        hipLaunchKernelGGL((hy_gated_norm_kernel<T>), dim3(n, d.norm_groups + (cv.w ? hy_cdiv(ch, 256) : 0)), dim3(256), 0, st, h->ssm_y, h->proj, np, 0, inner, d.norm_groups, L.ssm_norm, eps, mixo, ldo, cv, h->dyn, h->slot_floats);
     }
     return GL3_OK;
 }
@@ -1527,8 +1566,12 @@ static int32_t hy_mixer(gl3_ctx* ctx, HyLayer& L, int n, int pos0, int seq) {
         }
     } else
         hy_gemm<T>(ctx, (T*)h->h, h->W, L.proj, n, h->proj, np, false, nullptr, 0, HyGlu{});
-    int32_t r = hy_mixer_core<T>(ctx, L, np, L.mo_total, n, pos0, seq);
-    if (r == GL3_OK && L.side) r = hy_mixer_core<T>(ctx, *L.side, np, L.mo_total, n, pos0, seq);
+    int32_t r = GL3_OK;
+    if (n == 1 && L.side && hy_pair_one<T>(ctx, L, *L.side, np, pos0)) hy_pool(ctx, L, n, pos0);
+    else {
+        r = hy_mixer_core<T>(ctx, L, np, L.mo_total, n, pos0, seq);
+        if (r == GL3_OK && L.side) r = hy_mixer_core<T>(ctx, *L.side, np, L.mo_total, n, pos0, seq);
+    }
     if (r != GL3_OK) return r;
     hy_gemm<T>(ctx, (T*)h->mixo, L.mo_total, L.o, n, h->y, h->W, false, nullptr, 0, HyGlu{}, &h->y_parts);
     h->y_first = h->y_parts;
@@ -1642,15 +1685,18 @@ static void hy_moe(gl3_ctx* ctx, HyLayer& L, int n) {
     }
 }
 
-// logits of the nw rows listed in h->want: final norm of the gathered rows, the head's product, the optional cap * tanh(. / cap)
+// logits of the nw rows listed in h->want: final norm of the gathered rows (normed: the last sublayer's update has left it in h->xw), the head's product, the
+// optional cap * tanh(. / cap) (a few rows: in the product)
 template <typename T>
-static void hy_logits(gl3_ctx* ctx, int nw) {
+static void hy_logits(gl3_ctx* ctx, int nw, bool normed = false) {
     gl3_hybrid_state* h = ctx->hy;
     T* xw = (T*)h->xw;
-    hy_streams<T>(ctx, nw, h->X, h->W, h->S, (size_t)h->mb * h->W, (const float*)nullptr, 1, 0, (const float*)nullptr, (const float*)nullptr,
+    if (!normed) hy_streams<T>(ctx, nw, h->X, h->W, h->S, (size_t)h->mb * h->W, (const float*)nullptr, 1, 0, (const float*)nullptr, (const float*)nullptr,
                   h->ones, h->final_norm, ctx->d.rms_eps, xw, (float*)nullptr, h->want);
-    hy_gemm<T>(ctx, xw, h->W, h->head, nw, h->logits, ctx->d.vocab, false, nullptr, 0, HyGlu{});
-    if (h->softcap > 0.f) {
+    HyGlu g{};
+    if (nw <= 4) g.cap = h->softcap;
+    hy_gemm<T>(ctx, xw, h->W, h->head, nw, h->logits, ctx->d.vocab, false, nullptr, 0, g);
+    if (h->softcap > 0.f && nw > 4) {
         const size_t cnt = (size_t)nw * ctx->d.vocab;
         hipLaunchKernelGGL(hy_softcap_kernel, dim3((unsigned)std::min<size_t>(1024, (cnt + 255) / 256)), dim3(256), 0, ctx->stream, h->logits, cnt, h->softcap);
     }
@@ -1683,9 +1729,16 @@ static int32_t hy_portion_plain(gl3_ctx* ctx, int seq, const int32_t* tokens, in
     h->h_dyn[0] = pos0; h->h_dyn[1] = seq; h->h_dyn[2] = h->last_tok[seq];
     const int* host = n <= GL3_HOST_TOKENS ? h->h_dyn : nullptr;
     if (!host) HY_HIP(hipMemcpyAsync(h->dyn, h->h_dyn, (size_t)(4 + h->want_cap + n) * 4, hipMemcpyHostToDevice, st));
-    hipLaunchKernelGGL((hy_embed_kernel<T>), dim3(n, hy_cdiv(W, n <= 32 ? 256 : 1024)), dim3(256), 0, st, host, h->dyn, 4 + h->want_cap, nw, (const T*)h->emb.w, h->X, W, 1, lstride, h->emb_scale, h->depth ? h->hist : nullptr,
-                       HyBigram{h->bigram.w, h->bg_buckets, h->bg_prev, h->bg_cur});
     T* hb = (T*)h->h;
+    const HyBigram bg{h->bigram.w, h->bg_buckets, h->bg_prev, h->bg_cur};
+    const bool first = host && !h->shift;          // a few tokens: the first sublayer's norm with the embedding
+    if (first)
+        hipLaunchKernelGGL((hy_embed_norm_kernel<T>), dim3(n), dim3(1024), 0, st, host, h->dyn, 4 + h->want_cap, nw, (const T*)h->emb.w, h->X, W, 1, lstride, h->emb_scale, h->depth ? h->hist : nullptr,
+                           bg, (const float*)nullptr, h->L[0].norm1, eps, hb);
+    else
+        hipLaunchKernelGGL((hy_embed_kernel<T>), dim3(n, hy_cdiv(W, n <= 32 ? 256 : 1024)), dim3(256), 0, st, host, h->dyn, 4 + h->want_cap, nw, (const T*)h->emb.w, h->X, W, 1, lstride, h->emb_scale,
+                           h->depth ? h->hist : nullptr, bg);
+    const bool single = n == 1 && nw == 1 && h->L[nl - 1].d.identity == 0;          // its last update makes the final norm (identity choices read their input where that goes)
     HyResid base{};
     base.x = h->X; base.W = W; base.eps = eps; base.ya_parts = 1; base.ya_mul = 1.f;
     // a residual update that ends in the norm in front of layer l's mixer (l = nl: the last layer has run, no norm), with the token shift
@@ -1696,7 +1749,8 @@ static int32_t hy_portion_plain(gl3_ctx* ctx, int seq, const int32_t* tokens, in
             if (h->shift && n == 1) { r.shift_mu = N.shift_mu; r.shift_prev = h->slots + N.off_shift; r.slot_stride = h->slot_floats; r.dyn = h->dyn; }
             else if (h->shift) r.hf = h->hf;
         }
-        hy_resid<T>(ctx, n, r, h->no_pre ? hb : (T*)nullptr, hb);
+        else if (single) r.norm_w = h->final_norm;
+        hy_resid<T>(ctx, n, r, h->no_pre ? hb : (T*)nullptr, l == nl && single ? (T*)h->xw : hb);
         if (l < nl && r.hf) {
             float* prev = h->slots + h->L[l].off_shift;
             const int v = W % 4 == 0 ? 4 : 1;
@@ -1705,7 +1759,7 @@ static int32_t hy_portion_plain(gl3_ctx* ctx, int seq, const int32_t* tokens, in
             else hipLaunchKernelGGL((hy_shift_kernel<T, 1>), grid, dim3(256), 0, st, h->hf, W, n, h->L[l].shift_mu, prev, h->slot_floats, h->dyn, hb);
         }
     };
-    resid_to_mixer(base, 0);
+    if (!first) resid_to_mixer(base, 0);
     for (int l = 0; l < nl; ++l) {
         HyLayer& L = h->L[l];
         const bool last = l + 1 == nl;
@@ -1746,8 +1800,8 @@ static int32_t hy_portion_plain(gl3_ctx* ctx, int seq, const int32_t* tokens, in
             }
             r.ya_mul = h->resid_mul;
             if (h->taps) r.tap = h->taps + (size_t)l * lstride;
-            if (!last) r.norm_w = h->L[l + 1].norm1;
-            hy_resid<T>(ctx, n, r, (T*)nullptr, hb);
+            r.norm_w = !last ? h->L[l + 1].norm1 : single ? h->final_norm : nullptr;
+            hy_resid<T>(ctx, n, r, (T*)nullptr, last && single ? (T*)h->xw : hb);
             continue;
         }
         if (L.d.out_norm) { r.bw1 = L.branch_norm; r.bw2 = L.side->branch_norm; r.ya_first = h->y_first; }
@@ -1777,7 +1831,7 @@ static int32_t hy_portion_plain(gl3_ctx* ctx, int seq, const int32_t* tokens, in
         }
         finish(r);
     }
-    if (nw > 0) hy_logits<T>(ctx, nw);
+    if (nw > 0) hy_logits<T>(ctx, nw, single);
     HY_HIP(hipGetLastError());
     return GL3_OK;
 }
@@ -1795,33 +1849,39 @@ static int32_t hy_portion(gl3_ctx* ctx, int seq, const int32_t* tokens, int n, i
     h->h_dyn[0] = pos0; h->h_dyn[1] = seq;
     const int* host = n <= GL3_HOST_TOKENS ? h->h_dyn : nullptr;
     if (!host) HY_HIP(hipMemcpyAsync(h->dyn, h->h_dyn, (size_t)(4 + h->want_cap + n) * 4, hipMemcpyHostToDevice, st));
-    hipLaunchKernelGGL((hy_embed_kernel<T>), dim3(n, hy_cdiv(W, n <= 32 ? 256 : 1024)), dim3(256), 0, st, host, h->dyn, 4 + h->want_cap, nw, (const T*)h->emb.w, h->X, W, S, sstride, h->emb_scale, (float*)nullptr);
     T* hb = (T*)h->h;
     const int nl = (int)h->L.size();
-    hy_streams<T>(ctx, n, h->X, W, S, sstride, (const float*)nullptr, 1, 0, (const float*)nullptr, (const float*)nullptr,
-                       h->L[0].hc[0][0], h->L[0].norm1, eps, hb, (float*)nullptr, (const int*)nullptr);
+    if (host)          // a few tokens: the first sublayer's norm with the embedding
+        hipLaunchKernelGGL((hy_embed_norm_kernel<T>), dim3(n), dim3(1024), 0, st, host, h->dyn, 4 + h->want_cap, nw, (const T*)h->emb.w, h->X, W, S, sstride, h->emb_scale, (float*)nullptr, HyBigram{},
+                           h->L[0].hc[0][0], h->L[0].norm1, eps, hb);
+    else {
+        hipLaunchKernelGGL((hy_embed_kernel<T>), dim3(n, hy_cdiv(W, n <= 32 ? 256 : 1024)), dim3(256), 0, st, host, h->dyn, 4 + h->want_cap, nw, (const T*)h->emb.w, h->X, W, S, sstride, h->emb_scale, (float*)nullptr);
+        hy_streams<T>(ctx, n, h->X, W, S, sstride, (const float*)nullptr, 1, 0, (const float*)nullptr, (const float*)nullptr,
+                           h->L[0].hc[0][0], h->L[0].norm1, eps, hb, (float*)nullptr, (const int*)nullptr);
+    }
+    const bool single = n == 1 && nw == 1;          // its last update makes the final norm
     for (int l = 0; l < nl; ++l) {
         HyLayer& L = h->L[l];
         int32_t r = hy_mixer<T>(ctx, L, n, pos0, seq);
         if (r != GL3_OK) return r;
         const bool ff = L.d.ff > 0, last = l + 1 == nl;
         {   // write-back of the mixer sublayer + read of the next sublayer
-            const float* nin = ff ? L.hc[1][0] : last ? nullptr : h->L[l + 1].hc[0][0];
-            const float* nw_ = ff ? L.norm2 : last ? nullptr : h->L[l + 1].norm1;
-            hy_streams<T>(ctx, n, h->X, W, S, sstride, h->y, h->y_parts, (size_t)n * W, L.hc[0][2], L.hc[0][1], nin, nw_, eps, hb,
+            const float* nin = ff ? L.hc[1][0] : !last ? h->L[l + 1].hc[0][0] : single ? h->ones : nullptr;
+            const float* nw_ = ff ? L.norm2 : !last ? h->L[l + 1].norm1 : h->final_norm;
+            hy_streams<T>(ctx, n, h->X, W, S, sstride, h->y, h->y_parts, (size_t)n * W, L.hc[0][2], L.hc[0][1], nin, nw_, eps, !ff && last ? (T*)h->xw : hb,
                                (!ff && h->taps) ? h->taps + (size_t)l * sstride : nullptr, (const int*)nullptr);
         }
         if (ff) {
             T* act = (T*)h->mixo;
             hy_ff_up<T>(ctx, hb, L, n, act);
             hy_gemm<T>(ctx, act, L.ff_pad, L.down, n, h->y, W, false, nullptr, 0, HyGlu{}, &h->y_parts);
-            const float* nin = last ? nullptr : h->L[l + 1].hc[0][0];
-            const float* nw_ = last ? nullptr : h->L[l + 1].norm1;
-            hy_streams<T>(ctx, n, h->X, W, S, sstride, h->y, h->y_parts, (size_t)n * W, L.hc[1][2], L.hc[1][1], nin, nw_, eps, hb,
+            const float* nin = !last ? h->L[l + 1].hc[0][0] : single ? h->ones : nullptr;
+            const float* nw_ = !last ? h->L[l + 1].norm1 : h->final_norm;
+            hy_streams<T>(ctx, n, h->X, W, S, sstride, h->y, h->y_parts, (size_t)n * W, L.hc[1][2], L.hc[1][1], nin, nw_, eps, last ? (T*)h->xw : hb,
                                h->taps ? h->taps + (size_t)l * sstride : nullptr, (const int*)nullptr);
         }
     }
-    if (nw > 0) hy_logits<T>(ctx, nw);
+    if (nw > 0) hy_logits<T>(ctx, nw, single);
     HY_HIP(hipGetLastError());
     return GL3_OK;
 }

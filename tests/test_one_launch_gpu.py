@@ -84,3 +84,22 @@ def test_where_steps_go_over_to_many_workgroups(hy, tmp_path, name, positions):
     again = [p.step(s, toks[i:i + 1], i, [0])[0] for i in range(3)]          # the slot restarts
     p.close()
     assert N.err(np.array(got), want[positions - 4:]) < 3e-5 and N.err(np.array(again), want[:3]) < 3e-5
+
+
+@pytest.mark.parametrize("width", [6, 1022, 8196])
+@pytest.mark.parametrize("design", ["streams", "plain"])
+def test_embedding_with_the_first_norm(hy, tmp_path, design, width):
+    """One to four tokens: the embedding makes the first norm, a single token's last update the final one; rows around a thread's registers, five tokens beside them."""
+    mod = N if design == "streams" else K
+    cfg = mod.config([N.att(heads=2, kv_heads=1, dim=8, vdim=8, ff=0)] if design == "streams" else [K.mls(heads=2, dim=8, vdim=8, ff=8)], width=width, vocab=37)
+    m = mod.Model(hy, tmp_path, cfg, 7)
+    toks = np.random.default_rng(1).integers(0, 37, 24).astype(np.int32)
+    p = m.plan("float32", ctx=32, max_batch=32)
+    s, got, pos = p.acquire(), [], 0
+    for c in [1, 2, 4, 5, 3, 1, 1, 7]:
+        got.append(p.step(s, toks[pos:pos + c], pos, list(range(c))))
+        pos += c
+    again = p.step(s, toks[:3], 0, [2])          # (one wanted row of several)
+    p.close()
+    want = m.ref(toks)
+    assert N.err(np.concatenate(got), want) < 3e-5 and N.err(again, want[2:3]) < 3e-5
