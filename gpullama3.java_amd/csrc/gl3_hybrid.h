@@ -116,7 +116,10 @@ struct gl3_hybrid_state {
     void *h = nullptr, *mixo = nullptr, *xw = nullptr;
     float *logits = nullptr, *taps = nullptr, *ones = nullptr;
     int *tokens = nullptr, *dyn = nullptr, *want = nullptr;
-    int *h_tokens = nullptr, *h_dyn = nullptr, *h_want = nullptr;    // pinned
+    int *h_tokens = nullptr, *h_dyn = nullptr, *h_want = nullptr;    // pinned: the record of the portion being enqueued (one of two: h_rec)
+    int* h_rec = nullptr; int rec = 0;                               // the two records; portions of a call that nobody waits for take them in turn
+    hipEvent_t rec_ev[2] = {}; bool rec_busy[2] = {};                // ends of the portions that read them
+    void use_record(int r, int mb_) { h_dyn = h_rec + (size_t)r * (4 + want_cap + mb_); h_want = h_dyn + 4; h_tokens = h_want + want_cap; }
     float* h_logits = nullptr;                                       // pinned [want_cap][vocab]
     size_t part_rows = 0;
     int last_n = 0;

@@ -238,7 +238,7 @@ int32_t gl3_hy_create(const gl3_model_desc* desc, gl3_ctx** out, std::string& er
     h->want_cap = std::min(h->mb, 256);
     h->busy.assign(h->n_seqs, 0); h->len.assign(h->n_seqs, 0); h->last_tok.assign(h->n_seqs, 0);
     auto fail = [&](int32_t code) { err = ctx->err; gl3_hy_destroy(ctx); if (ctx->stream) hipStreamDestroy(ctx->stream); if (ctx->argmax) hipFree(ctx->argmax);
-                                    if (ctx->h_argmax) hipHostFree(ctx->h_argmax); if (ctx->h_dyn) hipHostFree(ctx->h_dyn); delete ctx; return code; };
+                                    if (ctx->h_argmax) hipHostFree(ctx->h_argmax); ctx->done.free(); if (ctx->h_dyn) hipHostFree(ctx->h_dyn); delete ctx; return code; };
 #define TRY(x) do { int32_t r_ = (x); if (r_ != GL3_OK) return fail(r_); } while (0)
 #define TRYHIP(call) do { hipError_t e_ = (call); if (e_ != hipSuccess) { ctx->err = std::string(#call) + ": " + hipGetErrorString(e_); return fail(e_ == hipErrorOutOfMemory ? GL3_E_OOM : GL3_E_HIP); } } while (0)
     TRYHIP(hipSetDevice(desc->device));
@@ -541,12 +541,14 @@ int32_t gl3_hy_create(const gl3_model_desc* desc, gl3_ctx** out, std::string& er
     // step record, wanted rows and token ids: [dyn 4 | want want_cap | tokens mb], copied to the device by the embedding
     TRY(hy_alloc(ctx, &h->dyn, (size_t)(4 + h->want_cap + mb) * 4));
     h->want = h->dyn + 4; h->tokens = h->want + h->want_cap;
-    TRYHIP(hipHostMalloc((void**)&h->h_dyn, (size_t)(4 + h->want_cap + mb) * 4, hipHostMallocCoherent));
-    h->h_want = h->h_dyn + 4; h->h_tokens = h->h_want + h->want_cap;
-    TRYHIP(hipHostMalloc((void**)&h->h_logits, (size_t)h->want_cap * V * 4));
+    TRYHIP(hipHostMalloc((void**)&h->h_rec, (size_t)2 * (4 + h->want_cap + mb) * 4, hipHostMallocCoherent));
+    h->use_record(0, mb);
+    for (hipEvent_t& e : h->rec_ev) TRYHIP(hipEventCreateWithFlags(&e, hipEventDisableTiming));
+    TRYHIP(hipHostMalloc((void**)&h->h_logits, (size_t)h->want_cap * V * 4, hipHostMallocCoherent));
     TRYHIP(hipMalloc((void**)&ctx->argmax, (2 + 2 * AMX_WGS) * sizeof(int)));
     TRYHIP(hipMemset(ctx->argmax, 0, (2 + 2 * AMX_WGS) * sizeof(int)));
-    TRYHIP(hipHostMalloc((void**)&ctx->h_argmax, sizeof(int)));
+    TRYHIP(hipHostMalloc((void**)&ctx->h_argmax, sizeof(int), hipHostMallocCoherent));
+    TRYHIP(ctx->done.make());
     TRYHIP(hipHostMalloc((void**)&ctx->h_dyn, 4 * sizeof(int)));          // the samplers' result words (gl3_sample.hip)
     {   // attention tiles above the 64 KB default of dynamic LDS
 #define HY_LDS(RW, DVL) TRYHIP(hipFuncSetAttribute((const void*)hy_attn_kernel<RW, DVL>, hipFuncAttributeMaxDynamicSharedMemorySize, 150 * 1024))
@@ -590,7 +592,8 @@ void gl3_hy_destroy(gl3_ctx* ctx) {
     f(h->slots); f(h->X); f(h->h); f(h->proj); f(h->y); f(h->mixo); f(h->conv); f(h->ssm_y); f(h->qa); f(h->oc); f(h->kx); f(h->vx); f(h->part_acc); f(h->part_ml); f(h->gates); f(h->rowr);
     f(h->cq); f(h->qfull); f(h->bigram.w); f(h->hf); f(h->ffz);
     f(h->xw); f(h->logits); f(h->taps); f(h->ones); f(h->dyn);
-    hf(h->h_dyn); hf(h->h_logits);
+    hf(h->h_rec); hf(h->h_logits);
+    for (hipEvent_t e : h->rec_ev) if (e) hipEventDestroy(e);
     if (ctx->logits == h->logits) ctx->logits = nullptr;
     delete h;
     ctx->hy = nullptr;
@@ -1909,6 +1912,8 @@ int32_t gl3_hy_step(gl3_ctx* ctx, int32_t seq, const int32_t* tokens, int32_t n,
         // the portion's wanted rows in groups of want_cap: the first group rides on the portion's run, further groups only redo the head
         int done = wi;
         bool ran = false;
+        if (h->rec_busy[h->rec]) { HY_HIP(hipEventSynchronize(h->rec_ev[h->rec])); h->rec_busy[h->rec] = false; }
+        h->use_record(h->rec, h->mb);
         do {
             const int g = std::min(h->want_cap, we - done);
             std::vector<int32_t> rel(std::max(g, 1));
@@ -1930,8 +1935,15 @@ int32_t gl3_hy_step(gl3_ctx* ctx, int32_t seq, const int32_t* tokens, int32_t n,
             }
             if (r != GL3_OK) return r;
             h->last_tok[seq] = tokens[off + pn - 1];
-            if (g > 0 && logits_out) { launch_to_host(h->logits, h->h_logits, (size_t)g * V, ctx->stream); HY_HIP(hipGetLastError()); }
-            HY_HIP(hipStreamSynchronize(ctx->stream));
+            if (g > 0 && logits_out) {
+                const int wgs = launch_to_host(ctx, h->logits, h->h_logits, (size_t)g * V, true);
+                HY_HIP(hipGetLastError());
+                HY_HIP(ctx->done.wait(wgs, ctx->stream));
+            } else if (g == 0 && off + pn < n) {          // nothing to hand out: the next portion follows at once, on the other record
+                HY_HIP(hipEventRecord(h->rec_ev[h->rec], ctx->stream));
+                h->rec_busy[h->rec] = true;
+                h->rec ^= 1;
+            } else HY_HIP(hipStreamSynchronize(ctx->stream));
             if (g > 0 && logits_out) memcpy(logits_out + (size_t)done * V, h->h_logits, (size_t)g * V * 4);
             done += g;
         } while (done < we);
@@ -1944,9 +1956,9 @@ int32_t gl3_hy_step(gl3_ctx* ctx, int32_t seq, const int32_t* tokens, int32_t n,
 }
 
 int32_t gl3_hy_argmax(gl3_ctx* ctx, int32_t* out) {
-    hipLaunchKernelGGL(argmax_kernel, dim3(AMX_WGS), dim3(256), 0, ctx->stream, ctx->hy->logits, ctx->d.vocab, ctx->argmax, ctx->h_argmax);
+    hipLaunchKernelGGL(argmax_kernel, dim3(AMX_WGS), dim3(256), 0, ctx->stream, ctx->hy->logits, ctx->d.vocab, ctx->argmax, ctx->h_argmax, ctx->done.words, ctx->done.next());
     HY_HIP(hipGetLastError());
-    HY_HIP(hipStreamSynchronize(ctx->stream));
+    HY_HIP(ctx->done.wait(1, ctx->stream));
     *out = *ctx->h_argmax;
     return GL3_OK;
 }

@@ -55,9 +55,9 @@ struct gl3_prefill_state {
     float* SUMS = nullptr;              // [M][n_heads] softmax denominators (pf_softmax_rows_kernel -> pf_pv_tiled_kernel)
     int tmx_tiles = 0;
     int32_t* seqpos = nullptr;          // [2][M] behind tokens: sequence id, position of every token of the step
+    hipEvent_t log_ev[PF_LOG_SLOTS] = {};
     int32_t* h_io = nullptr;            // pinned [4][M], behind ctx->h_logits: tokens, sequence ids, positions of the step on their way in, greedy ids on their way out
     uint8_t* h_log[PF_LOG_SLOTS] = {};  // pinned pieces of logits on their way to the caller (static-batched decode), made when first needed
-    hipEvent_t log_ev[PF_LOG_SLOTS] = {};
     float* LOGITS = nullptr;            // [rows][vocab], grown on demand (batched decode)
     int logits_rows = 0;
     std::vector<hipGraphExec_t> step_graphs;   // static-batched decode: one captured step per batch size (positions < AF_MAXN)
@@ -2742,8 +2742,9 @@ float* gl3_prefill_buf(gl3_ctx* ctx, int which) {
 }
 
 // x of token b from the rank-chunked X into the decode path's plain ctx->x (parity tap gl3_get_x)
-static __global__ void pf_unchunk_row_kernel(const float* __restrict__ X, int b, int dim, int cc, int ntok, float* __restrict__ out) {
+static __global__ void pf_unchunk_row_kernel(const float* __restrict__ X, int b, int dim, int cc, int ntok, float* __restrict__ out, int* done, int no) {
     for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < dim; i += gridDim.x * blockDim.x) out[i] = X[chunked(b, i, cc, ntok)];
+    say_done(done, no);
 }
 
 // Result memory the caller has just got from the system has no pages yet, and taking them one fault at a time costs more than the copy that follows
@@ -2777,7 +2778,7 @@ static int32_t pf_logits_out(gl3_ctx* ctx, float* out, size_t bytes) {
     const size_t pieces = pf_logits_pieces(bytes), per = ((bytes + pieces - 1) / pieces + 4095) & ~(size_t)4095;
     auto send = [&](size_t i) -> int32_t {
         if (i * per >= bytes) return GL3_OK;
-        launch_to_host(p->LOGITS + i * per / 4, (float*)p->h_log[i % PF_LOG_SLOTS], std::min(per, bytes - i * per) / 4, ctx->stream);
+        launch_to_host(ctx, p->LOGITS + i * per / 4, (float*)p->h_log[i % PF_LOG_SLOTS], std::min(per, bytes - i * per) / 4, false);
         GL3_HIP(hipGetLastError());
         GL3_HIP(hipEventRecord(p->log_ev[i % PF_LOG_SLOTS], ctx->stream));
         return GL3_OK;
@@ -2804,8 +2805,9 @@ int32_t gl3_prefill_run(gl3_ctx* ctx, int32_t seq, const int32_t* tokens, int32_
     int32_t r = pf_layers(ctx, n, start_pos + n - 1, seq);
     if (r != GL3_OK) return r;
     // keep the decode path's x in step with the last prefilled token (parity tap gl3_get_x)
-    hipLaunchKernelGGL(pf_unchunk_row_kernel, dim3(4), dim3(256), 0, ctx->stream, p->X, n - 1, d.dim, ctx->dim_l, n, ctx->x);
-    GL3_HIP(hipStreamSynchronize(ctx->stream));
+    hipLaunchKernelGGL(pf_unchunk_row_kernel, dim3(4), dim3(256), 0, ctx->stream, p->X, n - 1, d.dim, ctx->dim_l, n, ctx->x, ctx->done.words, ctx->done.next());
+    GL3_HIP(hipGetLastError());
+    GL3_HIP(d.tp_size == 1 ? ctx->done.wait(4, ctx->stream) : hipStreamSynchronize(ctx->stream));
     drain.passed = true;
     return gl3_tp_check(ctx);
 }
@@ -2869,15 +2871,17 @@ int32_t gl3_decode_batch_run(gl3_ctx* ctx, const int32_t* tokens, const int32_t*
         GL3_HIP(hipGraphLaunch(p->step_graphs[n], s));
     } else if ((r = enqueue_step(max_pos)) != GL3_OK) return r;
     const size_t logit_bytes = (size_t)n * d.vocab * 4;
+    bool waited = false;
     if (logits_out && d.tp_size == 1 && !pf_page_locked(logits_out) && pf_logits_slots(p, logit_bytes)) {
         if ((r = pf_logits_out(ctx, logits_out, logit_bytes)) != GL3_OK) return r;
+        waited = true;          // (the last piece's event is the step's end)
     } else if (logits_out) {      // un-chunk on the way out: [tp][n][vl] -> [n][vocab]
         for (int c = 0; c < d.tp_size; ++c)
             GL3_HIP(hipMemcpy2DAsync(logits_out + (size_t)c * vl, (size_t)d.vocab * 4, p->LOGITS + (size_t)c * n * vl, (size_t)vl * 4, (size_t)vl * 4, n,
                                      hipMemcpyDeviceToHost, s));
     }
     GL3_HIP(hipGetLastError());
-    GL3_HIP(hipStreamSynchronize(s));
+    if (!waited) GL3_HIP(hipStreamSynchronize(s));
     drain.passed = true;
     if (argmax_out) memcpy(argmax_out, p->h_io + 3 * p->max_batch, (size_t)n * sizeof(int32_t));
     return gl3_tp_check(ctx);
