@@ -209,6 +209,39 @@ static __global__ __launch_bounds__(256, DKC > 16 ? 1 : 2) void hy_attn_mfma_ker
         }
         __syncthreads();
     }
+    if (a.out) {          // one split: denominators, gate and the operand's type here (512 tokens x 32 heads of 128: a launch of 10 us, and 16 MB of parts written and read, less)
+        __shared__ float sF[32][2];
+        if (tid < 32) {
+            float L = 0.f;
+#pragma unroll
+            for (int w = 0; w < 4; ++w) if (sml[w][0][r32] > -INFINITY) L += expf(sml[w][0][r32] - M) * sml[w][1][r32];
+            const float z = a.sink_w ? a.sink_w[hr] : 0.f, top = a.sink ? fmaxf(M, z) : M, e = M > -INFINITY ? expf(M - top) : 0.f;
+            sF[tid][0] = e;
+            sF[tid][1] = e * L + (a.sink ? expf(z - top) : 0.f);
+        }
+        __syncthreads();
+        for (int i = tid; i < 32 * (DV / 4); i += 256) {
+            const int r = i / (DV / 4), c = i % (DV / 4), q = row0 + r;
+            if (q >= rows) continue;
+            const int t = q / hpg, h = g * hpg + q % hpg;
+            const float4 v4 = *reinterpret_cast<const float4*>(sO + r * OS + 4 * c);
+            const float e = sF[r][0], den = sF[r][1];
+            float v[4] = {v4.x * e / den, v4.y * e / den, v4.z * e / den, v4.w * e / den};
+            if (a.gate && a.gate_mode == 2) {
+                const float s = hy_sigmoid(a.gate[(size_t)t * a.ldg + h]);
+#pragma unroll
+                for (int k = 0; k < 4; ++k) v[k] *= s;
+            } else if (a.gate) {
+                const float4 z = *reinterpret_cast<const float4*>(a.gate + (size_t)t * a.ldg + h * DV + 4 * c);
+                v[0] *= hy_sigmoid(z.x); v[1] *= hy_sigmoid(z.y); v[2] *= hy_sigmoid(z.z); v[3] *= hy_sigmoid(z.w);
+            }
+#pragma unroll
+            for (int k = 0; k < 4; ++k) v[k] *= a.out_mul;
+            const size_t o = (size_t)t * a.ldo + h * DV + 4 * c;
+            if (a.out_f32) hy_stv<4>((float*)a.out + o, v); else hy_stv<4>((bf16_t*)a.out + o, v);
+        }
+        return;
+    }
     for (int i = tid; i < 32 * (DV / 4); i += 256) {
         const int r = i / (DV / 4), c = i % (DV / 4), q = row0 + r;
         if (q >= rows) continue;

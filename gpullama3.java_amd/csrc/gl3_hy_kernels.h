@@ -125,9 +125,9 @@ static __global__ __launch_bounds__(256) void hy_embed_kernel(const int* host, i
     }
 }
 
-// The same for a step of a few tokens together with the norm in front of the first sublayer (pre_in: the streams' weights, null = one stream; norm_w null: the row itself in
+// The same together with the norm in front of the first sublayer (pre_in: the streams' weights, null = one stream; norm_w null: the row itself in
 // the matrix type, if h_out is there at all): one workgroup per token, its first HY_EN entries per thread in registers.  One launch, and no second trip to memory, for
-// what took 4.2 + 3.7 us.
+// what took 4.2 + 3.7 us for one token and 9.8 + 10 for 512 of two streams.  host null: the record is in rec already.
 constexpr int HY_EN = 8;
 template <typename T>
 static __global__ __launch_bounds__(1024) void hy_embed_norm_kernel(const int* host, int* __restrict__ rec, int tok0, int nw, const T* __restrict__ emb, float* __restrict__ X,
@@ -138,10 +138,10 @@ static __global__ __launch_bounds__(1024) void hy_embed_norm_kernel(const int* h
     const int t = blockIdx.x, tid = threadIdx.x;
     if (tid < 3) {
         const int at = tid == 0 ? tok0 + t : tid == 2 ? 0 : t > 0 ? tok0 + t - 1 : 2;
-        if (tid == 0 || bg.table) sh[tid] = gl3::host_int(host + at);
+        if (tid == 0 || bg.table) sh[tid] = host ? gl3::host_int(host + at) : rec[at];
     }
-    if (t == 0) for (int i = tid - 64; i >= 0 && i < 4 + nw; i += 960) rec[i] = gl3::host_int(host + i);          // (wavefronts that do not wait for the token)
-    if (tid == 0) rec[tok0 + t] = sh[0];
+    if (host && t == 0) for (int i = tid - 64; i >= 0 && i < 4 + nw; i += 960) rec[i] = gl3::host_int(host + i);          // (wavefronts that do not wait for the token)
+    if (host && tid == 0) rec[tok0 + t] = sh[0];
     float ps = 1.f;
     if (pre_in) { ps = 0.f; for (int s = 0; s < S; ++s) ps += pre_in[s]; }
     __syncthreads();
@@ -720,7 +720,7 @@ struct HyPrepX {
 // moves on by this token (every thread the channels it has read).
 __device__ __forceinline__ void hy_conv_row(float* __restrict__ crow, const float* __restrict__ proj, int ld, int col, int t, int len, const float* __restrict__ w_, int C, int taps,
                                             float* __restrict__ tl, bool fresh, bool move_tail) {
-    const int lane = threadIdx.x, keep = taps - 1;
+    const int lane = threadIdx.x & 63, keep = taps - 1;
     const float* src = proj + (size_t)t * ld + col;
     // two channels and four taps at a time, their loads issued together (taps that are not there read the token's own row, times 0)
     for (int d0 = lane; d0 < len; d0 += 128) {
@@ -771,11 +771,14 @@ __device__ __forceinline__ void hy_turn_store(float* __restrict__ dst, const flo
     }
     for (int d = dims + lane; d < D; d += 64) dst[d] = val(d);
 }
-static __global__ __launch_bounds__(64) void hy_attn_prep_kernel(float* __restrict__ proj, int ld, int q_off, int k_off, int v_off, int H, int G, int D, int V,
+constexpr int HY_PREP_HEADS = 4;          // heads a workgroup, a wavefront each (one each: 512 tokens x 48 heads 13.7 us, the launching of 24576 workgroups)
+static __global__ __launch_bounds__(64 * HY_PREP_HEADS) void hy_attn_prep_kernel(float* __restrict__ proj, int ld, int q_off, int k_off, int v_off, int H, int G, int D, int V,
                                                                  int unit_norm, float eps, float* __restrict__ kc, float* __restrict__ vc, size_t slot_stride,
                                                                  const int* __restrict__ dyn, HyRot rot, HyPrepX x = HyPrepX{}) {
-    __shared__ float crow[HY_PREP_MAXD];
-    const int t = blockIdx.x, hh = blockIdx.y, lane = threadIdx.x;
+    __shared__ float crows[HY_PREP_HEADS][HY_PREP_MAXD];
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), t = blockIdx.x, hh = blockIdx.y * HY_PREP_HEADS + wave;
+    if (hh >= H + (x.v_from_k ? 1 : 2) * G) return;          // (no barrier follows)
+    float* crow = crows[wave];
     const int pos = dyn[0] + t;
     const size_t slot = (size_t)dyn[1] * slot_stride;
     if (hh < H + G) {
@@ -786,7 +789,7 @@ static __global__ __launch_bounds__(64) void hy_attn_prep_kernel(float* __restri
         float* dst = isq ? proj + (size_t)t * ld + col : kc + slot + (size_t)pos * (G * D) + (hh - H) * D;
         if (x.taps > 0) {
             hy_conv_row(crow, proj, ld, col, t, D, x.conv_w + hh * D, (H + G) * D, x.taps, x.tail + slot + hh * D, dyn[0] == 0, x.n == 1);
-            __syncthreads();
+            asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");          // (the row is this wavefront's own)
             src = crow;
             if (isq) dst = x.qout + (size_t)t * x.ldq + hh * D;
         }
@@ -1035,6 +1038,8 @@ struct HyAttnArgs {
     // pool > 0 (with a window): pooled rows pk / pv (laid out like kc / vc, one row per block of `pool` positions); query i also sees
     // the pooled rows of blocks b with b pool + pool - 1 <= i - window
     const float* pk; const float* pv; int pool;
+    // out != null (one split, hy_attn_mfma_kernel): the gated result itself, as hy_attn_merge_kernel makes it, instead of the parts; float32 if out_f32, else bfloat16
+    void* out; int ldo, out_f32; const float* gate; int ldg, gate_mode; int sink; const float* sink_w; float out_mul;
 };
 constexpr int HY_KT = 64;
 

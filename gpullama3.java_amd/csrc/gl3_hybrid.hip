@@ -1077,14 +1077,17 @@ static HyAttnPlan hy_attn_plan(int rows, int dk, int dv, bool shared_kv) {
     return p;
 }
 
+// What follows an attention core (hy_attn_merge_kernel's arguments): a core that can do it itself returns 0 splits.
+struct HyAttnOut { void* out; int ldo, f32; const float* gate; int ldg, gate_mode; int sink; const float* sink_w; float out_mul; };
 static int32_t hy_attention(gl3_ctx* ctx, const float* q, int ldq, const float* kc, const float* vc, int H, int G, int dk, int dv, float scale, float slope_log2,
-                            int n, int pos0, int* nsplit_out, bool in_slot = true, int window = 0, int keep = 0, const float* pk = nullptr, const float* pv = nullptr, int pool = 0) {
+                            int n, int pos0, int* nsplit_out, const HyAttnOut* fin = nullptr, bool in_slot = true, int window = 0, int keep = 0, const float* pk = nullptr,
+                            const float* pv = nullptr, int pool = 0) {
     gl3_hybrid_state* h = ctx->hy;
     const bool shared_kv = kc == vc && dk == dv;
     HyAttnArgs a;
     a.q = q; a.ldq = ldq; a.kc = kc; a.vc = vc; a.slot_stride = in_slot ? h->slot_floats : 0; a.H = H; a.G = G; a.dk = dk; a.dv = dv; a.scale = scale; a.slope_log2 = slope_log2;
     a.dyn = h->dyn; a.n = n; a.part_acc = h->part_acc; a.part_ml = h->part_ml; a.shared_kv = shared_kv ? 1 : 0; a.window = window; a.keep = keep;
-    a.pk = pk; a.pv = pv; a.pool = pool;
+    a.pk = pk; a.pv = pv; a.pool = pool; a.out = nullptr;
     // Matrix cores from 17 tokens on (up to 16 the keys are split over many workgroups, below), for the head sizes the kernel is built for.
     const bool aligned = ((ldq | H * dk | a.slot_stride) & 3) == 0 && (((uintptr_t)q | (uintptr_t)kc | (uintptr_t)vc | (uintptr_t)pk | (uintptr_t)pv) & 15) == 0;
     // A few tokens: one tile of 32 keys per split.  Heads of 64 with up to 8 rows a key / value head go to the vector kernel below once their tiles do not run side by side
@@ -1116,6 +1119,11 @@ static int32_t hy_attention(gl3_ctx* ctx, const float* q, int ldq, const float* 
         int nsplit = std::max(1, std::min({512 / blocks, HY_MFMA_SPLITS, hy_cdiv(pos0 + n, 512)}));
         if ((size_t)n * nsplit > h->part_rows) nsplit = std::max<size_t>(1, h->part_rows / n);
         a.nsplit = nsplit; a.kt = 32;
+        const int els = fin && fin->f32 ? 4 : 2;
+        if (nsplit == 1 && fin && !((fin->ldo | (fin->gate && fin->gate_mode != 2 ? fin->ldg : 0)) & 3) && !((uintptr_t)fin->out % (4 * els)) && !((uintptr_t)(fin->gate_mode != 2 ? fin->gate : nullptr) & 15)) {
+            a.out = fin->out; a.ldo = fin->ldo; a.out_f32 = fin->f32; a.gate = fin->gate; a.ldg = fin->ldg; a.gate_mode = fin->gate_mode; a.sink = fin->sink; a.sink_w = fin->sink_w;
+            a.out_mul = fin->out_mul;
+        }
         const dim3 grid(blocks, 1, nsplit);
         bool done = true;
 #define HY_AM(DKC, DVT) hipLaunchKernelGGL((hy_attn_mfma_kernel<DKC, DVT>), grid, dim3(256), 0, ctx->stream, a)
@@ -1125,7 +1133,7 @@ static int32_t hy_attention(gl3_ctx* ctx, const float* q, int ldq, const float* 
         else if (dk == 96 && dv == 64) HY_AM(12, 2);
         else done = false;
 #undef HY_AM
-        if (done) { *nsplit_out = nsplit; return GL3_OK; }
+        if (done) { *nsplit_out = a.out ? 0 : nsplit; return GL3_OK; }
     }
     HyAttnPlan p = hy_attn_plan(n * (H / G), dk, dv, shared_kv);
     if (p.smem > 150 * 1024) GL3_FAIL(GL3_E_UNSUPPORTED, "attention: key + value row too large for the LDS tile");
@@ -1152,6 +1160,7 @@ static int32_t hy_attention(gl3_ctx* ctx, const float* q, int ldq, const float* 
 // Joins the key splits of an attention core's launch: out[n][heads dv] (row stride ldo), gated and turned back where the layer asks for it.
 template <typename TO>
 static void hy_merge(gl3_ctx* ctx, const HyLayer& L, int n, int dv, int nsplit, const float* gate, int ldg, int gate_mode, TO* out, int ldo, const float* v_freq = nullptr, float out_mul = 1.f) {
+    if (nsplit == 0) return;          // (the core has made the result)
     gl3_hybrid_state* h = ctx->hy;
     const gl3_layer_desc& d = L.d;
     const float* sink_w = d.softmax_sink == 2 ? L.sink : nullptr;
@@ -1424,14 +1433,15 @@ static int32_t hy_mixer_core(gl3_ctx* ctx, HyLayer& L, int np, int ldo, int n, i
             if (n <= 32) hipLaunchKernelGGL((hy_rowrms_kernel<1024>), dim3(n, 2), dim3(1024), 0, st, h->proj, np, L.q_off, d.heads * d.dim, L.k_off, d.kv_heads * d.dim, px.bias, eps, h->rowr);
             else hipLaunchKernelGGL((hy_rowrms_kernel<256>), dim3(n, 2), dim3(256), 0, st, h->proj, np, L.q_off, d.heads * d.dim, L.k_off, d.kv_heads * d.dim, px.bias, eps, h->rowr);
         }
-        hipLaunchKernelGGL(hy_attn_prep_kernel, dim3(n, d.heads + (d.v_from_k ? 1 : 2) * d.kv_heads), dim3(64), 0, st, h->proj, np, L.q_off, L.k_off, L.v_off, d.heads, d.kv_heads, d.dim,
+        hipLaunchKernelGGL(hy_attn_prep_kernel, dim3(n, hy_cdiv(d.heads + (d.v_from_k ? 1 : 2) * d.kv_heads, HY_PREP_HEADS)), dim3(64 * HY_PREP_HEADS), 0, st, h->proj, np, L.q_off, L.k_off, L.v_off, d.heads, d.kv_heads, d.dim,
                            d.vdim, d.qk_unit_norm, eps, kc, vc, h->slot_floats, h->dyn, rot, px);
         if (d.qk_conv > 1 && n > 1)          // (q and k stand side by side in the projection row; a single token's tail moved on above)
             hipLaunchKernelGGL(hy_conv_tail_kernel, dim3(hy_cdiv(hy_qk_ch(d), 256)), dim3(256), 0, st, h->proj, np, L.q_off, hy_qk_ch(d), d.qk_conv, h->slots + L.off_tail,
                                h->slot_floats, h->dyn, n);
         hy_pool(ctx, L, n, pos0);
+        const HyAttnOut fin{mixo, ldo, sizeof(T) == 4, d.out_gate ? h->proj + L.g_off : nullptr, np, d.out_gate, d.softmax_sink, d.softmax_sink == 2 ? L.sink : nullptr, d.out_norm ? 1.f : L.out_mul};
         int32_t r = hy_by_heads(d) ? hy_attention_heads(ctx, L, q, ldq, kc, vc, n, pos0, &nsplit)
-                                   : hy_attention(ctx, q, ldq, kc, vc, d.heads, d.kv_heads, d.dim, d.vdim, d.scale, d.slope_log2, n, pos0, &nsplit, true, d.window, d.keep_first,
+                                   : hy_attention(ctx, q, ldq, kc, vc, d.heads, d.kv_heads, d.dim, d.vdim, d.scale, d.slope_log2, n, pos0, &nsplit, d.v_rot ? nullptr : &fin, true, d.window, d.keep_first,
                                                   pk, pv, d.pool);
         if (r != GL3_OK) return r;
         hy_merge<T>(ctx, L, n, d.vdim, nsplit, d.out_gate ? h->proj + L.g_off : nullptr, np, d.out_gate, mixo, ldo, d.v_rot ? L.vrot_freq : nullptr,
@@ -1501,7 +1511,8 @@ static int32_t hy_mixer_core(gl3_ctx* ctx, HyLayer& L, int np, int ldo, int n, i
             wvm.w = L.wv; wvm.rows = d.heads * d.vdim; wvm.k = R; wvm.ld = R;
             hy_gemm<float>(ctx, lat, R, wkm, M, h->kx, d.heads * De, false, nullptr, 0, HyGlu{});
             hy_gemm<float>(ctx, lat, R, wvm, M, h->vx, d.heads * d.vdim, false, nullptr, 0, HyGlu{});
-            int32_t r = hy_attention(ctx, q, ldq, h->kx, h->vx, d.heads, d.heads, De, d.vdim, d.scale, 0.f, n, pos0, &nsplit, false);
+            const HyAttnOut fin{mixo, ldo, sizeof(T) == 4, d.out_gate ? h->proj + L.g_off : nullptr, np, d.out_gate == 2 ? 2 : 1, d.softmax_sink, d.softmax_sink == 2 ? L.sink : nullptr, 1.f};
+            int32_t r = hy_attention(ctx, q, ldq, h->kx, h->vx, d.heads, d.heads, De, d.vdim, d.scale, 0.f, n, pos0, &nsplit, &fin, false);
             if (r != GL3_OK) return r;
             hy_merge<T>(ctx, L, n, d.vdim, nsplit, d.out_gate ? h->proj + L.g_off : nullptr, np, d.out_gate == 2 ? 2 : 1, mixo, ldo);
         } else {
@@ -1734,7 +1745,7 @@ static int32_t hy_portion_plain(gl3_ctx* ctx, int seq, const int32_t* tokens, in
     if (!host) HY_HIP(hipMemcpyAsync(h->dyn, h->h_dyn, (size_t)(4 + h->want_cap + n) * 4, hipMemcpyHostToDevice, st));
     T* hb = (T*)h->h;
     const HyBigram bg{h->bigram.w, h->bg_buckets, h->bg_prev, h->bg_cur};
-    const bool first = host && !h->shift;          // a few tokens: the first sublayer's norm with the embedding
+    const bool first = !h->shift;          // the first sublayer's norm with the embedding
     if (first)
         hipLaunchKernelGGL((hy_embed_norm_kernel<T>), dim3(n), dim3(1024), 0, st, host, h->dyn, 4 + h->want_cap, nw, (const T*)h->emb.w, h->X, W, 1, lstride, h->emb_scale, h->depth ? h->hist : nullptr,
                            bg, (const float*)nullptr, h->L[0].norm1, eps, hb);
@@ -1854,14 +1865,8 @@ static int32_t hy_portion(gl3_ctx* ctx, int seq, const int32_t* tokens, int n, i
     if (!host) HY_HIP(hipMemcpyAsync(h->dyn, h->h_dyn, (size_t)(4 + h->want_cap + n) * 4, hipMemcpyHostToDevice, st));
     T* hb = (T*)h->h;
     const int nl = (int)h->L.size();
-    if (host)          // a few tokens: the first sublayer's norm with the embedding
-        hipLaunchKernelGGL((hy_embed_norm_kernel<T>), dim3(n), dim3(1024), 0, st, host, h->dyn, 4 + h->want_cap, nw, (const T*)h->emb.w, h->X, W, S, sstride, h->emb_scale, (float*)nullptr, HyBigram{},
-                           h->L[0].hc[0][0], h->L[0].norm1, eps, hb);
-    else {
-        hipLaunchKernelGGL((hy_embed_kernel<T>), dim3(n, hy_cdiv(W, n <= 32 ? 256 : 1024)), dim3(256), 0, st, host, h->dyn, 4 + h->want_cap, nw, (const T*)h->emb.w, h->X, W, S, sstride, h->emb_scale, (float*)nullptr);
-        hy_streams<T>(ctx, n, h->X, W, S, sstride, (const float*)nullptr, 1, 0, (const float*)nullptr, (const float*)nullptr,
-                           h->L[0].hc[0][0], h->L[0].norm1, eps, hb, (float*)nullptr, (const int*)nullptr);
-    }
+    hipLaunchKernelGGL((hy_embed_norm_kernel<T>), dim3(n), dim3(1024), 0, st, host, h->dyn, 4 + h->want_cap, nw, (const T*)h->emb.w, h->X, W, S, sstride, h->emb_scale, (float*)nullptr, HyBigram{},
+                       h->L[0].hc[0][0], h->L[0].norm1, eps, hb);
     const bool single = n == 1 && nw == 1;          // its last update makes the final norm
     for (int l = 0; l < nl; ++l) {
         HyLayer& L = h->L[l];
@@ -1907,13 +1912,13 @@ int32_t gl3_hy_step(gl3_ctx* ctx, int32_t seq, const int32_t* tokens, int32_t n,
     int wi = 0;
     for (int off = 0; off < n; off += h->mb) {
         const int pn = std::min(h->mb, n - off);
+        if (h->rec_busy[h->rec]) { HY_HIP(hipEventSynchronize(h->rec_ev[h->rec])); h->rec_busy[h->rec] = false; }
+        h->use_record(h->rec, h->mb);
         int we = wi;
         while (we < n_want && want[we] < off + pn) ++we;
         // the portion's wanted rows in groups of want_cap: the first group rides on the portion's run, further groups only redo the head
         int done = wi;
         bool ran = false;
-        if (h->rec_busy[h->rec]) { HY_HIP(hipEventSynchronize(h->rec_ev[h->rec])); h->rec_busy[h->rec] = false; }
-        h->use_record(h->rec, h->mb);
         do {
             const int g = std::min(h->want_cap, we - done);
             std::vector<int32_t> rel(std::max(g, 1));
