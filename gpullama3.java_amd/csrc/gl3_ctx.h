@@ -130,8 +130,9 @@ constexpr size_t GL3_ARENA_HDR = 1024, GL3_ARENA_SEQ = 64, GL3_ARENA_ARRIVE = 68
 constexpr size_t GL3_ARENA_FOLD = 512, GL3_ARENA_FOLD_TICKET = 704, GL3_ARENA_STEP = 720;
 
 // Waiting for a step through words its last kernel sets (say_done): hipStreamSynchronize returns 6.5 us after the last kernel has ended, this within the reading of a
-// word.  The stream itself may be a few us behind; whatever is enqueued or freed next waits for it as ever.  A step that is not there after 5 ms is waited for, and its
-// errors reported, by the runtime.
+// word.  The stream itself may be a few us behind; whatever is enqueued or freed next waits for it as ever.  But a program that waits for the whole device next pays 45 - 100 us
+// there (15 behind a wait of the runtime's, which has tidied up): short steps only, of which many follow each other, not prompts.  A step that is not there after 5 ms
+// is waited for, and its errors reported, by the runtime.
 constexpr int GL3_DONE_WORD = 16, GL3_DONE_WGS = 256;
 struct gl3_done {
     int* words = nullptr;          // page-locked, coherent: [GL3_DONE_WGS][GL3_DONE_WORD]

@@ -771,7 +771,7 @@ __device__ __forceinline__ void hy_turn_store(float* __restrict__ dst, const flo
     }
     for (int d = dims + lane; d < D; d += 64) dst[d] = val(d);
 }
-constexpr int HY_PREP_HEADS = 4;          // heads a workgroup, a wavefront each (one each: 512 tokens x 48 heads 13.7 us, the launching of 24576 workgroups)
+constexpr int HY_PREP_HEADS = 4;          // heads a workgroup, a wavefront each (512 tokens x 48 heads of 128 13.2 us, 13.7 with a workgroup per head)
 static __global__ __launch_bounds__(64 * HY_PREP_HEADS) void hy_attn_prep_kernel(float* __restrict__ proj, int ld, int q_off, int k_off, int v_off, int H, int G, int D, int V,
                                                                  int unit_norm, float eps, float* __restrict__ kc, float* __restrict__ vc, size_t slot_stride,
                                                                  const int* __restrict__ dyn, HyRot rot, HyPrepX x = HyPrepX{}) {

@@ -1941,9 +1941,10 @@ int32_t gl3_hy_step(gl3_ctx* ctx, int32_t seq, const int32_t* tokens, int32_t n,
             if (r != GL3_OK) return r;
             h->last_tok[seq] = tokens[off + pn - 1];
             if (g > 0 && logits_out) {
-                const int wgs = launch_to_host(ctx, h->logits, h->h_logits, (size_t)g * V, true);
+                const bool words = n <= GL3_HOST_TOKENS;
+                const int wgs = launch_to_host(ctx, h->logits, h->h_logits, (size_t)g * V, words);
                 HY_HIP(hipGetLastError());
-                HY_HIP(ctx->done.wait(wgs, ctx->stream));
+                HY_HIP(words ? ctx->done.wait(wgs, ctx->stream) : hipStreamSynchronize(ctx->stream));
             } else if (g == 0 && off + pn < n) {          // nothing to hand out: the next portion follows at once, on the other record
                 HY_HIP(hipEventRecord(h->rec_ev[h->rec], ctx->stream));
                 h->rec_busy[h->rec] = true;

@@ -2742,9 +2742,8 @@ float* gl3_prefill_buf(gl3_ctx* ctx, int which) {
 }
 
 // x of token b from the rank-chunked X into the decode path's plain ctx->x (parity tap gl3_get_x)
-static __global__ void pf_unchunk_row_kernel(const float* __restrict__ X, int b, int dim, int cc, int ntok, float* __restrict__ out, int* done, int no) {
+static __global__ void pf_unchunk_row_kernel(const float* __restrict__ X, int b, int dim, int cc, int ntok, float* __restrict__ out) {
     for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < dim; i += gridDim.x * blockDim.x) out[i] = X[chunked(b, i, cc, ntok)];
-    say_done(done, no);
 }
 
 // Result memory the caller has just got from the system has no pages yet, and taking them one fault at a time costs more than the copy that follows
@@ -2805,9 +2804,8 @@ int32_t gl3_prefill_run(gl3_ctx* ctx, int32_t seq, const int32_t* tokens, int32_
     int32_t r = pf_layers(ctx, n, start_pos + n - 1, seq);
     if (r != GL3_OK) return r;
     // keep the decode path's x in step with the last prefilled token (parity tap gl3_get_x)
-    hipLaunchKernelGGL(pf_unchunk_row_kernel, dim3(4), dim3(256), 0, ctx->stream, p->X, n - 1, d.dim, ctx->dim_l, n, ctx->x, ctx->done.words, ctx->done.next());
-    GL3_HIP(hipGetLastError());
-    GL3_HIP(d.tp_size == 1 ? ctx->done.wait(4, ctx->stream) : hipStreamSynchronize(ctx->stream));
+    hipLaunchKernelGGL(pf_unchunk_row_kernel, dim3(4), dim3(256), 0, ctx->stream, p->X, n - 1, d.dim, ctx->dim_l, n, ctx->x);
+    GL3_HIP(hipStreamSynchronize(ctx->stream));
     drain.passed = true;
     return gl3_tp_check(ctx);
 }
