@@ -555,6 +555,9 @@ int32_t gl3_hy_create(const gl3_model_desc* desc, gl3_ctx** out, std::string& er
         HY_LDS(1, 1); HY_LDS(1, 2); HY_LDS(1, 4); HY_LDS(1, 8); HY_LDS(2, 1); HY_LDS(2, 2); HY_LDS(2, 4); HY_LDS(2, 8);
         HY_LDS(4, 1); HY_LDS(4, 2); HY_LDS(4, 4); HY_LDS(4, 8); HY_LDS(8, 1); HY_LDS(8, 2); HY_LDS(8, 4);
 #undef HY_LDS
+#define HY_LDS(NT, PC) TRYHIP(hipFuncSetAttribute((const void*)hy_scan_chunk_kernel<NT, PC>, hipFuncAttributeMaxDynamicSharedMemorySize, 2 * hy_chunk_floats(64 * NT, PC) * 4))
+        HY_LDS(1, 16); HY_LDS(2, 16); HY_LDS(2, 32); HY_LDS(4, 16); HY_LDS(4, 32);
+#undef HY_LDS
 #define HY_LDS(...) TRYHIP(hipFuncSetAttribute((const void*)hy_heads_attn_kernel<__VA_ARGS__>, hipFuncAttributeMaxDynamicSharedMemorySize, 150 * 1024))
         HY_LDS(1, 1, true); HY_LDS(1, 2, true); HY_LDS(1, 4, true); HY_LDS(2, 1, true); HY_LDS(2, 2, true); HY_LDS(2, 4, true);
         HY_LDS(4, 1, true); HY_LDS(4, 2, true); HY_LDS(4, 4, true); HY_LDS(1, 1, false); HY_LDS(1, 2, false); HY_LDS(1, 4, false);
@@ -1242,9 +1245,9 @@ static void hy_scan_chunk_launch(gl3_ctx* ctx, const HyScanArgs& a) {
     // with 16 and 61 with 32, 8 x 513 (264 or 136 workgroups) 112 and 96, 128 x 64 (512 or 256) 80 and 71.  64 states: always 16 (four layers of 64 heads x 80, 96 x 64,
     // 128 x 64, 32 x 129, 32 x 257, whole steps of 33 - 512 tokens: 32 columns take 0 - 6 % longer, with LDS of their own for the shares of y)
     const int pc = a.N == 64 || (long)a.heads * hy_cdiv(a.P, 16) <= 256 ? 16 : 32;
-    const size_t smem = (size_t)(2 * 32 * (a.N + 4) + 32 * (pc + 4) + 32 * 36 + 32 * 33 + 68) * 4;
+    const size_t smem = (size_t)2 * hy_chunk_floats(a.N, pc) * 4;          // (256 states x 32 columns: 157 KB)
     const dim3 grid(hy_cdiv(a.P, pc), a.heads);
-#define HY_SC(NT, PC) hipLaunchKernelGGL((hy_scan_chunk_kernel<NT, PC>), grid, dim3(256), smem, ctx->stream, a)
+#define HY_SC(NT, PC) hipLaunchKernelGGL((hy_scan_chunk_kernel<NT, PC>), grid, dim3(512), smem, ctx->stream, a)
     if (a.N == 64) HY_SC(1, 16);
     else if (a.N == 128) { if (pc == 32) HY_SC(2, 32); else HY_SC(2, 16); }
     else { if (pc == 32) HY_SC(4, 32); else HY_SC(4, 16); }
