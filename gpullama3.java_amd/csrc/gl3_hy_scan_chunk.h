@@ -24,16 +24,17 @@ __device__ __forceinline__ void hy_lds_barrier() { asm volatile("s_waitcnt lgkmc
 __device__ __forceinline__ hy_acc4 hy_mma4(float a, float b, hy_acc4 c) { return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0); }
 
 // Keys and queries of a whole portion in place, as the recurrence takes them: silu (act 1: keys, 2: queries), the multiplier, the turn by the
-// position (HyScanRot).  One workgroup per token; the angles are shared by the heads.
-static __global__ __launch_bounds__(256) void hy_scan_prep_kernel(float* __restrict__ proj, int ld, int q_off, int k_off, int heads, int N, float q_mul, float k_mul, int act,
+// position (HyScanRot).  One workgroup per token; the angles are shared by the heads.  (1024 threads: in place, a thread's pairs wait for each other; 88 and 512 tokens of 16 heads
+// x 128 5.0 and 8.0 us, 8.9 and 10.6 with 256 threads.)
+static __global__ __launch_bounds__(1024) void hy_scan_prep_kernel(float* __restrict__ proj, int ld, int q_off, int k_off, int heads, int N, float q_mul, float k_mul, int act,
                                                                   HyScanRot rot, const int* __restrict__ dyn) {
     extern __shared__ float sc[];          // cosines, sines of rot.dims / 2 angles
     const int half = rot.dims >> 1, pos = dyn[0] + blockIdx.x;
-    for (int j = threadIdx.x; j < half; j += 256) sincosf((float)pos * rot.freq[j], &sc[half + j], &sc[j]);
+    for (int j = threadIdx.x; j < half; j += 1024) sincosf((float)pos * rot.freq[j], &sc[half + j], &sc[j]);
     __syncthreads();
     float* row = proj + (size_t)blockIdx.x * ld;
     const int pairs = N - half;            // per head: half pairs, then single entries
-    for (int i = threadIdx.x; i < 2 * heads * pairs; i += 256) {
+    for (int i = threadIdx.x; i < 2 * heads * pairs; i += 1024) {
         const int which = i / (heads * pairs), h = i / pairs % heads, j = i % pairs;
         float* r = row + (which ? k_off : q_off) + h * N;
         const float mul = which ? k_mul : q_mul;

@@ -1046,7 +1046,8 @@ static void hy_streams(gl3_ctx* ctx, int blocks, float* X, int W, int S, size_t 
 #define HY_ST4(NT, NS) hipLaunchKernelGGL((hy_streams4_kernel<T, NT, NS>), dim3(blocks), dim3(NT), 0, ctx->stream, X, W, sstride, y, yparts, ystride, post_mix, post_out, pre_in, norm_w, eps, h_out, sum_out, rows)
 #define HY_ST4_S(NT) do { if (S == 1) HY_ST4(NT, 1); else if (S == 2) HY_ST4(NT, 2); else HY_ST4(NT, 4); } while (0)
     if (W % 4 == 0 && (S == 1 || S == 2 || S == 4)) {          // (every row then starts on 16 bytes: the plan's buffers do)
-        if (blocks <= 32) HY_ST4_S(1024); else HY_ST4_S(256);
+        // (a row on 1024 threads is read in one trip; past a row per CU the smaller workgroups hide theirs behind each other: 200 x 4096, two streams 7.2 us, 8.6 with 256, 512 14.6 and 12.8)
+        if (blocks <= 256) HY_ST4_S(1024); else HY_ST4_S(256);
         return;
     }
 #undef HY_ST4_S
@@ -1301,9 +1302,10 @@ static void hy_mem_out(gl3_ctx* ctx, const HyLayer& L, int n, int ldy, int P, co
     const int heads = whole ? 1 : d.heads, V = whole ? ldy : d.vdim;
     if (whole) P = ldy;
 #define HY_MO(NT) hipLaunchKernelGGL((hy_mem_out_kernel<T, NT>), dim3(n, heads), dim3(NT), 0, ctx->stream, h->ssm_y, ldy, P, V, ge, heads, w, gate, np, L.g_off, d.mem_gate_act, ctx->d.rms_eps, mul, mixo, ldo, w_stride)
-    // a whole row is heads x vdim wide: 1024 threads for a few tokens, 256 for many; a head: 256 / 64
+    // a whole row is heads x vdim wide: 1024 threads for a few tokens, 256 for many; a head: 256 / 64 by its columns (8 heads of 512: 88 tokens 4.8 us, 9.5 with 64 threads, 512 9.8 and
+    // 12.0; 16 of 128 stay with 64)
     if (whole ? (n <= 32 && V > 512) : false) HY_MO(1024);
-    else if (whole ? V > 128 : (n <= 32 && V > 128)) HY_MO(256);
+    else if (V > 128) HY_MO(256);
     else HY_MO(64);
 #undef HY_MO
 }
@@ -1433,7 +1435,8 @@ static int32_t hy_mixer_core(gl3_ctx* ctx, HyLayer& L, int np, int ldo, int n, i
         }
         if (n == 1 && hy_attn_one<T>(ctx, L, pos0, mixo)) { hy_pool(ctx, L, n, pos0); return GL3_OK; }          // (pooled blocks that this token completes: no window is passed yet)
         if (d.qk_unit_norm == 2) {
-            if (n <= 32) hipLaunchKernelGGL((hy_rowrms_kernel<1024>), dim3(n, 2), dim3(1024), 0, st, h->proj, np, L.q_off, d.heads * d.dim, L.k_off, d.kv_heads * d.dim, px.bias, eps, h->rowr);
+            // (projections of 4096 + 1024 columns: 88 tokens 4.8 us, 7.0 with 256 threads, 512 6.4 and 7.8; of 2048 + 512: 100 tokens 4.8 and 3.9)
+            if (n <= 32 || d.heads * d.dim > 2048) hipLaunchKernelGGL((hy_rowrms_kernel<1024>), dim3(n, 2), dim3(1024), 0, st, h->proj, np, L.q_off, d.heads * d.dim, L.k_off, d.kv_heads * d.dim, px.bias, eps, h->rowr);
             else hipLaunchKernelGGL((hy_rowrms_kernel<256>), dim3(n, 2), dim3(256), 0, st, h->proj, np, L.q_off, d.heads * d.dim, L.k_off, d.kv_heads * d.dim, px.bias, eps, h->rowr);
         }
         hipLaunchKernelGGL(hy_attn_prep_kernel, dim3(n, hy_cdiv(d.heads + (d.v_from_k ? 1 : 2) * d.kv_heads, HY_PREP_HEADS)), dim3(64 * HY_PREP_HEADS), 0, st, h->proj, np, L.q_off, L.k_off, L.v_off, d.heads, d.kv_heads, d.dim,
@@ -1477,7 +1480,7 @@ static int32_t hy_mixer_core(gl3_ctx* ctx, HyLayer& L, int np, int ldo, int n, i
                                h->slot_floats, h->dyn, n, ga, gb, ge);
         if (hy_scan_chunks(a) && ((a.act & 3) || a.rot.dims > 0 || a.k_mul != 1.f || a.q_mul != 1.f)) {
             // keys and queries are finished once, in place (the chunks' workgroups would each make them again for their few columns)
-            hipLaunchKernelGGL(hy_scan_prep_kernel, dim3(n), dim3(256), (size_t)std::max(1, d.rot_dims) * 4, st, h->proj, np, L.q_off, L.k_off, d.heads, d.dim, a.q_mul, a.k_mul, a.act, a.rot, h->dyn);
+            hipLaunchKernelGGL(hy_scan_prep_kernel, dim3(n), dim3(1024), (size_t)std::max(1, d.rot_dims) * 4, st, h->proj, np, L.q_off, L.k_off, d.heads, d.dim, a.q_mul, a.k_mul, a.act, a.rot, h->dyn);
             a.act &= 4; a.k_mul = a.q_mul = 1.f; a.rot = HyScanRot{};
         }
         if (cg && n > 32) {
@@ -1727,7 +1730,9 @@ static void hy_resid(gl3_ctx* ctx, int n, const HyResid& r, T* xt, T* h_out) {
         if (r.bw1) hipLaunchKernelGGL((hy_resid_kernel<T, NT, V, true>), dim3(n), dim3(NT), 0, ctx->stream, r, xt, h_out);               \
         else hipLaunchKernelGGL((hy_resid_kernel<T, NT, V, false>), dim3(n), dim3(NT), 0, ctx->stream, r, xt, h_out);                    \
     } while (0)
-    if (n <= 32) { if (v4) HY_RS(1024, 4); else HY_RS(1024, 1); }
+    // 1024 threads read a row of 4096 in one trip, whatever the number of rows (88 7.9 us, 15.5 with 256 threads; 250 10.8 and 17.6; 512 16.7 and 18.7); half of them have
+    // nothing of a row of 2048 (100 5.7 and 8.0, but 400 9.6 and 7.8)
+    if (n <= 256 || r.W > 2048) { if (v4) HY_RS(1024, 4); else HY_RS(1024, 1); }
     else { if (v4) HY_RS(256, 4); else HY_RS(256, 1); }
 #undef HY_RS
 }
