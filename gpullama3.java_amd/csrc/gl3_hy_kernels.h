@@ -1334,7 +1334,7 @@ static __global__ __launch_bounds__(256) void hy_attn_merge_few_kernel(const flo
 // One thread per channel and HY_CONV_T tokens: every input is loaded once (one token per thread loads it taps times: 28 -> 14 us for 512 tokens x
 // 10240 channels).  More than four taps do not stay in registers: a thread walks taps x tokens one load after the other, so it has one token (32 taps,
 // 2304 channels, two layers' steps of eight tokens: 200 us with eight tokens per thread, 143 with one; of 512: 657 and 581).  A portion that
-// fits one thread's tokens moves the tail on as well; longer ones leave that to hy_conv_tail_kernel.
+// fits one thread's tokens moves the tail on as well; longer ones leave that to the gated norm behind the recurrence, or to hy_conv_tail_kernel (more than four taps).
 constexpr int HY_CONV_T = 8;
 __host__ __device__ __forceinline__ int hy_conv_tokens(int taps) { return taps <= 4 ? HY_CONV_T : 1; }
 static __global__ __launch_bounds__(256) void hy_conv_kernel(const float* __restrict__ proj, int ld, int x_off, int ch, int taps, const float* __restrict__ w,
@@ -1571,7 +1571,7 @@ static __global__ __launch_bounds__(256) void hy_ssm_scan_kernel(HyScanArgs a) {
 // rows of 64 columns each on the way at once (256 states: one round trip); keys and queries of the head are made in LDS meanwhile.
 // With cv.w (a state-space layer with up to four taps) the sources are the raw projections: every workgroup makes the convolution of the channels it reads (one channel a
 // thread; the kernel behind this one moves the tail on, hy_conv_move), a launch of 5 us less.
-struct HyConvOne { const float* x; const float* w; const float* bias; float* tail; int ch, taps; };          // x: the token's raw channels
+struct HyConvOne { const float* x; const float* w; const float* bias; float* tail; int ch, taps; int ld, n; };          // x: the first token's raw channels; rows ld apart, n of them
 struct HyConvTaps { float v[4], w[4], b; };
 __device__ __forceinline__ void hy_conv_load(HyConvTaps& q, const HyConvOne& cv, const float* tl, bool fresh, int c) {
 #pragma unroll
@@ -1594,7 +1594,10 @@ __device__ __forceinline__ void hy_conv_move(const HyConvOne& cv, const int* dyn
     float *tl = cv.tail + (size_t)dyn[1] * slot_stride, v[3];
     const bool fresh = dyn[0] == 0;
 #pragma unroll
-    for (int i = 0; i < 3; ++i) v[i] = i + 2 == cv.taps ? cv.x[c] : i + 2 < cv.taps && !fresh ? tl[(size_t)(i + 1) * cv.ch + c] : 0.f;
+    for (int i = 0; i < 3; ++i) {          // the input at step-relative time n + i - (taps - 1)
+        const int tau = cv.n + i - (cv.taps - 1);
+        v[i] = i + 1 >= cv.taps ? 0.f : tau >= 0 ? cv.x[(size_t)tau * cv.ld + c] : fresh ? 0.f : tl[(size_t)(cv.taps - 1 + tau) * cv.ch + c];
+    }
 #pragma unroll
     for (int i = 0; i < 3; ++i)
         if (i + 1 < cv.taps) tl[(size_t)i * cv.ch + c] = v[i];
@@ -1761,15 +1764,15 @@ static __global__ __launch_bounds__(NT) void hy_mem_out_kernel(const float* __re
 }
 
 // y * silu(z), unit root mean square per part (ngroups equal parts of inner), times the weight; the first HY_GN entries of a thread stay in registers between the
-// two passes.  Workgroups behind the parts move the tail of a single token on
-// whose convolution hy_scan_one_kernel made (cv).
+// two passes.  Workgroups behind the parts move the convolution's tail on
+// where its kernel has not (cv.taps: up to four; a launch of 5 us less).
 constexpr int HY_GN = 4;
 template <typename TO>
 static __global__ __launch_bounds__(256) void hy_gated_norm_kernel(const float* __restrict__ y, const float* __restrict__ proj, int ld, int z_off, int inner,
                                                                    int ngroups, const float* __restrict__ w, float eps, TO* __restrict__ out, int ldo, HyConvOne cv, const int* __restrict__ dyn,
                                                                    size_t slot_stride) {
     __shared__ float red[4];
-    if ((int)blockIdx.y >= ngroups) { hy_conv_move(cv, dyn, slot_stride, (blockIdx.y - ngroups) * 256 + threadIdx.x); return; }
+    if ((int)blockIdx.y >= ngroups) { hy_conv_move(cv, dyn, slot_stride, ((blockIdx.y - ngroups) * gridDim.x + blockIdx.x) * 256 + threadIdx.x); return; }
     const int t = blockIdx.x, grp = blockIdx.y, len = inner / ngroups, c0 = grp * len;
     const float *yr = y + (size_t)t * inner + c0, *zr = proj + (size_t)t * ld + z_off + c0;
     float keep[HY_GN], wt[HY_GN], ss = 0.f;

@@ -1547,14 +1547,15 @@ static int32_t hy_mixer_core(gl3_ctx* ctx, HyLayer& L, int np, int ldo, int n, i
         const int inner = d.heads * d.vdim, ch = hy_conv_ch(d), dt_off = 2 * inner + 2 * d.groups * d.state;
         float* state = h->slots + L.off_state;
         float* tail = h->slots + L.off_tail;
-        HyConvOne cv{};          // one token: the recurrence makes the convolution itself
-        if (n == 1 && d.conv <= 4 && d.state <= 4096 && !hy_scan_forced(d.state)) { cv.x = h->proj + inner; cv.w = L.conv_w; cv.bias = L.conv_b; cv.tail = tail; cv.ch = ch; cv.taps = d.conv; }
-        else {
-            hipLaunchKernelGGL(hy_conv_kernel, dim3(hy_cdiv(ch, 256), hy_cdiv(n, hy_conv_tokens(d.conv))), dim3(256), 0, st, h->proj, np, inner, ch, d.conv, L.conv_w, L.conv_b, tail, h->slot_floats, h->dyn,
-                               n, h->conv);
-            if (d.conv > 1 && n > hy_conv_tokens(d.conv))
-                hipLaunchKernelGGL(hy_conv_tail_kernel, dim3(hy_cdiv(ch, 256)), dim3(256), 0, st, h->proj, np, inner, ch, d.conv, tail, h->slot_floats, h->dyn, n);
-        }
+        // one token: the recurrence makes the convolution itself; longer portions' tails move on in the gated norm's launch
+        HyConvOne cv{h->proj + inner, nullptr, L.conv_b, tail, ch, d.conv, np, n};
+        if (n == 1 && d.conv <= 4 && d.state <= 4096 && !hy_scan_forced(d.state)) cv.w = L.conv_w;
+        else
+            hipLaunchKernelGGL(hy_conv_kernel, dim3(hy_cdiv(ch, 256), hy_cdiv(n, hy_conv_tokens(d.conv))), dim3(256), 0, st, h->proj, np, inner, ch, d.conv, L.conv_w, L.conv_b, tail, h->slot_floats,
+                               h->dyn, n, h->conv);
+        const bool moves = d.conv <= 4 && (cv.w || n > hy_conv_tokens(d.conv));
+        if (d.conv > 4 && n > hy_conv_tokens(d.conv))
+            hipLaunchKernelGGL(hy_conv_tail_kernel, dim3(hy_cdiv(ch, 256)), dim3(256), 0, st, h->proj, np, inner, ch, d.conv, tail, h->slot_floats, h->dyn, n);
         HyScanArgs a{};
         a.ksrc = h->conv; a.ldk = ch; a.k_off = inner; a.k_hstride = d.state;
         a.qsrc = h->conv; a.ldq = ch; a.q_off = inner + d.groups * d.state; a.q_hstride = d.state;
@@ -1564,7 +1565,7 @@ static int32_t hy_mixer_core(gl3_ctx* ctx, HyLayer& L, int np, int ldo, int n, i
         a.heads = d.heads; a.P = d.vdim; a.N = d.state; a.G = d.groups;
         a.state = state; a.slot_stride = h->slot_floats; a.dyn = h->dyn; a.n = n; a.y = h->ssm_y; a.ldy = inner;
         hy_scan(ctx, a, cv);
-        hipLaunchKernelGGL((hy_gated_norm_kernel<T>), dim3(n, d.norm_groups + (cv.w ? hy_cdiv(ch, 256) : 0)), dim3(256), 0, st, h->ssm_y, h->proj, np, 0, inner, d.norm_groups, L.ssm_norm, eps, mixo, ldo, cv, h->dyn, h->slot_floats);
+        hipLaunchKernelGGL((hy_gated_norm_kernel<T>), dim3(n, d.norm_groups + (moves ? hy_cdiv(hy_cdiv(ch, 256), n) : 0)), dim3(256), 0, st, h->ssm_y, h->proj, np, 0, inner, d.norm_groups, L.ssm_norm, eps, mixo, ldo, cv, h->dyn, h->slot_floats);
     }
     return GL3_OK;
 }
