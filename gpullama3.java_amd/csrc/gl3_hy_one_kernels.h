@@ -19,6 +19,17 @@ __device__ __forceinline__ float hy_dot4(const float4& a, const float4& b, float
 __device__ __forceinline__ void hy_axpy4(float4& o, float p, const float4& v) { o.x = fmaf(p, v.x, o.x); o.y = fmaf(p, v.y, o.y); o.z = fmaf(p, v.z, o.z); o.w = fmaf(p, v.w, o.w); }
 __device__ __forceinline__ void hy_mul4(float4& o, float s) { o.x *= s; o.y *= s; o.z *= s; o.w *= s; }
 
+// p[0] + p[ld] + .. + p[(n - 1) ld], eight chains side by side that meet in pairs
+__device__ __forceinline__ float hy_sum_rows(const float* p, int ld, int n) {
+    float s[8];
+#pragma unroll
+    for (int u = 0; u < 8; ++u) s[u] = 0.f;
+    for (int k = 0; k < n; k += 8)
+#pragma unroll
+        for (int u = 0; u < 8; ++u)
+            if (k + u < n) s[u] += p[(k + u) * ld];
+    return ((s[0] + s[1]) + (s[2] + s[3])) + ((s[4] + s[5]) + (s[6] + s[7]));
+}
 // How the sums of sixteen wavefronts weigh in the result: lane w of 16 brings maximum and denominator of wavefront w and gets e^(m_w - M) / den, with the
 // sink's unit in the denominator.
 __device__ __forceinline__ float hy_join_weight(float mw, float lw, int sink, float z) {
@@ -302,9 +313,7 @@ static __global__ __launch_bounds__(1024) void hy_latent_one_kernel(HyLatentOne 
     }
     __syncthreads();
     for (int c = tid; c < R; c += 1024) {
-        float s = 0.f;
-        for (int k = 0; k < nkg; ++k) s += sO[k * R + c];
-        sA[c] = s;
+        sA[c] = hy_sum_rows(sO + c, R, nkg);
     }
     __syncthreads();
     float4 q[2], o[2];
@@ -384,8 +393,7 @@ static __global__ __launch_bounds__(1024) void hy_latent_one_kernel(HyLatentOne 
     }
     __syncthreads();
     for (int c = tid; c < V; c += 1024) {
-        float s = 0.f;
-        for (int k = 0; k < nvg; ++k) s += sO[k * V + c];
+        float s = hy_sum_rows(sO + c, V, nvg);
         if (a.gate) s *= hy_sigmoid(a.gate[a.gate_mode == 2 ? h : h * V + c]);
         hy_st(out + h * V + c, s);
     }
