@@ -151,7 +151,7 @@ __device__ __forceinline__ void hy_attn_one(const HyAttnOne& a, TO* __restrict__
         for (int i = 0; i < NI; ++i) hy_mul4(o[i], corr);
 #pragma unroll
         for (int u = 0; u < UU; ++u) {
-            const float p = any && dist[u] >= 0 ? expf(s[u] - mx) : 0.f;
+            const float p = dist[u] >= 0 && (any || s[u] != s[u]) ? expf(s[u] - mx) : 0.f;          // (fmaxf passes over a score that is not a number: a key alone must reach l all the same)
             l += p;
             if (dist[u] >= 0)
 #pragma unroll
@@ -342,7 +342,7 @@ static __global__ __launch_bounds__(1024) void hy_latent_one_kernel(HyLatentOne 
 #pragma unroll
         for (int u = 0; u < UU; ++u) {
             if (u >= n) break;
-            const float p = any ? expf(s[u] - mx) : 0.f;
+            const float p = any || s[u] != s[u] ? expf(s[u] - mx) : 0.f;
             l += p;
             hy_axpy4(o[0], p, k[u][0]); hy_axpy4(o[1], p, k[u][1]);
         }
