@@ -774,7 +774,6 @@ int32_t gl3_create(const gl3_model_desc* desc, gl3_ctx** out) {
     TRYHIP(hipHostMalloc((void**)&ctx->h_dyn, 4 * sizeof(int), hipHostMallocCoherent));          // (kernels read it: embed_q8t_kernel)
     TRYHIP(hipHostMalloc((void**)&ctx->h_logits, ((size_t)d.vocab + 4 * (size_t)(d.max_batch > 1 ? d.max_batch : 0)) * 4, hipHostMallocCoherent));      // + the batched steps' inputs and ids (gl3_prefill.hip: h_io)
     TRYHIP(hipHostMalloc((void**)&ctx->h_argmax, sizeof(int), hipHostMallocCoherent));
-    TRYHIP(ctx->done.make());
     // batched prefill / static-batched decode: int8 MFMA GEMMs for Q8_0 (any tensor-parallel degree); f32-MFMA / VALU GEMMs in the
     // Vector-API order for F16, Q4_0 and Q8_0 with the f32 activation (gl3_prefill_vl.h).  The scalar dot order
     // (GL3_FLAG_SCALAR_DOT) prefills token by token.
@@ -834,7 +833,6 @@ void gl3_destroy(gl3_ctx* ctx) {
     if (ctx->h_dyn) hipHostFree(ctx->h_dyn);
     if (ctx->h_logits) hipHostFree(ctx->h_logits);
     if (ctx->h_argmax) hipHostFree(ctx->h_argmax);
-    ctx->done.free();
     if (ctx->stream) hipStreamDestroy(ctx->stream);
     delete ctx;
 }
@@ -1075,12 +1073,9 @@ int32_t gl3_forward_decode(gl3_ctx* ctx, int32_t token, int32_t pos, float* logi
     const int amode = attn_mode(ctx, pos);
     if (ctx->graph_exec && want_logits) GL3_HIP(hipGraphLaunch(step_graph(ctx, amode), ctx->stream));
     else if ((r = enqueue_decode(ctx, want_logits, nullptr, amode)) != GL3_OK) return r;
-    const bool words = ctx->d.tp_size == 1;          // (ranks of a group end their steps by the runtime: their error words come with a copy)
-    int last = 0;                                // words the step's last kernel sets
     if (argmax_out) {
-        hipLaunchKernelGGL(argmax_kernel, dim3(AMX_WGS), dim3(256), 0, ctx->stream, ctx->logits, ctx->d.vocab, ctx->argmax, ctx->h_argmax, ctx->done.words, ctx->done.next());
+        hipLaunchKernelGGL(argmax_kernel, dim3(AMX_WGS), dim3(256), 0, ctx->stream, ctx->logits, ctx->d.vocab, ctx->argmax, ctx->h_argmax);
         GL3_HIP(hipGetLastError());
-        last = 1;
     }
     // logits D2H: straight into the caller's buffer when it is page-locked (gl3_pin_host_buffer), else through the plan's pinned
     // staging buffer + one host memcpy (513 KB for a 128 k vocabulary: ~40 us per token on the host)
@@ -1088,9 +1083,9 @@ int32_t gl3_forward_decode(gl3_ctx* ctx, int32_t token, int32_t pos, float* logi
     if (logits_out)
         for (const auto& pr : ctx->pinned)
             if ((uint8_t*)logits_out >= (uint8_t*)pr.first && (uint8_t*)logits_out + (size_t)ctx->d.vocab * 4 <= (uint8_t*)pr.first + pr.second) direct = true;
-    if (logits_out && direct) { GL3_HIP(hipMemcpyAsync(logits_out, ctx->logits, (size_t)ctx->d.vocab * 4, hipMemcpyDeviceToHost, ctx->stream)); last = 0; }
-    else if (logits_out) { last = launch_to_host(ctx, ctx->logits, ctx->h_logits, ctx->d.vocab, true); GL3_HIP(hipGetLastError()); }
-    GL3_HIP(last && words ? ctx->done.wait(last, ctx->stream) : hipStreamSynchronize(ctx->stream));
+    if (logits_out && direct) GL3_HIP(hipMemcpyAsync(logits_out, ctx->logits, (size_t)ctx->d.vocab * 4, hipMemcpyDeviceToHost, ctx->stream));
+    else if (logits_out) { launch_to_host(ctx, ctx->logits, ctx->h_logits, ctx->d.vocab); GL3_HIP(hipGetLastError()); }
+    GL3_HIP(hipStreamSynchronize(ctx->stream));
     drain.passed = true;
     if ((r = gl3_tp_check(ctx)) != GL3_OK) return r;
     if (logits_out && !direct) memcpy(logits_out, ctx->h_logits, (size_t)ctx->d.vocab * 4);

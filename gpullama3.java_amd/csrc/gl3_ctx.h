@@ -10,8 +10,6 @@
 #include <cstdlib>
 #include <mutex>
 #include <string>
-#include <cstring>
-#include <chrono>
 #include <vector>
 
 #include "../../include/gpullama3_hip.h"
@@ -129,34 +127,8 @@ constexpr size_t GL3_ARENA_HDR = 1024, GL3_ARENA_SEQ = 64, GL3_ARENA_ARRIVE = 68
 // rank p has completed into this arena), u32 ticket[3] (finished producer wavefronts of the running launch), u32 step (decode steps)
 constexpr size_t GL3_ARENA_FOLD = 512, GL3_ARENA_FOLD_TICKET = 704, GL3_ARENA_STEP = 720;
 
-// Waiting for a step through words its last kernel sets (say_done): hipStreamSynchronize returns 6.5 us after the last kernel has ended, this within the reading of a
-// word.  The stream itself may be a few us behind; whatever is enqueued or freed next waits for it as ever.  But a program that waits for the whole device next pays 45 - 100 us
-// there (15 behind a wait of the runtime's, which has tidied up): short steps only, of which many follow each other, not prompts.  A step that is not there after 5 ms
-// is waited for, and its errors reported, by the runtime.
-constexpr int GL3_DONE_WORD = 16, GL3_DONE_WGS = 256;
-struct gl3_done {
-    int* words = nullptr;          // page-locked, coherent: [GL3_DONE_WGS][GL3_DONE_WORD]
-    int no = 0;
-    hipError_t make() {
-        const size_t bytes = sizeof(int) * GL3_DONE_WGS * GL3_DONE_WORD;
-        const hipError_t e = hipHostMalloc((void**)&words, bytes, hipHostMallocCoherent);
-        if (e != hipSuccess) { words = nullptr; return e; }
-        memset(words, 0, bytes);
-        return e;
-    }
-    void free() { if (words) hipHostFree(words); words = nullptr; }
-    int next() { return no = no == 0x7fffffff ? 1 : no + 1; }
-    hipError_t wait(int wgs, hipStream_t stream) {          // until the first wgs words hold the number
-        const auto t0 = std::chrono::steady_clock::now();
-        for (int i = 0, spins = 0; i < wgs;) {
-            if (__atomic_load_n(words + (size_t)GL3_DONE_WORD * i, __ATOMIC_ACQUIRE) == no) { ++i; continue; }
-            __builtin_ia32_pause();
-            if ((++spins & 255) == 0 && std::chrono::steady_clock::now() - t0 > std::chrono::milliseconds(5)) return hipStreamSynchronize(stream);
-        }
-        return hipSuccess;
-    }
-};
-
+// Steps end by the runtime's wait.  (Words in page-locked memory that the last kernel sets are read 6 us earlier, but then the runtime tidies up behind whoever waits for
+// the device next.  One step and a device-wide wait, us, words / runtime: Llama 1B 191 / 189, Noditar 1B 194 / 174, Kugadra 1B 237 / 216; such a wait behind four steps: equal.)
 // Page-locked memory of a plan (h_dyn, h_io, h_logits, h_log) belongs to a call until the stream has passed it: a call that fails behind its first launch waits as well.
 struct gl3_drain {
     hipStream_t stream;
@@ -205,7 +177,6 @@ struct gl3_ctx {
     int* dyn_seq = nullptr;                       // [2 * dyn_seq_cap] pairs of a sequential (token-by-token) prefill chunk
     int dyn_seq_cap = 0;
     float* h_logits = nullptr;                    // pinned f32[vocab]
-    gl3_done done;                                // words of the steps' last kernels
     int* h_argmax = nullptr;
     float *sm_probs = nullptr, *sm_aux = nullptr, *h_probs = nullptr;   // sampling (gl3_sample.hip): probabilities, scratch, pinned copy
     int64_t topp_device = 0, topp_host = 0;       // top-p draws answered on the device / by the host heap (gl3_get_topp_counts)

@@ -558,25 +558,14 @@ __device__ __forceinline__ int step_token(int* dyn, const int* host) {
     if (blockIdx.x == 0 && threadIdx.x < 2) dyn[threadIdx.x] = sh[threadIdx.x];
     return sh[0];
 }
-// The end of a step, said by its last kernel: every workgroup's word (64 bytes apart, page-locked coherent memory) becomes the step's number when the workgroup's
-// stores have arrived.  done null: nobody waits that way.
-__device__ __forceinline__ void say_done(int* done, int no) {
-    if (!done) return;
-    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-    __syncthreads();
-    if (threadIdx.x == 0) __hip_atomic_store(done + GL3_DONE_WORD * blockIdx.x, no, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
-}
 // n floats to page-locked host memory; both ends start on 16 bytes
-static __global__ __launch_bounds__(256) void to_host_kernel(const float* __restrict__ src, float* __restrict__ dst, size_t n, int* done, int no) {
+static __global__ __launch_bounds__(256) void to_host_kernel(const float* __restrict__ src, float* __restrict__ dst, size_t n) {
     for (size_t i = (size_t)blockIdx.x * 256 + threadIdx.x; i < n / 4; i += (size_t)256 * gridDim.x) reinterpret_cast<float4*>(dst)[i] = reinterpret_cast<const float4*>(src)[i];
     if (blockIdx.x == 0 && threadIdx.x < n % 4) dst[n / 4 * 4 + threadIdx.x] = src[n / 4 * 4 + threadIdx.x];
-    say_done(done, no);
 }
-// say: it is the step's last kernel, and dst coherent memory; the number of words it sets is returned (gl3_done::wait)
-static inline int launch_to_host(gl3_ctx* ctx, const float* src, float* dst, size_t n, bool say) {
-    const size_t want = (n / 4 + 255) / 256, wgs = want < 1 ? 1 : want > GL3_DONE_WGS ? GL3_DONE_WGS : want;
-    hipLaunchKernelGGL(to_host_kernel, dim3((unsigned)wgs), dim3(256), 0, ctx->stream, src, dst, n, say ? ctx->done.words : (int*)nullptr, say ? ctx->done.next() : 0);
-    return (int)wgs;
+static inline void launch_to_host(gl3_ctx* ctx, const float* src, float* dst, size_t n) {
+    const size_t want = (n / 4 + 255) / 256, wgs = want < 1 ? 1 : want > 256 ? 256 : want;
+    hipLaunchKernelGGL(to_host_kernel, dim3((unsigned)wgs), dim3(256), 0, ctx->stream, src, dst, n);
 }
 
 // ---------------------------------------------------------------------------------------------------
@@ -1724,7 +1713,7 @@ constexpr int AMX_WGS = 64;
 __device__ __forceinline__ void amx_take(float& best, int& idx, float f, int i) {
     if (f > best || (f == best && i < idx)) { best = f; idx = i; }
 }
-static __global__ __launch_bounds__(256) void argmax_kernel(const float* __restrict__ v, int n, int* __restrict__ ws, int* __restrict__ host, int* done, int no) {
+static __global__ __launch_bounds__(256) void argmax_kernel(const float* __restrict__ v, int n, int* __restrict__ ws, int* __restrict__ host) {
     __shared__ float bv[4];
     __shared__ int bi[4];
     __shared__ int last;
@@ -1773,10 +1762,6 @@ static __global__ __launch_bounds__(256) void argmax_kernel(const float* __restr
         if (t == 0) {
             ws[0] = *host = idx == 0x7FFFFFFF ? 0 : idx;          // (host: page-locked)
             __hip_atomic_store(ws + 1, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            if (done) {          // (the only writer of the result says so: one word)
-                asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-                __hip_atomic_store(done, no, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
-            }
         }
     }
 }

@@ -238,7 +238,7 @@ int32_t gl3_hy_create(const gl3_model_desc* desc, gl3_ctx** out, std::string& er
     h->want_cap = std::min(h->mb, 256);
     h->busy.assign(h->n_seqs, 0); h->len.assign(h->n_seqs, 0); h->last_tok.assign(h->n_seqs, 0);
     auto fail = [&](int32_t code) { err = ctx->err; gl3_hy_destroy(ctx); if (ctx->stream) hipStreamDestroy(ctx->stream); if (ctx->argmax) hipFree(ctx->argmax);
-                                    if (ctx->h_argmax) hipHostFree(ctx->h_argmax); ctx->done.free(); if (ctx->h_dyn) hipHostFree(ctx->h_dyn); delete ctx; return code; };
+                                    if (ctx->h_argmax) hipHostFree(ctx->h_argmax); if (ctx->h_dyn) hipHostFree(ctx->h_dyn); delete ctx; return code; };
 #define TRY(x) do { int32_t r_ = (x); if (r_ != GL3_OK) return fail(r_); } while (0)
 #define TRYHIP(call) do { hipError_t e_ = (call); if (e_ != hipSuccess) { ctx->err = std::string(#call) + ": " + hipGetErrorString(e_); return fail(e_ == hipErrorOutOfMemory ? GL3_E_OOM : GL3_E_HIP); } } while (0)
     TRYHIP(hipSetDevice(desc->device));
@@ -548,7 +548,6 @@ int32_t gl3_hy_create(const gl3_model_desc* desc, gl3_ctx** out, std::string& er
     TRYHIP(hipMalloc((void**)&ctx->argmax, (2 + 2 * AMX_WGS) * sizeof(int)));
     TRYHIP(hipMemset(ctx->argmax, 0, (2 + 2 * AMX_WGS) * sizeof(int)));
     TRYHIP(hipHostMalloc((void**)&ctx->h_argmax, sizeof(int), hipHostMallocCoherent));
-    TRYHIP(ctx->done.make());
     TRYHIP(hipHostMalloc((void**)&ctx->h_dyn, 4 * sizeof(int)));          // the samplers' result words (gl3_sample.hip)
     {   // attention tiles above the 64 KB default of dynamic LDS
 #define HY_LDS(RW, DVL) TRYHIP(hipFuncSetAttribute((const void*)hy_attn_kernel<RW, DVL>, hipFuncAttributeMaxDynamicSharedMemorySize, 150 * 1024))
@@ -1950,11 +1949,10 @@ int32_t gl3_hy_step(gl3_ctx* ctx, int32_t seq, const int32_t* tokens, int32_t n,
             if (r != GL3_OK) return r;
             h->last_tok[seq] = tokens[off + pn - 1];
             if (g > 0 && logits_out) {
-                const bool words = n <= GL3_HOST_TOKENS;
-                const int wgs = launch_to_host(ctx, h->logits, h->h_logits, (size_t)g * V, words);
+                launch_to_host(ctx, h->logits, h->h_logits, (size_t)g * V);
                 HY_HIP(hipGetLastError());
-                HY_HIP(words ? ctx->done.wait(wgs, ctx->stream) : hipStreamSynchronize(ctx->stream));
-            } else if (g == 0 && off + pn < n) {          // nothing to hand out: the next portion follows at once, on the other record
+            }
+            if (g == 0 && off + pn < n) {          // nothing to hand out: the next portion follows at once, on the other record
                 HY_HIP(hipEventRecord(h->rec_ev[h->rec], ctx->stream));
                 h->rec_busy[h->rec] = true;
                 h->rec ^= 1;
@@ -1971,9 +1969,9 @@ int32_t gl3_hy_step(gl3_ctx* ctx, int32_t seq, const int32_t* tokens, int32_t n,
 }
 
 int32_t gl3_hy_argmax(gl3_ctx* ctx, int32_t* out) {
-    hipLaunchKernelGGL(argmax_kernel, dim3(AMX_WGS), dim3(256), 0, ctx->stream, ctx->hy->logits, ctx->d.vocab, ctx->argmax, ctx->h_argmax, ctx->done.words, ctx->done.next());
+    hipLaunchKernelGGL(argmax_kernel, dim3(AMX_WGS), dim3(256), 0, ctx->stream, ctx->hy->logits, ctx->d.vocab, ctx->argmax, ctx->h_argmax);
     HY_HIP(hipGetLastError());
-    HY_HIP(ctx->done.wait(1, ctx->stream));
+    HY_HIP(hipStreamSynchronize(ctx->stream));
     *out = *ctx->h_argmax;
     return GL3_OK;
 }

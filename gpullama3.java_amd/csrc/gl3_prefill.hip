@@ -2777,7 +2777,7 @@ static int32_t pf_logits_out(gl3_ctx* ctx, float* out, size_t bytes) {
     const size_t pieces = pf_logits_pieces(bytes), per = ((bytes + pieces - 1) / pieces + 4095) & ~(size_t)4095;
     auto send = [&](size_t i) -> int32_t {
         if (i * per >= bytes) return GL3_OK;
-        launch_to_host(ctx, p->LOGITS + i * per / 4, (float*)p->h_log[i % PF_LOG_SLOTS], std::min(per, bytes - i * per) / 4, false);
+        launch_to_host(ctx, p->LOGITS + i * per / 4, (float*)p->h_log[i % PF_LOG_SLOTS], std::min(per, bytes - i * per) / 4);
         GL3_HIP(hipGetLastError());
         GL3_HIP(hipEventRecord(p->log_ev[i % PF_LOG_SLOTS], ctx->stream));
         return GL3_OK;

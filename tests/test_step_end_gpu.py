@@ -1,5 +1,5 @@
-"""The end of a step as its last kernel says it (csrc/gl3_ctx.h, gl3_done): results are whole when the call returns, whatever stands behind them on the stream; steps with
-logits, with the greedy id and with both alternate, vocabularies need one word, several and more than there are, and prompts of several portions hand their records on in turn."""
+"""The end of a step: results are whole when the call returns, whatever stands behind them on the stream; steps with logits and with the greedy id alternate, vocabularies
+take one workgroup of the kernel that hands logits out, several and more than it has, and prompts of several portions hand their records on in turn."""
 import dataclasses
 
 import numpy as np
@@ -24,7 +24,7 @@ def test_logits_and_ids_of_single_steps(vocab):
     plan = plans.HipMasterPlan(pkg.synth.make_numpy(cfg, seed=3))
     toks = np.random.default_rng(0).integers(0, vocab, 60)
     first = [plan.forward_decode(int(t), i).copy() for i, t in enumerate(toks)]
-    for i, t in enumerate(toks):          # a late word or a stale one would show the step before
+    for i, t in enumerate(toks):          # a result read too early would show the step before
         if i % 3 == 0:
             assert np.array_equal(plan.forward_decode(int(t), i), first[i])
         else:
