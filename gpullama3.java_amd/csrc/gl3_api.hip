@@ -1198,7 +1198,10 @@ int32_t gl3_profile_decode(gl3_ctx* ctx, int32_t token, int32_t pos, gl3_kernel_
     memset(out, 0, sizeof(*out));
     int32_t r = set_dyn(ctx, token, pos);
     if (r != GL3_OK) return r;
-    return enqueue_decode(ctx, true, out, attn_mode(ctx, pos));
+    gl3_drain drain{ctx->stream};
+    if ((r = enqueue_decode(ctx, true, out, attn_mode(ctx, pos))) != GL3_OK) return r;
+    drain.passed = true;          // (the times have been waited for)
+    return GL3_OK;
 }
 
 int32_t gl3_profile_kernel(gl3_ctx* ctx, int32_t klass, int32_t iters, double* out_us, uint64_t* bytes_per_launch) {
