@@ -2761,7 +2761,7 @@ static inline void pf_touch_pages(void* mem, size_t bytes) {
 static size_t pf_logits_pieces(size_t bytes) { return (bytes + PF_LOG_PIECE - 1) / PF_LOG_PIECE; }
 static bool pf_logits_slots(gl3_prefill_state* p, size_t bytes) {
     for (size_t i = 0; i < PF_LOG_SLOTS && i < pf_logits_pieces(bytes); ++i) {
-        if (!p->h_log[i] && hipHostMalloc((void**)&p->h_log[i], PF_LOG_PIECE) != hipSuccess) { p->h_log[i] = nullptr; (void)hipGetLastError(); return false; }
+        if (!p->h_log[i] && hipHostMalloc((void**)&p->h_log[i], PF_LOG_PIECE, hipHostMallocCoherent) != hipSuccess) { p->h_log[i] = nullptr; (void)hipGetLastError(); return false; }
         if (!p->log_ev[i] && hipEventCreateWithFlags(&p->log_ev[i], hipEventDisableTiming) != hipSuccess) { p->log_ev[i] = nullptr; (void)hipGetLastError(); return false; }
     }
     return true;
