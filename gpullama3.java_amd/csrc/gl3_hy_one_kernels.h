@@ -47,7 +47,8 @@ __device__ __forceinline__ float hy_join_weight(float mw, float lw, int sink, fl
 // (NI pieces of 16 bytes each, DPP rotations add them up), keys and values on their way together, a running maximum and sums per sixteen lanes; the
 // token's own key joins from LDS.  One meeting in LDS, then the gated result itself.  Whole steps of one layer, us, with and without (three launches, four with a norm over the whole
 // projections): 32 heads of 64 behind 5 positions 92 / 99, 500 88 / 94, 1000 92 / 93, 2000 101 / 96; of 128 behind 5 154 / 161, 500 163 / 164, 1000 169 / 162: the line
-// lies at 384 KB of keys and values a head (HY_ATTN_ONE).  Splitting longer caches over workgroups behind it gains less than the runs differ.
+// lies at 384 KB of keys and values a head (HY_ATTN_ONE), with few heads as with many (us a layer, one launch / many, just behind it: 2 heads of 64 1000 positions 25.3 / 25.7, 64 heads 34.1 / 33.8; 2 heads of
+// 128 500 26.0 / 27.6, 64 heads 45.8 / 45.1; 4 heads of 256 250 28.8 / 33.0).  Splitting longer caches over workgroups behind it gains less than the runs differ.
 // Bound: latency (three dependent round trips), further back one CU's reads of the head's cache; the heads of a group read it side by side, which costs
 // an idle chip nothing, while four heads in a workgroup would queue their arithmetic.
 struct HyAttnOne {
@@ -226,8 +227,8 @@ static __global__ __launch_bounds__(1024) void hy_attn_one_kernel(HyAttnOne a, T
 // (a wavefront takes four rows at a time, 64 lanes to a row), the join in LDS and the value expansion with its gate.
 // It replaces five launches: cache row 3.6 us, query 2.9, attention 12.6 (7.2 for 256 entries), join 4.6 - 8.6, expansion 4.9 - 6.0.
 // Bound: one CU's share of the expansions (2 x 131 KB a head of 64 on 512-entry latents) and, further back, the cached rows, which every head reads.  Whole steps, us,
-// with and without: 512 entries, three layers, behind 5 positions 171 / 188, 250 178 / 191, 500 193 / 200, 1000 206 / 203; 256 entries, two layers, 5 205 / 217, 180
-// 208 / 221, 400 215 / 223, 800 222 / 221: the line lies at 640 positions (HY_LATENT_ONE_POS).
+// with and without: 512 entries, three layers, behind 5 positions 171 / 188, 250 178 / 191, 500 193 / 200; 256 entries, two layers, 5 205 / 217, 180 208 / 221, 400 215 / 223:
+// the line is hy_latent_one_line's, at most HY_LATENT_ONE_POS.
 struct HyLatentOne {
     const float* q; int D, P;                                // the head's query: D + P entries, the last P turn by the position
     const float* src; int R0; const float* lat_norm;         // the token's raw row (R0 + P entries); null: the cache holds the token's row already

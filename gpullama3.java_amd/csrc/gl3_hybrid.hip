@@ -1333,12 +1333,25 @@ static bool hy_attn_one(gl3_ctx* ctx, const HyLayer& L, int pos0, T* out) {
 #undef HY_A1
     return true;
 }
+// Positions up to which latent attention of one token goes in one launch.  A position costs its workgroup per head 0.023 us whatever the rank, and 0.001 - 0.01 in the kernels of many
+// workgroups, so the line lies where the launches saved are used up.  Ranks that hy_attn_few_kernel is built for, us a layer, one launch / many: 512 entries, heads of 64: 2 heads 640 positions
+// 41.5 / 41.3, 16 heads 720 45.1 / 44.9, 32 heads 800 48.2 / 48.1; 256: 2 heads 320 32.1 / 33.3, 400 33.9 / 33.2, 32 heads 480 38.7 / 39.5, 560 40.9 / 39.5; 128: 2 heads 280 31.2 / 31.5, 360
+// 32.8 / 31.5, 32 heads 360 36.6 / 37.4; 64: 2 heads 120 28.8 / 29.0, 240 31.6 / 29.3, 32 heads 180 34.2 / 34.8.  Wide expansions lie in one CU's way: 512 entries x heads of 160 (32 heads)
+// 500 57.8 / 58.8, 600 59.5 / 58.9; of 256 (16 heads) 320 56.1 / 56.3, 500 60.6 / 56.6; of 512 (8 heads) 100 63.5 / 60.1.  Other ranks' many workgroups are slower (vector kernel): 96: 4 heads
+// 300 32.7 / 35.1, 600 38.8 / 35.1; 40: 4 heads 100 30.1 / 31.7, 300 34.6 / 32.0 (37.7 / 39.4 on a host that launches more slowly), 32 heads 600 44.5 / 45.1; 384: 4 heads 500
+// 39.6 / 51.2.  Under 32 entries the expansion falls into so many shares that their sum costs more than the launches: 16: 4 heads 10 35.8 / 28.4, 32 heads 37.9 / 36.9.
+static int hy_latent_one_line(const HyLayer& L) {
+    const int R = L.Re, h = std::min(L.d.heads, 32), row = L.De + L.d.vdim, size = R * row;          // (size: floats of a head's expansions)
+    if (R < 32) return 0;
+    if (R != 64 && R != 128 && R != 256 && R != 512) return std::min(HY_LATENT_ONE_POS, 3 * R + 80 + 14 * h);
+    return std::min(HY_LATENT_ONE_POS - std::max(0, size - 128 * 1024) / 450, std::min(2 * R - 16, R + 104) + 3 * h + std::max(0, row - 128) / 4);
+}
 template <typename T>
 static bool hy_latent_one(gl3_ctx* ctx, const HyLayer& L, int pos0, const float* q, T* out) {
     gl3_hybrid_state* h = ctx->hy;
     const gl3_layer_desc& d = L.d;
     float* cc = h->slots + L.off_k;
-    if (L.Re > HY_LATENT_ONE || ((L.Re | d.vdim | (int)(h->slot_floats & 3)) & 3) || ((uintptr_t)cc & 15) || pos0 >= HY_LATENT_ONE_POS) return false;
+    if (L.Re > HY_LATENT_ONE || ((L.Re | d.vdim | (int)(h->slot_floats & 3)) & 3) || ((uintptr_t)cc & 15) || pos0 >= hy_latent_one_line(L)) return false;
     HyLatentOne a{};
     a.q = q; a.D = d.dim; a.P = d.rot_dim; a.src = d.kv_share > 0 ? nullptr : h->proj + L.c_off; a.R0 = d.kv_rank; a.lat_norm = L.lat_norm; a.eps = ctx->d.rms_eps;
     a.cc = cc; a.slot_stride = h->slot_floats; a.dyn = h->dyn; a.freq = L.lat_freq; a.mscale = L.rot_mscale; a.wk = L.wk; a.wvT = L.wvT; a.R = L.Re; a.V = d.vdim; a.scale = d.scale;
