@@ -12,6 +12,7 @@ typedef int v4i_t __attribute__((ext_vector_type(4)));
 typedef int v16i_t __attribute__((ext_vector_type(16)));
 typedef float v2f_t __attribute__((ext_vector_type(2)));
 typedef long v2l_t __attribute__((ext_vector_type(2)));
+typedef float v16f_bd __attribute__((ext_vector_type(16)));
 
 // ---------------------------------------------------------------------------------------------------
 // Batched Q8_0 matmul: out[b][n] = sum_blocks float(isum) * (wScale * aScale), blocks ascending
@@ -40,17 +41,19 @@ struct GemmArgs {
 //     load — and two v_permlane32_swap turn that into the 8 B x 4 k-groups of block 2j (low registers) and of block
 //     2j + 1 (high registers).  The int8 dot is exact, so the order of k inside a block is free; only A and B have to
 //     agree, and B (the int8 activations) is stored pre-split for exactly this access (XQ2 below): no swap on that side.
-//   * weight scales: the 128-byte f16 header of TWO tiles per load (lanes 0-31 / 32-63), converted once and parked in LDS
-//     as f32, read back as one broadcast float4 = the 4 rows a lane accumulates.  Activation scales: one float per lane
-//     and tile, parked in LDS twice ({s, s} = a ready v_pk_mul operand).
+//   * weight scales: the 128-byte f16 header of TWO tiles per load (lanes 0-31 / 32-63), converted once and parked in LDS as f32.  A lane reads
+//     the one of (row t, block g) and brings its own activation scale of (token t, block g): v_mfma_f32_16x16x1_4b_f32 makes the products
+//     wScale * aScale of the tile's four blocks in the lanes and registers that the int8 products have, each rounded once (K = 1, C = 0).
+//     Bound: the instructions of a lone wavefront.  Without packed f32 a block and matrix takes 12 VALU instructions and a quarter of an MFMA (16 with
+//     the products on the VALU, and six more LDS accesses a tile).  Qwen3-4B, 32 tokens, us, packed f32 / products on the VALU / this: wo + down 13.3 / 15.5 / 13.4,
+//     gate + up 20.1 / 20.7 / 20.6, qkv + logits 10.4 / 10.9 / 10.3; one float per token and block in LDS instead of a ready pair: 15.9, 20.6, 11.0.
 //   * a tile runs in two halves one iteration apart — front(i + 1): swaps + MFMAs, back(i): (float)isum * (wScale * aScale)
 //     and result += p, blocks ascending — so the MFMA latency sits behind the previous tile's arithmetic.
 //   * addresses are a uniform base (SGPRs, advanced by scalar adds) + a loop-invariant per-lane offset, and NOTHING is
 //     clamped or guarded: the rings read up to DA tiles past the end of a strip / of the activations, which is why
 //     every weight matrix and XQ2 / XS2 carry GL3_TAIL_PAD bytes of slack (alloc_mat, gl3_prefill_init).  A load under a
 //     condition makes the compiler wait vmcnt(0) at every use ("conditional loads"), and so did several other
-//     constructs here — ring slots must not be float4s whose odd elements feed v_pk_mul broadcasts, a later tile's swaps
-//     must not be scheduled behind their loads (sched_barrier per tile), the prologue has to issue in the loop's order,
+//     constructs here — a later tile's swaps must not be scheduled behind their loads (sched_barrier per tile), the prologue has to issue in the loop's order,
 //     loop exits inside the unrolled trip split the ring's live ranges, and since vmcnt counts in issue order every stream
 //     (weights from HBM, activations from L2) needs the same ring depth.
 //   * SwiGLU: gate and up rows of a strip in one wavefront (NM = 2): the activations are fetched once for both matrices.
@@ -79,7 +82,6 @@ __global__ __launch_bounds__(QOUT ? 128 : 64, WPE) void bdw_gemm_kernel(const Ge
     constexpr int NM = (EPI == EPI_SWIGLU) ? 2 : 1;
     static_assert(DA % 2 == 0, "ring slots are static under the unroll");
     __shared__ __attribute__((aligned(16))) float wsl_all[NWV][4 * NM * 64];   // [tile & 3][matrix][block][row] weight scales
-    __shared__ __attribute__((aligned(16))) float xsl_all[NWV][4 * 128];       // [tile & 3][blocks 01 | 23][token][2 blocks][2]: activation scale pairs, a token's float4s 16 B apart (no bank conflicts)
     __shared__ float amax_s[NWV][64];
     const int lane = threadIdx.x & 63, t = lane & 15, g = lane >> 4;
     const int wv = QOUT ? __builtin_amdgcn_readfirstlane(threadIdx.x >> 6) : 0;
@@ -87,7 +89,6 @@ __global__ __launch_bounds__(QOUT ? 128 : 64, WPE) void bdw_gemm_kernel(const Ge
     const unsigned long long bdw_t0 = __builtin_readcyclecounter(), bdw_w0 = wall_clock64();
 #endif
     float* wsl = wsl_all[wv];
-    float* xsl = xsl_all[wv];
     const int NTG = (a.ntok + 15) >> 4;                                         // token tiles of this launch
     const int nstrips = (a.rows + 15) >> 4;
     const int h = (blockIdx.x >> 3) % NTG;
@@ -129,7 +130,6 @@ __global__ __launch_bounds__(QOUT ? 128 : 64, WPE) void bdw_gemm_kernel(const Ge
                 make_float2(h2f((uint16_t)(hh & 0xffff)), h2f((uint16_t)(hh >> 16)));
         }
     };
-    auto park_x = [&](int u, int i) { *reinterpret_cast<float2*>(&xsl[(i & 3) * 128 + (g >> 1) * 64 + 4 * t + 2 * (g & 1)]) = make_float2(Xr[u], Xr[u]); };
     // 16 B per lane (two blocks x one half) -> lo = 8 B of block 2j, hi = 8 B of block 2j + 1 for all four k-groups:
     // v_permlane32_swap exchanges lo[lanes 32-63] with hi[lanes 0-31]
     auto split = [](const v4i_t v, long& lo, long& hi) {
@@ -138,19 +138,14 @@ __global__ __launch_bounds__(QOUT ? 128 : 64, WPE) void bdw_gemm_kernel(const Ge
         lo = (long)(((unsigned long)r1[0] << 32) | r0[0]);
         hi = (long)(((unsigned long)r1[1] << 32) | r0[1]);
     };
-    v2f_t acc[NM][2];
+    float acc[NM][4];
 #pragma unroll
-    for (int m = 0; m < NM; ++m) { acc[m][0] = v2f_t{0.f, 0.f}; acc[m][1] = v2f_t{0.f, 0.f}; }
+    for (int m = 0; m < NM; ++m) acc[m][0] = acc[m][1] = acc[m][2] = acc[m][3] = 0.f;
     const v4i_t cbias = {0x4B400000, 0x4B400000, 0x4B400000, 0x4B400000};      // 1.5 * 2^23: int accumulator read as float = bias + isum
-    const v2f_t fbias = {12582912.f, 12582912.f};
-    v4i_t Cb[2][NM][4]; float4 Wc[NM][4]; v2f_t Xc[4];
-    auto scales = [&](int i) {                           // weight / activation scales of tile i: LDS -> Wc / Xc
-        const float4 x01 = *reinterpret_cast<const float4*>(&xsl[(i & 3) * 128 + 4 * t]), x23 = *reinterpret_cast<const float4*>(&xsl[(i & 3) * 128 + 64 + 4 * t]);
-        Xc[0] = v2f_t{x01.x, x01.y}; Xc[1] = v2f_t{x01.z, x01.w}; Xc[2] = v2f_t{x23.x, x23.y}; Xc[3] = v2f_t{x23.z, x23.w};
+    v4i_t Cb[2][NM][4]; v16f_bd Sc[NM];
+    auto scales = [&](int i, int u) {                    // wScale * aScale of tile i (ring slot u), four blocks of 16 x 16 in one MFMA: register 4 block + r is row 4 g + r, token t
 #pragma unroll
-        for (int m = 0; m < NM; ++m)
-#pragma unroll
-            for (int bi = 0; bi < 4; ++bi) Wc[m][bi] = *reinterpret_cast<const float4*>(&wsl[((i & 3) * NM + m) * 64 + 16 * bi + 4 * g]);
+        for (int m = 0; m < NM; ++m) Sc[m] = __builtin_amdgcn_mfma_f32_16x16x1f32(wsl[((i & 3) * NM + m) * 64 + lane], Xr[u], v16f_bd{0.f}, 0, 0, 0);
     };
     auto front = [&](int u) {                            // ring slot u: swaps + 4 MFMAs per matrix -> Cb[u & 1]
         const int q = u & 1;
@@ -177,11 +172,8 @@ __global__ __launch_bounds__(QOUT ? 128 : 64, WPE) void bdw_gemm_kernel(const Ge
 #pragma unroll
             for (int m = 0; m < NM; ++m) {
                 const v4i_t c = Cb[q][m][bi];
-                const float4 w4 = Wc[m][bi];
-                const v2f_t ca = v2f_t{__int_as_float(c[0]), __int_as_float(c[1])} - fbias;
-                const v2f_t cb = v2f_t{__int_as_float(c[2]), __int_as_float(c[3])} - fbias;
-                acc[m][0] = acc[m][0] + ca * (v2f_t{w4.x, w4.y} * Xc[bi]);      // result += isum * (wScale * aScale)
-                acc[m][1] = acc[m][1] + cb * (v2f_t{w4.z, w4.w} * Xc[bi]);
+#pragma unroll
+                for (int r = 0; r < 4; ++r) acc[m][r] = acc[m][r] + (__int_as_float(c[r]) - 12582912.f) * Sc[m][4 * bi + r];      // result += isum * (wScale * aScale)
             }
         }
     };
@@ -189,7 +181,7 @@ __global__ __launch_bounds__(QOUT ? 128 : 64, WPE) void bdw_gemm_kernel(const Ge
 #pragma unroll
     for (int u = 0; u < DA; ++u) { fetch(u); __builtin_amdgcn_sched_barrier(0); }
     park_h(0, 0);
-    park_x(0, 0);
+    scales(0, 0);
     front(0);
     const int nfull = a.nb >> 2;                         // full tiles
     int base = 0;
@@ -197,11 +189,10 @@ __global__ __launch_bounds__(QOUT ? 128 : 64, WPE) void bdw_gemm_kernel(const Ge
 #pragma unroll
         for (int u = 0; u < DA; ++u) {
             const int i = base + u;
-            scales(i);
             if ((u & 1) == 0) park_h(((u + 2) % DA) / 2, i + 2);               // scales of tiles i + 2, i + 3 (fetched DA - 2 tiles ago)
-            park_x((u + 1) % DA, i + 1);
             front((u + 1) % DA);
             back(std::true_type{}, u, 4);
+            scales(i + 1, (u + 1) % DA);
             fetch(u);
             __builtin_amdgcn_sched_barrier(0);           // or the scheduler hoists a later tile's swaps to just behind their loads (vmcnt(0))
         }
@@ -213,11 +204,10 @@ __global__ __launch_bounds__(QOUT ? 128 : 64, WPE) void bdw_gemm_kernel(const Ge
         for (int u = 0; u < DA; ++u) {
             const int i = base + u;
             if (i < ntiles) {
-                scales(i);
                 if ((u & 1) == 0) park_h(((u + 2) % DA) / 2, i + 2);
-                park_x((u + 1) % DA, i + 1);
                 front((u + 1) % DA);
                 back(std::false_type{}, u, min(4, a.nb - 4 * i));
+                scales(i + 1, (u + 1) % DA);
                 fetch(u);
             }
             __builtin_amdgcn_sched_barrier(0);
@@ -240,9 +230,9 @@ __global__ __launch_bounds__(QOUT ? 128 : 64, WPE) void bdw_gemm_kernel(const Ge
         float hv[4];
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
-            float gt = acc[0][i >> 1][i & 1];
+            float gt = acc[0][i];
             gt = gt / (float)(1.0 + exp(-(double)gt));
-            hv[i] = gt * acc[NM - 1][i >> 1][i & 1];
+            hv[i] = gt * acc[NM - 1][i];
         }
         amax_s[wv][lane] = fmaxf(fmaxf(fabsf(hv[0]), fabsf(hv[1])), fmaxf(fabsf(hv[2]), fabsf(hv[3])));
         __syncthreads();
@@ -271,11 +261,11 @@ __global__ __launch_bounds__(QOUT ? 128 : 64, WPE) void bdw_gemm_kernel(const Ge
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
         if (rbase + i >= a.rows) continue;
-        const float v0 = acc[0][i >> 1][i & 1];
+        const float v0 = acc[0][i];
         if (EPI == EPI_SWIGLU) {
             float gt = v0;
             gt = gt / (float)(1.0 + exp(-(double)gt));
-            o[i] = gt * acc[NM - 1][i >> 1][i & 1];
+            o[i] = gt * acc[NM - 1][i];
         } else if (EPI == EPI_STORE) o[i] = v0 * a.out_scale;
         else o[i] = o[i] + v0 * a.out_scale;
     }
