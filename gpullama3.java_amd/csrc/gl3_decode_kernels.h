@@ -195,8 +195,8 @@ __device__ __forceinline__ float seq_sum_lds(const float* v, int n, float start 
     return s;
 }
 
-// a * b as one v_mul_f32 the SLP vectoriser cannot pair: v_pk_mul_f32 wants its operands in aligned register pairs, and the
-// v_mov shuffles it inserts for that read freshly issued LDS results, i.e. wait for them — which is what a read ring is there to avoid.
+// a * b as one v_mul_f32 written out, which stays where the read ring puts it: left to the compiler the products move to their freshly issued LDS reads and wait for them
+// (scores behind 8000 positions, 32 heads of 128: 16.1 us, 12.0 like this).
 __device__ __forceinline__ float mul_f32_scalar(float a, float b) {
     float r;
     asm("v_mul_f32 %0, %1, %2" : "=v"(r) : "v"(a), "v"(b));

@@ -59,8 +59,8 @@ def test_prefill_attention_forms(env, select):
                                     pf_softmax_rows_kernel -> pf_pv_mfma_kernel (kvMul 4, head size 128 / 64; other shapes: the VALU kernels)
        GL3_PF_FUSED_ATTN=0          the three kernels from position 0
        GL3_PF_SOFTMAX_ROWS=0        the r1 softmax kernel (one row per wavefront, normalises in place) and the r1 V-sum kernel
-       GL3_PF_SCORES_MFMA=0 / GL3_PF_PV_MFMA=0     packed-f32 VALU products (pf_scores_pk_kernel, pf_pv_ring_kernel); + _PK=0 / _RING=0: the scalar r1 kernels
-       GL3_PF_FUSED_MFMA=0 / GL3_PF_FUSED_V1=1     the one-launch kernel with packed-f32 VALU products (fused2) / the r4 kernel
+       GL3_PF_SCORES_MFMA=0 / GL3_PF_PV_MFMA=0     VALU products, four chains side by side (pf_scores_pk_kernel, pf_pv_ring_kernel); + _PK=0 / _RING=0: the r1 kernels
+       GL3_PF_FUSED_MFMA=0 / GL3_PF_FUSED_V1=1     the one-launch kernel with VALU products (fused2) / the r4 kernel
     Ragged chunks, chunks at non-zero positions, the 8B / 1B layers at 512 tokens and behind 1000 positions."""
     e = dict(os.environ, **env)
     out = subprocess.run([sys.executable, "-m", "pytest", os.path.join(ROOT, "tests", "test_gpu_decode.py"), os.path.join(ROOT, "tests", "test_gpu_fullsize.py"),
