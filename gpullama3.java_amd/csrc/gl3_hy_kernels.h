@@ -126,7 +126,7 @@ static __global__ __launch_bounds__(256) void hy_embed_kernel(const int* host, i
 }
 
 // The same together with the norm in front of the first sublayer (pre_in: the streams' weights, null = one stream; norm_w null: the row itself in
-// the matrix type, if h_out is there at all): one workgroup per token, its first HY_EN entries per thread in registers.  One launch, and no second trip to memory, for
+// the matrix type): one workgroup per token, its first HY_EN entries per thread in registers.  One launch, and no second trip to memory, for
 // what took 4.2 + 3.7 us for one token and 9.8 + 10 for 512 of two streams.  host null: the record is in rec already.
 constexpr int HY_EN = 8;
 template <typename T>
@@ -169,7 +169,6 @@ static __global__ __launch_bounds__(1024) void hy_embed_norm_kernel(const int* h
     for (int u = 0; u < HY_EN; ++u)
         if (tid + u * 1024 < W) put(tid + u * 1024, keep[u]);
     for (int w = tid + HY_EN * 1024; w < W; w += 1024) put(w, hy_ld(row + w) * scale + (pair ? hy_ld(pair + w) : 0.f));
-    if (!h_out) return;
     ss = hy_block_sum<1024>(ss, red);
     const float r = norm_w ? ps / sqrtf(ss / (float)W + eps) : 1.f;
 #pragma unroll

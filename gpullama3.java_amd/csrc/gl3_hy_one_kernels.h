@@ -1,8 +1,7 @@
 // gl3_hy_one_kernels.h — the mixers of the layer-list family for ONE token behind few positions, each in one launch.
 //
 // A token's small launches cost 2 us of boundary and one or two round trips to memory each, whatever they compute; behind a few hundred positions the
-// work of all of them fits one workgroup per key / value head (attention) or per head (latent attention): cache row, queries, scores, softmax,
-// weighted sum, gate.  All float32; longer caches, windows in use and other forms stay with the kernels of many workgroups (gl3_hy_kernels.h, gl3_hy_attn_mfma.h).
+// work of all of them fits one workgroup per query head: cache row, queries, scores, softmax, weighted sum, gate.  All float32; longer caches, windows in use and other forms stay with the kernels of many workgroups (gl3_hy_kernels.h, gl3_hy_attn_mfma.h).
 #pragma once
 #include "gl3_hy_kernels.h"
 
