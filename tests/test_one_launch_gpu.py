@@ -69,7 +69,7 @@ def test_tokens_one_by_one(hy, tmp_path, name, dtype):
         assert N.err(np.concatenate(got[i]), m.ref(toks[i])) < (3e-5 if dtype == "float32" else 6e-2)
 
 
-@pytest.mark.parametrize("name,positions", [("heads_64", 768), ("heads_132_and_256", 253), ("latent_512", 640), ("latent_260", 640)])
+@pytest.mark.parametrize("name,positions", [("heads_64", 768), ("heads_132_and_256", 253), ("latent_512", 204), ("latent_260", 640)])
 def test_where_steps_go_over_to_many_workgroups(hy, tmp_path, name, positions):
     mod, layer = LAYERS[name]
     cfg = mod.config([layer])
