@@ -15,9 +15,14 @@
 // The tile is picked per shape (hy_ring_pick in gl3_hybrid.hip).  Measured against hy_gemm_kernel, 512 tokens, W cold in HBM (us):
 //   28672 x 4096 220 -> 107 - 125, 18560 x 4096 200 -> 75 - 83, 10240 x 4096 98 -> 49, 4096 x 4096 50 -> 31 (K split in 2: 24), 4096 x 14336 157 -> 65 - 75;
 //   88 tokens, 4096 x 14336: 56; 24 tokens, 28672 x 4096: 89 -> 52 (4.5 TB/s of weights).
-// float32 matrices (v_mfma_f32_32x32x2_f32): a lane's 16-byte chunk holds 4 k of its row, so one read feeds four MFMAs (the half-wave's
-// chunks pair up; k enters in the order 0, 4, 1, 5, ...); the accumulators are added to a second set every HY_FLUSH stages (128 k), so that the
-// rounding of a long K grows with the number of blocks and not with K.
+// float32 matrices.  The float32 MFMAs (v_mfma_f32_32x32x2_f32) take 16 times as long per product as the bfloat16 ones AND the vector units' time with them (measured: the
+// times of f32 MFMAs and of vector instructions of a SIMD add up, those of bfloat16 MFMAs overlap).  So an operand is split into three bfloat16 planes on its way from
+// LDS (x = p0 + p1 + p2, every plane the rounded rest: all 24 bits) and the plane products of at least 2^-16 go to v_mfma_f32_32x32x16_bf16: six, or three where the
+// matrix's values are bfloat16 already (HyMat::b16: what most checkpoints hold; exact).  A sum has a rounding per 16 k and product instead of one per k, and the accumulators
+// are added to a second set every HY_FLUSH stages (256 k; 512 costs 2 % less, 128 3 % more): whole requests err by 8.1e-7 and 1.25e-6 against 64 bits (181 and 400 tokens, means of 12),
+// with the float32 MFMAs 8.2e-7 and 1.31e-6.  An infinity's planes are not a number: results that are not finite are made again in float32 at the end, one by one.
+// Bound now by the issue of one wavefront per SIMD (58 % of its cycles, 148 vector instructions a stage; planes made ahead by a kernel of their own, and eight wavefronts, were
+// no faster).  181 tokens (us): 8192 x 2048 80 -> 40, 16384 x 2048 with the gate 135 -> 58, 2048 x 8192 79 -> 40, experts 181 + 91 -> 132 + 67; 512 tokens, 4096 x 512 23 -> 14.
 #pragma once
 #include "gl3_hy_kernels.h"
 
@@ -29,26 +34,40 @@ __device__ __forceinline__ void hy_dma16(const void* src, void* lds_wave_base) {
 // all but the newest N loads of this wavefront have landed, its LDS reads are done, and so are everybody's
 template <int N> __device__ __forceinline__ void hy_wait_barrier() { asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" :: "n"(N) : "memory"); }
 
-constexpr int HY_FLUSH = 4;
+constexpr int HY_FLUSH = 8;
+typedef float hy_v8f __attribute__((ext_vector_type(8)));
 template <typename T> struct HyFrag;
 template <> struct HyFrag<bf16_t> { typedef hy_v8bf V; static constexpr int K = 64; };
 template <> struct HyFrag<float> { typedef hy_v4f V; static constexpr int K = 32; };
 __device__ __forceinline__ void hy_mma(hy_v16f& c, const hy_v8bf& a, const hy_v8bf& b) { c = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, c, 0, 0, 0); }
-__device__ __forceinline__ void hy_mma(hy_v16f& c, const hy_v4f& a, const hy_v4f& b) {
-#pragma unroll
-    for (int e = 0; e < 4; ++e) c = __builtin_amdgcn_mfma_f32_32x32x2f32(a[e], b[e], c, 0, 0, 0);
+typedef __bf16 hy_v2bf __attribute__((ext_vector_type(2)));
+typedef float hy_v2f __attribute__((ext_vector_type(2)));
+typedef uint32_t hy_v4u __attribute__((ext_vector_type(4)));
+template <int I, int N, typename F> __device__ __forceinline__ void hy_static_for(F f) { if constexpr (I < N) { f(std::integral_constant<int, I>{}); hy_static_for<I + 1, N>(f); } }
+// Two values as bfloat16, and (REST) what is left of them.  Three times over all 24 bits are held; once for values that are bfloat16 already.
+template <bool REST> __device__ __forceinline__ uint32_t hy_plane(float& x, float& y) {
+    const uint32_t d = __builtin_bit_cast(uint32_t, __builtin_convertvector((hy_v2f{x, y}), hy_v2bf));
+    if constexpr (REST) { x -= __uint_as_float(d << 16); y -= __uint_as_float(d & 0xffff0000u); }
+    return d;
+}
+// one result in float32 throughout (the planes of an infinity are not a number, and so is their product)
+__device__ __attribute__((noinline)) float hy_dot_again(const float* __restrict__ a, const float* __restrict__ w, int n) {
+    float s = 0.f;
+#pragma unroll 1
+    for (int k = 0; k < n; ++k) s = fmaf(a[k], w[k], s);
+    return s;
 }
 
 // WM x WN wavefronts, BM x BN results; EPI, GR and HyGroup as for hy_gemm_kernel (GR: blockIdx.y = row tile of the list, BM rows at most).
 // Grid: x = mt nt ks workgroups (row tiles x column tiles x K splits of kper) rounded up to a multiple of 8; GR: x = column tiles.
-template <typename T, int BM, int BN, int WM, int WN, int SA, int SW, int EPI, int GR = 0>
+template <typename T, int BM, int BN, int WM, int WN, int SA, int SW, int EPI, int GR = 0, int WP = 3>
 static __global__ __launch_bounds__(WM * WN * 64) void hy_gemm_ring_kernel(const T* __restrict__ A, int lda, const T* __restrict__ Wt, int ldw, int M, int N, int K,
                                                                            float* __restrict__ C, int ldc, T* __restrict__ act, int ld_act, HyGlu glu, int mt, int nt, int ks,
                                                                            int kper, HyGroup grp = HyGroup{}) {
     constexpr int NW = WM * WN, TM = BM / WM / 32, TN = BN / WN / 32, BK = HyFrag<T>::K;
     constexpr int PA = BM / 8, PW = BN / 8, NPA = (PA + NW - 1) / NW, NPW = (PW + NW - 1) / NW, NP = NPA + NPW;      // 1 KB pieces (8 rows) of a stage, per wavefront
     constexpr int SZA = BM * 128, SZW = BN * 128, OW = SA * SZA;
-    static_assert(SW > SA && SA >= 2 && NPA * NW < 2 * PA + NW && TM * WM * 32 == BM && TN * WN * 32 == BN, "tile layout");
+    static_assert(SW >= SA + (sizeof(T) == 2) && SA >= 2 && NPA * NW < 2 * PA + NW && TM * WM * 32 == BM && TN * WN * 32 == BN, "tile layout");
     static_assert(SA * SZA + SW * SZW <= 160 * 1024, "LDS");
     __shared__ __attribute__((aligned(1024))) uint8_t smem[SA * SZA + SW * SZW];
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), wm = wave / WN, wn = wave % WN;
@@ -128,6 +147,107 @@ static __global__ __launch_bounds__(WM * WN * 64) void hy_gemm_ring_kernel(const
 #pragma unroll
     for (int q = 0; q < 4; ++q) ca[q] = ((2 * q + kh) ^ ((r32 >> 1) & 7)) * 16;
     const uint32_t aw = (wm * (BM / WM) + r32) * 128, ww = OW + (wn * (BN / WN) + r32) * 128;
+    if constexpr (sizeof(T) == 4) {
+        // Half a stage (16 k) at a time, three deep: while the MFMAs take half h's planes, half h + 1 is split and half h + 2 comes from LDS.  Barrier s finds the stage's last
+        // chunks in registers, so the loads behind it (A's stage s + SA, W's s + SW) go into the stage's own slots.
+        constexpr int LEFT = SW > SA ? NPW + (SA - 2) * NP : (SA - 2) * NP;          // loads started behind stage s + 1's when barrier s waits for them (a step starts A's, then W's)
+        hy_v4f xa[2][TM][2], xw[2][TN][2];
+        hy_v4u qa[2][TM][3], qw[2][TN][WP];
+        auto rd = [&](int set, int sa, int sw, int h) {
+#pragma unroll
+            for (int u = 0; u < 2; ++u) {
+#pragma unroll
+                for (int j = 0; j < TN; ++j) xw[set][j][u] = *reinterpret_cast<const hy_v4f*>(smem + sw * SZW + ww + j * 4096 + ca[2 * h + u]);
+#pragma unroll
+                for (int i = 0; i < TM; ++i) xa[set][i][u] = *reinterpret_cast<const hy_v4f*>(smem + sa * SZA + aw + i * 4096 + ca[2 * h + u]);
+            }
+        };
+        // the split of a half in UN steps, a plane of one pair of values each
+        constexpr int UN = 4 * (WP * TN + 3 * TM);
+        auto cut = [&](auto c, int set) {
+            constexpr int u = decltype(c)::value, w = 4 * WP * TN, f = u < w ? u / (4 * WP) : (u - w) / 12, pl = u < w ? u / 4 % WP : (u - w) / 4 % 3, e = u % 4;
+            if constexpr (u < w) qw[set][f][pl][e] = hy_plane<(pl + 1 < WP)>(*((float*)&xw[set][f][e / 2] + e % 2 * 2), *((float*)&xw[set][f][e / 2] + e % 2 * 2 + 1));
+            else qa[set][f][pl][e] = hy_plane<(pl < 2)>(*((float*)&xa[set][f][e / 2] + e % 2 * 2), *((float*)&xa[set][f][e / 2] + e % 2 * 2 + 1));
+        };
+        // the products of at least 2^-16 (planes a + b <= 2), the small ones first
+        constexpr int NM = (WP == 3 ? 6 : 3) * TM * TN;
+        auto mm = [&](auto c, int set) {
+            constexpr int q = decltype(c)::value / (TM * TN), i = decltype(c)::value / TN % TM, j = decltype(c)::value % TN;
+            constexpr int a_ = WP == 3 ? (q == 0 ? 2 : q == 1 || q == 3 ? 1 : 0) : 2 - q, b_ = WP == 3 ? (q == 1 || q == 4 ? 1 : q == 2 ? 2 : 0) : 0;
+            hy_mma(acc[i][j], __builtin_bit_cast(hy_v8bf, qa[set][i][a_]), __builtin_bit_cast(hy_v8bf, qw[set][j][b_]));
+        };
+        // (pinned: left to the compiler the splits stand in one piece behind the MFMAs)
+        auto both = [&](auto mset, int cset, auto load) {
+            hy_static_for<0, NM>([&](auto c) {
+                constexpr int q = decltype(c)::value, u0 = q * UN / NM, u1 = (q + 1) * UN / NM, h = NM * decltype(mset)::value, l0 = (h + q) * NP / (2 * NM), l1 = (h + q + 1) * NP / (2 * NM);
+                mm(c, decltype(mset)::value);
+                hy_static_for<l0, l1>(load);
+                hy_static_for<u0, u1>([&](auto u) { cut(u, cset); });
+                __builtin_amdgcn_sched_barrier(0);
+            });
+        };
+        constexpr std::integral_constant<int, 0> H0{};
+        constexpr std::integral_constant<int, 1> H1{};
+#pragma unroll
+        for (int s = -SW; s < 0; ++s) {
+            if (s + SA >= 0 && s + SA < n_it) issue_a(s + SA, s + SA);
+            if (s + SW < n_it) issue_w(s + SW, s + SW, 0, NPW);
+        }
+        if (n_it >= SW) hy_wait_barrier<LEFT + NP>(); else hy_wait_barrier<0>();
+        int sa = 0, sw = 0, it = 0;
+        rd(0, 0, 0, 0);
+        rd(1, 0, 0, 1);
+        hy_static_for<0, UN>([&](auto u) { cut(u, 0); });
+        while (it < n_it - SW) {
+            const int stop = min(n_it - SW, it + HY_FLUSH);
+#pragma unroll 1
+            for (; it < stop; ++it) {
+                __builtin_amdgcn_s_waitcnt(0xc07f);          // lgkmcnt(0) where the compiler sees it: it would wait for the reads behind the barrier as well
+                hy_wait_barrier<LEFT>();
+                const uint8_t *na = (const uint8_t*)A + (size_t)(it + SA) * 128, *nw = (const uint8_t*)Wt + (size_t)(it + SW) * 128;
+                uint8_t *da = smem + sa * SZA, *dw = smem + sw * SZW;
+                auto load = [&](auto c) {          // piece c of this step
+                    constexpr int u = decltype(c)::value;
+                    if constexpr (u < NPA) hy_dma16(na + offa[u], da + pa[u]); else hy_dma16(nw + offw[u - NPA], dw + pw[u - NPA]);
+                };
+                if (++sa == SA) sa = 0;
+                if (++sw == SW) sw = 0;
+                rd(0, sa, sw, 0);
+                __builtin_amdgcn_sched_barrier(0);
+                both(H0, 1, load);
+                rd(1, sa, sw, 1);
+                __builtin_amdgcn_sched_barrier(0);
+                both(H1, 0, load);
+            }
+            flush();
+        }
+        for (; it < n_it; ++it) {          // the last SW stages: nothing (A: little) left to load
+            hy_wait_barrier<0>();
+            if (it + SA < n_it) issue_a(it + SA, sa);
+            if (++sa == SA) sa = 0;
+            if (++sw == SW) sw = 0;
+            const bool more = it + 1 < n_it;
+            if (more) rd(0, sa, sw, 0);
+            both(H0, 1, [](auto) {});
+            if (more) rd(1, sa, sw, 1);
+            both(H1, 0, [](auto) {});          // (nothing behind the last stage: the chunks are those of before, the planes unused)
+        }
+        flush();
+#pragma unroll
+        for (int i = 0; i < TM; ++i)
+#pragma unroll
+            for (int j = 0; j < TN; ++j) acc[i][j] = tot[i][j];
+    } else {
+    // step s (behind barrier s) starts the loads of A's stage s + SA (into the slot the barrier freed) and, in the two quarters after it,
+    // of W's stage s + SW; the steps before 0 are the prologue, the last one's W belongs to the loop's first round
+    constexpr int LEFT = (SA - 2) * NP + NPW;          // loads started behind A's stage s + 1 when barrier s waits for it
+#pragma unroll
+    for (int s = -SW; s < 0; ++s) {
+        if (s + SA >= 0 && s + SA < n_it) issue_a(s + SA, s + SA);
+        if (s < -1 && s + SW < n_it) issue_w(s + SW, s + SW, 0, NPW);
+    }
+    if (n_it >= SW) hy_wait_barrier<(SA - 1) * NP>(); else hy_wait_barrier<0>();
+    int sa = 0, sw = 0, sp = SW - 1, it = 0;          // slots of the current stage; sp: the W slot that the step before fills
     typedef typename HyFrag<T>::V V;
     V fa[2][TM], fw[2][TN];
     auto rd = [&](int set, int sa, int sw, int q) {
@@ -143,28 +263,18 @@ static __global__ __launch_bounds__(WM * WN * 64) void hy_gemm_ring_kernel(const
             for (int j = 0; j < TN; ++j) hy_mma(acc[i][j], fa[set][i], fw[set][j]);
     };
     // a quarter's order: fragment reads and the quarter's loads (ND of them) between the MFMAs
-    constexpr int NR = TM + TN, MPR = sizeof(T) == 2 ? 1 : 4, NM = TM * TN * MPR;
+    constexpr int NR = TM + TN, NM = TM * TN;
 #define HY_QUARTER(ND)                                                              \
     do {                                                                            \
         _Pragma("unroll") for (int q_ = 0; q_ < NR; ++q_) {                         \
             __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);                      \
-            if ((q_ + 1) * MPR <= NM) __builtin_amdgcn_sched_group_barrier(0x8, MPR, 0); \
+            if (q_ + 1 <= NM) __builtin_amdgcn_sched_group_barrier(0x8, 1, 0);     \
             if (q_ < (ND)) __builtin_amdgcn_sched_group_barrier(0x20, 1, 0);        \
         }                                                                           \
-        if (NM > NR * MPR) __builtin_amdgcn_sched_group_barrier(0x8, NM - NR * MPR, 0); \
+        if (NM > NR) __builtin_amdgcn_sched_group_barrier(0x8, NM - NR, 0);          \
         __builtin_amdgcn_sched_barrier(0);                                          \
     } while (0)
-    // step s (behind barrier s) starts the loads of A's stage s + SA (into the slot the barrier freed) and, in the two quarters after it,
-    // of W's stage s + SW; the steps before 0 are the prologue, the last one's W belongs to the loop's first round
-    constexpr int LEFT = (SA - 2) * NP + NPW;          // loads started behind A's stage s + 1 when barrier s waits for it
-#pragma unroll
-    for (int s = -SW; s < 0; ++s) {
-        if (s + SA >= 0 && s + SA < n_it) issue_a(s + SA, s + SA);
-        if (s < -1 && s + SW < n_it) issue_w(s + SW, s + SW, 0, NPW);
-    }
-    if (n_it >= SW) hy_wait_barrier<(SA - 1) * NP>(); else hy_wait_barrier<0>();
     rd(0, 0, 0, 0);
-    int sa = 0, sw = 0, sp = SW - 1, it = 0;          // slots of the current stage; sp: the W slot that the step before fills
     for (; it < n_it - SW; ++it) {
         rd(1, sa, sw, 1); mm(0); issue_w(it - 1 + SW, sp, 0, WH); HY_QUARTER(WH);
         rd(0, sa, sw, 2); mm(1); issue_w(it - 1 + SW, sp, WH, NPW); HY_QUARTER(NPW - WH);
@@ -175,7 +285,6 @@ static __global__ __launch_bounds__(WM * WN * 64) void hy_gemm_ring_kernel(const
         if (++sa == SA) sa = 0;
         if (++sw == SW) sw = 0;
         rd(0, sa, sw, 0); mm(1); issue_a(it + SA, freed); HY_QUARTER(NPA);
-        if (sizeof(T) == 4 && it % HY_FLUSH == HY_FLUSH - 1) flush();
     }
     if (it - 1 + SW < n_it) issue_w(it - 1 + SW, sp, 0, NPW);
     for (; it < n_it; ++it) {          // the last SW stages: nothing (A: little) left to load
@@ -189,18 +298,29 @@ static __global__ __launch_bounds__(WM * WN * 64) void hy_gemm_ring_kernel(const
         if (it + 1 < n_it) rd(0, sa, sw, 0);
         mm(1);
         __builtin_amdgcn_sched_barrier(0);
-        if (sizeof(T) == 4 && it % HY_FLUSH == HY_FLUSH - 1) flush();
     }
-    if constexpr (sizeof(T) == 4) {
-        flush();
-#pragma unroll
-        for (int i = 0; i < TM; ++i)
-#pragma unroll
-            for (int j = 0; j < TN; ++j) acc[i][j] = tot[i][j];
     }
 #undef HY_QUARTER
     // lane holds column lane % 32 and rows 8 (r / 4) + 4 (lane / 32) + r % 4 of every 32 x 32 tile
     const int mb = m0 + wm * (BM / WM) + 4 * kh, nb = n0 + wn * (BN / WN) + r32;
+    if constexpr (sizeof(T) == 4) {          // an operand or a sum that is not finite: float32 all the way (rare)
+#pragma unroll
+        for (int i = 0; i < TM; ++i)
+#pragma unroll
+            for (int j = 0; j < TN; ++j) {
+                bool odd = false;
+#pragma unroll
+                for (int r = 0; r < 16; ++r) odd |= !(fabsf(acc[i][j][r]) < INFINITY);
+                if (__builtin_expect(__any(odd), 0)) {
+#pragma unroll
+                    for (int r = 0; r < 16; ++r) {
+                        const int m = mb + i * 32 + 8 * (r >> 2) + (r & 3), n = nb + j * 32;
+                        if (!(fabsf(acc[i][j][r]) < INFINITY) && m < M && n < N)
+                            acc[i][j][r] = hy_dot_again((const float*)A + (size_t)m * lda + kbeg, (const float*)Wt + (size_t)n * ldw + kbeg, n_it * BK);
+                    }
+                }
+            }
+    }
     if constexpr (EPI == HY_EPI_GLU) {
         static_assert(EPI != HY_EPI_GLU || TN % 2 == 0, "gate / up pairs need a wavefront tile of 64 features");
 #pragma unroll

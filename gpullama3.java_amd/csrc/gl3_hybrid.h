@@ -14,6 +14,7 @@ typedef std::bitset<GL3_T_COUNT> HyHave;      // tensors that have arrived, by i
 struct HyMat {                 // [rows][ld] of the plan's matrix type (bfloat16 or float32), K-contiguous, zero padded
     void* w = nullptr;
     int rows = 0, k = 0, ld = 0;
+    bool b16 = true;           // float32 matrices: every entry is a bfloat16 value (checked as it arrives)
 };
 
 struct HyLayer {
@@ -64,6 +65,7 @@ struct HyLayer {
     // De = dim + rot_dim entries; the expansions are padded to these sizes (key expansion: identity behind the latent's columns, value
     // expansion: zeros), so every kernel of the latent path runs on (De, Re) as it does on (dim, kv_rank) without a rotated part.
     float *lat_norm = nullptr, *wk = nullptr, *wv = nullptr, *wvT = nullptr;
+    bool wk16 = false, wv16 = false;          // every entry of wk / wv is a bfloat16 value
     int De = 0, Re = 0;
     HyMat uq;                  // latent with q_rank: query expansion [heads De x q_rank]
     float* qlat_norm = nullptr;// norm weight of the query latent [q_rank]

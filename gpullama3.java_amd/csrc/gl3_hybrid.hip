@@ -615,6 +615,11 @@ static bool hy_to_f32(const void* host, uint64_t bytes, int type, size_t n, std:
         return false;
     return true;
 }
+static bool hy_all_bf16(const float* x, size_t n) {
+    uint32_t low = 0;
+    for (size_t i = 0; i < n; ++i) { uint32_t u; memcpy(&u, x + i, 4); low |= u & 0xffffu; }
+    return low == 0;
+}
 static int32_t hy_put_vec(gl3_ctx* ctx, float* dst, size_t n, const void* host, uint64_t bytes, int type, float add = 0.f) {
     std::vector<float> f;
     if (!hy_to_f32(host, bytes, type, n, f)) GL3_FAIL(GL3_E_ARG, "tensor size or type mismatch");
@@ -631,6 +636,7 @@ static int32_t hy_put_rows(gl3_ctx* ctx, HyMat& m, int dst_row0, int rows, int k
     if ((type != GL3_TYPE_BF16 && type != GL3_TYPE_F32) || bytes != n * (type == GL3_TYPE_BF16 ? 2 : 4)) GL3_FAIL(GL3_E_ARG, "tensor size or type mismatch");
     if (dst_col0 < 0 || dst_col0 + k > m.k) GL3_FAIL(GL3_E_ARG, "tensor row length mismatch");
     std::vector<uint8_t> img(n * es, 0);
+    if (f32 && type == GL3_TYPE_F32) m.b16 = m.b16 && hy_all_bf16((const float*)host, n);
     for (size_t i = 0; i < n; ++i) {
         if (f32) ((float*)img.data())[i] = type == GL3_TYPE_BF16 ? hy_bf16_to_f32(((const uint16_t*)host)[i]) : ((const float*)host)[i];
         else ((uint16_t*)img.data())[i] = type == GL3_TYPE_BF16 ? ((const uint16_t*)host)[i] : hy_f32_to_bf16(((const float*)host)[i]);
@@ -760,6 +766,7 @@ int32_t gl3_hy_upload(gl3_ctx* ctx, int32_t id, int32_t layer, const void* host,
                     for (int j = 0; j < d.rot_dim; ++j) wk[((size_t)hh * De + d.dim + j) * Re + R + j] = 1.f;
                 }
                 HY_HIP(hipMemcpy(L.wk, wk.data(), wk.size() * 4, hipMemcpyHostToDevice));
+                L.wk16 = hy_all_bf16(wk.data(), wk.size());
                 r = GL3_OK;
             }
             break;
@@ -778,6 +785,7 @@ int32_t gl3_hy_upload(gl3_ctx* ctx, int32_t id, int32_t layer, const void* host,
                         }
                 HY_HIP(hipMemcpy(L.wvT, tr.data(), n * 4, hipMemcpyHostToDevice));
                 HY_HIP(hipMemcpy(L.wv, wv.data(), n * 4, hipMemcpyHostToDevice));
+                L.wv16 = hy_all_bf16(wv.data(), n);
                 r = GL3_OK;
             }
             break;
@@ -893,6 +901,7 @@ int32_t gl3_hy_finalize(gl3_ctx* ctx) {
     if ((h->have & g) != g) GL3_FAIL(GL3_E_STATE, "missing global tensors (token embedding / output norm / side embedding / token-pair embedding)");
     if (!h->have.test(GL3_T_OUTPUT)) {           // tied head
         HY_HIP(hipMemcpy(h->head.w, h->emb.w, (size_t)h->emb.rows * h->emb.ld * (h->f32 ? 4 : 2), hipMemcpyDeviceToDevice));
+        h->head.b16 = h->emb.b16;
     }
     for (size_t l = 0; l < h->L.size(); ++l) {
         const HyHave need = hy_needed(h, h->L[l].d);
@@ -920,24 +929,25 @@ static HyGlu hy_ff_glu(const HyLayer& L) { return HyGlu{L.dense_limit, L.d.ff_al
 enum { HY_R256x256, HY_R256x224, HY_R256x192, HY_R256x160, HY_R256x128, HY_R128x256, HY_R128x160, HY_R128x128, HY_R64x128, HY_R64x64, HY_R_COUNT };
 static const struct { int bm, bn; } HY_RING_TILES[HY_R_COUNT] = {{256, 256}, {256, 224}, {256, 192}, {256, 160}, {256, 128}, {128, 256}, {128, 160}, {128, 128}, {64, 128}, {64, 64}};
 // Which tile and K split: the one with the least estimated time.  A stage of a BM x BN tile takes a CU 0.00154 (BM + BN) us for its operand bytes (83 GB/s per CU,
-// what the loads of all 256 sustain) + 0.0000128 BM BN us that its MFMAs add (fits 64 x 64 ... 256 x 256 within 8 %; float32 MFMAs are 16 x slower for half the
-// K); 256 CUs take the workgroups in rounds of whole tiles (two workgroups of a small tile share a CU, and its loads) — what decides for most shapes: 10240 x 4096 at
+// what the loads of all 256 sustain) + 0.0000128 BM BN us that its MFMAs add (fits 64 x 64 ... 256 x 256 within 8 %).  A float32 stage is bound by the issue of its
+// one wavefront per SIMD: 0.43 / 0.58 / 0.78 us for 64 x 64 / 64 x 128 / 128 x 128 with weights of one plane (0.55 / 0.9 / 1.4 with three), and two workgroups on a CU take
+// 1.55 times as long as one (128 x 128 fill its registers alone).  256 CUs take the workgroups in rounds of whole tiles (two workgroups of a small tile share a CU, and its loads) — what decides for most shapes: 10240 x 4096 at
 // 512 tokens is 256 tiles of 128 x 160 (49 us) but 320 of 128 x 128 (65 us) or 160 of 256 x 128 (53 us).  A K split writes and re-reads its part of C at ~4 TB/s.
-static double hy_ring_pick(bool f32, int M, int N, int K, bool glu, bool actmul, int max_parts, int* tile, int* ks_out) {
+static double hy_ring_pick(bool f32, bool b16, int M, int N, int K, bool glu, bool actmul, int max_parts, int* tile, int* ks_out) {
     const int stages = K / (f32 ? 32 : 64);
     double best = 1e30;
     for (int t = 0; t < HY_R_COUNT; ++t) {
         const int bm = HY_RING_TILES[t].bm, bn = HY_RING_TILES[t].bn;
         if (glu ? (t != HY_R256x256 && t != HY_R128x256 && t != HY_R128x128 && t != HY_R64x128) : t == HY_R256x256) continue;
         if (actmul && t != HY_R256x224 && t != HY_R128x128 && t != HY_R64x64) continue;
-        if (f32 && (t < HY_R256x128 || t == HY_R128x256)) continue;          // (two sets of accumulators)
-        const double stage = 0.00154 * (bm + bn) + (f32 ? 0.000105 : 0.0000128) * bm * bn;
-        const long mn = (long)hy_cdiv(M, bm) * hy_cdiv(N, bn), pair = t >= HY_R128x128 ? 2 : 1;
+        if (f32 && t < HY_R128x128) continue;          // (two sets of accumulators; 128 x 160 takes 1.15 times 128 x 128)
+        const double stage = !f32 ? 0.00154 * (bm + bn) + 0.0000128 * bm * bn : b16 ? 0.30 + 0.000031 * bm * bn : 0.28 + 0.00007 * bm * bn, both = f32 ? 1.55 : 2.0;
+        const long mn = (long)hy_cdiv(M, bm) * hy_cdiv(N, bn), pair = t >= (f32 ? HY_R64x128 : HY_R128x128) ? 2 : 1;
         for (int ks = 1; ks <= max_parts && (ks == 1 || stages / ks >= 4); ++ks) {
             const int per = hy_cdiv(stages, ks);
             if (hy_cdiv(stages, per) != ks) continue;
             const long wgs = mn * ks, rest = wgs % (256 * pair);
-            const double rounds = (double)(wgs / (256 * pair)) * pair * (per * stage + 3.0), last = rest == 0 ? 0.0 : (rest <= 256 ? 1 : 2) * (per * stage + 3.0);
+            const double rounds = (double)(wgs / (256 * pair)) * (pair == 2 ? both : 1.0) * (per * stage + 3.0), last = rest == 0 ? 0.0 : (rest <= 256 ? 1.0 : both) * (per * stage + 3.0);
             const double us = rounds + last + (ks - 1) * (double)M * N * 8 / 4e6;
             if (us < best) { best = us; *tile = t; *ks_out = ks; }
         }
@@ -954,13 +964,17 @@ static bool hy_gemm_ring(gl3_ctx* ctx, const T* A, int lda, const HyMat& w, int 
     if ((uint64_t)M * lda * sizeof(T) >= 0xffff0000ull || (uint64_t)N * w.ld * sizeof(T) >= 0xffff0000ull) return false;      // 32-bit offsets inside an operand
     const bool actmul = !glu && (gp.mul_table || gp.act == 2);
     int tile = HY_R128x128, ks = 1;
-    if (hy_ring_pick(sizeof(T) == 4, M, N, K, glu, actmul, parts && !glu && !actmul ? max_parts : 1, &tile, &ks) >= limit_us) return false;
+    if (hy_ring_pick(sizeof(T) == 4, w.b16, M, N, K, glu, actmul, parts && !glu && !actmul ? max_parts : 1, &tile, &ks) >= limit_us) return false;
     const int kper = hy_cdiv(K / BK, ks) * BK, mt = hy_cdiv(M, HY_RING_TILES[tile].bm), nt = hy_cdiv(N, HY_RING_TILES[tile].bn);
     if (parts) *parts = ks;
     const dim3 grid((unsigned)hy_cdiv(mt * nt * ks, 8) * 8);
+#define HY_RG1(BM, BN, WM, WN, SA, SW, EPI, WP)                                                                                                         \
+    hipLaunchKernelGGL((hy_gemm_ring_kernel<T, BM, BN, WM, WN, SA, SW, EPI, 0, sizeof(T) == 4 ? WP : 1>), grid, dim3((WM) * (WN) * 64), 0, ctx->stream, A, lda, (const T*)w.w, w.ld, \
+                       M, N, K, C, ldc, act, ld_act, gp, mt, nt, ks, kper)
 #define HY_RG(BM, BN, WM, WN, SA, SW, EPI)                                                                                                              \
-    hipLaunchKernelGGL((hy_gemm_ring_kernel<T, BM, BN, WM, WN, SA, SW, EPI>), grid, dim3(WM * WN * 64), 0, ctx->stream, A, lda, (const T*)w.w, w.ld, M, N, K, C, ldc, act, \
-                       ld_act, gp, mt, nt, ks, kper)
+    do {                                                                                                                                                \
+        if (sizeof(T) == 4 && !w.b16) HY_RG1(BM, BN, WM, WN, SA, SW, EPI, 3); else HY_RG1(BM, BN, WM, WN, SA, SW, EPI, 1);                               \
+    } while (0)
     // The rings: A has to be on its way for more than one stage as well (L2's answer takes 0.4 us; 64 x 64 with a ring of 2 + 6 took that long per stage and 0.25 with
     // 4 + 5: 88 tokens, 4096 x 14336 90 -> 56 us; 512 tokens, 2048 x 8192 51 -> 37).  What two workgroups of a CU cannot have one alone takes (64 x 128: 4096 x 4096 at 512
     // tokens 35 -> 31 us; 128 x 128: 6144 x 4096 41 -> 39).
@@ -971,16 +985,18 @@ static bool hy_gemm_ring(gl3_ctx* ctx, const T* A, int lda, const HyMat& w, int 
         if (tile == HY_R256x224) { if (actmul) HY_RG(256, 224, 8, 1, 2, 3, HY_EPI_ACTMUL); else HY_RG(256, 224, 8, 1, 2, 3, HY_EPI_STORE); return true; }
         if (tile == HY_R256x192) { HY_RG(256, 192, 4, 2, 2, 4, HY_EPI_STORE); return true; }
         if (tile == HY_R256x160) { HY_RG(256, 160, 8, 1, 2, 4, HY_EPI_STORE); return true; }
+        if (tile == HY_R256x128) { HY_RG(256, 128, 4, 2, 3, 4, HY_EPI_STORE); return true; }
+        if (tile == HY_R128x160) { HY_RG(128, 160, 4, 1, 3, 5, HY_EPI_STORE); return true; }
     }
-#define HY_RG_64x128(EPI) do { if (lone) HY_RG(64, 128, 2, 2, 3, 4, EPI); else HY_RG(64, 128, 2, 2, 2, 4, EPI); } while (0)
-#define HY_RG_128x128(EPI) do { if (lone) HY_RG(128, 128, 4, 2, 3, 4, EPI); else HY_RG(128, 128, 4, 2, 2, 3, EPI); } while (0)
+    // float32: two workgroups of 64 x 128 share a CU whatever their number (a ring of 6 + 6 is no faster alone: 181 tokens, 8192 x 2048 39 us both)
+    constexpr bool F = sizeof(T) == 4;
+#define HY_RG_64x128(EPI) do { if (!F && lone) HY_RG(64, 128, 2, 2, 3, 4, EPI); else HY_RG(64, 128, 2, 2, F ? 3 : 2, F ? 3 : 4, EPI); } while (0)
+#define HY_RG_128x128(EPI) do { if (F || lone) HY_RG(128, 128, 4, 2, F ? 4 : 3, F ? 5 : 4, EPI); else HY_RG(128, 128, 4, 2, 2, 3, EPI); } while (0)
     if (glu) {
         if (tile == HY_R64x128) HY_RG_64x128(HY_EPI_GLU); else HY_RG_128x128(HY_EPI_GLU);
     } else if (actmul) {
         if (tile == HY_R64x64) HY_RG(64, 64, 2, 2, 4, 5, HY_EPI_ACTMUL); else HY_RG_128x128(HY_EPI_ACTMUL);
     } else switch (tile) {
-        case HY_R256x128: HY_RG(256, 128, 4, 2, 3, 4, HY_EPI_STORE); break;
-        case HY_R128x160: HY_RG(128, 160, 4, 1, 3, 5, HY_EPI_STORE); break;
         case HY_R64x128: HY_RG_64x128(HY_EPI_STORE); break;
         case HY_R64x64: HY_RG(64, 64, 2, 2, 4, 5, HY_EPI_STORE); break;
         default: HY_RG_128x128(HY_EPI_STORE);
@@ -988,6 +1004,7 @@ static bool hy_gemm_ring(gl3_ctx* ctx, const T* A, int lda, const HyMat& w, int 
 #undef HY_RG_64x128
 #undef HY_RG_128x128
 #undef HY_RG
+#undef HY_RG1
     return true;
 }
 
@@ -1525,8 +1542,8 @@ static int32_t hy_mixer_core(gl3_ctx* ctx, HyLayer& L, int np, int ldo, int n, i
             const int M = pos0 + n;
             const float* lat = cc + (size_t)seq * h->slot_floats;
             HyMat wkm, wvm;
-            wkm.w = L.wk; wkm.rows = d.heads * De; wkm.k = R; wkm.ld = R;
-            wvm.w = L.wv; wvm.rows = d.heads * d.vdim; wvm.k = R; wvm.ld = R;
+            wkm.w = L.wk; wkm.rows = d.heads * De; wkm.k = R; wkm.ld = R; wkm.b16 = L.wk16;
+            wvm.w = L.wv; wvm.rows = d.heads * d.vdim; wvm.k = R; wvm.ld = R; wvm.b16 = L.wv16;
             hy_gemm<float>(ctx, lat, R, wkm, M, h->kx, d.heads * De, false, nullptr, 0, HyGlu{});
             hy_gemm<float>(ctx, lat, R, wvm, M, h->vx, d.heads * d.vdim, false, nullptr, 0, HyGlu{});
             const HyAttnOut fin{mixo, ldo, sizeof(T) == 4, d.out_gate ? h->proj + L.g_off : nullptr, np, d.out_gate == 2 ? 2 : 1, d.softmax_sink, d.softmax_sink == 2 ? L.sink : nullptr, 1.f};
@@ -1662,11 +1679,14 @@ static void hy_gemm_grouped(gl3_ctx* ctx, const T* A, int lda, const HyMat& w, s
     const dim3 grid(hy_cdiv(N, 128), max_tiles, 1);
     constexpr int PE = 16 / (int)sizeof(T), BK = 128 / (int)sizeof(T);
     if (K % BK == 0 && lda % PE == 0 && w.ld % PE == 0 && wstride % PE == 0 && (((uintptr_t)A | (uintptr_t)Wt) & 15) == 0 && (uint64_t)N * w.ld * sizeof(T) < 0xffff0000ull) {
-#define HY_RGG(BM, WM, EPI) hipLaunchKernelGGL((hy_gemm_ring_kernel<T, BM, 128, WM, 2, BM == 32 ? 3 : 2, 4, EPI, 1>), grid, dim3(WM * 128), 0, st, A, lda, Wt, w.ld, 0, N, K, C, ldc, act, ld_act, gp, 0, 0, 1, K, grp)
+    // float32 tiles of 32 rows: four workgroups a CU hide each other's stages (rings of 2 + 2; 3 + 4, two a CU: 181 tokens x 4 of 32 experts 132 + 67 us, 145 + 73)
+#define HY_RGG1(BM, WM, EPI, WP) hipLaunchKernelGGL((hy_gemm_ring_kernel<T, BM, 128, WM, 2, sizeof(T) == 2 && BM == 32 ? 3 : 2, sizeof(T) == 2 ? 4 : BM == 32 ? 2 : 3, EPI, 1, sizeof(T) == 4 ? WP : 1>), grid, dim3(WM * 128), 0, st, A, lda, Wt, w.ld, 0, N, K, C, ldc, act, ld_act, gp, 0, 0, 1, K, grp)
+#define HY_RGG(BM, WM, EPI) do { if (sizeof(T) == 4 && !w.b16) HY_RGG1(BM, WM, EPI, 3); else HY_RGG1(BM, WM, EPI, 1); } while (0)
 #define HY_RGG_EPI(BM, WM) do { if (glu) HY_RGG(BM, WM, HY_EPI_GLU); else if (gp.act == 2) HY_RGG(BM, WM, HY_EPI_ACTMUL); else HY_RGG(BM, WM, HY_EPI_STORE); } while (0)
         if (bm == HY_MOE_BM_FEW) HY_RGG_EPI(HY_MOE_BM_FEW, 1); else HY_RGG_EPI(HY_MOE_BM, 2);
 #undef HY_RGG_EPI
 #undef HY_RGG
+#undef HY_RGG1
         return;
     }
     if (glu) hipLaunchKernelGGL((hy_gemm_kernel<T, T, HY_MOE_BM, 128, HY_EPI_GLU, 1>), grid, dim3(256), 0, st, A, lda, Wt, w.ld, 0, N, K, C, ldc, act, ld_act, gp, K, grp);

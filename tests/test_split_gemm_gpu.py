@@ -1,0 +1,81 @@
+"""float32 products of many tokens as products of bfloat16 planes (csrc/gl3_hy_gemm.h): matrices whose entries need all 24 bits (three planes, six products; the other tests'
+weights are bfloat16 values and take one plane), at the edges of the tiles and of the rings, and values the planes cannot hold.
+
+Yardstick: float64.  Bound: a float32 sum of K terms errs by a few 1e-6 of the logits' root mean square; a plane left out is 2^-8 or 2^-17 of every product (4e-3 or 8e-6)
+and two layers of products see it, so 3e-6 on the root mean square is below what the smallest plane would cost and above what the sums cost (measured up to 1.1e-6)."""
+import numpy as np
+import pytest
+
+import __graft_entry__ as ge
+import kugadra_ref as KR
+import noditar_ref as R
+import test_kugadra_gpu as U
+from test_noditar_gpu import att, config, err, lat, tokens_for
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def hy():
+    from importlib import import_module
+    ge.load_package()
+    return import_module(ge.PKG_NAME + ".hybrid")
+
+
+def full_bits(ref, cfg, seed):
+    """The design's random weights with every matrix entry moved by up to a part in 200: float32 values with all their bits."""
+    rng = np.random.default_rng(seed)
+    return {k: (v * (1.0 + 0.005 * rng.standard_normal(v.shape))).astype(np.float32) if v.ndim == 2 else v.astype(np.float32) for k, v in ref.random_weights(cfg, seed).items()}
+
+
+def logits(hy, path, cfg, w, toks):
+    hy.save_model_dir(str(path), cfg, w, dtype="F32")
+    p = hy.HybridPlan.from_dir(str(path), dtype="float32", ctx=len(toks) + 8, max_batch=512)
+    got = p.step(p.acquire(), toks, 0, list(range(len(toks))))
+    p.close()
+    return got
+
+
+# stages of 32 k: fewer than a ring (64), the ring (96 - 160), behind it, across the 8-stage sums (544, 1056); rows and columns around 32, 64 and 128
+@pytest.mark.parametrize("n,width,vocab,ff", [(9, 64, 211, 96), (33, 96, 1003, 160), (65, 128, 8195, 544), (130, 160, 451, 1056), (300, 192, 20003, 96)])
+def test_all_bits_of_the_weights(hy, tmp_path, n, width, vocab, ff):
+    cfg = config([att(heads=4, kv_heads=2, dim=16, vdim=24, ff=ff), lat(heads=2, dim=16, vdim=32, kv_rank=64, ff=ff)], width=width, vocab=vocab, streams=1)
+    w = full_bits(R, cfg, n)
+    toks = tokens_for(cfg, n)
+    got, want = logits(hy, tmp_path / "m", cfg, w, toks), R.forward(cfg, R.to_f64(w), toks, None)
+    assert err(got, want) < 3e-6
+    assert np.abs(got - want).max() < 3e-5 * np.sqrt((want ** 2).mean())
+
+
+@pytest.mark.parametrize("n,experts,top", [(40, 6, 2), (200, 3, 2)])          # tiles of 32 and of 64 rows
+def test_all_bits_of_the_experts(hy, tmp_path, n, experts, top):
+    cfg = U.config([U.lig(heads=2, dim=16, vdim=16, mlp=U.moe(experts=experts, top=top, ff=96, shared=64))], width=128)
+    w = full_bits(KR, cfg, n)
+    toks = tokens_for(cfg, n)
+    got, want = logits(hy, tmp_path / "m", cfg, w, toks), KR.forward(cfg, KR.to_f64(w), toks)
+    assert np.median(np.sqrt(((got - want) ** 2).mean(axis=1)) / np.sqrt((want ** 2).mean())) < 3e-6          # (a near tie of two experts may fall the other way)
+
+
+@pytest.mark.parametrize("bits", [16, 24])
+def test_values_that_planes_do_not_hold(hy, tmp_path, bits):
+    """Head rows of 3.395e38 (finite, rounds to infinity in bfloat16), of infinity and of mixed signs: every logit is what float32 products give."""
+    cfg = config([att(heads=2, kv_heads=2, dim=16, vdim=16, ff=32)], width=64, vocab=300, streams=1)
+    w = full_bits(R, cfg, 5) if bits == 24 else {k: R.bf16_round(v) for k, v in R.random_weights(cfg, 5).items()}
+    toks = tokens_for(cfg, 40)
+    base = logits(hy, tmp_path / "a", cfg, w, toks)
+    head = w["head"].copy()
+    head[7] = 0.0
+    head[7, 3] = np.float32(3.395e38) * np.float32(1e-3 if bits == 16 else 1.0)
+    head[11, 5] = np.inf
+    head[12] = 0.0
+    head[12, 5], head[12, 6] = np.inf, -np.inf
+    got = logits(hy, tmp_path / "b", cfg, dict(w, head=head), toks)
+    h = R.forward(cfg, R.to_f64(dict(w, head=np.eye(64)[np.arange(300) % 64])), toks, None)          # the normed rows themselves
+    with np.errstate(over="ignore"):
+        want7 = (h[:, 3] * np.float64(head[7, 3])).astype(np.float32)
+    ok = np.abs(h[:, 3]) < 0.99 if bits == 24 else np.ones(40, bool)
+    assert ok.sum() > 10 and np.all(np.abs(got[ok, 7] - want7[ok]) <= 2e-5 * np.abs(want7[ok]) + 1e-6 * np.abs(head[7, 3]))
+    assert np.array_equal(got[:, 11], np.where(h[:, 5] > 0, np.inf, -np.inf))
+    assert np.isnan(got[np.sign(h[:, 5]) == np.sign(h[:, 6]), 12]).all()
+    rest = np.setdiff1d(np.arange(300), [7, 11, 12])
+    assert np.abs(got[:, rest] - base[:, rest]).max() <= 1e-5 * np.abs(base).max()
