@@ -11,6 +11,14 @@ constexpr int HY_YPARTS = 2 * HY_KSPLIT;      // copies of y: in a parallel bloc
 
 typedef std::bitset<GL3_T_COUNT> HyHave;      // tensors that have arrived, by id
 
+// x <- mix^T x + po y_mul post(y) (S streams; one stream without tables: x + y_mul post(y)); h = rms norm of (pi . x), weighted.  y = sum of yparts rows.
+struct HyPre {
+    const float* x; size_t xs; float* x_out; size_t xos; int W;
+    const float* y; int yparts; size_t ystride; float y_mul; const float* post_w;
+    const float *mix, *po, *pi, *norm_w; float eps;
+    void* h_out;
+};
+
 struct HyMat {                 // [rows][ld] of the plan's matrix type (bfloat16 or float32), K-contiguous, zero padded
     void* w = nullptr;
     int rows = 0, k = 0, ld = 0;
@@ -112,6 +120,10 @@ struct gl3_hybrid_state {
     std::vector<int> len;      // tokens a slot holds
     std::vector<int> last_tok; // the last of them
     // scratch of one portion of a step (<= mb tokens)
+    float* X2 = nullptr;                // single tokens: the residual's other buffer (an update that a product makes reads one and writes the other)
+    bool pre_on = false;                // ... and such an update that waits for its product (pre)
+    int pre_streams = 1;
+    HyPre pre{};
     float *X = nullptr, *proj = nullptr, *y = nullptr, *conv = nullptr, *ssm_y = nullptr, *qa = nullptr, *oc = nullptr, *kx = nullptr, *vx = nullptr, *part_acc = nullptr, *part_ml = nullptr;
     float *gates = nullptr, *rowr = nullptr;     // matrix memory: a, b, e^(-m) per (token, head), [3][mb][max heads]; attention: 1 / rms of the whole q and k rows [mb][2]
     int max_heads = 1;

@@ -25,6 +25,7 @@
 #include "gl3_hy_heads_kernels.h"
 #include "gl3_hy_one_kernels.h"
 #include "gl3_hy_plain_kernels.h"
+#include "gl3_hy_pre_kernels.h"
 
 using gl3::AMX_WGS;
 using gl3::argmax_kernel;
@@ -484,6 +485,7 @@ int32_t gl3_hy_create(const gl3_model_desc* desc, gl3_ctx** out, std::string& er
     h->slot_floats = slot;
     TRY(hy_alloc(ctx, &h->slots, slot * h->n_seqs * 4));
     TRY(hy_alloc(ctx, &h->X, (size_t)S * mb * W * 4));
+    TRY(hy_alloc(ctx, &h->X2, (size_t)S * W * 4));
     TRY(hy_alloc(ctx, &h->h, (size_t)mb * W * es));
     TRY(hy_alloc(ctx, &h->proj, (size_t)mb * max_proj * 4));
     TRY(hy_alloc(ctx, &h->y, (size_t)HY_YPARTS * mb * W * 4));          // K-split partial sums of the output / down projections
@@ -591,7 +593,7 @@ void gl3_hy_destroy(gl3_ctx* ctx) {
         f(L.router.w); f(L.egu.w); f(L.edown.w); f(L.depth_mix); f(L.side_gate.w); f(L.side_proj.w); f(L.side_norm);
     }
     f(h->side_emb.w); f(h->sgz); f(h->hist); f(h->side_z); f(h->moe_z); f(h->wsel); f(h->eout); f(h->xb); f(h->side_g); f(h->ea); f(h->eact); f(h->sel); f(h->pair_row); f(h->tiles); f(h->ntiles);
-    f(h->slots); f(h->X); f(h->h); f(h->proj); f(h->y); f(h->mixo); f(h->conv); f(h->ssm_y); f(h->qa); f(h->oc); f(h->kx); f(h->vx); f(h->part_acc); f(h->part_ml); f(h->gates); f(h->rowr);
+    f(h->slots); f(h->X); f(h->X2); f(h->h); f(h->proj); f(h->y); f(h->mixo); f(h->conv); f(h->ssm_y); f(h->qa); f(h->oc); f(h->kx); f(h->vx); f(h->part_acc); f(h->part_ml); f(h->gates); f(h->rowr);
     f(h->cq); f(h->qfull); f(h->bigram.w); f(h->hf); f(h->ffz);
     f(h->xw); f(h->logits); f(h->taps); f(h->ones); f(h->dyn);
     hf(h->h_rec); hf(h->h_logits);
@@ -1008,10 +1010,42 @@ static bool hy_gemm_ring(gl3_ctx* ctx, const T* A, int lda, const HyMat& w, int 
     return true;
 }
 
+// ---- single tokens: residual updates that the next product makes (gl3_hy_pre_kernels.h) -------------------------------------------------
+template <typename T, int EPI>
+static void hy_pre_launch(gl3_ctx* ctx, const HyPre& p, int S, const T* Wt, int ldw, int N, float* C, T* act, int ld_act, const HyGlu& gp) {
+    const int pairs = (N + 1) / 2, wgs = std::max(1, std::min(256, pairs));
+    // up to four pairs a workgroup: four wavefronts share one (2048 x 2048: all of the matrix is on its way at once)
+#define HY_PRE(S_) do { if (hy_cdiv(pairs, wgs) <= 4) hipLaunchKernelGGL((hy_matvec_pre_kernel<T, S_, EPI, 4>), dim3(wgs), dim3(1024), 0, ctx->stream, p, Wt, ldw, N, C, act, ld_act, gp);   \
+                    else hipLaunchKernelGGL((hy_matvec_pre_kernel<T, S_, EPI, 1>), dim3(wgs), dim3(1024), 0, ctx->stream, p, Wt, ldw, N, C, act, ld_act, gp); } while (0)
+    if (S == 1) HY_PRE(1); else if (S == 2) HY_PRE(2); else HY_PRE(4);
+#undef HY_PRE
+}
+// a deferred update that no product has taken: one workgroup without rows
+template <typename T>
+static void hy_pre_flush(gl3_ctx* ctx) {
+    gl3_hybrid_state* h = ctx->hy;
+    if (!h->pre_on) return;
+    h->pre_on = false;
+    hy_pre_launch<T, HY_EPI_STORE>(ctx, h->pre, h->pre_streams, (const T*)nullptr, 0, 0, nullptr, (T*)nullptr, 0, HyGlu{});
+}
+// the product of one token's row that a deferred update makes (true), or the update alone
+template <typename T>
+static bool hy_pre_gemm(gl3_ctx* ctx, const T* A, const HyMat& w, int M, float* C, bool glu, T* act, int ld_act, const HyGlu& gp) {
+    gl3_hybrid_state* h = ctx->hy;
+    constexpr int PE = 16 / (int)sizeof(T);
+    if (M != 1 || (const void*)A != h->pre.h_out || w.k != h->pre.W || w.ld % PE || ((uintptr_t)w.w & 15) || gp.mul_table) { hy_pre_flush<T>(ctx); return false; }
+    h->pre_on = false;
+    if (glu) hy_pre_launch<T, HY_EPI_GLU>(ctx, h->pre, h->pre_streams, (const T*)w.w, w.ld, w.rows, nullptr, act, ld_act, gp);
+    else if (gp.act == 2) hy_pre_launch<T, HY_EPI_ACTMUL>(ctx, h->pre, h->pre_streams, (const T*)w.w, w.ld, w.rows, nullptr, act, ld_act, gp);
+    else hy_pre_launch<T, HY_EPI_STORE>(ctx, h->pre, h->pre_streams, (const T*)w.w, w.ld, w.rows, C, (T*)nullptr, 0, gp);
+    return true;
+}
+
 // parts != null: C has room for HY_KSPLIT copies and the caller sums them (the streams kernel does); *parts = copies written
 template <typename T>
 static void hy_gemm(gl3_ctx* ctx, const T* A, int lda, const HyMat& w, int M, float* C, int ldc, bool glu, T* act, int ld_act, HyGlu gp, int* parts = nullptr, int max_parts = HY_KSPLIT) {
     if (parts) *parts = 1;
+    if (ctx->hy->pre_on && hy_pre_gemm<T>(ctx, A, w, M, C, glu, act, ld_act, gp)) return;
     const T* Wt = (const T*)w.w;
     const int N = w.rows, K = w.k;
     hipStream_t st = ctx->stream;
@@ -1779,6 +1813,7 @@ static int32_t hy_portion_plain(gl3_ctx* ctx, int seq, const int32_t* tokens, in
     const int W = h->W, nl = (int)h->L.size();
     const size_t lstride = (size_t)h->mb * W;
     const float eps = ctx->d.rms_eps;
+    h->pre_on = false;          // (a call that failed may have left one)
     memcpy(h->h_tokens, tokens, (size_t)n * 4);
     if (nw > 0) memcpy(h->h_want, want, (size_t)nw * 4);
     h->h_dyn[0] = pos0; h->h_dyn[1] = seq; h->h_dyn[2] = h->last_tok[seq];
@@ -1794,7 +1829,17 @@ static int32_t hy_portion_plain(gl3_ctx* ctx, int seq, const int32_t* tokens, in
         hipLaunchKernelGGL((hy_embed_kernel<T>), dim3(n, hy_cdiv(W, n <= 32 ? 256 : 1024)), dim3(256), 0, st, host, h->dyn, 4 + h->want_cap, nw, (const T*)h->emb.w, h->X, W, 1, lstride, h->emb_scale,
                            h->depth ? h->hist : nullptr, bg);
     const bool single = n == 1 && nw == 1 && h->L[nl - 1].d.identity == 0;          // its last update makes the final norm (identity choices read their input where that goes)
+    // One token: an update of sums and norms alone waits for the product that reads its norm, and the residual moves from one buffer to the other
+    float* x2 = h->X2;
+    const bool may_defer = n == 1 && (single || nw == 0) && !h->taps && !h->depth && !h->shift && h->side_dim == 0 && !h->no_pre && W % 8 == 0 && W <= 4096;
     HyResid base{};
+    auto defer = [&](HyResid& r, T* out) {
+        if (!may_defer || !r.norm_w || !r.ya || r.gate_z || r.bw1 || r.eo || r.lw || r.yc) return false;
+        h->pre = HyPre{base.x, (size_t)W, x2, (size_t)W, W, r.ya, r.ya_parts, r.ya_stride, r.ya_mul, r.post_w, nullptr, nullptr, nullptr, r.norm_w, eps, out};
+        h->pre_on = true; h->pre_streams = 1;
+        std::swap(base.x, x2);
+        return true;
+    };
     base.x = h->X; base.W = W; base.eps = eps; base.ya_parts = 1; base.ya_mul = 1.f;
     // a residual update that ends in the norm in front of layer l's mixer (l = nl: the last layer has run, no norm), with the token shift
     auto resid_to_mixer = [&](HyResid r, int l) {
@@ -1805,6 +1850,7 @@ static int32_t hy_portion_plain(gl3_ctx* ctx, int seq, const int32_t* tokens, in
             else if (h->shift) r.hf = h->hf;
         }
         else if (single) r.norm_w = h->final_norm;
+        if (defer(r, l == nl && single ? (T*)h->xw : hb)) return;
         hy_resid<T>(ctx, n, r, h->no_pre ? hb : (T*)nullptr, l == nl && single ? (T*)h->xw : hb);
         if (l < nl && r.hf) {
             float* prev = h->slots + h->L[l].off_shift;
@@ -1856,7 +1902,7 @@ static int32_t hy_portion_plain(gl3_ctx* ctx, int seq, const int32_t* tokens, in
             r.ya_mul = h->resid_mul;
             if (h->taps) r.tap = h->taps + (size_t)l * lstride;
             r.norm_w = !last ? h->L[l + 1].norm1 : single ? h->final_norm : nullptr;
-            hy_resid<T>(ctx, n, r, (T*)nullptr, last && single ? (T*)h->xw : hb);
+            if (!defer(r, last && single ? (T*)h->xw : hb)) hy_resid<T>(ctx, n, r, (T*)nullptr, last && single ? (T*)h->xw : hb);
             continue;
         }
         if (L.d.out_norm) { r.bw1 = L.branch_norm; r.bw2 = L.side->branch_norm; r.ya_first = h->y_first; }
@@ -1864,7 +1910,7 @@ static int32_t hy_portion_plain(gl3_ctx* ctx, int seq, const int32_t* tokens, in
         r.lw = L.ls1;                 // null without layer scales
         if (L.d.ff > 0) {
             r.norm_w = L.norm2;
-            hy_resid<T>(ctx, n, r, h->no_pre ? hb : (T*)nullptr, hb);
+            if (!defer(r, hb)) hy_resid<T>(ctx, n, r, h->no_pre ? hb : (T*)nullptr, hb);
             r = base;
             r.post_w = L.norm2b;
             r.lw = L.ls2;
@@ -1887,6 +1933,7 @@ static int32_t hy_portion_plain(gl3_ctx* ctx, int seq, const int32_t* tokens, in
         finish(r);
     }
     if (nw > 0) hy_logits<T>(ctx, nw, single);
+    hy_pre_flush<T>(ctx);
     HY_HIP(hipGetLastError());
     return GL3_OK;
 }
@@ -1899,6 +1946,7 @@ static int32_t hy_portion(gl3_ctx* ctx, int seq, const int32_t* tokens, int n, i
     const int W = h->W, S = h->S;
     const size_t sstride = (size_t)h->mb * W;
     const float eps = ctx->d.rms_eps;
+    h->pre_on = false;          // (a call that failed may have left one)
     memcpy(h->h_tokens, tokens, (size_t)n * 4);
     if (nw > 0) memcpy(h->h_want, want, (size_t)nw * 4);
     h->h_dyn[0] = pos0; h->h_dyn[1] = seq;
@@ -1909,6 +1957,16 @@ static int32_t hy_portion(gl3_ctx* ctx, int seq, const int32_t* tokens, int n, i
     hipLaunchKernelGGL((hy_embed_norm_kernel<T>), dim3(n), dim3(1024), 0, st, host, h->dyn, 4 + h->want_cap, nw, (const T*)h->emb.w, h->X, W, S, sstride, h->emb_scale, (float*)nullptr, HyBigram{},
                        h->L[0].hc[0][0], h->L[0].norm1, eps, hb);
     const bool single = n == 1 && nw == 1;          // its last update makes the final norm
+    // One token: the updates wait for the product that reads their norm, and the residual moves from one buffer to the other.  (Rows of up to 4096: four columns a thread.)
+    float *x = h->X, *x2 = h->X2;
+    size_t xs = sstride, xs2 = W;
+    const bool defer = n == 1 && !h->taps && W % 8 == 0 && W <= 4096 && (S == 1 || S == 2 || S == 4);
+    auto update = [&](const float* mix, const float* po, const float* nin, const float* norm, T* out, float* tap) {
+        if (!defer || !nin) { hy_streams<T>(ctx, n, x, W, S, xs, h->y, h->y_parts, (size_t)n * W, mix, po, nin, norm, eps, out, tap, (const int*)nullptr); return; }
+        h->pre = HyPre{x, xs, x2, xs2, W, h->y, h->y_parts, (size_t)W, 1.f, nullptr, mix, po, nin, norm, eps, out};
+        h->pre_on = true; h->pre_streams = S;
+        std::swap(x, x2); std::swap(xs, xs2);
+    };
     for (int l = 0; l < nl; ++l) {
         HyLayer& L = h->L[l];
         int32_t r = hy_mixer<T>(ctx, L, n, pos0, seq);
@@ -1917,8 +1975,7 @@ static int32_t hy_portion(gl3_ctx* ctx, int seq, const int32_t* tokens, int n, i
         {   // write-back of the mixer sublayer + read of the next sublayer
             const float* nin = ff ? L.hc[1][0] : !last ? h->L[l + 1].hc[0][0] : single ? h->ones : nullptr;
             const float* nw_ = ff ? L.norm2 : !last ? h->L[l + 1].norm1 : h->final_norm;
-            hy_streams<T>(ctx, n, h->X, W, S, sstride, h->y, h->y_parts, (size_t)n * W, L.hc[0][2], L.hc[0][1], nin, nw_, eps, !ff && last ? (T*)h->xw : hb,
-                               (!ff && h->taps) ? h->taps + (size_t)l * sstride : nullptr, (const int*)nullptr);
+            update(L.hc[0][2], L.hc[0][1], nin, nw_, !ff && last ? (T*)h->xw : hb, (!ff && h->taps) ? h->taps + (size_t)l * sstride : nullptr);
         }
         if (ff) {
             T* act = (T*)h->mixo;
@@ -1926,11 +1983,11 @@ static int32_t hy_portion(gl3_ctx* ctx, int seq, const int32_t* tokens, int n, i
             hy_gemm<T>(ctx, act, L.ff_pad, L.down, n, h->y, W, false, nullptr, 0, HyGlu{}, &h->y_parts);
             const float* nin = !last ? h->L[l + 1].hc[0][0] : single ? h->ones : nullptr;
             const float* nw_ = !last ? h->L[l + 1].norm1 : h->final_norm;
-            hy_streams<T>(ctx, n, h->X, W, S, sstride, h->y, h->y_parts, (size_t)n * W, L.hc[1][2], L.hc[1][1], nin, nw_, eps, last ? (T*)h->xw : hb,
-                               h->taps ? h->taps + (size_t)l * sstride : nullptr, (const int*)nullptr);
+            update(L.hc[1][2], L.hc[1][1], nin, nw_, last ? (T*)h->xw : hb, h->taps ? h->taps + (size_t)l * sstride : nullptr);
         }
     }
     if (nw > 0) hy_logits<T>(ctx, nw, single);
+    hy_pre_flush<T>(ctx);
     HY_HIP(hipGetLastError());
     return GL3_OK;
 }

@@ -1,0 +1,72 @@
+"""Single tokens whose residual updates and norms the next product makes (csrc/gl3_hy_pre_kernels.h): widths around what a wavefront's places and a workgroup's threads cover (8 ... 4096, and 4104,
+which keeps the launch of its own), rows that leave pairs and wavefronts over, four wavefronts a pair and one, one, two and four streams, post norms, gates, squared ReLU,
+capped logits, and a step that hands no logits out between two that do.
+
+Yardstick: the same steps in a plan with layer taps, whose updates stay launches of their own, and the designs' float64 restatements.  Bound: float32 sums of K terms in another
+order, some 1e-6 of the logits' root mean square; bfloat16 plans round rows that differ so far apart now and then, 2^-9 of an operand."""
+import numpy as np
+import pytest
+
+import __graft_entry__ as ge
+import test_kosusun_gpu as K
+import test_kugadra_gpu as U
+import test_noditar_gpu as N
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def hy():
+    from importlib import import_module
+    ge.load_package()
+    return import_module(ge.PKG_NAME + ".hybrid")
+
+
+def noditar(width, vocab, streams=2, ff=72):
+    return N, N.config([N.att(heads=4, kv_heads=2, dim=16, vdim=16, ff=ff), N.ssm(heads=2, vdim=16, state=16), N.lat(heads=2, dim=16, vdim=16, kv_rank=32, ff=ff)], width=width, vocab=vocab, streams=streams)
+
+
+def kosusun(width, vocab, ff=56):
+    return K, K.config([K.par(ff=ff), K.mls(heads=2, dim=16, vdim=16, ff=ff)], width=width, vocab=vocab)
+
+
+def kugadra(width, vocab, ff=56):
+    return U, U.config([U.lig(heads=2, dim=16, vdim=16, mlp=U.dense(ff)), U.lat(mlp=U.moe())], width=width, vocab=vocab)
+
+
+CASES = [(noditar, 8, 3, 1, 40), (noditar, 104, 211, 2, 72), (noditar, 264, 2051, 4, 2050), (noditar, 2048, 2047, 1, 8200), (noditar, 4096, 1025, 2, 300), (noditar, 4104, 257, 2, 72),
+         (kosusun, 88, 131, None, 56), (kosusun, 520, 4099, None, 8200), (kosusun, 2056, 515, None, 1030), (kugadra, 96, 131, None, 56), (kugadra, 1032, 2055, None, 4100), (kugadra, 4096, 259, None, 96)]
+
+
+@pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
+@pytest.mark.parametrize("make,width,vocab,streams,ff", CASES)
+def test_same_as_updates_of_their_own(hy, tmp_path, make, width, vocab, streams, ff, dtype):
+    mod, cfg = make(width, vocab, streams, ff) if streams else make(width, vocab, ff)
+    m = mod.Model(hy, tmp_path, cfg, seed=width % 97 + 1)
+    toks = np.random.default_rng(width).integers(0, vocab, 12).astype(np.int32)
+    out = []
+    for taps in (False, True):
+        p = m.plan(dtype, ctx=32, max_batch=16, layer_taps=taps)
+        s = p.acquire()
+        rows = [p.step(s, toks[:3], 0, want=[2])]
+        for i in range(3, 12):
+            r = p.step(s, toks[i:i + 1], i, want=[] if i == 6 else [0])
+            if i != 6:
+                rows.append(r)
+        out.append(np.concatenate(rows).astype(np.float64))
+        p.close()
+    got, own = out
+    scale = np.sqrt((own ** 2).mean())
+    assert np.sqrt(((got - own) ** 2).mean()) < (4e-6 if dtype == "float32" else 2e-2) * scale
+    assert np.abs(got - own).max() < (4e-5 if dtype == "float32" else 2e-1) * scale
+
+
+def test_against_the_restatement(hy, tmp_path):
+    cfg = N.config([N.att(ff=72), N.ssm(), N.lat(ff=72)], width=136, vocab=211, streams=4)
+    m = N.Model(hy, tmp_path, cfg, seed=3)
+    toks = N.tokens_for(cfg, 14)
+    p = m.plan("float32", ctx=32, max_batch=16)
+    s = p.acquire()
+    got = np.concatenate([p.step(s, toks[i:i + 1], i, want=[0]) for i in range(14)])
+    p.close()
+    assert N.err(got, m.ref(toks)) < 2e-5
