@@ -1,24 +1,27 @@
 // gl3_hy_attn_mfma.h — the attention core of the layer-list family for portions of many tokens, its products on the matrix cores
-// (v_mfma_f32_32x32x2_f32: float32 products and sums, the precision hy_attn_kernel has on the vector units).
+// (many tokens: float32 operands as three bfloat16 planes, the products of at least 2^-16 on v_mfma_f32_32x32x16_bf16, see gl3_hy_gemm.h; a few: v_mfma_f32_32x32x2_f32).
 //
 // Workgroup = (32 rows of a key / value head, key split): rows are (token, head of the group) pairs, token-major, as in hy_attn_kernel; its four
 // wavefronts deal the key tiles of 32 out between them and join their sums in LDS at the end, so that 512 tokens x 32 heads are 512
 // workgroups and no wavefront waits for another inside the key loop.  Both products are taken transposed, keys x rows and value columns x
 // rows: a lane then holds ONE query row in all of them, the running maximum and sum are its own registers (one exchange with
-// lane ^ 32 per tile), and the scores' accumulators ARE the second product's operand (register r of a lane is key 8 (r / 4) +
-// 4 (lane / 32) + r % 4, which is the pair of keys MFMA r takes from the half-waves) — nothing is transposed through LDS.
-// Keys and values come straight from the cache (each wavefront its own tile): a lane reads its key row 16 bytes at a time (element 8 c + 4 (lane / 32)
-// + e is step e of chunk c) and DVT consecutive value columns of the keys r (value column DVT m + i is row m of tile i); the values travel under the first product
+// lane ^ 32 per tile), and the scores' accumulators ARE the second product's operand: register r of a lane is key 8 (r / 4) + 4 (lane / 32) + r % 4, so a half-wave's
+// registers 0 - 7 and 8 - 15 are its eight keys of two MFMA steps, in the order in which it holds the values — nothing is transposed through LDS.
+// Keys and values come straight from the cache (each wavefront its own tile): a lane reads its key row 32 bytes at a time (elements 16 c + 8 (lane / 32) .. + 7 of chunk c)
+// and DVT consecutive value columns of the keys r (value column DVT m + i is row m of tile i); the values travel under the first product
 // and the softmax, the next tile's keys under the second half of the second product (all at once do not fit 256 registers, and a second wavefront
-// per SIMD is what keeps the matrix cores busy during the softmax).  Queries (scaled) stay in LDS, rows dk + 4 floats apart.
+// per SIMD is what covers the waits).  Queries (scaled) stay in LDS as planes; a step's MFMAs stand between the splits of the next step's keys or values, which the vector units
+// make under them.  One chain of scores: a second one was 16 registers spilled and 14 % of the kernel.
 // A value that is not finite must stay with the rows that see its key, and the second product carries it to every row of the tile (p = 0 times infinity).  Nothing in the
 // loops below looks for one (values cleaned in the tiles with unseen keys cost 1 and 5 % of the two kernels, right in front of every MFMA 6 - 12 %): sums that hold a
 // not-a-number at the end are made once more, key by key on the vector units (hy_attn_again), which costs other inputs the look at the sums: 1 % of the kernel of
-// many tokens, of that of few 2 % with 64 and 256 entries and 7 % with 512.  It stands behind the last exchange in LDS, which the loop's last MFMAs run under.
-// Bound: 153 TFLOP/s of float32 MFMAs.  Measured against hy_attn_kernel (8 key / value heads x 4, head size 128, us):
-//   512 tokens at position 0 131 -> 45, four such portions of 2041 tokens 1795 -> 428 in all.
+// many tokens, of that of few 2 % with 64 and 256 entries and 7 % with 512.  It stands behind the last exchange in LDS, which the loop's last MFMAs run under.  An infinite key
+// or query entry has no planes: scores that are not numbers are made again in float32 (hy_score_again).
+// What bounds it: at position 0 a wavefront has two tiles on average and waits for memory half of its time (queries, first keys and the gate are asked for as early as they are
+// known); behind many positions the splits (11 vector instructions per pair of values).  8 key / value heads x 4, head size 128 (us): 512 tokens at position 0 131 (hy_attn_kernel) -> 52
+// (float32 MFMAs) -> 42, four such portions of 2041 tokens 1795 -> 458 -> 355 in all.
 #pragma once
-#include "gl3_hy_kernels.h"
+#include "gl3_hy_gemm.h"
 
 typedef float hy_acc4 __attribute__((ext_vector_type(4)));
 template <int DVT> struct HyVec;
@@ -68,28 +71,41 @@ __device__ __forceinline__ void hy_attn_again(hy_v16f* o, const HyAttnArgs& a, c
     }
 }
 
+// A score in float32 throughout: a key's or query's infinity has no planes (rare).
+__device__ __attribute__((noinline)) float hy_score_again(const float* __restrict__ k, const float* __restrict__ q, float scale, int n) {
+    float s = 0.f;
+#pragma unroll 1
+    for (int d = 0; d < n; ++d) s = fmaf(k[d], q[d] * scale, s);
+    return s;
+}
+
 template <int DKC, int DVT>          // dk = 8 DKC, dv = 32 DVT
 static __global__ __launch_bounds__(256, DKC > 16 ? 1 : 2) void hy_attn_mfma_kernel(HyAttnArgs a) {
-    constexpr int DK = 8 * DKC, DV = 32 * DVT, QS = DK + 4, OS = DV + 4;
+    constexpr int DK = 8 * DKC, DV = 32 * DVT, CH = DK / 16, QB = 6 * DK + 16, OS = DV + 4;
     typedef typename HyVec<DVT>::V VV;
-    __shared__ __attribute__((aligned(16))) float sQ[32 * QS];
+    __shared__ __attribute__((aligned(16))) uint8_t sQ[32 * QB];          // a row: its three planes
     __shared__ __attribute__((aligned(16))) float sO[32 * OS];
     __shared__ float sml[4][2][32];
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), r32 = lane & 31, kh = lane >> 5;
     // the LAST row block first: late tokens see the most keys
     const int g = blockIdx.x % a.G, rb = (int)(gridDim.x / a.G) - 1 - (int)(blockIdx.x / a.G), split = blockIdx.z, hpg = a.H / a.G;
-    const int rows = a.n * hpg, row0 = rb * 32, pos0 = a.dyn[0];
+    const int rows = a.n * hpg, row0 = rb * 32;
+    // queries, then the first keys: both are on their way before the first is waited for
+    constexpr int QI = (32 * (DK / 8) + 255) / 256;
+    hy_v4f qs[QI][2];
+#pragma unroll
+    for (int u = 0; u < QI; ++u) {
+        const int i = min(tid + 256 * u, 32 * (DK / 8) - 1), p = min(row0 + i / (DK / 8), rows - 1);          // (a row that is not there repeats the last one: its results are not stored)
+        const float* src = a.q + (size_t)(p / hpg) * a.ldq + (size_t)(g * hpg + p % hpg) * DK + 8 * (i % (DK / 8));
+        qs[u][0] = *reinterpret_cast<const hy_v4f*>(src);
+        qs[u][1] = *reinterpret_cast<const hy_v4f*>(src + 4);
+    }
+    const int pos0 = a.dyn[0];
     const int minpos = pos0 + row0 / hpg, maxpos = pos0 + min(rows - 1, row0 + 31) / hpg;
     const int rho = row0 + r32, pr = rho < rows ? pos0 + rho / hpg : -1;          // this lane's row: position (-1: no such row), head
     const int hr = g * hpg + (rho < rows ? rho % hpg : 0);
     const float slope = a.slope_log2 != 0.f ? exp2f(-a.slope_log2 * (float)(hr + 1) / (float)a.H) : 0.f;
-    for (int i = tid; i < 32 * (DK / 4); i += 256) {
-        const int r = i / (DK / 4), c = i % (DK / 4), p = row0 + r;
-        float4 v = make_float4(0.f, 0.f, 0.f, 0.f);
-        if (p < rows) v = *reinterpret_cast<const float4*>(a.q + (size_t)(p / hpg) * a.ldq + (size_t)(g * hpg + p % hpg) * DK + 4 * c);
-        v.x *= a.scale; v.y *= a.scale; v.z *= a.scale; v.w *= a.scale;
-        *reinterpret_cast<float4*>(sQ + r * QS + 4 * c) = v;
-    }
+    const float* qrow = a.q + (size_t)(min(rho, rows - 1) / hpg) * a.ldq + (size_t)hr * DK;
     const size_t slot = (size_t)a.dyn[1] * a.slot_stride;
     const float *kc = a.kc + slot + (size_t)g * DK, *vc = a.vc + slot + (size_t)g * DV;
     const int ldk = a.G * DK, ldv = a.G * DV;
@@ -100,13 +116,13 @@ static __global__ __launch_bounds__(256, DKC > 16 ? 1 : 2) void hy_attn_mfma_ker
     const int np_t = (nb_wg + 31) >> 5, nv = np_t + nk + hi_t - lo_t + 1;
     const float *pkc = P > 0 ? a.pk + slot + (size_t)g * DK : kc, *pvc = P > 0 ? a.pv + slot + (size_t)g * DV : vc;
     auto first_key = [&](int vt) { const int w = vt - np_t; return (vt < np_t ? vt : w < nk ? w : lo_t + w - nk) << 5; };
-    float4 kr[DKC];
+    hy_v4f kr[CH][2];          // elements 16 c + 8 (lane / 32) .. + 7 of key lane % 32
     auto load_keys = [&](int vt) {          // (rows past the last one repeat it: masked)
         const bool pooled = vt < np_t;
         const char* p = (const char*)(pooled ? pkc : kc);          // uniform base + 32-bit byte offset
-        const uint32_t off = ((uint32_t)min(first_key(vt) + r32, pooled ? nb_wg - 1 : maxpos) * (uint32_t)ldk + 4 * kh) * 4;
+        const uint32_t off = ((uint32_t)min(first_key(vt) + r32, pooled ? nb_wg - 1 : maxpos) * (uint32_t)ldk + 8 * kh) * 4;
 #pragma unroll
-        for (int c = 0; c < DKC; ++c) kr[c] = *reinterpret_cast<const float4*>(p + off + 32 * c);
+        for (int c = 0; c < CH; ++c) { kr[c][0] = *reinterpret_cast<const hy_v4f*>(p + off + 64 * c); kr[c][1] = *reinterpret_cast<const hy_v4f*>(p + off + 64 * c + 16); }
     };
     hy_v16f o[DVT];
 #pragma unroll
@@ -116,7 +132,22 @@ static __global__ __launch_bounds__(256, DKC > 16 ? 1 : 2) void hy_attn_mfma_ker
     float m = -INFINITY, l = 0.f;
     int vt = split * 4 + wave;
     if (vt < nv) load_keys(vt);
+#pragma unroll
+    for (int u = 0; u < QI; ++u) {
+        const int i = tid + 256 * u, r = i / (DK / 8), c = i % (DK / 8);
+        if (i >= 32 * (DK / 8)) continue;
+        qs[u][0] *= a.scale; qs[u][1] *= a.scale;
+#pragma unroll
+        for (int pl = 0; pl < 3; ++pl) {
+            hy_v4u d;
+#pragma unroll
+            for (int e = 0; e < 4; ++e) d[e] = hy_plane<true>(*((float*)&qs[u][e / 2] + e % 2 * 2), *((float*)&qs[u][e / 2] + e % 2 * 2 + 1));
+            *reinterpret_cast<hy_v4u*>(sQ + r * QB + pl * 2 * DK + 16 * c) = d;
+        }
+    }
     __syncthreads();
+    // product q of a step: planes PA and PB, the small ones first (those of less than 2^-16 are left out); a step's MFMAs stand between the splits of the next one's operand
+    constexpr int PA[6] = {2, 1, 0, 1, 0, 0}, PB[6] = {0, 1, 2, 0, 1, 0};
     for (; vt < nv; vt += 4 * a.nsplit) {
         const bool pooled = vt < np_t;
         const int j0 = first_key(vt), last = pooled ? nb_wg - 1 : maxpos;
@@ -128,29 +159,52 @@ static __global__ __launch_bounds__(256, DKC > 16 ? 1 : 2) void hy_attn_mfma_ker
         };
         load_values(0);
         __builtin_amdgcn_sched_barrier(0);
-        hy_v16f s0, s1;          // two chains of sums
+        hy_v16f s0;
 #pragma unroll
-        for (int r = 0; r < 16; ++r) s0[r] = s1[r] = 0.f;
-        const float* qp = sQ + r32 * QS + 4 * kh;
+        for (int r = 0; r < 16; ++r) s0[r] = 0.f;
+        {
+            hy_v4u ka[2][3];
+            hy_v8bf qv[2][3];
+            auto cut = [&](auto uc, auto cc) {          // step u of chunk c's split
+                constexpr int u = decltype(uc)::value, c = decltype(cc)::value, e = u % 4;
+                ka[c & 1][u / 4][e] = hy_plane<(u < 8)>(*((float*)&kr[c][e / 2] + e % 2 * 2), *((float*)&kr[c][e / 2] + e % 2 * 2 + 1));
+            };
+            auto rq = [&](auto cc) {
+                constexpr int c = decltype(cc)::value;
 #pragma unroll
-        for (int c = 0; c < DKC; ++c) {
-            const float4 q = *reinterpret_cast<const float4*>(qp + 8 * c);
-            s0 = __builtin_amdgcn_mfma_f32_32x32x2f32(kr[c].x, q.x, s0, 0, 0, 0);
-            s1 = __builtin_amdgcn_mfma_f32_32x32x2f32(kr[c].y, q.y, s1, 0, 0, 0);
-            s0 = __builtin_amdgcn_mfma_f32_32x32x2f32(kr[c].z, q.z, s0, 0, 0, 0);
-            s1 = __builtin_amdgcn_mfma_f32_32x32x2f32(kr[c].w, q.w, s1, 0, 0, 0);
+                for (int pl = 0; pl < 3; ++pl) qv[c & 1][pl] = *reinterpret_cast<const hy_v8bf*>(sQ + r32 * QB + pl * 2 * DK + 32 * c + 16 * kh);
+            };
+            rq(std::integral_constant<int, 0>{});
+            hy_static_for<0, 12>([&](auto u) { cut(u, std::integral_constant<int, 0>{}); });
+            __builtin_amdgcn_sched_barrier(0);
+            hy_static_for<0, CH>([&](auto cc) {
+                constexpr int c = decltype(cc)::value;
+                constexpr std::integral_constant<int, c + 1 < CH ? c + 1 : c> nx{};
+                if constexpr (c + 1 < CH) rq(nx);
+                hy_static_for<0, 6>([&](auto qc) {
+                    constexpr int q = decltype(qc)::value;
+                    hy_mma(s0, __builtin_bit_cast(hy_v8bf, ka[c & 1][PA[q]]), qv[c & 1][PB[q]]);
+                    if constexpr (c + 1 < CH) hy_static_for<2 * q, 2 * q + 2>([&](auto u) { cut(u, nx); });
+                    __builtin_amdgcn_sched_barrier(0);
+                });
+            });
         }
-        __builtin_amdgcn_sched_group_barrier(0x100, 2, 0);          // two query chunks ahead of their MFMAs
-#pragma unroll
-        for (int c = 0; c < DKC; ++c) { __builtin_amdgcn_sched_group_barrier(0x8, 4, 0); if (c + 2 < DKC) __builtin_amdgcn_sched_group_barrier(0x100, 1, 0); }
-        __builtin_amdgcn_sched_barrier(0);
         load_values(8);
         __builtin_amdgcn_sched_barrier(0);
-        float p[16], mx = m;
+        float p[16], mx = m, bad = 0.f;
+#pragma unroll
+        for (int r = 0; r < 16; ++r) { p[r] = s0[r]; bad += p[r]; }
+        if (__builtin_expect(__any(bad != bad), 0)) {
+#pragma unroll
+            for (int r = 0; r < 16; ++r) {
+                const int j = j0 + 8 * (r >> 2) + 4 * kh + (r & 3);
+                if (p[r] != p[r] && j <= last) p[r] = hy_score_again((pooled ? pkc : kc) + (size_t)j * ldk, qrow, a.scale, DK);
+            }
+        }
 #pragma unroll
         for (int r = 0; r < 16; ++r) {
             const int j = j0 + 8 * (r >> 2) + 4 * kh + (r & 3);
-            const float s = s0[r] + s1[r];
+            const float s = p[r];
             if (pooled) p[r] = j < nbr ? s : -INFINITY;
             else p[r] = (j <= pr && (pr - j < win || j < a.keep)) ? s - slope * (float)(pr - j) : -INFINITY;
             mx = fmaxf(mx, p[r]);
@@ -163,28 +217,46 @@ static __global__ __launch_bounds__(256, DKC > 16 ? 1 : 2) void hy_attn_mfma_ker
         for (int r = 0; r < 16; ++r) { p[r] = any ? expf(p[r] - mx) : 0.f; ls += p[r]; }
         l = l * corr + ls;
         m = mx;
+        hy_v4u pp[2][3], va[2][3];          // weights of keys 0 .. 7 and 8 .. 15 of the lane, a value tile's column
+#pragma unroll
+        for (int h = 0; h < 2; ++h)
+#pragma unroll
+            for (int u = 0; u < 12; ++u) pp[h][u / 4][u % 4] = u < 8 ? hy_plane<true>(p[8 * h + 2 * (u % 4)], p[8 * h + 2 * (u % 4) + 1]) : hy_plane<false>(p[8 * h + 2 * (u % 4)], p[8 * h + 2 * (u % 4) + 1]);
+        auto cut = [&](auto uc, auto tc) {          // step u of item t = (half, value tile)
+            constexpr int u = decltype(uc)::value, t = decltype(tc)::value, i = t % DVT, r = 8 * (t / DVT) + 2 * (u % 4);
+            va[t & 1][u / 4][u % 4] = hy_plane<(u < 8)>(*((float*)&vr[r] + i), *((float*)&vr[r + 1] + i));
+        };
+        hy_static_for<0, 12>([&](auto u) { cut(u, std::integral_constant<int, 0>{}); });
 #pragma unroll
         for (int i = 0; i < DVT; ++i)
 #pragma unroll
             for (int r = 0; r < 16; ++r) o[i][r] *= corr;
-        auto add_values = [&](int r0) {
-#pragma unroll
-            for (int r = r0; r < r0 + 8; ++r) {
-                o[0] = __builtin_amdgcn_mfma_f32_32x32x2f32(vr[r].x, p[r], o[0], 0, 0, 0);
-                o[1] = __builtin_amdgcn_mfma_f32_32x32x2f32(vr[r].y, p[r], o[1], 0, 0, 0);
-                if constexpr (DVT == 4) {
-                    o[2] = __builtin_amdgcn_mfma_f32_32x32x2f32(vr[r].z, p[r], o[2], 0, 0, 0);
-                    o[3] = __builtin_amdgcn_mfma_f32_32x32x2f32(vr[r].w, p[r], o[3], 0, 0, 0);
-                }
+        __builtin_amdgcn_sched_barrier(0);
+        hy_static_for<0, 2 * DVT>([&](auto tc) {
+            constexpr int t = decltype(tc)::value;
+            constexpr std::integral_constant<int, t + 1 < 2 * DVT ? t + 1 : t> nx{};
+            if constexpr (t == DVT) {
+                if (vt + 4 * a.nsplit < nv) load_keys(vt + 4 * a.nsplit);
+                __builtin_amdgcn_sched_barrier(0);
             }
-        };
-        add_values(0);
-        __builtin_amdgcn_sched_barrier(0);
-        if (vt + 4 * a.nsplit < nv) load_keys(vt + 4 * a.nsplit);
-        __builtin_amdgcn_sched_barrier(0);
-        add_values(8);
-        __builtin_amdgcn_sched_barrier(0);
+            hy_static_for<0, 6>([&](auto qc) {
+                constexpr int q = decltype(qc)::value;
+                hy_mma(o[t % DVT], __builtin_bit_cast(hy_v8bf, va[t & 1][PA[q]]), __builtin_bit_cast(hy_v8bf, pp[t / DVT][PB[q]]));
+                if constexpr (t + 1 < 2 * DVT) hy_static_for<2 * q, 2 * q + 2>([&](auto u) { cut(u, nx); });
+                __builtin_amdgcn_sched_barrier(0);
+            });
+        });
     }
+    // the gate's values travel while the wavefronts join
+    constexpr int GI = 32 * (DV / 4) / 256;
+    float4 gz[GI];
+    const bool gated = a.out && a.gate && a.gate_mode != 2;
+    if (gated)
+#pragma unroll
+        for (int u = 0; u < GI; ++u) {
+            const int i = tid + 256 * u, q = min(row0 + i / (DV / 4), rows - 1), c = i % (DV / 4);
+            gz[u] = *reinterpret_cast<const float4*>(a.gate + (size_t)(q / hpg) * a.ldg + (g * hpg + q % hpg) * DV + 4 * c);
+        }
     // join the wavefronts: every lane scales by e^(m - M), the wavefronts add up in LDS one after the other
     l += __shfl_xor(l, 32, 64);
     if (kh == 0) { sml[wave][0][r32] = m; sml[wave][1][r32] = l; }
@@ -192,7 +264,7 @@ static __global__ __launch_bounds__(256, DKC > 16 ? 1 : 2) void hy_attn_mfma_ker
     const float M = fmaxf(fmaxf(sml[0][0][r32], sml[1][0][r32]), fmaxf(sml[2][0][r32], sml[3][0][r32]));
     const float sc = m > -INFINITY ? expf(m - M) : 0.f;
     if (__builtin_expect(__any(hy_attn_nan<DVT>(o) && pr >= 0), 0))
-        hy_attn_again<DK, DVT>(o, a, sQ + r32 * QS, 1.f, m, slope, pr, nbr, win, kc, vc, pkc, pvc, 0, kh, split * 4 + wave, 4 * a.nsplit, nv,
+        hy_attn_again<DK, DVT>(o, a, qrow, a.scale, m, slope, pr, nbr, win, kc, vc, pkc, pvc, 0, kh, split * 4 + wave, 4 * a.nsplit, nv,
                                [&](int t, int& j, int& last, bool& pooled) { pooled = t < np_t; j = first_key(t); last = pooled ? nb_wg - 1 : maxpos; });
     for (int w = 0; w < 4; ++w) {
         if (wave == w) {
@@ -220,8 +292,9 @@ static __global__ __launch_bounds__(256, DKC > 16 ? 1 : 2) void hy_attn_mfma_ker
             sF[tid][1] = e * L + (a.sink ? expf(z - top) : 0.f);
         }
         __syncthreads();
-        for (int i = tid; i < 32 * (DV / 4); i += 256) {
-            const int r = i / (DV / 4), c = i % (DV / 4), q = row0 + r;
+#pragma unroll
+        for (int u = 0; u < GI; ++u) {
+            const int i = tid + 256 * u, r = i / (DV / 4), c = i % (DV / 4), q = row0 + r;
             if (q >= rows) continue;
             const int t = q / hpg, h = g * hpg + q % hpg;
             const float4 v4 = *reinterpret_cast<const float4*>(sO + r * OS + 4 * c);
@@ -232,7 +305,7 @@ static __global__ __launch_bounds__(256, DKC > 16 ? 1 : 2) void hy_attn_mfma_ker
 #pragma unroll
                 for (int k = 0; k < 4; ++k) v[k] *= s;
             } else if (a.gate) {
-                const float4 z = *reinterpret_cast<const float4*>(a.gate + (size_t)t * a.ldg + h * DV + 4 * c);
+                const float4 z = gz[u];
                 v[0] *= hy_sigmoid(z.x); v[1] *= hy_sigmoid(z.y); v[2] *= hy_sigmoid(z.z); v[3] *= hy_sigmoid(z.w);
             }
 #pragma unroll

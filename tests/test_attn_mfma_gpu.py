@@ -174,3 +174,30 @@ def test_few_rows_of_many_tiles(hy, tmp_path, heads, kv_heads):
         pos += k
     p.close()
     assert N.err(np.concatenate(got), m.ref(toks)[fill:]) < 2e-5
+
+
+@pytest.mark.parametrize("size", [64, 128])
+def test_infinite_key_entries(hy, tmp_path, size):
+    """Three tokens whose keys hold an infinity (a latent entry that only they have, past the largest float when expanded): a row with a score of plus infinity is not a number, one
+    with minus infinity leaves the key out.  One portion against portions of 16, whose kernel multiplies in float32."""
+    def tweak(w):
+        w["embed"][:, 0], w["embed"][3, 0], w["embed"][4, 0] = 0.0, 30.0, -30.0
+        w["l0.mix.dkv"][5] = 0.0
+        w["l0.mix.dkv"][5, 0] = 1.0
+        w["l0.mix.uk"][:, 5] = 0.0
+        w["l0.mix.uk"][7, 5] = 3e38
+        w["l0.mix.uv"][:, 5] = 0.0
+    cfg = N.config([N.lat(heads=1, dim=size, vdim=size, kv_rank=96, ff=0, scale=0.05)])
+    m = N.Model(hy, tmp_path, cfg, seed=size, tweak=tweak)
+    toks = N.tokens_for(cfg, 192)
+    toks[(toks == 3) | (toks == 4)] = 5
+    toks[[20, 90, 150]] = 3, 4, 3
+    out = []
+    for batch in (256, 16):
+        p = m.plan("float32", ctx=200, max_batch=batch)
+        out.append(p.step(p.acquire(), toks, 0, list(range(192))))
+        p.close()
+    whole, short = out
+    bad = np.isnan(short).any(axis=1)
+    assert 20 < bad.sum() < 180 and not bad[:20].any() and np.array_equal(np.isnan(whole).any(axis=1), bad)
+    assert np.abs(whole[~bad] - short[~bad]).max() < 1e-4 * np.sqrt((short[~bad] ** 2).mean())
