@@ -4,16 +4,35 @@
 // four to six times a token, while a product of 8 MB waits.  Here every workgroup of the product makes the whole row itself (24 - 48 KB from L2, 16 bytes a thread) under
 // the first weights it has already asked for; workgroup 0 keeps the new residual (in the other of two buffers: the others still read the old one) and the normed row for
 // later readers.  That wants few workgroups (every one reads the row): one of sixteen wavefronts per CU, pairs of weight rows dealt out over the wavefronts, the next
-// pair's pieces on their way while one is multiplied.  Few pairs a workgroup (up to four): four wavefronts share one.
+// pair's pieces on their way while one is multiplied.
+//
+// Every sum is taken in the order of the kernels it stands for (hy_streams4_kernel or hy_resid_kernel on 1024 threads, then hy_matvec_kernel), to the bit: a plan's results do
+// not depend on whether an update was deferred, and a lane's chain of products is no longer here than there.  So four wavefronts share a pair (KS = 4) where that kernel splits K:
+// up to 16384 rows of 1024 columns and more; a lane of one wavefront alone would add K / 64 products in one chain instead of K / 256, an error of 1.2e-7 instead of 0.95e-7
+// (K = 2048, float32 plans).  Both splits take the same time once the sums cross the wavefront in registers: 4608 - 12000 x 2048 in bfloat16 10.2 - 11.0 us (one wavefront a
+// pair 10.8 - 11.3), 8192 x 2048 in float32 14.9 (15.1).
 #pragma once
 #include "gl3_hybrid.h"
 #include "gl3_hy_kernels.h"
+#include "gl3_hy_heads_kernels.h"
 
-template <typename T, int S, int EPI, int KS>
+// hy_wave_sum without LDS, the same sums in the same order: lanes l ^ 32, l ^ 16, then within rows of 16, whose values repeat every 8, 4, 2 by then (a turn by as many is the exchange)
+__device__ __forceinline__ float hy_wave_sum_vec(float v) {
+    auto swap = [](uint32_t x, auto f) { const auto r = f(x); return __uint_as_float(r[0]) + __uint_as_float(r[1]); };
+    v = swap(__float_as_uint(v), [](uint32_t x) { return __builtin_amdgcn_permlane32_swap(x, x, false, false); });
+    v = swap(__float_as_uint(v), [](uint32_t x) { return __builtin_amdgcn_permlane16_swap(x, x, false, false); });
+    v += hy_dpp<0x128>(v);          // row_ror 8, 4, 2, 1
+    v += hy_dpp<0x124>(v);
+    v += hy_dpp<0x122>(v);
+    return v + hy_dpp<0x121>(v);
+}
+
+// UN: a wavefront's places of the walk that are loaded together
+template <typename T, int S, int EPI, int KS, int UN>
 static __global__ __launch_bounds__(1024) void hy_matvec_pre_kernel(HyPre p, const T* __restrict__ Wt, int ldw, int N, float* __restrict__ C, T* __restrict__ act, int ld_act, HyGlu glu) {
-    constexpr int PE = HyPiece<T>::N, UN = KS == 1 ? 4 : 2, STEP = KS * 64 * PE;
+    constexpr int PE = HyPiece<T>::N, STEP = KS * 64 * PE;
     __shared__ __attribute__((aligned(16))) T sh[4096];
-    __shared__ float red[16], part[16][2];
+    __shared__ float red[16], part[HY_PRE_SPLIT_PAIRS * 4][2];
     const int K = p.W, tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int pairs = (N + 1) >> 1, mine = (int)blockIdx.x < pairs ? (pairs - 1 - (int)blockIdx.x) / (int)gridDim.x + 1 : 0;          // pairs blockIdx.x + i gridDim.x
     const int kp = wave % KS, slots = 16 / KS, first = wave / KS, chunks = (K + UN * STEP - 1) / (UN * STEP), todo = first < mine ? ((mine - 1 - first) / slots + 1) * chunks : 0;
@@ -50,13 +69,11 @@ static __global__ __launch_bounds__(1024) void hy_matvec_pre_kernel(HyPre p, con
             for (int i = 0; i < 4; ++i) yv[i] += q[i];
         }
     }
-#pragma unroll
-    for (int i = 0; i < 4; ++i) yv[i] *= p.y_mul;
     if (p.post_w) {
         float sd = 0.f;
         if (on)
 #pragma unroll
-            for (int i = 0; i < 4; ++i) sd += yv[i] * yv[i];
+            for (int i = 0; i < 4; ++i) { yv[i] *= p.y_mul; sd = fmaf(yv[i], yv[i], sd); }
         sd = hy_block_sum<1024>(sd, red);
         const float r = 1.f / sqrtf(sd / (float)K + p.eps);
         if (on)
@@ -71,12 +88,12 @@ static __global__ __launch_bounds__(1024) void hy_matvec_pre_kernel(HyPre p, con
         for (int u = 0; u < S; ++u)
 #pragma unroll
             for (int i = 0; i < 4; ++i) {
-                if constexpr (S == 1) nx[0][i] = p.mix ? p.mix[0] * xs[0][i] + p.po[0] * yv[i] : xs[0][i] + yv[i];
+                if (S == 1 && !p.mix) nx[0][i] = p.post_w ? xs[0][i] + yv[i] : fmaf(p.y_mul, yv[i], xs[0][i]);
                 else {
-                    float t = 0.f;
+                    float t = p.mix[u] * xs[0][i];
 #pragma unroll
-                    for (int s = 0; s < S; ++s) t += p.mix[s * S + u] * xs[s][i];
-                    nx[u][i] = t + p.po[u] * yv[i];
+                    for (int s = 1; s < S; ++s) t = fmaf(p.mix[s * S + u], xs[s][i], t);
+                    nx[u][i] = fmaf(p.po[u], yv[i], t);
                 }
             }
         if (blockIdx.x == 0)
@@ -84,10 +101,10 @@ static __global__ __launch_bounds__(1024) void hy_matvec_pre_kernel(HyPre p, con
             for (int s = 0; s < S; ++s) hy_stv<4>(p.x_out + s * p.xos + w, nx[s]);
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
-            h[i] = 0.f;
+            h[i] = (p.pi ? p.pi[0] : 1.f) * nx[0][i];
 #pragma unroll
-            for (int s = 0; s < S; ++s) h[i] += (p.pi ? p.pi[s] : 1.f) * nx[s][i];
-            ss += h[i] * h[i];
+            for (int s = 1; s < S; ++s) h[i] = fmaf(p.pi[s], nx[s][i], h[i]);
+            ss = fmaf(h[i], h[i], ss);
         }
     }
     ss = hy_block_sum<1024>(ss, red);
@@ -128,9 +145,9 @@ static __global__ __launch_bounds__(1024) void hy_matvec_pre_kernel(HyPre p, con
             for (int i = 0; i < PE; ++i) { a0 = fmaf(fx[i], f0[i], a0); a1 = fmaf(fx[i], f1[i], a1); }
         }
         if (c + 1 == chunks) {
-            const float s0 = hy_wave_sum(a0), s1 = hy_wave_sum(a1);
-            if constexpr (KS == 1) { if (lane == 0) store(first + q / chunks * slots, s0, s1); }
-            else if (lane == 0) { part[wave][0] = s0; part[wave][1] = s1; }          // (one pair a wavefront: the host sees to it)
+            const float s0 = hy_wave_sum_vec(a0), s1 = hy_wave_sum_vec(a1);
+            const int i = first + q / chunks * slots;
+            if (lane == 0) { if constexpr (KS == 1) store(i, s0, s1); else { part[i * KS + kp][0] = s0; part[i * KS + kp][1] = s1; } }
         }
     };
     int q = 0;
@@ -144,10 +161,8 @@ static __global__ __launch_bounds__(1024) void hy_matvec_pre_kernel(HyPre p, con
     if constexpr (KS > 1) {
         __syncthreads();
         if (tid < mine) {
-            float s0 = 0.f, s1 = 0.f;
-#pragma unroll
-            for (int z = 0; z < KS; ++z) { s0 += part[tid * KS + z][0]; s1 += part[tid * KS + z][1]; }
-            store(tid, s0, s1);
+            const float (*s)[2] = part + tid * KS;
+            store(tid, (s[0][0] + s[1][0]) + (s[2][0] + s[3][0]), (s[0][1] + s[1][1]) + (s[2][1] + s[3][1]));
         }
     }
 }

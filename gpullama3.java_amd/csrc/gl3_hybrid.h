@@ -11,6 +11,9 @@ constexpr int HY_YPARTS = 2 * HY_KSPLIT;      // copies of y: in a parallel bloc
 
 typedef std::bitset<GL3_T_COUNT> HyHave;      // tensors that have arrived, by id
 
+constexpr int HY_SPLIT_PAIRS = 8192, HY_SPLIT_K = 1024;          // one token's products: below so many pairs of rows of at least so many columns four wavefronts share a pair
+constexpr int HY_PRE_WGS = 256, HY_PRE_SPLIT_PAIRS = HY_SPLIT_PAIRS / HY_PRE_WGS;
+
 // x <- mix^T x + po y_mul post(y) (S streams; one stream without tables: x + y_mul post(y)); h = rms norm of (pi . x), weighted.  y = sum of yparts rows.
 struct HyPre {
     const float* x; size_t xs; float* x_out; size_t xos; int W;

@@ -1013,12 +1013,14 @@ static bool hy_gemm_ring(gl3_ctx* ctx, const T* A, int lda, const HyMat& w, int 
 // ---- single tokens: residual updates that the next product makes (gl3_hy_pre_kernels.h) -------------------------------------------------
 template <typename T, int EPI>
 static void hy_pre_launch(gl3_ctx* ctx, const HyPre& p, int S, const T* Wt, int ldw, int N, float* C, T* act, int ld_act, const HyGlu& gp) {
-    const int pairs = (N + 1) / 2, wgs = std::max(1, std::min(256, pairs));
-    // up to four pairs a workgroup: four wavefronts share one (2048 x 2048: all of the matrix is on its way at once)
-#define HY_PRE(S_) do { if (hy_cdiv(pairs, wgs) <= 4) hipLaunchKernelGGL((hy_matvec_pre_kernel<T, S_, EPI, 4>), dim3(wgs), dim3(1024), 0, ctx->stream, p, Wt, ldw, N, C, act, ld_act, gp);   \
-                    else hipLaunchKernelGGL((hy_matvec_pre_kernel<T, S_, EPI, 1>), dim3(wgs), dim3(1024), 0, ctx->stream, p, Wt, ldw, N, C, act, ld_act, gp); } while (0)
+    const int pairs = (N + 1) / 2, wgs = std::max(1, std::min(HY_PRE_WGS, pairs));
+    // the split of K that hy_gemm's kernel has (below); its places are loaded one or two at a time
+    const bool ksplit = pairs < HY_SPLIT_PAIRS && p.W >= HY_SPLIT_K, two = p.W > 4 * 64 * HyPiece<T>::N;
+#define HY_PRE1(S_, KS, UN) hipLaunchKernelGGL((hy_matvec_pre_kernel<T, S_, EPI, KS, UN>), dim3(wgs), dim3(1024), 0, ctx->stream, p, Wt, ldw, N, C, act, ld_act, gp)
+#define HY_PRE(S_) do { if (!ksplit) HY_PRE1(S_, 1, 4); else if (two) HY_PRE1(S_, 4, 2); else HY_PRE1(S_, 4, 1); } while (0)
     if (S == 1) HY_PRE(1); else if (S == 2) HY_PRE(2); else HY_PRE(4);
 #undef HY_PRE
+#undef HY_PRE1
 }
 // a deferred update that no product has taken: one workgroup without rows
 template <typename T>
@@ -1054,7 +1056,7 @@ static void hy_gemm(gl3_ctx* ctx, const T* A, int lda, const HyMat& w, int M, fl
     if (M > 4 && M <= 8 && sizeof(T) == 2 && hy_gemm_ring<T>(ctx, A, lda, w, M, C, ldc, glu, act, ld_act, gp, parts, max_parts, 2.1 * N * K * 2 / 5.6e6 + 3.0)) return;
     if (M <= 8) {
         const int pairs = hy_cdiv(N, 2);
-        const bool ksplit = pairs < 8192 && K >= 1024;       // few rows: a workgroup's four wavefronts share one pair's K
+        const bool ksplit = pairs < HY_SPLIT_PAIRS && K >= HY_SPLIT_K;       // few rows: a workgroup's four wavefronts share one pair's K
         const int wgs = ksplit ? pairs : hy_cdiv(pairs, 4);
 #define HY_MV2(MT, KS)                                                                                                                              \
     do {                                                                                                                                            \

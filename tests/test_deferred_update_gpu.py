@@ -38,11 +38,10 @@ CASES = [(noditar, 8, 3, 1, 40), (noditar, 104, 211, 2, 72), (noditar, 264, 2051
          (kosusun, 88, 131, None, 56), (kosusun, 520, 4099, None, 8200), (kosusun, 2056, 515, None, 1030), (kugadra, 96, 131, None, 56), (kugadra, 1032, 2055, None, 4100), (kugadra, 4096, 259, None, 96)]
 
 
-@pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
-@pytest.mark.parametrize("make,width,vocab,streams,ff", CASES)
-def test_same_as_updates_of_their_own(hy, tmp_path, make, width, vocab, streams, ff, dtype):
+def both_ways(hy, path, make, width, vocab, streams, ff, dtype):
+    """Logits of twelve tokens, the first three at once: updates deferred, and launches of their own."""
     mod, cfg = make(width, vocab, streams, ff) if streams else make(width, vocab, ff)
-    m = mod.Model(hy, tmp_path, cfg, seed=width % 97 + 1)
+    m = mod.Model(hy, path, cfg, seed=width % 97 + 1)
     toks = np.random.default_rng(width).integers(0, vocab, 12).astype(np.int32)
     out = []
     for taps in (False, True):
@@ -55,10 +54,26 @@ def test_same_as_updates_of_their_own(hy, tmp_path, make, width, vocab, streams,
                 rows.append(r)
         out.append(np.concatenate(rows).astype(np.float64))
         p.close()
-    got, own = out
+    return out
+
+
+@pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
+@pytest.mark.parametrize("make,width,vocab,streams,ff", CASES)
+def test_same_as_updates_of_their_own(hy, tmp_path, make, width, vocab, streams, ff, dtype):
+    got, own = both_ways(hy, tmp_path, make, width, vocab, streams, ff, dtype)
     scale = np.sqrt((own ** 2).mean())
     assert np.sqrt(((got - own) ** 2).mean()) < (4e-6 if dtype == "float32" else 2e-2) * scale
     assert np.abs(got - own).max() < (4e-5 if dtype == "float32" else 2e-1) * scale
+
+
+# widths around where a wavefront's places are one or two (1024, 2048), both sides of 16384 rows, and up to 32 pairs a workgroup
+@pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
+@pytest.mark.parametrize("make,width,vocab,streams,ff", CASES + [(noditar, 1016, 4099, 1, 72), (noditar, 1024, 16381, 4, 8160), (noditar, 1032, 16387, 2, 8200), (kosusun, 2048, 12001, None, 2100),
+                                                                 (kugadra, 2056, 9001, None, 96)])
+def test_same_bits(hy, tmp_path, make, width, vocab, streams, ff, dtype):
+    """The sums are those of the launches that a deferred update stands for, term by term."""
+    got, own = both_ways(hy, tmp_path, make, width, vocab, streams, ff, dtype)
+    assert np.array_equal(got, own)
 
 
 def test_against_the_restatement(hy, tmp_path):
