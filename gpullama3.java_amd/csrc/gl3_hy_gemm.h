@@ -18,9 +18,10 @@
 // float32 matrices.  The float32 MFMAs (v_mfma_f32_32x32x2_f32) take 16 times as long per product as the bfloat16 ones AND the vector units' time with them (measured: the
 // times of f32 MFMAs and of vector instructions of a SIMD add up, those of bfloat16 MFMAs overlap).  So an operand is split into three bfloat16 planes on its way from
 // LDS (x = p0 + p1 + p2, every plane the rounded rest: all 24 bits) and the plane products of at least 2^-16 go to v_mfma_f32_32x32x16_bf16: six, or three where the
-// matrix's values are bfloat16 already (HyMat::b16: what most checkpoints hold; exact).  A sum has a rounding per 16 k and product instead of one per k, and the accumulators
-// are added to a second set every HY_FLUSH stages (256 k; 512 costs 2 % less, 128 3 % more): whole requests err by 8.1e-7 and 1.25e-6 against 64 bits (181 and 400 tokens, means of 12),
-// with the float32 MFMAs 8.2e-7 and 1.31e-6.  An infinity's planes are not a number: results that are not finite are made again in float32 at the end, one by one.
+// matrix's values are bfloat16 already (HyMat::b16: what most checkpoints hold; exact).  Only the largest plane product is added in the main chain, a rounding per 16 k, which goes to
+// a second set of accumulators every HY_FLUSH stages (128 k); the others, 2^-8 of it and less, have a chain of their own (in one chain they are rounded to its size: 2.3e-7 below).
+// Relative error of a product against 64 bits, weights of 24 bits / of bfloat16 values: 181 tokens, 8192 x 2048 0.93e-7 / 0.90e-7 (float32 MFMAs 2.1e-7), 2048 x 8192 1.1e-7 (2.2e-7),
+// 512 tokens, 4096 x 512 0.8e-7 (2.1e-7); of positive operands 0.49e-7 / 0.47e-7 (0.58e-7).  An infinity's planes are not a number: results that are not finite are made again in float32 at the end, one by one.
 // Bound now by the issue of one wavefront per SIMD (58 % of its cycles, 148 vector instructions a stage; planes made ahead by a kernel of their own, and eight wavefronts, were
 // no faster).  181 tokens (us): 8192 x 2048 80 -> 40, 16384 x 2048 with the gate 135 -> 58, 2048 x 8192 79 -> 40, experts 181 + 91 -> 132 + 67; 512 tokens, 4096 x 512 23 -> 14.
 #pragma once
@@ -34,7 +35,7 @@ __device__ __forceinline__ void hy_dma16(const void* src, void* lds_wave_base) {
 // all but the newest N loads of this wavefront have landed, its LDS reads are done, and so are everybody's
 template <int N> __device__ __forceinline__ void hy_wait_barrier() { asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" :: "n"(N) : "memory"); }
 
-constexpr int HY_FLUSH = 8;
+constexpr int HY_FLUSH = 4;
 typedef float hy_v8f __attribute__((ext_vector_type(8)));
 template <typename T> struct HyFrag;
 template <> struct HyFrag<bf16_t> { typedef hy_v8bf V; static constexpr int K = 64; };
@@ -61,7 +62,7 @@ __device__ __attribute__((noinline)) float hy_dot_again(const float* __restrict_
 // WM x WN wavefronts, BM x BN results; EPI, GR and HyGroup as for hy_gemm_kernel (GR: blockIdx.y = row tile of the list, BM rows at most).
 // Grid: x = mt nt ks workgroups (row tiles x column tiles x K splits of kper) rounded up to a multiple of 8; GR: x = column tiles.
 template <typename T, int BM, int BN, int WM, int WN, int SA, int SW, int EPI, int GR = 0, int WP = 3>
-static __global__ __launch_bounds__(WM * WN * 64) void hy_gemm_ring_kernel(const T* __restrict__ A, int lda, const T* __restrict__ Wt, int ldw, int M, int N, int K,
+static __global__ __launch_bounds__(WM * WN * 64, sizeof(T) == 4 ? 2 : 1) void hy_gemm_ring_kernel(const T* __restrict__ A, int lda, const T* __restrict__ Wt, int ldw, int M, int N, int K,
                                                                            float* __restrict__ C, int ldc, T* __restrict__ act, int ld_act, HyGlu glu, int mt, int nt, int ks,
                                                                            int kper, HyGroup grp = HyGroup{}) {
     constexpr int NW = WM * WN, TM = BM / WM / 32, TN = BN / WN / 32, BK = HyFrag<T>::K;
@@ -169,12 +170,17 @@ static __global__ __launch_bounds__(WM * WN * 64) void hy_gemm_ring_kernel(const
             if constexpr (u < w) qw[set][f][pl][e] = hy_plane<(pl + 1 < WP)>(*((float*)&xw[set][f][e / 2] + e % 2 * 2), *((float*)&xw[set][f][e / 2] + e % 2 * 2 + 1));
             else qa[set][f][pl][e] = hy_plane<(pl < 2)>(*((float*)&xa[set][f][e / 2] + e % 2 * 2), *((float*)&xa[set][f][e / 2] + e % 2 * 2 + 1));
         };
-        // the products of at least 2^-16 (planes a + b <= 2), the small ones first
+        // the products of at least 2^-16 (planes a + b <= 2); all but the largest add up in a chain of their own, where they are rounded to their size
+        hy_v16f low[TM][TN];
+#pragma unroll
+        for (int i = 0; i < TM; ++i)
+#pragma unroll
+            for (int j = 0; j < TN; ++j) low[i][j] = acc[i][j];
         constexpr int NM = (WP == 3 ? 6 : 3) * TM * TN;
         auto mm = [&](auto c, int set) {
             constexpr int q = decltype(c)::value / (TM * TN), i = decltype(c)::value / TN % TM, j = decltype(c)::value % TN;
             constexpr int a_ = WP == 3 ? (q == 0 ? 2 : q == 1 || q == 3 ? 1 : 0) : 2 - q, b_ = WP == 3 ? (q == 1 || q == 4 ? 1 : q == 2 ? 2 : 0) : 0;
-            hy_mma(acc[i][j], __builtin_bit_cast(hy_v8bf, qa[set][i][a_]), __builtin_bit_cast(hy_v8bf, qw[set][j][b_]));
+            hy_mma(a_ + b_ ? low[i][j] : acc[i][j], __builtin_bit_cast(hy_v8bf, qa[set][i][a_]), __builtin_bit_cast(hy_v8bf, qw[set][j][b_]));
         };
         // (pinned: left to the compiler the splits stand in one piece behind the MFMAs)
         auto both = [&](auto mset, int cset, auto load) {
@@ -236,7 +242,7 @@ static __global__ __launch_bounds__(WM * WN * 64) void hy_gemm_ring_kernel(const
 #pragma unroll
         for (int i = 0; i < TM; ++i)
 #pragma unroll
-            for (int j = 0; j < TN; ++j) acc[i][j] = tot[i][j];
+            for (int j = 0; j < TN; ++j) acc[i][j] = tot[i][j] + low[i][j];
     } else {
     // step s (behind barrier s) starts the loads of A's stage s + SA (into the slot the barrier freed) and, in the two quarters after it,
     // of W's stage s + SW; the steps before 0 are the prologue, the last one's W belongs to the loop's first round

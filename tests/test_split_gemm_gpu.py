@@ -57,6 +57,22 @@ def test_all_bits_of_the_experts(hy, tmp_path, n, experts, top):
 
 
 @pytest.mark.parametrize("bits", [16, 24])
+@pytest.mark.parametrize("n,k", [(181, 2048), (64, 512)])
+def test_error_of_one_product(hy, tmp_path, n, k, bits):
+    """The head's product alone: with an identity in its place the logits are its operand, to the bit.  Float32 MFMAs err by 2.1e-7 here, a chain that rounds every plane's product to the sum's
+    size by 1.7e-7 (bfloat16 values) and 2.3e-7; one rounding of 2^-24 per 16 k in blocks of 128 k by 0.8e-7 to 1.0e-7."""
+    cfg = config([att(heads=2, kv_heads=2, dim=16, vdim=16, ff=32)], width=k, vocab=k, streams=1)
+    rng = np.random.default_rng(k + bits)
+    w = dict(R.random_weights(cfg, 7), head=np.eye(k, dtype=np.float32))
+    toks = tokens_for(cfg, n)
+    rows = logits(hy, tmp_path / "a", cfg, w, toks).astype(np.float64)
+    head = (0.02 * rng.standard_normal((k, k))).astype(np.float32)
+    head = head if bits == 24 else R.bf16_round(head)
+    got, want = logits(hy, tmp_path / "b", cfg, dict(w, head=head), toks), rows @ head.astype(np.float64).T
+    assert np.linalg.norm(got - want) < 1.4e-7 * np.linalg.norm(want)
+
+
+@pytest.mark.parametrize("bits", [16, 24])
 def test_values_that_planes_do_not_hold(hy, tmp_path, bits):
     """Head rows of 3.395e38 (finite, rounds to infinity in bfloat16), of infinity and of mixed signs: every logit is what float32 products give."""
     cfg = config([att(heads=2, kv_heads=2, dim=16, vdim=16, ff=32)], width=64, vocab=300, streams=1)
