@@ -11,15 +11,18 @@
 // and DVT consecutive value columns of the keys r (value column DVT m + i is row m of tile i); the values travel under the first product
 // and the softmax, the next tile's keys under the second half of the second product (all at once do not fit 256 registers, and a second wavefront
 // per SIMD is what covers the waits).  Queries (scaled) stay in LDS as planes; a step's MFMAs stand between the splits of the next step's keys or values, which the vector units
-// make under them.  One chain of scores: a second one was 16 registers spilled and 14 % of the kernel.
+// make under them.  The scores have one chain (a second one was 16 registers spilled and 14 % of the kernel) in two passes: every chunk's small plane products, rounded to their own size,
+// then the largest products of all chunks, whose key planes wait in registers.  Each product in turn as its chunk comes rounds six times per 16 entries to the size of the score: relative
+// error of a head's output against 64 bits, head size 128, scores of one / of four, 512 tokens behind 1529: 4.5e-7 / 9.7e-7 against 3.5e-7 / 4.7e-7 as it is (float32 MFMAs
+// 4.5e-7 / 7.9e-7; 192 entries, scores of four 7.1e-7, 3.2e-7, 5.2e-7), for 1 % (behind many positions) to 4 % (at position 0) of the kernel.
 // A value that is not finite must stay with the rows that see its key, and the second product carries it to every row of the tile (p = 0 times infinity).  Nothing in the
 // loops below looks for one (values cleaned in the tiles with unseen keys cost 1 and 5 % of the two kernels, right in front of every MFMA 6 - 12 %): sums that hold a
 // not-a-number at the end are made once more, key by key on the vector units (hy_attn_again), which costs other inputs the look at the sums: 1 % of the kernel of
 // many tokens, of that of few 2 % with 64 and 256 entries and 7 % with 512.  It stands behind the last exchange in LDS, which the loop's last MFMAs run under.  An infinite key
 // or query entry has no planes: scores that are not numbers are made again in float32 (hy_score_again).
 // What bounds it: at position 0 a wavefront has two tiles on average and waits for memory half of its time (queries, first keys and the gate are asked for as early as they are
-// known); behind many positions the splits (11 vector instructions per pair of values).  8 key / value heads x 4, head size 128 (us): 512 tokens at position 0 131 (hy_attn_kernel) -> 52
-// (float32 MFMAs) -> 42, four such portions of 2041 tokens 1795 -> 458 -> 355 in all.
+// known); behind many positions the splits (11 vector instructions per pair of values).  8 key / value heads x 4, head size 128, 512 tokens (us, float32 MFMAs -> now): at position 0 45 -> 35,
+// behind 1529 176 -> 145 (launched over and over, caches warm; inside a prompt of 2041 tokens hy_attn_kernel took 131 at position 0, 1795 for the four portions).
 #pragma once
 #include "gl3_hy_gemm.h"
 
@@ -163,30 +166,35 @@ static __global__ __launch_bounds__(256, DKC > 16 ? 1 : 2) void hy_attn_mfma_ker
 #pragma unroll
         for (int r = 0; r < 16; ++r) s0[r] = 0.f;
         {
-            hy_v4u ka[2][3];
-            hy_v8bf qv[2][3];
+            hy_v4u k0[CH], ka[2][2];          // largest planes of all chunks, the smaller two of this and the next one
+            hy_v8bf qv[3];
             auto cut = [&](auto uc, auto cc) {          // step u of chunk c's split
                 constexpr int u = decltype(uc)::value, c = decltype(cc)::value, e = u % 4;
-                ka[c & 1][u / 4][e] = hy_plane<(u < 8)>(*((float*)&kr[c][e / 2] + e % 2 * 2), *((float*)&kr[c][e / 2] + e % 2 * 2 + 1));
+                const uint32_t d = hy_plane<(u < 8)>(*((float*)&kr[c][e / 2] + e % 2 * 2), *((float*)&kr[c][e / 2] + e % 2 * 2 + 1));
+                if constexpr (u < 4) k0[c][e] = d; else ka[c & 1][u / 4 - 1][e] = d;
             };
-            auto rq = [&](auto cc) {
-                constexpr int c = decltype(cc)::value;
+            auto rq = [&](int pl, int c) { return *reinterpret_cast<const hy_v8bf*>(sQ + r32 * QB + pl * 2 * DK + 32 * c + 16 * kh); };
 #pragma unroll
-                for (int pl = 0; pl < 3; ++pl) qv[c & 1][pl] = *reinterpret_cast<const hy_v8bf*>(sQ + r32 * QB + pl * 2 * DK + 32 * c + 16 * kh);
-            };
-            rq(std::integral_constant<int, 0>{});
+            for (int pl = 0; pl < 3; ++pl) qv[pl] = rq(pl, 0);
             hy_static_for<0, 12>([&](auto u) { cut(u, std::integral_constant<int, 0>{}); });
             __builtin_amdgcn_sched_barrier(0);
             hy_static_for<0, CH>([&](auto cc) {
                 constexpr int c = decltype(cc)::value;
-                constexpr std::integral_constant<int, c + 1 < CH ? c + 1 : c> nx{};
-                if constexpr (c + 1 < CH) rq(nx);
-                hy_static_for<0, 6>([&](auto qc) {
-                    constexpr int q = decltype(qc)::value;
-                    hy_mma(s0, __builtin_bit_cast(hy_v8bf, ka[c & 1][PA[q]]), qv[c & 1][PB[q]]);
-                    if constexpr (c + 1 < CH) hy_static_for<2 * q, 2 * q + 2>([&](auto u) { cut(u, nx); });
+                hy_static_for<0, 5>([&](auto qc) {
+                    constexpr int q = decltype(qc)::value, ka_ = q < 2 ? 0 : q < 4 ? 1 : 2, qb = q == 0 ? 2 : q < 3 ? 1 : 0;
+                    hy_mma(s0, __builtin_bit_cast(hy_v8bf, ka_ ? ka[c & 1][ka_ ? ka_ - 1 : 0] : k0[c]), qv[qb]);
+                    if constexpr (c + 1 < CH) {
+                        if constexpr (q != 1 && q != 3) qv[qb] = rq(qb, c + 1);
+                        hy_static_for<q * 12 / 5, (q + 1) * 12 / 5>([&](auto u) { cut(u, std::integral_constant<int, c + 1>{}); });
+                    } else if constexpr (q == 0 || q == 2) qv[qb] = rq(0, q == 0 ? 0 : 1);
                     __builtin_amdgcn_sched_barrier(0);
                 });
+            });
+            hy_static_for<0, CH>([&](auto cc) {          // the largest products
+                constexpr int c = decltype(cc)::value;
+                hy_mma(s0, __builtin_bit_cast(hy_v8bf, k0[c]), qv[c & 1 ? 1 : 2]);
+                if constexpr (c + 2 < CH) qv[c & 1 ? 1 : 2] = rq(0, c + 2);
+                __builtin_amdgcn_sched_barrier(0);
             });
         }
         load_values(8);

@@ -201,3 +201,36 @@ def test_infinite_key_entries(hy, tmp_path, size):
     bad = np.isnan(short).any(axis=1)
     assert 20 < bad.sum() < 180 and not bad[:20].any() and np.array_equal(np.isnan(whole).any(axis=1), bad)
     assert np.abs(whole[~bad] - short[~bad]).max() < 1e-4 * np.sqrt((short[~bad] ** 2).mean())
+
+
+def exact_rows(size, seed, spread=4.0):
+    """One latent attention layer whose queries, keys and values are matrix columns picked by the token, to the bit (every norm is of one entry, its mean square 1), and whose outputs are the logits but
+    for a factor per row.  Scores of about `spread`."""
+    W, R, heads = 1024, 256, 512 // size
+    cfg = N.config([N.lat(heads=heads, dim=size, vdim=size, kv_rank=R, ff=0, scale=size ** -0.5)], width=W, vocab=512, streams=1, eps=1e-30)
+    rng = np.random.default_rng(seed)
+    w = {k: np.zeros_like(v, dtype=np.float32) for k, v in N.R.random_weights(cfg, 1).items()}
+    w["embed"][np.arange(512), np.arange(512)] = 32.0
+    w["l0.mix.dkv"][np.arange(512) % R, np.arange(512)] = 0.5
+    for k in ("l0.norm1", "final.norm", "l0.mix.dkv.norm", "l0.hc1.in", "l0.hc1.mix", "l0.hc1.out"):
+        w[k][...] = 1.0
+    for k, scale in (("q", spread / 32), ("uk", 1 / 16), ("uv", 1 / 16)):
+        w["l0.mix." + k][...] = scale * rng.standard_normal(w["l0.mix." + k].shape)
+    w["l0.mix.o"][512 + np.arange(512), np.arange(512)] = 1.0
+    w["head"][np.arange(512), 512 + np.arange(512)] = 1.0
+    return cfg, w
+
+
+@pytest.mark.parametrize("size,n,bound", [(64, 100, 2.5e-7), (64, 400, 3.1e-7), (128, 100, 3.2e-7), (128, 400, 4.0e-7)])
+def test_error_of_the_attention_alone(hy, tmp_path, size, n, bound):
+    """Scores of four, against float64.  The small plane products in front of the largest ones err by 1.8e-7, 2.3e-7, 2.2e-7 and 2.8e-7, float32 MFMAs by 2.9e-7, 3.6e-7, 3.8e-7 and 4.7e-7, and one chain
+    in which every product is rounded to the size of the score by 3.3e-7, 4.4e-7, 5.0e-7 and 6.3e-7: the bounds lie between the first two."""
+    cfg, w = exact_rows(size, n)
+    hy.save_model_dir(str(tmp_path), cfg, w, dtype="F32")
+    toks = np.random.default_rng(n).integers(0, 512, n).astype(np.int32)
+    p = hy.HybridPlan.from_dir(str(tmp_path), dtype="float32", ctx=n + 8, max_batch=512)
+    got = p.step(p.acquire(), toks, 0, list(range(n))).astype(np.float64)
+    p.close()
+    want = N.R.forward(cfg, N.R.to_f64(w), toks)
+    got *= ((got * want).sum(axis=1) / (got * got).sum(axis=1))[:, None]          # (the last norm's factor)
+    assert np.linalg.norm(got - want) < bound * np.linalg.norm(want)
