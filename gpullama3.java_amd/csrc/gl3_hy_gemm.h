@@ -21,7 +21,8 @@
 // matrix's values are bfloat16 already (HyMat::b16: what most checkpoints hold; exact).  Only the largest plane product is added in the main chain, a rounding per 16 k, which goes to
 // a second set of accumulators every HY_FLUSH stages (128 k); the others, 2^-8 of it and less, have a chain of their own (in one chain they are rounded to its size: 2.3e-7 below).
 // Relative error of a product against 64 bits, weights of 24 bits / of bfloat16 values: 181 tokens, 8192 x 2048 0.93e-7 / 0.90e-7 (float32 MFMAs 2.1e-7), 2048 x 8192 1.1e-7 (2.2e-7),
-// 512 tokens, 4096 x 512 0.8e-7 (2.1e-7); of positive operands 0.49e-7 / 0.47e-7 (0.58e-7).  An infinity's planes are not a number: results that are not finite are made again in float32 at the end, one by one.
+// 512 tokens, 4096 x 512 0.8e-7 (2.1e-7); of positive operands 0.49e-7 / 0.47e-7 (0.58e-7).  An infinity's planes are not a number: tiles with a result that is not finite make it again in float32
+// at the end (hy_tile_again).
 // Bound now by the issue of one wavefront per SIMD (58 % of its cycles, 148 vector instructions a stage; planes made ahead by a kernel of their own, and eight wavefronts, were
 // no faster).  181 tokens (us): 8192 x 2048 80 -> 40, 16384 x 2048 with the gate 135 -> 58, 2048 x 8192 79 -> 40, experts 181 + 91 -> 132 + 67; 512 tokens, 4096 x 512 23 -> 14.
 #pragma once
@@ -51,12 +52,47 @@ template <bool REST> __device__ __forceinline__ uint32_t hy_plane(float& x, floa
     if constexpr (REST) { x -= __uint_as_float(d << 16); y -= __uint_as_float(d & 0xffff0000u); }
     return d;
 }
-// one result in float32 throughout (the planes of an infinity are not a number, and so is their product)
-__device__ __attribute__((noinline)) float hy_dot_again(const float* __restrict__ a, const float* __restrict__ w, int n) {
-    float s = 0.f;
+// Which of 32 rows hold a value that is not a number (bit r: row r); p: row lane % 32.
+__device__ __forceinline__ uint32_t hy_nan_rows(const float* __restrict__ p, int n, int kh) {
+    bool nan = false;
+#pragma unroll 16
+    for (int k = 0; k < n; k += 8) {
+        const hy_v4f v = *reinterpret_cast<const hy_v4f*>(p + k + 4 * kh);
+        nan |= __builtin_isunordered(v[0], v[1]) || __builtin_isunordered(v[2], v[3]);
+    }
+    const uint64_t b = __ballot(nan);
+    return (uint32_t)b | (uint32_t)(b >> 32);
+}
+// The results `odd` (bit r: register r) of a 32 x 32 tile once more, in float32 MFMAs straight from memory: the planes of an infinity are not a number, and so is their product.  a, w: the
+// lane's row (lane % 32) of either operand, n a multiple of 8.  Rows and columns with an operand that is not a number have their results already: a spoiled row costs the look at its operands
+// (a prompt of 181 rows of 1024, none a number: 0.25 ms instead of 0.21; one lane's chain per result took 6.1 ms) and only infinities the products.
+__device__ __attribute__((noinline)) hy_v16f hy_tile_again(hy_v16f c, uint32_t odd, const float* __restrict__ a, const float* __restrict__ w, int n, float scale) {
+    const int lane = threadIdx.x & 63, r32 = lane & 31, kh = lane >> 5;
+    const uint32_t na = hy_nan_rows(a, n, kh);
+#pragma unroll
+    for (int r = 0; r < 16; ++r) if (na >> (8 * (r >> 2) + 4 * kh + (r & 3)) & 1) odd &= ~(1u << r);
+    if (!__any(odd)) return c;
+    if (hy_nan_rows(w, n, kh) >> r32 & 1) odd = 0;
+    if (!__any(odd)) return c;
+    hy_v16f tot;
+#pragma unroll
+    for (int r = 0; r < 16; ++r) tot[r] = 0.f;
 #pragma unroll 1
-    for (int k = 0; k < n; ++k) s = fmaf(a[k], w[k], s);
-    return s;
+    for (int k0 = 0; k0 < n; k0 += 128) {
+        hy_v16f d;
+#pragma unroll
+        for (int r = 0; r < 16; ++r) d[r] = 0.f;
+#pragma unroll 4
+        for (int k = k0; k < min(n, k0 + 128); k += 8) {
+            const hy_v4f x = *reinterpret_cast<const hy_v4f*>(a + k + 4 * kh), y = *reinterpret_cast<const hy_v4f*>(w + k + 4 * kh) * scale;
+#pragma unroll
+            for (int e = 0; e < 4; ++e) d = __builtin_amdgcn_mfma_f32_32x32x2f32(x[e], y[e], d, 0, 0, 0);
+        }
+        tot += d;
+    }
+#pragma unroll
+    for (int r = 0; r < 16; ++r) if (odd >> r & 1) c[r] = tot[r];
+    return c;
 }
 
 // WM x WN wavefronts, BM x BN results; EPI, GR and HyGroup as for hy_gemm_kernel (GR: blockIdx.y = row tile of the list, BM rows at most).
@@ -309,21 +345,20 @@ static __global__ __launch_bounds__(WM * WN * 64, sizeof(T) == 4 ? 2 : 1) void h
 #undef HY_QUARTER
     // lane holds column lane % 32 and rows 8 (r / 4) + 4 (lane / 32) + r % 4 of every 32 x 32 tile
     const int mb = m0 + wm * (BM / WM) + 4 * kh, nb = n0 + wn * (BN / WN) + r32;
-    if constexpr (sizeof(T) == 4) {          // an operand or a sum that is not finite: float32 all the way (rare)
+    if constexpr (sizeof(T) == 4) {          // an operand or a sum that is not finite (rare)
 #pragma unroll
         for (int i = 0; i < TM; ++i)
 #pragma unroll
             for (int j = 0; j < TN; ++j) {
-                bool odd = false;
+                uint32_t odd = 0;
 #pragma unroll
-                for (int r = 0; r < 16; ++r) odd |= !(fabsf(acc[i][j][r]) < INFINITY);
+                for (int r = 0; r < 16; ++r) odd |= !(fabsf(acc[i][j][r]) < INFINITY) ? 1u << r : 0u;
                 if (__builtin_expect(__any(odd), 0)) {
+                    const int ma = m0 + wm * (BM / WM) + i * 32 + r32, n = nb + j * 32;
 #pragma unroll
-                    for (int r = 0; r < 16; ++r) {
-                        const int m = mb + i * 32 + 8 * (r >> 2) + (r & 3), n = nb + j * 32;
-                        if (!(fabsf(acc[i][j][r]) < INFINITY) && m < M && n < N)
-                            acc[i][j][r] = hy_dot_again((const float*)A + (size_t)m * lda + kbeg, (const float*)Wt + (size_t)n * ldw + kbeg, n_it * BK);
-                    }
+                    for (int r = 0; r < 16; ++r) if (mb + i * 32 + 8 * (r >> 2) + (r & 3) >= M || n >= N) odd &= ~(1u << r);          // (repeated rows: not stored)
+                    if (__any(odd))
+                        acc[i][j] = hy_tile_again(acc[i][j], odd, (const float*)A + (size_t)min(ma, M - 1) * lda + kbeg, (const float*)Wt + (size_t)min(n, N - 1) * ldw + kbeg, n_it * BK, 1.f);
                 }
             }
     }

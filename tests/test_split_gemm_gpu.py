@@ -3,6 +3,8 @@ weights are bfloat16 values and take one plane), at the edges of the tiles and o
 
 Yardstick: float64.  Bound: a float32 sum of K terms errs by a few 1e-6 of the logits' root mean square; a plane left out is 2^-8 or 2^-17 of every product (4e-3 or 8e-6)
 and two layers of products see it, so 3e-6 on the root mean square is below what the smallest plane would cost and above what the sums cost (measured up to 1.1e-6)."""
+import time
+
 import numpy as np
 import pytest
 
@@ -10,7 +12,7 @@ import __graft_entry__ as ge
 import kugadra_ref as KR
 import noditar_ref as R
 import test_kugadra_gpu as U
-from test_noditar_gpu import att, config, err, lat, tokens_for
+from test_noditar_gpu import att, config, err, lat, ssm, tokens_for
 
 pytestmark = pytest.mark.gpu
 
@@ -95,3 +97,53 @@ def test_values_that_planes_do_not_hold(hy, tmp_path, bits):
     assert np.isnan(got[np.sign(h[:, 5]) == np.sign(h[:, 6]), 12]).all()
     rest = np.setdiff1d(np.arange(300), [7, 11, 12])
     assert np.abs(got[:, rest] - base[:, rest]).max() <= 1e-5 * np.abs(base).max()
+
+
+@pytest.mark.parametrize("bits", [16, 24])
+def test_time_of_a_prompt_that_is_not_a_number(hy, tmp_path, bits):
+    """A result that is not a number because an operand is not is what it has to be: a prompt of such rows takes about as long as any other (0.25 ms against 0.21; a serial
+    float32 chain per result, 6.1 ms)."""
+    cfg = config([ssm(heads=4, vdim=64, state=16, ff=2048)], width=1024, vocab=4096, streams=1)
+    w = {k: v.copy() for k, v in (full_bits(R, cfg, 3) if bits == 24 else R.random_weights(cfg, 3)).items()}
+    w["embed"][7] = np.nan
+    hy.save_model_dir(str(tmp_path), cfg, w, dtype="F32")
+    p = hy.HybridPlan.from_dir(str(tmp_path), dtype="float32", ctx=256, max_batch=256)
+    toks = tokens_for(cfg, 181)
+    toks[toks == 7] = 8
+    best = []
+    for t in (toks, np.full_like(toks, 7)):
+        took = []
+        for _ in range(6):
+            s = p.acquire()
+            t0 = time.perf_counter()
+            got = p.step(s, t, 0, [0, 180])
+            took.append(time.perf_counter() - t0)
+            p.release(s)
+        best.append(min(took))
+    p.close()
+    assert np.isnan(got).all()
+    assert best[1] < 3 * best[0]
+
+
+def test_infinite_rows(hy, tmp_path):
+    """Rows that hold an infinity among rows that are numbers and rows that are not: float32's results for each, and nobody else's change."""
+    cfg = config([ssm(heads=2, vdim=16, state=16, ff=0)], width=256, vocab=300, streams=1)
+    w = full_bits(R, cfg, 5)
+    w["l0.mix.o"][:] = 0.0
+    w["final.norm"][9], w["final.norm"][10] = 0.0, 3.0e38          # the operand's entry 10 is past the largest float where the row's is more than 1.13
+    w["embed"][:, 10] = 0.01
+    w["embed"][[3, 4], 10] = 4.0, -4.0
+    w["embed"][5] = np.nan
+    w["head"][:, 10] = np.random.default_rng(2).choice([0.0, 0.25, -0.25], 300) * 1e-30
+    toks = tokens_for(cfg, 70) % 200 + 6
+    toks[[2, 40]], toks[[9, 33]], toks[60] = 3, 4, 5          # (the recurrence carries the last one on)
+    x = w["embed"][toks].astype(np.float64)
+    x[60:] = np.nan
+    got = logits(hy, tmp_path, cfg, w, toks)
+    with np.errstate(all="ignore"):
+        h = (x / np.sqrt((x ** 2).mean(axis=1, keepdims=True) + cfg["norm"]["eps"]) * w["final.norm"].astype(np.float64)).astype(np.float32)
+        want = h.astype(np.float64) @ w["head"].astype(np.float64).T
+    assert np.isinf(h).any(axis=1).sum() == 4 and np.isfinite(h).all(axis=1).sum() == 56
+    assert np.array_equal(np.isnan(got), np.isnan(want)) and np.array_equal(got[np.isinf(want)], want[np.isinf(want)].astype(np.float32))
+    ok = np.isfinite(want)
+    assert np.abs(got[ok] - want[ok]).max() < 1e-5 * np.sqrt((want[ok] ** 2).mean())
