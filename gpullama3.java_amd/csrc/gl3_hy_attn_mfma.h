@@ -14,15 +14,16 @@
 // make under them.  The scores have one chain (a second one was 16 registers spilled and 14 % of the kernel) in two passes: every chunk's small plane products, rounded to their own size,
 // then the largest products of all chunks, whose key planes wait in registers.  Each product in turn as its chunk comes rounds six times per 16 entries to the size of the score: relative
 // error of a head's output against 64 bits, head size 128, scores of one / of four, 512 tokens behind 1529: 4.5e-7 / 9.7e-7 against 3.5e-7 / 4.7e-7 as it is (float32 MFMAs
-// 4.5e-7 / 7.9e-7; 192 entries, scores of four 7.1e-7, 3.2e-7, 5.2e-7), for 1 % (behind many positions) to 4 % (at position 0) of the kernel.
+// 4.5e-7 / 7.9e-7; 192 entries, scores of four 7.1e-7, 3.2e-7, 5.2e-7), in the same time.
 // A value that is not finite must stay with the rows that see its key, and the second product carries it to every row of the tile (p = 0 times infinity).  Nothing in the
 // loops below looks for one (values cleaned in the tiles with unseen keys cost 1 and 5 % of the two kernels, right in front of every MFMA 6 - 12 %): sums that hold a
 // not-a-number at the end are made once more, key by key on the vector units (hy_attn_again), which costs other inputs the look at the sums: 1 % of the kernel of
 // many tokens, of that of few 2 % with 64 and 256 entries and 7 % with 512.  It stands behind the last exchange in LDS, which the loop's last MFMAs run under.  An infinite key
-// or query entry has no planes: scores that are not numbers are made again in float32 (hy_score_again).
+// or query entry has no planes: a row whose sum is not a number has its maximum and sum made again, in front of that exchange (hy_softmax_again), up to the first score that is none in float32
+// either.  (Looking at the scores inside the loop: 2 % of the kernel, and 0.1 -> 1.0 - 4.9 ms for 512 tokens with queries or keys that are not numbers, 0.15 this way.)
 // What bounds it: at position 0 a wavefront has two tiles on average and waits for memory half of its time (queries, first keys and the gate are asked for as early as they are
-// known); behind many positions the splits (11 vector instructions per pair of values).  8 key / value heads x 4, head size 128, 512 tokens (us, float32 MFMAs -> now): at position 0 45 -> 35,
-// behind 1529 176 -> 145 (launched over and over, caches warm; inside a prompt of 2041 tokens hy_attn_kernel took 131 at position 0, 1795 for the four portions).
+// known); behind many positions the splits (11 vector instructions per pair of values).  8 key / value heads x 4, head size 128, 512 tokens (us, float32 MFMAs -> now): at position 0 45 -> 34.5,
+// behind 1529 176 -> 140 (launched over and over, caches warm; inside a prompt of 2041 tokens hy_attn_kernel took 131 at position 0, 1795 for the four portions).
 #pragma once
 #include "gl3_hy_gemm.h"
 
@@ -31,6 +32,44 @@ template <int DVT> struct HyVec;
 template <> struct HyVec<2> { typedef float2 V; };
 template <> struct HyVec<4> { typedef float4 V; };
 
+// The rare second passes: a lane's row, key by key in float32.  A score of k and q (which is multiplied first, as the planes' are).
+template <int DK> __device__ __forceinline__ float hy_score(const float* __restrict__ k, const float* __restrict__ q, float qscale) {
+    float s = 0.f;
+#pragma unroll 4
+    for (int d = 0; d < DK; d += 4) {
+        const hy_v4f x = *reinterpret_cast<const hy_v4f*>(k + d), y = *reinterpret_cast<const hy_v4f*>(q + d);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) s = fmaf(x[e], y[e] * qscale, s);
+    }
+    return s;
+}
+// Maximum and sum of a row whose sum is not a number: an infinity's planes and their products are none.  A score that is not a number without planes either leaves the row as it is: none.
+template <int DK, typename Key>
+__device__ __forceinline__ void hy_softmax_again(float& m, float& l, const HyAttnArgs& a, const float* q, float slope, int pr, int nbr, int win, const float* kc, const float* pkc, int vt0, int step,
+                                                 int nv, Key key) {
+    const int ldk = a.G * DK;
+    float mx = -INFINITY, sum = 0.f;
+    bool nan = false;
+#pragma unroll 1
+    for (int pass = 0; pass < 2; ++pass)
+#pragma unroll 1
+        for (int vt = vt0; vt < nv && !nan; vt += step) {
+            int j, last;
+            bool pooled;
+            key(vt, j, last, pooled);
+            last = min(j + 31, last);
+#pragma unroll 1
+            for (; j <= last && !nan; ++j) {
+                if (!(pooled ? j < nbr : (j <= pr && (pr - j < win || j < a.keep)))) continue;
+                float s = hy_score<DK>((pooled ? pkc : kc) + (size_t)j * ldk, q, a.scale);
+                s = pooled ? s : s - slope * (float)(pr - j);
+                if (pass == 0) { mx = fmaxf(mx, s); nan = s != s; }
+                else sum += expf(s - (mx > -INFINITY ? mx : 0.f));
+            }
+        }
+    if (!nan) { m = mx; l = sum; }
+    if (l != l) m = INFINITY;          // (whoever joins the sums has none left)
+}
 // The weighted sums of a lane's row over the keys it sees, vt0, vt0 + step ... of the tile list (key(vt): first key, last one, pooled or not): register r of tile i is
 // value column DVT (8 (r / 4) + 4 (lane / 32) + r % 4) + i behind col0.  q: the row's query; m: its maximum.
 template <int DVT> __device__ __forceinline__ bool hy_attn_nan(const hy_v16f* o) {
@@ -42,7 +81,7 @@ template <int DVT> __device__ __forceinline__ bool hy_attn_nan(const hy_v16f* o)
     return nan;
 }
 template <int DK, int DVT, typename Key>
-__device__ __forceinline__ void hy_attn_again(hy_v16f* o, const HyAttnArgs& a, const float* q, float scale, float m, float slope, int pr, int nbr, int win, const float* kc, const float* vc,
+__device__ __forceinline__ void hy_attn_again(hy_v16f* o, const HyAttnArgs& a, const float* q, float qscale, float scale, float m, float slope, int pr, int nbr, int win, const float* kc, const float* vc,
                                               const float* pkc, const float* pvc, int col0, int kh, int vt0, int step, int nv, Key key) {
 #pragma unroll
     for (int i = 0; i < DVT; ++i)
@@ -59,10 +98,7 @@ __device__ __forceinline__ void hy_attn_again(hy_v16f* o, const HyAttnArgs& a, c
         for (; j <= last; ++j) {
             if (!(pooled ? j < nbr : (j <= pr && (pr - j < win || j < a.keep)))) continue;
             const float *k = (pooled ? pkc : kc) + (size_t)j * ldk, *v = (pooled ? pvc : vc) + (size_t)j * ldv + col0 + DVT * 4 * kh;
-            float s = 0.f;
-#pragma unroll 4
-            for (int d = 0; d < DK; ++d) s = fmaf(k[d], q[d], s);
-            s *= scale;
+            const float s = hy_score<DK>(k, q, qscale) * scale;
             const float p = expf((pooled ? s : s - slope * (float)(pr - j)) - m);
 #pragma unroll
             for (int r = 0; r < 16; ++r) {
@@ -72,14 +108,6 @@ __device__ __forceinline__ void hy_attn_again(hy_v16f* o, const HyAttnArgs& a, c
             }
         }
     }
-}
-
-// A score in float32 throughout: a key's or query's infinity has no planes (rare).
-__device__ __attribute__((noinline)) float hy_score_again(const float* __restrict__ k, const float* __restrict__ q, float scale, int n) {
-    float s = 0.f;
-#pragma unroll 1
-    for (int d = 0; d < n; ++d) s = fmaf(k[d], q[d] * scale, s);
-    return s;
 }
 
 template <int DKC, int DVT>          // dk = 8 DKC, dv = 32 DVT
@@ -199,30 +227,21 @@ static __global__ __launch_bounds__(256, DKC > 16 ? 1 : 2) void hy_attn_mfma_ker
         }
         load_values(8);
         __builtin_amdgcn_sched_barrier(0);
-        float p[16], mx = m, bad = 0.f;
-#pragma unroll
-        for (int r = 0; r < 16; ++r) { p[r] = s0[r]; bad += p[r]; }
-        if (__builtin_expect(__any(bad != bad), 0)) {
-#pragma unroll
-            for (int r = 0; r < 16; ++r) {
-                const int j = j0 + 8 * (r >> 2) + 4 * kh + (r & 3);
-                if (p[r] != p[r] && j <= last) p[r] = hy_score_again((pooled ? pkc : kc) + (size_t)j * ldk, qrow, a.scale, DK);
-            }
-        }
+        float p[16], mx = m;
 #pragma unroll
         for (int r = 0; r < 16; ++r) {
             const int j = j0 + 8 * (r >> 2) + 4 * kh + (r & 3);
-            const float s = p[r];
+            const float s = s0[r];
             if (pooled) p[r] = j < nbr ? s : -INFINITY;
             else p[r] = (j <= pr && (pr - j < win || j < a.keep)) ? s - slope * (float)(pr - j) : -INFINITY;
             mx = fmaxf(mx, p[r]);
         }
         mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
-        const bool any = mx > -INFINITY;                         // false: this row has seen no key yet
-        const float corr = any ? expf(m - mx) : 1.f;             // exp(-inf) = 0 the first time
+        const bool any = mx > -INFINITY;                         // false: this row has seen no key yet, or none whose score is a number
+        const float corr = any ? expf(m - mx) : 1.f, top = any ? mx : 0.f;             // exp(-inf) = 0 the first time
         float ls = 0.f;
 #pragma unroll
-        for (int r = 0; r < 16; ++r) { p[r] = any ? expf(p[r] - mx) : 0.f; ls += p[r]; }
+        for (int r = 0; r < 16; ++r) { p[r] = expf(p[r] - top); ls += p[r]; }
         l = l * corr + ls;
         m = mx;
         hy_v4u pp[2][3], va[2][3];          // weights of keys 0 .. 7 and 8 .. 15 of the lane, a value tile's column
@@ -267,13 +286,14 @@ static __global__ __launch_bounds__(256, DKC > 16 ? 1 : 2) void hy_attn_mfma_ker
         }
     // join the wavefronts: every lane scales by e^(m - M), the wavefronts add up in LDS one after the other
     l += __shfl_xor(l, 32, 64);
+    const auto tile = [&](int t, int& j, int& last, bool& pooled) { pooled = t < np_t; j = first_key(t); last = pooled ? nb_wg - 1 : maxpos; };
+    if (__builtin_expect(l != l, 0)) hy_softmax_again<DK>(m, l, a, qrow, slope, pr, nbr, win, kc, pkc, split * 4 + wave, 4 * a.nsplit, nv, tile);
     if (kh == 0) { sml[wave][0][r32] = m; sml[wave][1][r32] = l; }
     __syncthreads();
     const float M = fmaxf(fmaxf(sml[0][0][r32], sml[1][0][r32]), fmaxf(sml[2][0][r32], sml[3][0][r32]));
     const float sc = m > -INFINITY ? expf(m - M) : 0.f;
-    if (__builtin_expect(__any(hy_attn_nan<DVT>(o) && pr >= 0), 0))
-        hy_attn_again<DK, DVT>(o, a, qrow, a.scale, m, slope, pr, nbr, win, kc, vc, pkc, pvc, 0, kh, split * 4 + wave, 4 * a.nsplit, nv,
-                               [&](int t, int& j, int& last, bool& pooled) { pooled = t < np_t; j = first_key(t); last = pooled ? nb_wg - 1 : maxpos; });
+    if (__builtin_expect(__any(hy_attn_nan<DVT>(o) && pr >= 0 && l == l), 0))
+        hy_attn_again<DK, DVT>(o, a, qrow, a.scale, 1.f, m, slope, pr, nbr, win, kc, vc, pkc, pvc, 0, kh, split * 4 + wave, 4 * a.nsplit, nv, tile);
     for (int w = 0; w < 4; ++w) {
         if (wave == w) {
 #pragma unroll
@@ -470,7 +490,7 @@ static __global__ __launch_bounds__(64 * NW, 1) void hy_attn_few_kernel(HyAttnAr
     if (__builtin_expect(!__any(nan), 1)) store(o);          // (the rare way out of line: 256 entries 9.2 -> 8.6 us, 64 6.1 -> 6.0)
     else if (nan) {
         hy_v16f again[DVT];
-        hy_attn_again<DK, DVT>(again, a, a.q + (size_t)(rho / hpg) * a.ldq + (size_t)hr * DK, a.scale, m, slope, pr, nbr, win, kc, vc, pkc, pvc, col0, kh, split, a.nsplit, nv,
+        hy_attn_again<DK, DVT>(again, a, a.q + (size_t)(rho / hpg) * a.ldq + (size_t)hr * DK, 1.f, a.scale, m, slope, pr, nbr, win, kc, vc, pkc, pvc, col0, kh, split, a.nsplit, nv,
                                [&](int t, int& j, int& last, bool& pooled) { const int w = t - np_t; pooled = t < np_t; j = (pooled ? t : w < nk ? w : lo_t + w - nk) << 5; last = pooled ? nb_wg - 1 : maxpos; });
         store(again);
     } else store(o);
