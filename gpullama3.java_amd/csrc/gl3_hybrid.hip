@@ -1031,11 +1031,15 @@ static void hy_pre_flush(gl3_ctx* ctx) {
     hy_pre_launch<T, HY_EPI_STORE>(ctx, h->pre, h->pre_streams, (const T*)nullptr, 0, 0, nullptr, (T*)nullptr, 0, HyGlu{});
 }
 // the product of one token's row that a deferred update makes (true), or the update alone
+// Long products run on more wavefronts than the 256 workgroups have, for 1 - 6 % less time, which passes the launch saved from some 400 MB on.  Whole steps with heads of rows x columns (us, a launch of
+// its own / deferred): bfloat16 24000 x 2048 (98 MB) 58.1 / 57.4, 131072 x 1024 (268 MB) 100.0 / 97.7, 131072 x 2048 (537 MB) 148 / 153, 131072 x 4096 239 / 244; float32 24000 x 2048 (197 MB) 70.9 / 70.6,
+// 32000 x 2048 (262 MB) 82.9 / 83.2, 24000 x 4096 (393 MB) 113.7 / 115.2, 32000 x 4096 (524 MB) 136 / 140, 131072 x 4096 (2.1 GB) 403 / 430; gate and up of 36864 x 2048 to 36864 x 4096 within 3 us.
+constexpr size_t HY_PRE_BYTES = (size_t)384 << 20;
 template <typename T>
 static bool hy_pre_gemm(gl3_ctx* ctx, const T* A, const HyMat& w, int M, float* C, bool glu, T* act, int ld_act, const HyGlu& gp) {
     gl3_hybrid_state* h = ctx->hy;
     constexpr int PE = 16 / (int)sizeof(T);
-    if (M != 1 || (const void*)A != h->pre.h_out || w.k != h->pre.W || w.ld % PE || ((uintptr_t)w.w & 15) || gp.mul_table) { hy_pre_flush<T>(ctx); return false; }
+    if (M != 1 || (const void*)A != h->pre.h_out || w.k != h->pre.W || (size_t)w.rows * w.ld * sizeof(T) > HY_PRE_BYTES || w.ld % PE || ((uintptr_t)w.w & 15) || gp.mul_table) { hy_pre_flush<T>(ctx); return false; }
     h->pre_on = false;
     if (glu) hy_pre_launch<T, HY_EPI_GLU>(ctx, h->pre, h->pre_streams, (const T*)w.w, w.ld, w.rows, nullptr, act, ld_act, gp);
     else if (gp.act == 2) hy_pre_launch<T, HY_EPI_ACTMUL>(ctx, h->pre, h->pre_streams, (const T*)w.w, w.ld, w.rows, nullptr, act, ld_act, gp);

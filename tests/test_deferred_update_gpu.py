@@ -41,11 +41,14 @@ CASES = [(noditar, 8, 3, 1, 40), (noditar, 104, 211, 2, 72), (noditar, 264, 2051
 def both_ways(hy, path, make, width, vocab, streams, ff, dtype):
     """Logits of twelve tokens, the first three at once: updates deferred, and launches of their own."""
     mod, cfg = make(width, vocab, streams, ff) if streams else make(width, vocab, ff)
-    m = mod.Model(hy, path, cfg, seed=width % 97 + 1)
+    return both_plans(mod.Model(hy, path, cfg, seed=width % 97 + 1).plan, width, vocab, dtype)
+
+
+def both_plans(plan, width, vocab, dtype):
     toks = np.random.default_rng(width).integers(0, vocab, 12).astype(np.int32)
     out = []
     for taps in (False, True):
-        p = m.plan(dtype, ctx=32, max_batch=16, layer_taps=taps)
+        p = plan(dtype, ctx=32, max_batch=16, layer_taps=taps)
         s = p.acquire()
         rows = [p.step(s, toks[:3], 0, want=[2])]
         for i in range(3, 12):
@@ -74,6 +77,17 @@ def test_same_bits(hy, tmp_path, make, width, vocab, streams, ff, dtype):
     """The sums are those of the launches that a deferred update stands for, term by term."""
     got, own = both_ways(hy, tmp_path, make, width, vocab, streams, ff, dtype)
     assert np.array_equal(got, own)
+
+
+@pytest.mark.parametrize("vocab", [24575, 24577])          # 384 MB: the last head whose product makes the update, the first behind a launch
+def test_heads_of_many_bytes(hy, tmp_path, vocab):
+    _, cfg = noditar(4096, vocab, 2)
+    w = N.R.random_weights(dict(cfg, vocab=64), 5)
+    for k in ("embed", "head"):
+        w[k] = np.ascontiguousarray(np.resize(w[k], (vocab, 4096)))
+    hy.save_model_dir(str(tmp_path), cfg, w)
+    got, own = both_plans(lambda dtype, **kw: hy.HybridPlan.from_dir(str(tmp_path), dtype=dtype, **kw), 4096, vocab, "float32")
+    assert np.array_equal(got, own) and np.abs(got).max() > 0
 
 
 def test_against_the_restatement(hy, tmp_path):
