@@ -932,8 +932,8 @@ enum { HY_R256x256, HY_R256x224, HY_R256x192, HY_R256x160, HY_R256x128, HY_R128x
 static const struct { int bm, bn; } HY_RING_TILES[HY_R_COUNT] = {{256, 256}, {256, 224}, {256, 192}, {256, 160}, {256, 128}, {128, 256}, {128, 160}, {128, 128}, {64, 128}, {64, 64}};
 // Which tile and K split: the one with the least estimated time.  A stage of a BM x BN tile takes a CU 0.00154 (BM + BN) us for its operand bytes (83 GB/s per CU,
 // what the loads of all 256 sustain) + 0.0000128 BM BN us that its MFMAs add (fits 64 x 64 ... 256 x 256 within 8 %).  A float32 stage is bound by the issue of its
-// one wavefront per SIMD: 0.43 / 0.58 / 0.78 us for 64 x 64 / 64 x 128 / 128 x 128 with weights of one plane (0.55 / 0.9 / 1.4 with three), and two workgroups on a CU take
-// 1.55 times as long as one (128 x 128 fill its registers alone).  256 CUs take the workgroups in rounds of whole tiles (two workgroups of a small tile share a CU, and its loads) — what decides for most shapes: 10240 x 4096 at
+// wavefronts (one per SIMD in the tiles of 64 rows, two in 128 x 128): 0.43 / 0.58 / 0.78 us for 64 x 64 / 64 x 128 / 128 x 128 with weights of one plane (0.55 / 0.9 / 1.4 with three), and two
+// workgroups of 64 rows on a CU take 1.55 times as long as one (128 x 128 fill its registers alone).  256 CUs take the workgroups in rounds of whole tiles (two workgroups of a small tile share a CU, and its loads) — what decides for most shapes: 10240 x 4096 at
 // 512 tokens is 256 tiles of 128 x 160 (49 us) but 320 of 128 x 128 (65 us) or 160 of 256 x 128 (53 us).  A K split writes and re-reads its part of C at ~4 TB/s.
 static double hy_ring_pick(bool f32, bool b16, int M, int N, int K, bool glu, bool actmul, int max_parts, int* tile, int* ks_out) {
     const int stages = K / (f32 ? 32 : 64);
@@ -992,8 +992,8 @@ static bool hy_gemm_ring(gl3_ctx* ctx, const T* A, int lda, const HyMat& w, int 
     }
     // float32: two workgroups of 64 x 128 share a CU whatever their number (a ring of 6 + 6 is no faster alone: 181 tokens, 8192 x 2048 39 us both)
     constexpr bool F = sizeof(T) == 4;
-#define HY_RG_64x128(EPI) do { if (!F && lone) HY_RG(64, 128, 2, 2, 3, 4, EPI); else HY_RG(64, 128, 2, 2, F ? 3 : 2, F ? 3 : 4, EPI); } while (0)
-#define HY_RG_128x128(EPI) do { if (F || lone) HY_RG(128, 128, 4, 2, F ? 4 : 3, F ? 5 : 4, EPI); else HY_RG(128, 128, 4, 2, 2, 3, EPI); } while (0)
+#define HY_RG_64x128(EPI) do { if constexpr (F) HY_RG(64, 128, 2, 2, 3, 3, EPI); else if (lone) HY_RG(64, 128, 2, 2, 3, 4, EPI); else HY_RG(64, 128, 2, 2, 2, 4, EPI); } while (0)
+#define HY_RG_128x128(EPI) do { if constexpr (F) HY_RG(128, 128, 4, 2, 4, 5, EPI); else if (lone) HY_RG(128, 128, 4, 2, 3, 4, EPI); else HY_RG(128, 128, 4, 2, 2, 3, EPI); } while (0)
     if (glu) {
         if (tile == HY_R64x128) HY_RG_64x128(HY_EPI_GLU); else HY_RG_128x128(HY_EPI_GLU);
     } else if (actmul) {

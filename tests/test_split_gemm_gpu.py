@@ -1,8 +1,8 @@
 """float32 products of many tokens as products of bfloat16 planes (csrc/gl3_hy_gemm.h): matrices whose entries need all 24 bits (three planes, six products; the other tests'
 weights are bfloat16 values and take one plane), at the edges of the tiles and of the rings, and values the planes cannot hold.
 
-Yardstick: float64.  Bound: a float32 sum of K terms errs by a few 1e-6 of the logits' root mean square; a plane left out is 2^-8 or 2^-17 of every product (4e-3 or 8e-6)
-and two layers of products see it, so 3e-6 on the root mean square is below what the smallest plane would cost and above what the sums cost (measured up to 1.1e-6)."""
+Yardstick: float64.  Bound of whole models: a float32 sum of K terms errs by a few 1e-6 of the logits' root mean square (measured up to 1.1e-6), the second plane left out is 2^-9 of every product (4e-3).  The
+third is 2^-18 at most and 2e-6 on average, which a whole model's error does not show for one matrix (0.7e-6 to 2.5e-6 of the logits): test_the_smallest_plane looks for it in the direction in which its loss would move them."""
 import time
 
 import numpy as np
@@ -56,6 +56,33 @@ def test_all_bits_of_the_experts(hy, tmp_path, n, experts, top):
     toks = tokens_for(cfg, n)
     got, want = logits(hy, tmp_path / "m", cfg, w, toks), KR.forward(cfg, KR.to_f64(w), toks)
     assert np.median(np.sqrt(((got - want) ** 2).mean(axis=1)) / np.sqrt((want ** 2).mean())) < 3e-6          # (a near tie of two experts may fall the other way)
+
+
+ONE = {"head": None, "mlp.gate": None, "mlp.down": None, "mix.o": None, "mix.uk": None, "mix.uv": None, "mlp.e1.gate": 40, "mlp.e2.up": 200, "mlp.e1.down": 40, "mlp.e2.down": 200}
+
+
+@pytest.mark.parametrize("name", ONE)
+def test_the_smallest_plane(hy, tmp_path, name):
+    """One matrix alone holds 24 bits (of the experts' one of one expert).  What is left between the logits and float64's must not point where the loss of its third plane points: the share is 1 if it
+    is lost, 0 if not."""
+    if ONE[name]:          # tiles of 32 and of 64 rows
+        ref, n, cfg = KR, ONE[name], U.config([U.lig(heads=2, dim=16, vdim=16, mlp=U.moe(experts=3, top=2, ff=96, shared=64))], width=128)
+    else:
+        ref, n, cfg = R, 130, config([lat(heads=2, dim=16, vdim=32, kv_rank=64, ff=96)], width=128, vocab=451, streams=1)
+    name = name if name == "head" else "l0." + name
+    w = {k: R.bf16_round(v) for k, v in ref.random_weights(cfg, 11).items()}
+    w[name] = (w[name] * (1.0 + 0.005 * np.random.default_rng(1).standard_normal(w[name].shape))).astype(np.float32)
+    p0 = R.bf16_round(w[name])
+    two = p0.astype(np.float64) + R.bf16_round(w[name] - p0)
+    toks = tokens_for(cfg, n)
+    got, full = logits(hy, tmp_path, cfg, w, toks).astype(np.float64), ref.forward(cfg, ref.to_f64(w), toks)
+    lost = ref.forward(cfg, dict(ref.to_f64(w), **{name: two}), toks) - full
+    left = got - full
+    same = np.abs(left).max(axis=1) < 1e-4 * np.abs(full).max()          # (a near tie of two experts may fall the other way)
+    assert same.mean() > 0.9
+    left, lost = left[same], lost[same]
+    share = (left * lost).sum() / (lost * lost).sum()
+    assert abs(share) < 0.25
 
 
 @pytest.mark.parametrize("bits", [16, 24])
