@@ -5,7 +5,7 @@
 // under load) that is 60 - 75 GB/s per CU, while 256 x 256 results need 60 GB/s to keep the matrix cores busy and 128 x 128 twice that.  So:
 //   * operands go straight to LDS (global_load_lds, 16 bytes per lane: no staging registers, no store pass) into two rings, SA stages of A
 //     (re-read by every workgroup: L2 hits, 0.4 us under load — a ring of two leaves it one stage's time, less than that in the small tiles) and SW > SA stages of
-//     W (each row read once: HBM misses, hence the longer lead);
+//     W (each row read once: HBM misses, hence the longer lead; the float32 tiles of 64 x 128 and 32 x 128 have as many of either, two and four workgroups of them share a CU);
 //   * the barrier of a stage sits a quarter of a stage before its end: the last quarter's MFMAs run behind it while the next stage's first
 //     fragments are read, and it waits with a counted vmcnt for everything but the loads that have a whole stage left to travel;
 //   * the loads are spread between the MFMAs (issued in one go they hold the wavefront for ~1000 cycles: the address unit takes 16 cycles each);
@@ -17,14 +17,16 @@
 //   88 tokens, 4096 x 14336: 56; 24 tokens, 28672 x 4096: 89 -> 52 (4.5 TB/s of weights).
 // float32 matrices.  The float32 MFMAs (v_mfma_f32_32x32x2_f32) take 16 times as long per product as the bfloat16 ones AND the vector units' time with them (measured: the
 // times of f32 MFMAs and of vector instructions of a SIMD add up, those of bfloat16 MFMAs overlap).  So an operand is split into three bfloat16 planes on its way from
-// LDS (x = p0 + p1 + p2, every plane the rounded rest: all 24 bits) and the plane products of at least 2^-16 go to v_mfma_f32_32x32x16_bf16: six, or three where the
+// LDS (x = p0 + p1 + p2, every plane the rounded rest: all 24 bits
+// of values above 2^-108, below which the planes run out of bfloat16's range: a matrix of size 2^-112 errs by 1.6e-7, of 2^-116 by 2.2e-6, of 2^-120 by 3.5e-5) and the plane products of at least 2^-16 go to v_mfma_f32_32x32x16_bf16: six, or three where the
 // matrix's values are bfloat16 already (HyMat::b16: what most checkpoints hold; exact).  Only the largest plane product is added in the main chain, a rounding per 16 k, which goes to
 // a second set of accumulators every HY_FLUSH stages (128 k); the others, 2^-8 of it and less, have a chain of their own (in one chain they are rounded to its size: 2.3e-7 below).
 // Relative error of a product against 64 bits, weights of 24 bits / of bfloat16 values: 181 tokens, 8192 x 2048 0.93e-7 / 0.90e-7 (float32 MFMAs 2.1e-7), 2048 x 8192 1.1e-7 (2.2e-7),
 // 512 tokens, 4096 x 512 0.8e-7 (2.1e-7); of positive operands 0.49e-7 / 0.47e-7 (0.58e-7).  An infinity's planes are not a number: tiles with a result that is not finite make it again in float32
 // at the end (hy_tile_again).
-// Bound now by the issue of one wavefront per SIMD (58 % of its cycles, 148 vector instructions a stage; planes made ahead by a kernel of their own, and eight wavefronts, were
-// no faster).  181 tokens (us): 8192 x 2048 80 -> 40, 16384 x 2048 with the gate 135 -> 58, 2048 x 8192 79 -> 40, experts 181 + 91 -> 132 + 67; 512 tokens, 4096 x 512 23 -> 14.
+// Bound now by issue: the one wavefront per SIMD of a 64 x 128 tile is at work 58 % of its cycles (148 vector instructions a stage with weights of one plane; planes made ahead by a kernel of their own,
+// and the tile on eight wavefronts, were no faster).  Products alone, us, float32 MFMAs -> weights of one plane / of three: 181 tokens, 8192 x 2048 79 -> 40 / 60, 16384 x 2048 with the gate 135 -> 58 / 98,
+// 2048 x 8192 with K split 79 -> 39 / 60, 512 tokens, 4096 x 512 23 -> 13 / 19.  Inside a request (float32 chat, 181 tokens): 8192 x 2048 with its activation 84 -> 50 / 76, experts 183 + 91 -> 121 + 64 / 143 + 75.
 #pragma once
 #include "gl3_hy_kernels.h"
 
@@ -46,7 +48,7 @@ typedef __bf16 hy_v2bf __attribute__((ext_vector_type(2)));
 typedef float hy_v2f __attribute__((ext_vector_type(2)));
 typedef uint32_t hy_v4u __attribute__((ext_vector_type(4)));
 template <int I, int N, typename F> __device__ __forceinline__ void hy_static_for(F f) { if constexpr (I < N) { f(std::integral_constant<int, I>{}); hy_static_for<I + 1, N>(f); } }
-// Two values as bfloat16, and (REST) what is left of them.  Three times over all 24 bits are held; once for values that are bfloat16 already.
+// Two values as bfloat16, and (REST) what is left of them.  Three times over all 24 bits are held (see above); once for values that are bfloat16 already.
 template <bool REST> __device__ __forceinline__ uint32_t hy_plane(float& x, float& y) {
     const uint32_t d = __builtin_bit_cast(uint32_t, __builtin_convertvector((hy_v2f{x, y}), hy_v2bf));
     if constexpr (REST) { x -= __uint_as_float(d << 16); y -= __uint_as_float(d & 0xffff0000u); }

@@ -1719,7 +1719,7 @@ static void hy_gemm_grouped(gl3_ctx* ctx, const T* A, int lda, const HyMat& w, s
     const dim3 grid(hy_cdiv(N, 128), max_tiles, 1);
     constexpr int PE = 16 / (int)sizeof(T), BK = 128 / (int)sizeof(T);
     if (K % BK == 0 && lda % PE == 0 && w.ld % PE == 0 && wstride % PE == 0 && (((uintptr_t)A | (uintptr_t)Wt) & 15) == 0 && (uint64_t)N * w.ld * sizeof(T) < 0xffff0000ull) {
-    // float32 tiles of 32 rows: four workgroups a CU hide each other's stages (rings of 2 + 2; 3 + 4, two a CU: 181 tokens x 4 of 32 experts 132 + 67 us, 145 + 73)
+    // float32 tiles of 32 rows: four workgroups a CU hide each other's stages (rings of 2 + 2; 3 + 4, two a CU: 181 tokens x 4 of 32 experts, weights of one plane, 132 + 67 us, 145 + 73; with the small products in a chain of their own 121 + 64)
 #define HY_RGG1(BM, WM, EPI, WP) hipLaunchKernelGGL((hy_gemm_ring_kernel<T, BM, 128, WM, 2, sizeof(T) == 2 && BM == 32 ? 3 : 2, sizeof(T) == 2 ? 4 : BM == 32 ? 2 : 3, EPI, 1, sizeof(T) == 4 ? WP : 1>), grid, dim3(WM * 128), 0, st, A, lda, Wt, w.ld, 0, N, K, C, ldc, act, ld_act, gp, 0, 0, 1, K, grp)
 #define HY_RGG(BM, WM, EPI) do { if (sizeof(T) == 4 && !w.b16) HY_RGG1(BM, WM, EPI, 3); else HY_RGG1(BM, WM, EPI, 1); } while (0)
 #define HY_RGG_EPI(BM, WM) do { if (glu) HY_RGG(BM, WM, HY_EPI_GLU); else if (gp.act == 2) HY_RGG(BM, WM, HY_EPI_ACTMUL); else HY_RGG(BM, WM, HY_EPI_STORE); } while (0)
