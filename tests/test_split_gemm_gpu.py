@@ -101,6 +101,17 @@ def test_error_of_one_product(hy, tmp_path, n, k, bits):
     assert np.linalg.norm(got - want) < 1.4e-7 * np.linalg.norm(want)
 
 
+@pytest.mark.parametrize("log2,bound", [(100, 1.4e-7), (-108, 1.4e-7), (-116, 4e-6)])
+def test_planes_of_large_and_tiny_values(hy, tmp_path, log2, bound):
+    """Planes hold all bits of values above 2^-108; below, they run out of bfloat16's range (2.2e-6 at 2^-116, float32 MFMAs 2.1e-7)."""
+    cfg = config([att(heads=2, kv_heads=2, dim=16, vdim=16, ff=32)], width=512, vocab=512, streams=1)
+    w, toks = dict(R.random_weights(cfg, 7), head=np.eye(512, dtype=np.float32)), tokens_for(cfg, 64)
+    rows = logits(hy, tmp_path / "a", cfg, w, toks).astype(np.float64)
+    head = (np.random.default_rng(3).standard_normal((512, 512)) * 2.0 ** log2).astype(np.float32)
+    got, want = logits(hy, tmp_path / "b", cfg, dict(w, head=head), toks), rows @ head.astype(np.float64).T
+    assert np.linalg.norm(got * 2.0 ** -log2 - want * 2.0 ** -log2) < bound * np.linalg.norm(want * 2.0 ** -log2)
+
+
 @pytest.mark.parametrize("bits", [16, 24])
 def test_values_that_planes_do_not_hold(hy, tmp_path, bits):
     """Head rows of 3.395e38 (finite, rounds to infinity in bfloat16), of infinity and of mixed signs: every logit is what float32 products give."""
