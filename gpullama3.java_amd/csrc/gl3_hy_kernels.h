@@ -561,15 +561,14 @@ __device__ __forceinline__ void hy_widen(const uint4& p, float* f, const float*)
 // the wavefronts in flight for matrices with few rows.  EPI_GLU: the pair is (gate row, up row) of one feature in the block layout above.
 // Grouped form (GR = 1, mixture of experts, MT = 1): blockIdx.y = a (token, choice) pair whose expert sel[pair] picks the N rows of the
 // stacked matrix; row `pair` of A, C and act belongs to it.  A choice that is no expert (sel[pair] >= n_sel, identity) has no products.
-template <typename T, typename TO, int MT, int EPI, int KS, int GR = 0>
-static __global__ __launch_bounds__(256) void hy_matvec_kernel(const T* __restrict__ A, int lda, const T* __restrict__ Wt, int ldw, int M, int N, int K,
-                                                               float* __restrict__ C, int ldc, TO* __restrict__ act, int ld_act, HyGlu glu,
-                                                               const int* __restrict__ sel = nullptr, size_t wstride = 0, int a_div = 1,
-                                                               const float* __restrict__ row_scale = nullptr, int n_sel = 0) {
+// SUB: groups of four wavefronts in the workgroup, each a workgroup of its own (gl3_hy_beside_kernels.h); (bx, by): place in the grid.
+template <typename T, typename TO, int MT, int EPI, int KS, int GR, int SUB>
+__device__ __forceinline__ void hy_matvec(int bx, int by, const T* __restrict__ A, int lda, const T* __restrict__ Wt, int ldw, int M, int N, int K, float* __restrict__ C, int ldc,
+                                          TO* __restrict__ act, int ld_act, const HyGlu& glu, const int* __restrict__ sel, size_t wstride, int a_div, const float* __restrict__ row_scale, int n_sel) {
     constexpr int PE = HyPiece<T>::N;
     float rs = 1.f;          // grouped: the pair's products are multiplied by row_scale[pair] (a score that scales the expert's input scales W x)
     if constexpr (GR) {
-        const int pair_ = blockIdx.y;
+        const int pair_ = by;
         if (sel[pair_] >= n_sel) return;
         A += (size_t)(pair_ / a_div) * lda;          // a_div = choices per token: the pairs of a token share its row
         if (row_scale) rs = row_scale[pair_];
@@ -577,14 +576,15 @@ static __global__ __launch_bounds__(256) void hy_matvec_kernel(const T* __restri
         if (C) C += (size_t)pair_ * ldc;
         if (act) act += (size_t)pair_ * ld_act;
     }
-    __shared__ float red[3][2 * MT];
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const int pair = KS == 1 ? blockIdx.x * 4 + wave : blockIdx.x;
-    const int kt = KS == 1 ? lane : threadIdx.x, kstep = KS == 1 ? 64 : 256;          // this thread's place in the walk over K
+    __shared__ float red_[SUB][3][2 * MT];
+    const int sub = SUB > 1 ? threadIdx.x >> 8 : 0, tid = SUB > 1 ? threadIdx.x & 255 : threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    float (*red)[2 * MT] = red_[sub];
+    const int pair = KS == 1 ? (bx * SUB + sub) * 4 + wave : bx * SUB + sub;
+    const int kt = KS == 1 ? lane : tid, kstep = KS == 1 ? 64 : 256;          // this thread's place in the walk over K
     int r0, r1;
     if constexpr (EPI == HY_EPI_GLU) { r0 = (pair >> 5) * 64 + (pair & 31); r1 = r0 + 32; }
     else { r0 = 2 * pair; r1 = r0 + 1; }
-    if (r0 >= N) return;                                                               // uniform per workgroup when KS = 4
+    if (r0 >= N) return;                                                               // uniform per workgroup when KS = 4 (with SUB > 1: N a multiple of 64)
     const bool has1 = r1 < N;
     const T* w0 = Wt + (size_t)r0 * ldw;
     const T* w1 = Wt + (size_t)(has1 ? r1 : r0) * ldw;
@@ -676,6 +676,13 @@ static __global__ __launch_bounds__(256) void hy_matvec_kernel(const T* __restri
             }
         }
     }
+}
+template <typename T, typename TO, int MT, int EPI, int KS, int GR = 0>
+static __global__ __launch_bounds__(256) void hy_matvec_kernel(const T* __restrict__ A, int lda, const T* __restrict__ Wt, int ldw, int M, int N, int K,
+                                                               float* __restrict__ C, int ldc, TO* __restrict__ act, int ld_act, HyGlu glu,
+                                                               const int* __restrict__ sel = nullptr, size_t wstride = 0, int a_div = 1,
+                                                               const float* __restrict__ row_scale = nullptr, int n_sel = 0) {
+    hy_matvec<T, TO, MT, EPI, KS, GR, 1>(blockIdx.x, blockIdx.y, A, lda, Wt, ldw, M, N, K, C, ldc, act, ld_act, glu, sel, wstride, a_div, row_scale, n_sel);
 }
 
 // ---- attention: cache writers ---------------------------------------------------------------------------------------------------

@@ -343,10 +343,9 @@ static __global__ __launch_bounds__(256) void hy_side_act_kernel(const float* __
 constexpr int HY_RT_PER = 16;
 struct HyRoute { int softmax; const float* bias; int renorm; float mul; int groups, keep; int real, group_max; };
 template <int PER>          // router rows per lane: rows <= 64 PER
-static __global__ __launch_bounds__(64) void hy_route_kernel(const float* __restrict__ z, int ldz, int parts, size_t pstride, int E, int top, int* __restrict__ sel,
-                                                             float* __restrict__ wgt, int* __restrict__ pair_row, float* __restrict__ extra_out,
-                                                             HyRoute rt) {
-    const int t = blockIdx.x, lane = threadIdx.x;
+__device__ __forceinline__ void hy_route(const int t, const float* __restrict__ z, int ldz, int parts, size_t pstride, int E, int top, int* __restrict__ sel, float* __restrict__ wgt,
+                                         int* __restrict__ pair_row, float* __restrict__ extra_out, const HyRoute& rt) {          // threads 0 .. 63 alone
+    const int lane = threadIdx.x;
     constexpr float GONE = -3.0e38f;
     __shared__ float pick_w[64];
     __shared__ int pick_e[64];
@@ -446,6 +445,12 @@ static __global__ __launch_bounds__(64) void hy_route_kernel(const float* __rest
         wgt[t * top + lane] = (rt.renorm || rt.mul != 1.f) ? myw * (rt.mul / (rt.renorm ? wsum + 1e-20f : 1.f)) : myw;
         if (pair_row) pair_row[t * top + lane] = mysel < rt.real ? t * top + lane : -1;
     }
+}
+template <int PER>
+static __global__ __launch_bounds__(64) void hy_route_kernel(const float* __restrict__ z, int ldz, int parts, size_t pstride, int E, int top, int* __restrict__ sel,
+                                                             float* __restrict__ wgt, int* __restrict__ pair_row, float* __restrict__ extra_out,
+                                                             HyRoute rt) {
+    hy_route<PER>(blockIdx.x, z, ldz, parts, pstride, E, top, sel, wgt, pair_row, extra_out, rt);
 }
 
 // Grouping for portions of many tokens: the P = n top (token, choice) pairs are ordered by expert.  pair_row[p] = the pair's row in that

@@ -131,6 +131,7 @@ struct gl3_hybrid_state {
     float *gates = nullptr, *rowr = nullptr;     // matrix memory: a, b, e^(-m) per (token, head), [3][mb][max heads]; attention: 1 / rms of the whole q and k rows [mb][2]
     int max_heads = 1;
     void *h = nullptr, *mixo = nullptr, *xw = nullptr;
+    void* act1 = nullptr;      // parallel blocks, one token: the feed-forward's activation [max ff_pad], matrix type (made while mixo is)
     float *logits = nullptr, *taps = nullptr, *ones = nullptr;
     int *tokens = nullptr, *dyn = nullptr, *want = nullptr;
     int *h_tokens = nullptr, *h_dyn = nullptr, *h_want = nullptr;    // pinned: the record of the portion being enqueued (one of two: h_rec)

@@ -26,6 +26,7 @@
 #include "gl3_hy_one_kernels.h"
 #include "gl3_hy_plain_kernels.h"
 #include "gl3_hy_pre_kernels.h"
+#include "gl3_hy_beside_kernels.h"
 
 using gl3::AMX_WGS;
 using gl3::argmax_kernel;
@@ -495,6 +496,7 @@ int32_t gl3_hy_create(const gl3_model_desc* desc, gl3_ctx** out, std::string& er
     TRY(hy_alloc(ctx, &h->gates, (size_t)3 * mb * max_heads * 4));
     TRY(hy_alloc(ctx, &h->rowr, (size_t)2 * mb * 4));
     TRY(hy_alloc(ctx, &h->mixo, (size_t)mb * max_mix * es));
+    if (h->parallel) TRY(hy_alloc(ctx, &h->act1, (size_t)max_mix * es));
     TRY(hy_alloc(ctx, &h->conv, (size_t)mb * max_ch * 4));
     TRY(hy_alloc(ctx, &h->ssm_y, (size_t)mb * max_inner * 4));
     TRY(hy_alloc(ctx, &h->qa, (size_t)mb * max_hr * 4));
@@ -593,7 +595,7 @@ void gl3_hy_destroy(gl3_ctx* ctx) {
         f(L.router.w); f(L.egu.w); f(L.edown.w); f(L.depth_mix); f(L.side_gate.w); f(L.side_proj.w); f(L.side_norm);
     }
     f(h->side_emb.w); f(h->sgz); f(h->hist); f(h->side_z); f(h->moe_z); f(h->wsel); f(h->eout); f(h->xb); f(h->side_g); f(h->ea); f(h->eact); f(h->sel); f(h->pair_row); f(h->tiles); f(h->ntiles);
-    f(h->slots); f(h->X); f(h->X2); f(h->h); f(h->proj); f(h->y); f(h->mixo); f(h->conv); f(h->ssm_y); f(h->qa); f(h->oc); f(h->kx); f(h->vx); f(h->part_acc); f(h->part_ml); f(h->gates); f(h->rowr);
+    f(h->slots); f(h->X); f(h->X2); f(h->h); f(h->proj); f(h->y); f(h->mixo); f(h->act1); f(h->conv); f(h->ssm_y); f(h->qa); f(h->oc); f(h->kx); f(h->vx); f(h->part_acc); f(h->part_ml); f(h->gates); f(h->rowr);
     f(h->cq); f(h->qfull); f(h->bigram.w); f(h->hf); f(h->ffz);
     f(h->xw); f(h->logits); f(h->taps); f(h->ones); f(h->dyn);
     hf(h->h_rec); hf(h->h_logits);
@@ -1639,6 +1641,15 @@ static int32_t hy_mixer_core(gl3_ctx* ctx, HyLayer& L, int np, int ldo, int n, i
     return GL3_OK;
 }
 
+// Every mixer of a layer on the n rows of the fused projection.
+template <typename T>
+static int32_t hy_mixers(gl3_ctx* ctx, HyLayer& L, int np, int n, int pos0, int seq) {
+    if (n == 1 && L.side && hy_pair_one<T>(ctx, L, *L.side, np, pos0)) { hy_pool(ctx, L, n, pos0); return GL3_OK; }
+    int32_t r = hy_mixer_core<T>(ctx, L, np, L.mo_total, n, pos0, seq);
+    if (r == GL3_OK && L.side) r = hy_mixer_core<T>(ctx, *L.side, np, L.mo_total, n, pos0, seq);
+    return r;
+}
+
 // The mixer sublayer of a layer on the n normed rows in h->h: one product for the inputs of every mixer of the layer, the mixers'
 // kernels, one product for their outputs (K-split parts in h->y, h->y_parts of them).
 template <typename T>
@@ -1656,12 +1667,7 @@ static int32_t hy_mixer(gl3_ctx* ctx, HyLayer& L, int n, int pos0, int seq) {
         }
     } else
         hy_gemm<T>(ctx, (T*)h->h, h->W, L.proj, n, h->proj, np, false, nullptr, 0, HyGlu{});
-    int32_t r = GL3_OK;
-    if (n == 1 && L.side && hy_pair_one<T>(ctx, L, *L.side, np, pos0)) hy_pool(ctx, L, n, pos0);
-    else {
-        r = hy_mixer_core<T>(ctx, L, np, L.mo_total, n, pos0, seq);
-        if (r == GL3_OK && L.side) r = hy_mixer_core<T>(ctx, *L.side, np, L.mo_total, n, pos0, seq);
-    }
+    int32_t r = hy_mixers<T>(ctx, L, np, n, pos0, seq);
     if (r != GL3_OK) return r;
     hy_gemm<T>(ctx, (T*)h->mixo, L.mo_total, L.o, n, h->y, h->W, false, nullptr, 0, HyGlu{}, &h->y_parts);
     h->y_first = h->y_parts;
@@ -1688,6 +1694,77 @@ static void hy_ff_up(gl3_ctx* ctx, const T* hb, HyLayer& L, int n, T* act) {
             hipLaunchKernelGGL((hy_polynorm_kernel<T, 256>), dim3(n), dim3(256), 0, ctx->stream, h->ffz, L.ff_pad, L.dense_ff, parts, (size_t)n * L.ff_pad, L.poly, ctx->d.rms_eps, act);
     } else if (act_id == 2) hy_gemm<T>(ctx, hb, h->W, L.gu, n, nullptr, 0, false, act, L.ff_pad, HyGlu{0.f, 0.f, 0.f, nullptr, nullptr, 0, 0, 2});      // no gate: relu(up)^2
     else hy_gemm<T>(ctx, hb, h->W, L.gu, n, nullptr, 0, true, act, L.ff_pad, hy_ff_glu(L));
+}
+
+// ---- one token: launches side by side (gl3_hy_beside_kernels.h) -------------------------------------------------------------------------
+static bool hy_mv_split(long pairs, int K) { return pairs < HY_SPLIT_PAIRS && K >= HY_SPLIT_K; }          // (hy_gemm's and hy_gemm_grouped's rule)
+template <typename T>
+static HyMv<T> hy_mv(const T* A, int lda, const HyMat& w, float* C, T* act, int ld_act, const HyGlu& g) { return HyMv<T>{A, lda, (const T*)w.w, w.ld, w.rows, w.k, C, 0, act, ld_act, g, nullptr, 0, 1, nullptr, 0}; }
+// The mixer of a parallel block in its one-launch form and the feed-forward's gate and up rows; false: another form or position, nothing has run.  us, launches apart / like this, 16384 x 2048 in bfloat16
+// beside attention of 32 heads of 64 and retention of 16 x 64 x 128: 7.3 + 14.3 / 17, beside mLSTM of 8 x 128 x 256: 12.4 + 14.3 / 18 (the mixer's workgroups are through before the rows are).
+template <typename T>
+static bool hy_mixer_up(gl3_ctx* ctx, const HyLayer& L, int np, int pos0, T* act) {
+    gl3_hybrid_state* h = ctx->hy;
+    const gl3_layer_desc& d = L.d;
+    if (hy_ungated(d) || d.out_norm) return false;
+    HyAttnOne a{};
+    HyScanOut b{};
+    const HyLayer *at = d.mixer == GL3_MIX_ATTENTION ? &L : nullptr, *me = d.mixer == GL3_MIX_MEMORY ? &L : nullptr;
+    if (L.side) {
+        const HyLayer*& other = L.side->d.mixer == GL3_MIX_ATTENTION ? at : me;
+        if (other) return false;
+        other = L.side;
+    }
+    if (!at && !me) return false;
+    if (at && (!hy_attn_one_args(ctx, *at, pos0, a) || std::max(a.D, a.V) > 128)) return false;
+    if (me && (!hy_scan_out_args(ctx, *me, np, b) || b.s.N > 128)) return false;
+    const HyMv<T> f = hy_mv<T>((const T*)h->h, h->W, L.gu, nullptr, act, L.ff_pad, hy_ff_glu(L));
+    const int pairs = L.ff_pad;
+    const bool ks = hy_mv_split(pairs, h->W), wide = at && std::max(a.D, a.V) > 64, deep = me && b.s.N > 64;
+    constexpr int PE = 16 / (int)sizeof(T);
+    const int mixers = a.H + b.s.heads;
+    const bool walk = !ks && h->W % PE == 0 && h->W <= HY_WALK_K && L.gu.ld % PE == 0 && mixers <= 128;
+    const dim3 grid(mixers + (walk ? std::min(256 - mixers, hy_cdiv(pairs, 16)) : ks ? hy_cdiv(pairs, 4) : hy_cdiv(pairs, 16)));
+    T *oa = at ? (T*)h->mixo + at->o0 : nullptr, *ob = me ? (T*)h->mixo + me->o0 : nullptr;
+#define HY_MU1(NI, QN, KS) hipLaunchKernelGGL((hy_mixer_up_kernel<T, NI, QN, KS>), grid, dim3(1024), 0, ctx->stream, a, oa, b, ob, f)
+#define HY_MU(NI, QN) do { if (walk) HY_MU1(NI, QN, 0); else if (ks) HY_MU1(NI, QN, 4); else HY_MU1(NI, QN, 1); } while (0)
+    if (wide) { if (deep) HY_MU(2, 8); else HY_MU(2, 4); }
+    else { if (deep) HY_MU(1, 8); else HY_MU(1, 4); }
+#undef HY_MU
+#undef HY_MU1
+    if (at) hy_pool(ctx, *at, 1, pos0);
+    return true;
+}
+// Two plain products of one token whose results both add to the residual (C0 = w0 A0, C1 = w1 A1).
+template <typename T>
+static void hy_two(gl3_ctx* ctx, const T* A0, const HyMat& w0, float* C0, const T* A1, const HyMat& w1, float* C1) {
+    const int p0 = hy_cdiv(w0.rows, 2), p1 = hy_cdiv(w1.rows, 2);
+    const bool ks = hy_mv_split(p0, w0.k);
+    if (ctx->hy->pre_on || ks != hy_mv_split(p1, w1.k)) {
+        hy_gemm<T>(ctx, A0, w0.k, w0, 1, C0, w0.rows, false, nullptr, 0, HyGlu{});
+        hy_gemm<T>(ctx, A1, w1.k, w1, 1, C1, w1.rows, false, nullptr, 0, HyGlu{});
+        return;
+    }
+    const int g0 = ks ? p0 : hy_cdiv(p0, 4), g1 = ks ? p1 : hy_cdiv(p1, 4);
+    const HyMv<T> m0 = hy_mv<T>(A0, w0.k, w0, C0, nullptr, 0, HyGlu{}), m1 = hy_mv<T>(A1, w1.k, w1, C1, nullptr, 0, HyGlu{});
+    if (ks) hipLaunchKernelGGL((hy_matvec_two_kernel<T, 4, 0>), dim3(g0 + g1), dim3(256), 0, ctx->stream, m0, g0, m1, g1);
+    else hipLaunchKernelGGL((hy_matvec_two_kernel<T, 1, 0>), dim3(g0 + g1), dim3(256), 0, ctx->stream, m0, g0, m1, g1);
+}
+// A layer of a parallel block for one token (dense feed-forward): h->y holds the mixer's output and the feed-forward's, two parts.
+template <typename T>
+static int32_t hy_parallel_one(gl3_ctx* ctx, HyLayer& L, int pos0, int seq) {
+    gl3_hybrid_state* h = ctx->hy;
+    const int np = L.proj.rows;
+    T* act = (T*)h->act1;          // (mixo is read beside it)
+    hy_gemm<T>(ctx, (T*)h->h, h->W, L.proj, 1, h->proj, np, false, nullptr, 0, HyGlu{});
+    if (!hy_mixer_up<T>(ctx, L, np, pos0, act)) {
+        int32_t r = hy_mixers<T>(ctx, L, np, 1, pos0, seq);
+        if (r != GL3_OK) return r;
+        hy_ff_up<T>(ctx, (const T*)h->h, L, 1, act);
+    }
+    hy_two<T>(ctx, act, L.down, h->y + h->W, (const T*)h->mixo, L.o, h->y);
+    h->y_parts = 2;
+    return GL3_OK;
 }
 
 // ---- mixture of experts -------------------------------------------------------------------------------------------------------------
@@ -1752,10 +1829,22 @@ static void hy_moe(gl3_ctx* ctx, HyLayer& L, int n) {
     const int max_tiles = P / bm + std::min(E, P);
     const bool on_out = d.route_on_output != 0;          // the weights multiply the experts' outputs (in the residual update) instead of their inputs
     const HyRoute rt{d.route_softmax, L.route_bias, d.route_renorm, d.route_scale != 0.f ? d.route_scale : 1.f, d.route_groups, d.route_keep, E, d.route_group_max};
-#define HY_RT(PER) hipLaunchKernelGGL((hy_route_kernel<PER>), dim3(n), dim3(64), 0, st, h->moe_z, RZ, zparts, (size_t)n * RZ, E + d.identity, top, h->sel, h->wsel,          \
-                                      few ? h->pair_row : nullptr, (d.shared_ff > 0 && !d.shared_ungated) ? h->sgz : nullptr, rt)
-    if (RZ <= 64) HY_RT(1); else if (RZ <= 256) HY_RT(4); else HY_RT(HY_RT_PER);
+    const HyRouteArgs ra{h->moe_z, RZ, zparts, (size_t)n * RZ, E + d.identity, top, h->sel, h->wsel, few ? h->pair_row : nullptr, (d.shared_ff > 0 && !d.shared_ungated) ? h->sgz : nullptr, rt};
+    // one token: the shared expert's gate and up rows beside the choice, its down projection beside the chosen experts'
+    const bool up_beside = n == 1 && d.shared_ff > 0 && !hy_ungated(d), down_beside = n == 1 && d.shared_ff > 0 && hy_mv_split((long)hy_cdiv(W, 2) * P, L.edown.k) == hy_mv_split(hy_cdiv(W, 2), L.down.k);
+    T* shared_act = (T*)h->mixo;
+    if (up_beside) {
+        const bool ks = hy_mv_split(L.ff_pad, W);
+        const HyMv<T> f = hy_mv<T>(hb, W, L.gu, nullptr, shared_act, L.ff_pad, hy_ff_glu(L));
+        const dim3 grid(1 + (ks ? L.ff_pad : hy_cdiv(L.ff_pad, 4)));
+#define HY_RU(PER) do { if (ks) hipLaunchKernelGGL((hy_route_up_kernel<T, PER, 4>), grid, dim3(256), 0, st, ra, f); else hipLaunchKernelGGL((hy_route_up_kernel<T, PER, 1>), grid, dim3(256), 0, st, ra, f); } while (0)
+        if (RZ <= 64) HY_RU(1); else if (RZ <= 256) HY_RU(4); else HY_RU(HY_RT_PER);
+#undef HY_RU
+    } else {
+#define HY_RT(PER) hipLaunchKernelGGL((hy_route_kernel<PER>), dim3(n), dim3(64), 0, st, ra.z, ra.ldz, ra.parts, ra.pstride, ra.E, ra.top, ra.sel, ra.wgt, ra.pair_row, ra.extra_out, rt)
+        if (RZ <= 64) HY_RT(1); else if (RZ <= 256) HY_RT(4); else HY_RT(HY_RT_PER);
 #undef HY_RT
+    }
     HyMat one_gu = L.egu, one_down = L.edown;
     const bool glu = !hy_ungated(d);
     one_gu.rows = (glu ? 2 : 1) * L.eff_pad; one_down.rows = W;
@@ -1770,12 +1859,21 @@ static void hy_moe(gl3_ctx* ctx, HyLayer& L, int n) {
         hy_gemm_grouped<T>(ctx, (const T*)h->ea, W, one_gu, gu_stride, P, bm, max_tiles, false, nullptr, 0, glu, (T*)h->eact, L.eff_pad,
                            HyGlu{d.ff_limit, d.ff_alpha, d.ff_shift, nullptr, nullptr, 0, 0, d.ff_act}, E);
     }
-    hy_gemm_grouped<T>(ctx, (const T*)h->eact, L.eff_pad, one_down, (size_t)W * L.edown.ld, P, bm, max_tiles, few, h->eout, W, false, nullptr, 0, HyGlu{}, E);
-    if (d.shared_ff > 0) {
-        T* act = (T*)h->mixo;
-        hy_ff_up<T>(ctx, hb, L, n, act);
-        hy_gemm<T>(ctx, act, L.ff_pad, L.down, n, h->y, W, false, nullptr, 0, HyGlu{}, &h->y_parts);
+    if (d.shared_ff > 0 && !up_beside) hy_ff_up<T>(ctx, hb, L, n, shared_act);
+    if (down_beside) {
+        const int pairs = hy_cdiv(W, 2);
+        const bool ks = hy_mv_split(pairs, L.down.k);
+        const int gx = ks ? pairs : hy_cdiv(pairs, 4);
+        HyMv<T> e = hy_mv<T>((const T*)h->eact, L.eff_pad, one_down, h->eout, nullptr, 0, HyGlu{});
+        e.ldc = W; e.sel = h->sel; e.wstride = (size_t)W * L.edown.ld; e.n_sel = E;
+        const HyMv<T> s = hy_mv<T>(shared_act, L.ff_pad, L.down, h->y, nullptr, 0, HyGlu{});
+        if (ks) hipLaunchKernelGGL((hy_matvec_two_kernel<T, 4, 1>), dim3(gx * (1 + P)), dim3(256), 0, st, s, gx, e, gx);
+        else hipLaunchKernelGGL((hy_matvec_two_kernel<T, 1, 1>), dim3(gx * (1 + P)), dim3(256), 0, st, s, gx, e, gx);
+        h->y_parts = 1;
+        return;
     }
+    hy_gemm_grouped<T>(ctx, (const T*)h->eact, L.eff_pad, one_down, (size_t)W * L.edown.ld, P, bm, max_tiles, few, h->eout, W, false, nullptr, 0, HyGlu{}, E);
+    if (d.shared_ff > 0) hy_gemm<T>(ctx, shared_act, L.ff_pad, L.down, n, h->y, W, false, nullptr, 0, HyGlu{}, &h->y_parts);
 }
 
 // logits of the nw rows listed in h->want: final norm of the gathered rows (normed: the last sublayer's update has left it in h->xw), the head's product, the
@@ -1891,14 +1989,15 @@ static int32_t hy_portion_plain(gl3_ctx* ctx, int seq, const int32_t* tokens, in
             if (h->taps) r.tap = h->taps + (size_t)l * lstride;
             resid_to_mixer(r, l + 1);
         };
-        int32_t rc = hy_mixer<T>(ctx, L, n, pos0, seq);
+        const bool beside = n == 1 && h->parallel && L.d.ff > 0 && !L.d.out_norm;
+        int32_t rc = beside ? hy_parallel_one<T>(ctx, L, pos0, seq) : hy_mixer<T>(ctx, L, n, pos0, seq);
         if (rc != GL3_OK) return rc;
         HyResid r = base;
         r.ya = h->y; r.ya_parts = h->y_parts; r.ya_stride = (size_t)n * W;
         if (h->parallel) {
             // one norm, two readers: the feed-forward takes the same normed rows as the mixer, its down projection's parts follow the
             // mixer's in y, and one residual update adds them all: x += residual multiplier * (mixer + feed-forward)
-            if (L.d.ff > 0) {
+            if (L.d.ff > 0 && !beside) {
                 T* act = (T*)h->mixo;
                 int p2 = 1;
                 hy_ff_up<T>(ctx, hb, L, n, act);
