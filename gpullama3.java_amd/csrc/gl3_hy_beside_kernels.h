@@ -53,8 +53,8 @@ __device__ __forceinline__ void hy_walk_glu(int wg, int wgs, const HyMv<T>& p) {
 #pragma unroll
         for (int u = 0; u < UN; ++u) {
             const int ku = min(k + u * STEP, K - PE);
-            a[set][u] = *reinterpret_cast<const uint4*>(w0 + ku);
-            b[set][u] = *reinterpret_cast<const uint4*>(w1 + ku);
+            a[set][u] = hy_ld_once(w0 + ku);
+            b[set][u] = hy_ld_once(w1 + ku);
         }
     };
     const uint4 row = *reinterpret_cast<const uint4*>(p.A + min(tid * PE, K - PE));          // first: the weights' answers come in order behind it

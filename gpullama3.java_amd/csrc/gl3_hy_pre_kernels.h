@@ -45,8 +45,8 @@ static __global__ __launch_bounds__(1024) void hy_matvec_pre_kernel(HyPre p, con
 #pragma unroll
         for (int u = 0; u < UN; ++u) {
             const int ku = min(k + u * STEP, K - PE);
-            a[set][u] = *reinterpret_cast<const uint4*>(w0 + ku);
-            b[set][u] = *reinterpret_cast<const uint4*>(w1 + ku);
+            a[set][u] = hy_ld_once(w0 + ku);
+            b[set][u] = hy_ld_once(w1 + ku);
         }
     };
     const int w = 4 * tid;
