@@ -35,6 +35,13 @@ typedef float hy_v4f __attribute__((ext_vector_type(4)));
 __device__ __forceinline__ void hy_dma16(const void* src, void* lds_wave_base) {
     __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)src, (__attribute__((address_space(3))) void*)lds_wave_base, 16, 0, 0);
 }
+// The same for W, which leaves HBM once (the row tiles that share a tile of it run side by side on one XCD).  bfloat16: past the caches.  Prompts, us, without / with: Kosusun 8B, 600 tokens 1321 / 1272,
+// 88 460 / 439, Noditar 8B 30 tokens 441 / 420, 200 650 / 654, 512 967 / 957.  float32 row tiles are smaller and more of them read a tile again: experts' tiles
+// of 32 rows alone (Kugadra 1B: 12 tokens 789 / 774, 60 852 / 831, 181 1339 / 1342; every product: 60 tokens 854 / 828, but 181 1333 / 1355, 480 1327 / 1344).
+template <bool ONCE>
+__device__ __forceinline__ void hy_dma16_w(const void* src, void* lds_wave_base) {
+    __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)src, (__attribute__((address_space(3))) void*)lds_wave_base, 16, 0, ONCE ? 2 : 0);
+}
 // all but the newest N loads of this wavefront have landed, its LDS reads are done, and so are everybody's
 template <int N> __device__ __forceinline__ void hy_wait_barrier() { asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" :: "n"(N) : "memory"); }
 
@@ -108,6 +115,7 @@ static __global__ __launch_bounds__(WM * WN * 64, sizeof(T) == 4 ? 2 : 1) void h
     constexpr int SZA = BM * 128, SZW = BN * 128, OW = SA * SZA;
     static_assert(SW >= SA + (sizeof(T) == 2) && SA >= 2 && NPA * NW < 2 * PA + NW && TM * WM * 32 == BM && TN * WN * 32 == BN, "tile layout");
     static_assert(SA * SZA + SW * SZW <= 160 * 1024, "LDS");
+    constexpr bool ONCE = sizeof(T) == 2 || (GR && BM == 32);
     __shared__ __attribute__((aligned(1024))) uint8_t smem[SA * SZA + SW * SZW];
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), wm = wave / WN, wn = wave % WN;
     int m0, n0, z = 0;
@@ -155,7 +163,7 @@ static __global__ __launch_bounds__(WM * WN * 64, sizeof(T) == 4 ? 2 : 1) void h
         const uint8_t* w = (const uint8_t*)Wt + (size_t)it * 128;
 #pragma unroll
         for (int u = 0; u < NPW; ++u)
-            if (u >= u0 && u < u1) hy_dma16(w + offw[u], smem + slot * SZW + pw[u]);
+            if (u >= u0 && u < u1) hy_dma16_w<ONCE>(w + offw[u], smem + slot * SZW + pw[u]);
     };
     hy_v16f acc[TM][TN];
 #pragma unroll
@@ -252,7 +260,7 @@ static __global__ __launch_bounds__(WM * WN * 64, sizeof(T) == 4 ? 2 : 1) void h
                 uint8_t *da = smem + sa * SZA, *dw = smem + sw * SZW;
                 auto load = [&](auto c) {          // piece c of this step
                     constexpr int u = decltype(c)::value;
-                    if constexpr (u < NPA) hy_dma16(na + offa[u], da + pa[u]); else hy_dma16(nw + offw[u - NPA], dw + pw[u - NPA]);
+                    if constexpr (u < NPA) hy_dma16(na + offa[u], da + pa[u]); else hy_dma16_w<ONCE>(nw + offw[u - NPA], dw + pw[u - NPA]);
                 };
                 if (++sa == SA) sa = 0;
                 if (++sw == SW) sw = 0;
