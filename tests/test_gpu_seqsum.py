@@ -44,3 +44,19 @@ def test_exact_sumsq_matches_sequential_chain(pkg):
         assert L.gl3_debug_sumsq(0, x.ctypes.data_as(C.c_void_p), x.size, C.byref(out)) == 0
         ref = seq_sumsq(x)
         assert np.float32(out.value).view(np.uint32) == np.float32(ref).view(np.uint32), (name, x.size, out.value, float(ref))
+
+
+@pytest.mark.parametrize("n", [1024, 1028, 2560, 4092, 5120])
+def test_passes_of_the_replay(pkg, n):
+    """Segments with a rounding tie are replayed one after the other, 61 in a pass: counts around one, two and three passes, spread over the wavefronts' spans or side by side.  5000^2 starts the sum in
+    the middle of a binade with ulp 2: a term of 4 is easy, a term of 1 a tie."""
+    from importlib import import_module
+    L = import_module(ge.PKG_NAME + ".hip").lib()
+    out = C.c_float()
+    for hard in (0, 1, 59, 60, 61, 62, 121, 122, 123, 183, 184):
+        for at in (np.linspace(1, n // 4 - 1, hard).astype(int), n // 4 - hard + np.arange(hard)):
+            x = np.full(n, 2.0, np.float32)
+            x[0] = 5000.0
+            x[4 * at + hard % 4] = 1.0
+            assert L.gl3_debug_sumsq(0, x.ctypes.data_as(C.c_void_p), n, C.byref(out)) == 0
+            assert np.float32(out.value) == seq_sumsq(x), (hard, at[:4])
