@@ -68,7 +68,7 @@ static hipError_t allow_big_lds() {
 
 // rows_valid / out / resid_in may address a slice (tensor parallel row split); w holds exactly that slice.
 static void launch_matvec(gl3_ctx* ctx, int pro, int epi, const Q8Mat& w, const Q8Mat* w2, const float* x,
-                          const float* norm_w, float* out, const float* resid_in, float out_scale = 1.0f, const TpRec* tp = nullptr) {
+                          const float* norm_w, float* out, const float* resid_in, float out_scale = 1.0f, const TpRec* tp = nullptr, float* host = nullptr) {
     if (w.fmt != GL3_TYPE_Q8_0) {      // F16 / Q4_0: element-wise chains, one output row per lane (gl3_rowlane_kernels.h)
         hipStream_t s = ctx->stream;
         // Vector-order kernels normalise in their own prologue (matvec_vl_kernel<.., RMS>); GL3_VL_RMS=0: separate rmsnorm launch
@@ -88,6 +88,7 @@ static void launch_matvec(gl3_ctx* ctx, int pro, int epi, const Q8Mat& w, const 
         if (w.vl) {                   // Vector-API order (8 accumulator lanes per row): lane = (row, accumulator), HBM-bound
             VlArgs v{};
             v.w = w.w; v.w2 = w2 ? w2->w : nullptr; v.rows = w.rows; v.k = w.k; v.x = x; v.out = out; v.resid_in = resid_in; v.out_scale = out_scale;
+            v.host = host; v.host_on = ctx->dyn + 2;
             v.tp = tp;      // folded gathers (gate/up -> hb, down -> x): producer side only, the consumers get wait launches
             const dim3 vg(((w.rows + 7) / 8 + VL_WAVES - 1) / VL_WAVES), vb(64 * VL_WAVES);
             const size_t vs = vl_smem_bytes(w.k);
@@ -161,7 +162,7 @@ static void launch_matvec(gl3_ctx* ctx, int pro, int epi, const Q8Mat& w, const 
     MatvecArgs a{};
     a.w = w.w; a.w2 = w2 ? w2->w : nullptr; a.rows = w.rows; a.k = w.k; a.ng = w.ng; a.nstrips = w.nstrips;
     a.x = x; a.norm_w = norm_w; a.eps = ctx->d.rms_eps; a.out = out; a.resid_in = resid_in; a.out_scale = out_scale;
-    a.tp = tp;
+    a.tp = tp; a.host = host; a.host_on = ctx->dyn + 2;
     const int wgs = w.nstrips < max_wgs ? w.nstrips : max_wgs;
     const size_t smem = matvec_smem(pro, epi, w);
     if (pro == PRO_RMS && epi == EPI_STORE) launch_matvec_t<PRO_RMS, EPI_STORE>(ctx, a, wgs, smem, nt);
@@ -438,6 +439,8 @@ static void launch_attention(gl3_ctx* ctx, int l, int which /* 0 both, 1 scores,
 }
 
 // amode: attn_mode(position) — the host knows the position of the step
+// The logits' kernel can write the host's copy itself (one rank, not the row-per-lane kernels).
+static bool logits_leave(const gl3_ctx* ctx) { return ctx->d.tp_size <= 1 && (ctx->wcls.fmt == GL3_TYPE_Q8_0 || ctx->wcls.vl); }
 static int32_t enqueue_decode(gl3_ctx* ctx, bool want_logits, gl3_kernel_times* kt, int amode) {
     const gl3_model_desc& d = ctx->d;
     hipStream_t s = ctx->stream;
@@ -509,7 +512,7 @@ static int32_t enqueue_decode(gl3_ctx* ctx, bool want_logits, gl3_kernel_times* 
         pr.begin(GL3_K_MATVEC_LOGITS, mv_bytes(ctx->wcls) + d.dim * 4, q8);
         { Gl3Range g("final rmsnorm + logits");
           launch_matvec(ctx, PRO_RMS, EPI_STORE, ctx->wcls, nullptr, ctx->x, ctx->out_norm,
-                        ctx->logits + (size_t)rank * ctx->vocab_l, nullptr, ctx->logit_scale, (fmask & TF_LOGITS) ? tp_rec(ctx, L_, 1) : nullptr); }
+                        ctx->logits + (size_t)rank * ctx->vocab_l, nullptr, ctx->logit_scale, (fmask & TF_LOGITS) ? tp_rec(ctx, L_, 1) : nullptr, host && logits_leave(ctx) ? ctx->h_logits : nullptr); }
         pr.end();
         if ((r = all_gather(ctx, GB_LOGITS, ctx->vocab_l, pr)) != GL3_OK) return r;
     }
@@ -1053,7 +1056,7 @@ static int32_t set_dyn(gl3_ctx* ctx, int32_t token, int32_t pos) {
     if (token < 0 || token >= ctx->d.vocab) GL3_FAIL(GL3_E_ARG, "token id out of range");
     if (pos < 0 || pos >= ctx->d.ctx) GL3_FAIL(GL3_E_ARG, "position outside the KV cache (context length)");
     GL3_HIP(hipSetDevice(ctx->d.device));
-    ctx->h_dyn[0] = token; ctx->h_dyn[1] = pos;          // (every step that read the pair has been waited for)
+    ctx->h_dyn[0] = token; ctx->h_dyn[1] = pos; ctx->h_dyn[2] = 0;          // (every step that read them has been waited for)
     return GL3_OK;
 }
 
@@ -1071,20 +1074,22 @@ int32_t gl3_forward_decode(gl3_ctx* ctx, int32_t token, int32_t pos, float* logi
     gl3_drain drain{ctx->stream};
     const bool want_logits = logits_out || argmax_out;
     const int amode = attn_mode(ctx, pos);
-    if (ctx->graph_exec && want_logits) GL3_HIP(hipGraphLaunch(step_graph(ctx, amode), ctx->stream));
-    else if ((r = enqueue_decode(ctx, want_logits, nullptr, amode)) != GL3_OK) return r;
-    if (argmax_out) {
-        hipLaunchKernelGGL(argmax_kernel, dim3(AMX_WGS), dim3(256), 0, ctx->stream, ctx->logits, ctx->d.vocab, ctx->argmax, ctx->h_argmax);
-        GL3_HIP(hipGetLastError());
-    }
     // logits D2H: straight into the caller's buffer when it is page-locked (gl3_pin_host_buffer), else through the plan's pinned
     // staging buffer + one host memcpy (513 KB for a 128 k vocabulary: ~40 us per token on the host)
     bool direct = false;
     if (logits_out)
         for (const auto& pr : ctx->pinned)
             if ((uint8_t*)logits_out >= (uint8_t*)pr.first && (uint8_t*)logits_out + (size_t)ctx->d.vocab * 4 <= (uint8_t*)pr.first + pr.second) direct = true;
+    const bool leave = logits_out && !direct && logits_leave(ctx);
+    ctx->h_dyn[2] = leave;
+    if (ctx->graph_exec && want_logits) GL3_HIP(hipGraphLaunch(step_graph(ctx, amode), ctx->stream));
+    else if ((r = enqueue_decode(ctx, want_logits, nullptr, amode)) != GL3_OK) return r;
+    if (argmax_out) {
+        hipLaunchKernelGGL(argmax_kernel, dim3(AMX_WGS), dim3(256), 0, ctx->stream, ctx->logits, ctx->d.vocab, ctx->argmax, ctx->h_argmax);
+        GL3_HIP(hipGetLastError());
+    }
     if (logits_out && direct) GL3_HIP(hipMemcpyAsync(logits_out, ctx->logits, (size_t)ctx->d.vocab * 4, hipMemcpyDeviceToHost, ctx->stream));
-    else if (logits_out) { launch_to_host(ctx, ctx->logits, ctx->h_logits, ctx->d.vocab); GL3_HIP(hipGetLastError()); }
+    else if (logits_out && !leave) { launch_to_host(ctx, ctx->logits, ctx->h_logits, ctx->d.vocab); GL3_HIP(hipGetLastError()); }
     GL3_HIP(hipStreamSynchronize(ctx->stream));
     drain.passed = true;
     if ((r = gl3_tp_check(ctx)) != GL3_OK) return r;

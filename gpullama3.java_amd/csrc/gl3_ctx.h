@@ -171,7 +171,7 @@ struct gl3_ctx {
     float *moe_logits = nullptr, *moe_w = nullptr, *moe_hb = nullptr, *moe_y = nullptr;
     int* moe_sel = nullptr;                       // [topk] expert ids, then the router kernel's arrival ticket
     void* moe_slots = nullptr;                    // MoeSlots[n_layers][3]: gate/up with the shared expert merged, gate/up alone, down
-    int *dyn = nullptr, *argmax = nullptr;        // dyn[0] = token, dyn[1] = position
+    int *dyn = nullptr, *argmax = nullptr;        // dyn[0] = token, dyn[1] = position, dyn[2] = the logits' kernel writes the host's copy too
     int* h_dyn = nullptr;                         // pinned
     int* dyn_cur = nullptr;                       // (token, position) pair the next launches read: dyn, or an entry of dyn_seq
     int* dyn_seq = nullptr;                       // [2 * dyn_seq_cap] pairs of a sequential (token-by-token) prefill chunk

@@ -134,6 +134,8 @@ struct MatvecArgs {
     const float* resid_in;   // may be NULL (tensor-parallel ranks > 0)
     float out_scale;         // EPI_STORE / EPI_RESID: the row result is multiplied by this first (1 except Granite: residualScale after wo /
                              // down, logitScale on the logits — InferenceCore.forwardGranite :893-894, :911-912, :921; x * 1.0f is exact)
+    float* host;             // EPI_STORE, may be null: page-locked memory that takes the results too if *host_on (step_token)
+    const int* host_on;
     const struct MoeSlots* moe;   // SEL instantiations only (Qwen2-MoE): what each blockIdx.y slot of the launch works on
     const TpRec* tp;         // tensor parallel, folded gathers: what this launch pushes to the peers / waits for (NULL: nothing)
 };
@@ -494,6 +496,7 @@ __global__ __launch_bounds__(mv_threads(NPW), NPW == 4 ? 4 : 2) void matvec_q8t_
     if (wave != MV_PRODUCERS) return;                    // waves 5-7 retire; wave 4 becomes the chain wavefront
 
     // ---------------------------------------------------------------------- chain wavefront
+    const bool to_host = EPI == EPI_STORE && a.host && *a.host_on;
     int it = 0;
     for (int strip = blockIdx.x; strip < a.nstrips; strip += gridDim.x, ++it) {
         __syncthreads();
@@ -535,6 +538,7 @@ __global__ __launch_bounds__(mv_threads(NPW), NPW == 4 ? 4 : 2) void matvec_q8t_
                     res = gte * v1;
                 }
                 a.out[row] = res;
+                if (EPI == EPI_STORE && to_host) a.host[row] = res;
                 if (TPF) tp_push_store(a.tp->p, a.out + row, res);
             }
         }
@@ -548,14 +552,17 @@ __global__ __launch_bounds__(mv_threads(NPW), NPW == 4 ? 4 : 2) void matvec_q8t_
 // Tokens of a step whose ids the embedding reads over the link itself; more take one copy in front of it, for the link answers a read every ~35 ns (whole steps, us,
 // copy / own reads: batched prompt of 2 tokens 137 / 132, 4 137 / 135, 8 142 / 141; layer-list steps, whose embedding has 8 - 16 workgroups a token: 1 token 112 / 109,
 // 4 152 / 152, 16 143 / 152, 32 146 / 164).
+// A single step's logits go over the link from the kernel that makes them, row by row under the rest of it, where the host takes them as they are (third word of the step's record): a kernel behind
+// the captured step takes 4.6 us for 64 KB and stands some us apart from it.  Four layers, us, a kernel behind / like this: Llama 8B Q8_0, 8 tokens behind 389 2569 / 2546, Llama 1B, one token 182 / 178,
+// 8 tokens and 128256 rows of logits 1877 / 1857, F16 1889 / 1860.
 constexpr int GL3_HOST_TOKENS = 4;
 __device__ __forceinline__ int host_int(const int* p) { return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM); }
 __device__ __forceinline__ int step_token(int* dyn, const int* host) {
     if (!host) return dyn[0];
-    __shared__ int sh[2];          // (one read over the link per workgroup)
-    if (threadIdx.x < 2) sh[threadIdx.x] = host_int(host + threadIdx.x);
+    __shared__ int sh[3];          // (one read over the link per workgroup)
+    if (threadIdx.x < 3) sh[threadIdx.x] = host_int(host + threadIdx.x);
     __syncthreads();
-    if (blockIdx.x == 0 && threadIdx.x < 2) dyn[threadIdx.x] = sh[threadIdx.x];
+    if (blockIdx.x == 0 && threadIdx.x < 3) dyn[threadIdx.x] = sh[threadIdx.x];
     return sh[0];
 }
 // n floats to page-locked host memory; both ends start on 16 bytes

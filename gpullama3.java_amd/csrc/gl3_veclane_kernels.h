@@ -108,6 +108,7 @@ struct VlArgs {
     float* out; const float* resid_in;      // EPI_RESID: out[i] = resid_in[i] + result
     float out_scale;                        // result *= out_scale first (Granite residual / logit scaling; 1 otherwise)
     const float* norm_w; float eps;         // RMS variant: x is the raw residual stream, normalised in the kernel's prologue
+    float* host; const int* host_on;        // as MatvecArgs
     const TpRec* tp;                        // tensor parallel, folded gathers (r6): results also go to the peers' arenas, the last wavefront publishes (NULL: no)
 };
 
@@ -391,6 +392,7 @@ static __global__ __launch_bounds__(64 * VW, WT == WT_F16 ? 1 : 2) void matvec_v
             o = gte * res[NM - 1];
         }
         a.out[row] = o;
+        if (EPI == EPI_STORE && a.host && *a.host_on) a.host[row] = o;
         if (a.tp) tp_push_store(a.tp->p, a.out + row, o);
     }
     if (a.tp && a.tp->p.npeers) tp_publish(a.tp->p, ngroups);      // every live wavefront of the launch reaches its epilogue
@@ -601,6 +603,7 @@ static __global__ __launch_bounds__(64 * MAXW) void matvec_vlq_kernel(const VlAr
             o = gte * res[NM - 1];
         }
         a.out[row] = o;
+        if (EPI == EPI_STORE && a.host && *a.host_on) a.host[row] = o;
         if (a.tp) tp_push_store(a.tp->p, a.out + row, o);
     }
     if (a.tp && a.tp->p.npeers) tp_publish(a.tp->p, gridDim.x);      // wavefront 0 of every workgroup
