@@ -384,7 +384,16 @@ typedef float hy_v16f __attribute__((ext_vector_type(16)));
 // type: gelu_tanh(product) times an entry of a per-token table row (mul_table[mul_rows[m]][mul_col0 + feature], the per-layer token
 // input), or relu(product)^2 alone (act = 2, mul_table = null: a feed-forward without a gate).
 enum { HY_EPI_STORE = 0, HY_EPI_GLU = 1, HY_EPI_ACTMUL = 2 };
-struct HyGlu { float limit, alpha, shift; const void* mul_table; const int* mul_rows; int mul_ld, mul_col0; int act; float cap; };      // act 1: gelu_tanh(g) u; 2: relu(u)^2, no gate; cap: plain products of a few tokens become cap tanh(. / cap)
+struct HyGlu { float limit, alpha, shift; const void* mul_table; const int* mul_rows; int mul_ld, mul_col0; int act; float cap; float* host; };      // act 1: gelu_tanh(g) u; 2: relu(u)^2, no gate; cap: plain products of a few tokens become cap tanh(. / cap)
+// One token's plain results of two rows.  glu.host (one token's logits): they also go over the link to page-locked memory, from the kernel that makes them.
+__device__ __forceinline__ void hy_put2(float* C, int r0, bool has1, float s0, float s1, const HyGlu& glu) {
+    if (glu.cap > 0.f) { s0 = glu.cap * tanhf(s0 / glu.cap); s1 = glu.cap * tanhf(s1 / glu.cap); }
+    C[r0] = s0;
+    if (has1) C[r0 + 1] = s1;
+    if (glu.host) {          // (r0 is even)
+        if (has1) *reinterpret_cast<float2*>(glu.host + r0) = make_float2(s0, s1); else glu.host[r0] = s0;
+    }
+}
 __device__ __forceinline__ float hy_gelu_tanh(float z) { return 0.5f * z * (1.f + tanhf(0.7978845608028654f * (z + 0.044715f * z * z * z))); }
 template <typename T>
 __device__ __forceinline__ float hy_actmul(float a, int m, int feature, const HyGlu& p) {
@@ -679,8 +688,11 @@ __device__ __forceinline__ void hy_matvec(int bx, int by, const T* __restrict__ 
                 hy_st(act + (size_t)m * ld_act + r0, hy_actmul<T>(a0[m], m, r0, glu));
                 if (has1) hy_st(act + (size_t)m * ld_act + r1, hy_actmul<T>(a1[m], m, r1, glu));
             } else {
-                C[(size_t)m * ldc + r0] = glu.cap > 0.f ? glu.cap * tanhf(a0[m] / glu.cap) : a0[m];
-                if (has1) C[(size_t)m * ldc + r1] = glu.cap > 0.f ? glu.cap * tanhf(a1[m] / glu.cap) : a1[m];
+                if constexpr (MT == 1) hy_put2(C, r0, has1, a0[m], a1[m], glu);
+                else {
+                    C[(size_t)m * ldc + r0] = glu.cap > 0.f ? glu.cap * tanhf(a0[m] / glu.cap) : a0[m];
+                    if (has1) C[(size_t)m * ldc + r1] = glu.cap > 0.f ? glu.cap * tanhf(a1[m] / glu.cap) : a1[m];
+                }
             }
         }
     }

@@ -34,9 +34,10 @@ static __global__ __launch_bounds__(1024) void hy_matvec_pre_kernel(HyPre p, con
     __shared__ __attribute__((aligned(16))) T sh[4096];
     __shared__ float red[16], part[HY_PRE_SPLIT_PAIRS * 4][2];
     const int K = p.W, tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int pairs = (N + 1) >> 1, mine = (int)blockIdx.x < pairs ? (pairs - 1 - (int)blockIdx.x) / (int)gridDim.x + 1 : 0;          // pairs blockIdx.x + i gridDim.x
+    const int pairs = (N + 1) >> 1, each = pairs / (int)gridDim.x, over = pairs % (int)gridDim.x;
+    const int pair0 = (int)blockIdx.x * each + min((int)blockIdx.x, over), mine = each + ((int)blockIdx.x < over);          // pairs in a row, so that results leave in whole lines
     const int kp = wave % KS, slots = 16 / KS, first = wave / KS, chunks = (K + UN * STEP - 1) / (UN * STEP), todo = first < mine ? ((mine - 1 - first) / slots + 1) * chunks : 0;
-    auto row0 = [&](int i) { const int pr = blockIdx.x + i * gridDim.x; return EPI == HY_EPI_GLU ? (pr >> 5) * 64 + (pr & 31) : 2 * pr; };
+    auto row0 = [&](int i) { const int pr = pair0 + i; return EPI == HY_EPI_GLU ? (pr >> 5) * 64 + (pr & 31) : 2 * pr; };
     auto row1 = [&](int r0) { return EPI == HY_EPI_GLU ? r0 + 32 : r0 + 1; };
     uint4 a[2][UN], b[2][UN];
     auto fetch = [&](int set, int q) {          // chunk q of this wavefront's walk (places past K repeat the last one: not multiplied)
@@ -126,8 +127,7 @@ static __global__ __launch_bounds__(1024) void hy_matvec_pre_kernel(HyPre p, con
             hy_st(act + r0, hy_actmul<T>(s0, 0, r0, glu));
             if (has1) hy_st(act + r1, hy_actmul<T>(s1, 0, r1, glu));
         } else {
-            C[r0] = glu.cap > 0.f ? glu.cap * tanhf(s0 / glu.cap) : s0;
-            if (has1) C[r1] = glu.cap > 0.f ? glu.cap * tanhf(s1 / glu.cap) : s1;
+            hy_put2(C, r0, has1, s0, s1, glu);
         }
     };
     float a0 = 0.f, a1 = 0.f;

@@ -1879,13 +1879,14 @@ static void hy_moe(gl3_ctx* ctx, HyLayer& L, int n) {
 // logits of the nw rows listed in h->want: final norm of the gathered rows (normed: the last sublayer's update has left it in h->xw), the head's product, the
 // optional cap * tanh(. / cap) (a few rows: in the product)
 template <typename T>
-static void hy_logits(gl3_ctx* ctx, int nw, bool normed = false) {
+static void hy_logits(gl3_ctx* ctx, int nw, bool normed = false) {          // one row: to h->leave too where that is set
     gl3_hybrid_state* h = ctx->hy;
     T* xw = (T*)h->xw;
     if (!normed) hy_streams<T>(ctx, nw, h->X, h->W, h->S, (size_t)h->mb * h->W, (const float*)nullptr, 1, 0, (const float*)nullptr, (const float*)nullptr,
                   h->ones, h->final_norm, ctx->d.rms_eps, xw, (float*)nullptr, h->want);
     HyGlu g{};
     if (nw <= 4) g.cap = h->softcap;
+    if (nw == 1) g.host = h->leave;
     hy_gemm<T>(ctx, xw, h->W, h->head, nw, h->logits, ctx->d.vocab, false, nullptr, 0, g);
     if (h->softcap > 0.f && nw > 4) {
         const size_t cnt = (size_t)nw * ctx->d.vocab;
@@ -2127,6 +2128,7 @@ int32_t gl3_hy_step(gl3_ctx* ctx, int32_t seq, const int32_t* tokens, int32_t n,
             std::vector<int32_t> rel(std::max(g, 1));
             for (int i = 0; i < g; ++i) rel[i] = want[done + i] - off;
             int32_t r;
+            h->leave = g == 1 && logits_out ? h->h_logits : nullptr;
             if (!ran) {
                 if (h->plain)
                     r = h->f32 ? hy_portion_plain<float>(ctx, seq, tokens + off, pn, start_pos + off, rel.data(), g)
@@ -2143,7 +2145,7 @@ int32_t gl3_hy_step(gl3_ctx* ctx, int32_t seq, const int32_t* tokens, int32_t n,
             }
             if (r != GL3_OK) return r;
             h->last_tok[seq] = tokens[off + pn - 1];
-            if (g > 0 && logits_out) {
+            if (g > 1 && logits_out) {
                 launch_to_host(ctx, h->logits, h->h_logits, (size_t)g * V);
                 HY_HIP(hipGetLastError());
             }
