@@ -951,8 +951,11 @@ __host__ __device__ inline size_t attn_head_smem(int hs, int group = 1) {
 }
 
 // HS: head size as a compile-time constant (64 / 128: LDS row strides become immediate offsets and the index arithmetic folds), 0 = a.hs
-template <int HS>
-static __global__ __launch_bounds__(256, 1) void attn_head_kernel(const AttnArgs a) {
+// NT: 256 threads for one query head, 512 for a group: its (head, position) and (head, column) pairs then take one pass each instead of two, and the chip has one workgroup per CU anyway
+// (LDS).  Bound: strictly ordered chains (scores head_size terms, sums and outputs `positions` terms), so their operands are read from LDS a group of four quads ahead.
+// 32 sequences x 8 groups of four heads of 128 behind 117 positions: 20.2 us on 256 threads with reads one quad ahead, 16.3 like this.
+template <int HS, int NT>
+static __global__ __launch_bounds__(NT, 1) void attn_head_kernel(const AttnArgs a) {
     extern __shared__ __attribute__((aligned(16))) float sm[];
     const int hs = HS > 0 ? HS : a.hs, kvmul = a.n_heads / a.n_kv_heads, half = hs >> 1, pitch = hs + 4, q4 = hs >> 2;
     // float4 index -> (row, column quad) of a K / V tile: shift / mask for the power-of-two head sizes, division otherwise
@@ -981,32 +984,32 @@ static __global__ __launch_bounds__(256, 1) void attn_head_kernel(const AttnArgs
     ATT_STAMP(0);
     // ---- one global round trip: cached K / V rows (both in flight at once), raw q / k / v of this token, the RoPE row
     const int nk4 = pos * q4;
-    constexpr int KMAX = 16;                         // 127 rows x 32 float4 / 256 threads (head_size 128)
+    constexpr int KMAX = 4096 / NT;                  // 127 rows x 32 float4 (head_size 128)
     float4 kreg[KMAX], vreg[KMAX];                   // initialised + uniform condition + clamped index: stays in VGPRs (see attn_scores_kernel)
-    const bool in_regs = nk4 <= KMAX * 256;
-    const int per = in_regs ? (nk4 + 255) >> 8 : 0;
+    const bool in_regs = nk4 <= KMAX * NT;
+    const int per = in_regs ? (nk4 + NT - 1) / NT : 0;
 #pragma unroll
     for (int u = 0; u < KMAX; ++u) {
         kreg[u] = make_float4(0.f, 0.f, 0.f, 0.f);
         vreg[u] = make_float4(0.f, 0.f, 0.f, 0.f);
         if (u < per) {
-            const int i = min(t + u * 256, nk4 - 1), ri = row_of(i);
+            const int i = min(t + u * NT, nk4 - 1), ri = row_of(i);
             const size_t off = (size_t)ri * a.kv_dim + kvh * hs + 4 * col_of(i, ri);
             kreg[u] = *reinterpret_cast<const float4*>(kcache + off);
             vreg[u] = *reinterpret_cast<const float4*>(vcache + off);
         }
     }
-    for (int i = t; i < G * hs; i += 256) q_s[i] = a.bq ? qkv[h0 * hs + i] + a.bq[h0 * hs + i] : qkv[h0 * hs + i];
-    for (int i = t; i < half; i += 256) { cr_s[i] = a.rope_cr[(size_t)pos * half + i]; ci_s[i] = a.rope_ci[(size_t)pos * half + i]; }
+    for (int i = t; i < G * hs; i += NT) q_s[i] = a.bq ? qkv[h0 * hs + i] + a.bq[h0 * hs + i] : qkv[h0 * hs + i];
+    for (int i = t; i < half; i += NT) { cr_s[i] = a.rope_cr[(size_t)pos * half + i]; ci_s[i] = a.rope_ci[(size_t)pos * half + i]; }
     float* krow = kt + pos * pitch;
-    for (int i = t; i < hs; i += 256) {
+    for (int i = t; i < hs; i += NT) {
         krow[i] = a.bk ? qkv[a.q_dim + kvh * hs + i] + a.bk[kvh * hs + i] : qkv[a.q_dim + kvh * hs + i];
         vt[pos * hs + i] = a.bv ? qkv[a.q_dim + a.kv_dim + kvh * hs + i] + a.bv[kvh * hs + i] : qkv[a.q_dim + a.kv_dim + kvh * hs + i];
     }
     if (in_regs) {
 #pragma unroll
         for (int u = 0; u < KMAX; ++u) {
-            const int i = t + u * 256;
+            const int i = t + u * NT;
             if (i < nk4) {
                 const int ri = row_of(i), ci = col_of(i, ri);
                 *reinterpret_cast<float4*>(kt + ri * pitch + 4 * ci) = kreg[u];
@@ -1014,7 +1017,7 @@ static __global__ __launch_bounds__(256, 1) void attn_head_kernel(const AttnArgs
             }
         }
     } else {                                         // head_size 256: straight to LDS
-        for (int i = t; i < nk4; i += 256) {
+        for (int i = t; i < nk4; i += NT) {
             const int ri = row_of(i), ci = col_of(i, ri);
             const size_t off = (size_t)ri * a.kv_dim + kvh * hs + 4 * ci;
             *reinterpret_cast<float4*>(kt + ri * pitch + 4 * ci) = *reinterpret_cast<const float4*>(kcache + off);
@@ -1024,15 +1027,15 @@ static __global__ __launch_bounds__(256, 1) void attn_head_kernel(const AttnArgs
     __syncthreads();
     ATT_STAMP(1);
     if (a.arch == 1) {                               // qwen3: per-head RMSNorm of q and k (strict-order sum, one wavefront per head)
-        for (int vec = wave; vec <= G; vec += 4)                   // G query heads + the key: one wavefront each
+        for (int vec = wave; vec <= G; vec += NT / 64)                   // G query heads + the key: one wavefront each
             head_rmsnorm_wave(vec < G ? q_s + vec * hs : krow, vec < G ? a.qnorm : a.knorm, hs, a.eps, lane);
         __syncthreads();
     }
-    for (int g = 0; g < G; ++g) rope_head(q_s + g * hs, hs, cr_s, ci_s, a.arch, t, 256);
-    rope_head(krow, hs, cr_s, ci_s, a.arch, t, 256);
+    for (int g = 0; g < G; ++g) rope_head(q_s + g * hs, hs, cr_s, ci_s, a.arch, t, NT);
+    rope_head(krow, hs, cr_s, ci_s, a.arch, t, NT);
     __syncthreads();
     if (owner) {                                     // KV write, InferenceCore.java:92-93
-        for (int i = t; i < hs; i += 256) {
+        for (int i = t; i < hs; i += NT) {
             kcache[(size_t)pos * a.kv_dim + kvh * hs + i] = krow[i];
             vcache[(size_t)pos * a.kv_dim + kvh * hs + i] = vt[pos * hs + i];
         }
@@ -1041,24 +1044,43 @@ static __global__ __launch_bounds__(256, 1) void attn_head_kernel(const AttnArgs
     // ---- scores: one (query head, timestep) pair per thread and pass; strict j order, mul then add (FloatTensor.scalarDot)
     const float sqrt_hs = (float)sqrt((double)hs);
     float sc = -INFINITY;                            // group == 1: this thread's score (timestep t)
-    for (int idx = t; idx < G * n; idx += 256) {
+    for (int idx = t; idx < G * n; idx += NT) {
         const int g = idx / n, tt = idx - g * n;
         const float* q = q_s + g * hs;
         const float* kk = kt + tt * pitch;
         float score = 0.f;
-        float4 qv = *reinterpret_cast<const float4*>(q), kv = *reinterpret_cast<const float4*>(kk);
-        for (int j = 4; j < hs; j += 4) {
-            const float4 qn = *reinterpret_cast<const float4*>(q + j), kn = *reinterpret_cast<const float4*>(kk + j);
-            score = score + qv.x * kv.x; score = score + qv.y * kv.y; score = score + qv.z * kv.z; score = score + qv.w * kv.w;
-            qv = qn; kv = kn;
-        }
-        score = score + qv.x * kv.x; score = score + qv.y * kv.y; score = score + qv.z * kv.z; score = score + qv.w * kv.w;
+        const float4 *q4p = reinterpret_cast<const float4*>(q), *k4p = reinterpret_cast<const float4*>(kk);
+        auto use = [&](const float4& qv, const float4& kv) {
+            score = score + mul_f32_scalar(qv.x, kv.x); score = score + mul_f32_scalar(qv.y, kv.y); score = score + mul_f32_scalar(qv.z, kv.z); score = score + mul_f32_scalar(qv.w, kv.w);
+        };
+        if constexpr (HS > 0) {                      // (the sched_barriers keep the reads ahead, as in attn_scores_loop_kernel)
+            float4 qa[4], ka[4], qb[4], kb[4];
+            auto rd = [&](float4 (&Q)[4], float4 (&K)[4], int c) {
+#pragma unroll
+                for (int u = 0; u < 4; ++u) { Q[u] = q4p[c + u]; K[u] = k4p[c + u]; }
+            };
+            rd(qa, ka, 0);
+#pragma unroll
+            for (int c = 0; c < HS / 4; c += 8) {
+                rd(qb, kb, c + 4);
+                __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+                for (int u = 0; u < 4; ++u) use(qa[u], ka[u]);
+                __builtin_amdgcn_sched_barrier(0);
+                if (c + 8 < HS / 4) rd(qa, ka, c + 8);
+                __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+                for (int u = 0; u < 4; ++u) use(qb[u], kb[u]);
+                __builtin_amdgcn_sched_barrier(0);
+            }
+        } else
+            for (int j = 0; j < q4; ++j) use(q4p[j], k4p[j]);
         sc = a.att_mul != 0.f ? score * a.att_mul : score / sqrt_hs;
         if (G > 1) e_s[g * AF_MAXN + tt] = sc;
     }
     ATT_STAMP(3);
     // ---- softmax (FloatTensor.softmaxInPlace :211-219): max, exp in double, strict sum, divide
-    if (G == 1) {                                    // one head: all timesteps in parallel across the workgroup
+    if (NT == 256 && G == 1) {                       // one head: all timesteps in parallel across the workgroup
         {
             const float wm = wave_max(t < n ? sc : -INFINITY);
             if (lane == 0) red[wave] = wm;
@@ -1075,7 +1097,7 @@ static __global__ __launch_bounds__(256, 1) void attn_head_kernel(const AttnArgs
         __syncthreads();
     } else {                                         // a group: one wavefront per head, everything wave-local (LDS runs a wavefront in order)
         __syncthreads();
-        for (int g = wave; g < G; g += 4) {
+        for (int g = wave; g < G; g += NT / 64) {
             float* e = e_s + g * AF_MAXN;
             const float s0 = lane < n ? e[lane] : -INFINITY, s1 = lane + 64 < n ? e[lane + 64] : -INFINITY;
             const float mx = wave_max(fmaxf(s0, s1));
@@ -1094,7 +1116,7 @@ static __global__ __launch_bounds__(256, 1) void attn_head_kernel(const AttnArgs
     }
     ATT_STAMP(5);
     // ---- weighted V sum, t ascending: xb[j] = a_t * v[t][j] + xb[j] (saxpyInPlace :221-227); one (head, output column) per thread and pass
-    for (int idx = t; idx < G * hs; idx += 256) {
+    for (int idx = t; idx < G * hs; idx += NT) {
         const int g = idx / hs, j = idx - g * hs;
         const float* e = e_s + g * AF_MAXN;
         const float* vj = vt + j;
@@ -1155,15 +1177,15 @@ static __global__ __launch_bounds__(256, 1) void attn_head_kernel(const AttnArgs
         }
     }
     ATT_STAMP(6);
-    if (a.tp) tp_publish(a.tp->p, gridDim.x * gridDim.y * 4);
+    if (a.tp) tp_publish(a.tp->p, gridDim.x * gridDim.y * (NT / 64));
 }
 
 // Picks the instantiation for the head size (host side).
-template <typename F>
+template <int NT, typename F>
 static inline void attn_head_dispatch(int hs, F&& f) {
-    if (hs == 128) f(attn_head_kernel<128>);
-    else if (hs == 64) f(attn_head_kernel<64>);
-    else f(attn_head_kernel<0>);
+    if (hs == 128) f(attn_head_kernel<128, NT>);
+    else if (hs == 64) f(attn_head_kernel<64, NT>);
+    else f(attn_head_kernel<0, NT>);
 }
 
 // Decode attention, part 2: softmax + weighted V sum.   Grid = n_heads x hs/16, block = 256.

@@ -117,9 +117,20 @@ __global__ __launch_bounds__(256) void pf_norm_quant_kernel(const float* __restr
     auto xquad = [&](int qd) { return *reinterpret_cast<const float4*>(in + chunked(b, 4 * qd, cc, nt)); };
     const int nquads = k >> 2;
     float scale = 1.0f;
+    constexpr int QN = 5;                                        // rows of up to 5120 and their norm weights: on their way together, read once (32 rows of 2560: 7.2 -> 6.3 us)
+    float4 xr[QN], wr[QN];
+    const bool in_regs = NORM && nquads <= QN * 256;
     if (NORM) {
-        for (int qd = t; qd < nquads; qd += 256)
-            *reinterpret_cast<float4*>(xf + 4 * qd) = xquad(qd);
+        if (in_regs) {                                           // (uniform conditions and clamped places: see attn_scores_kernel)
+#pragma unroll
+            for (int u = 0; u < QN; ++u) { xr[u] = make_float4(0.f, 0.f, 0.f, 0.f); if (u * 256 < nquads) xr[u] = xquad(min(t + u * 256, nquads - 1)); }
+#pragma unroll
+            for (int u = 0; u < QN; ++u) { wr[u] = make_float4(0.f, 0.f, 0.f, 0.f); if (u * 256 < nquads) wr[u] = *reinterpret_cast<const float4*>(norm_w + 4 * min(t + u * 256, nquads - 1)); }
+#pragma unroll
+            for (int u = 0; u < QN; ++u) if (t + u * 256 < nquads) *reinterpret_cast<float4*>(xf + 4 * (t + u * 256)) = xr[u];
+        } else
+            for (int qd = t; qd < nquads; qd += 256)
+                *reinterpret_cast<float4*>(xf + 4 * qd) = xquad(qd);
         if (t < 32) xf[k + t] = 0.f;
         __syncthreads();
         float ss;
@@ -137,16 +148,11 @@ __global__ __launch_bounds__(256) void pf_norm_quant_kernel(const float* __restr
     }
     uint8_t* xq = XQ + (size_t)b * maxk;
     float* xs = XS + (size_t)b * (maxk >> 5);
-    for (int qd = t + 256 * blockIdx.y; qd < nquads; qd += 256 * gridDim.y) {
-        float4 v;
+    auto emit = [&](const int qd, float4 v, const float4 w) {
         if (NORM) {
-            v = *reinterpret_cast<const float4*>(xf + 4 * qd);
-            const float4 w = *reinterpret_cast<const float4*>(norm_w + 4 * qd);
             v.x = w.x * (scale * v.x); v.y = w.y * (scale * v.y); v.z = w.z * (scale * v.z); v.w = w.w * (scale * v.w);
-        } else {
-            v = xquad(qd);
         }
-        if (MODE == PQ_NORM_F32 || MODE == PQ_PLAIN_F32) { *reinterpret_cast<float4*>(XS + (size_t)b * k + 4 * qd) = v; continue; }
+        if (MODE == PQ_NORM_F32 || MODE == PQ_PLAIN_F32) { *reinterpret_cast<float4*>(XS + (size_t)b * k + 4 * qd) = v; return; }
         if (tslots == 0) {
             float qs;
             const uint32_t packed = quantize_quad_pack(v, qs);
@@ -179,7 +185,15 @@ __global__ __launch_bounds__(256) void pf_norm_quant_kernel(const float* __restr
             *reinterpret_cast<uint32_t*>(XQ + bdq_offset(qd, b, tslots)) = packed;
             if ((qd & 7) == 0) XS[bds_offset(qd >> 3, b, tslots)] = qs;
         }
-    }
+    };
+    if (in_regs) {
+#pragma unroll
+        for (int u = 0; u < QN; ++u) if (t + u * 256 < nquads) emit(t + u * 256, xr[u], wr[u]);
+    } else
+        for (int qd = t + 256 * blockIdx.y; qd < nquads; qd += 256 * gridDim.y) {
+            if (NORM) emit(qd, *reinterpret_cast<const float4*>(xf + 4 * qd), *reinterpret_cast<const float4*>(norm_w + 4 * qd));
+            else emit(qd, xquad(qd), float4{});
+        }
 }
 
 
@@ -2456,7 +2470,8 @@ static bool pf_attention(gl3_ctx* ctx, int l, int n, int max_pos, int one_seq, f
         ha.eps = d.rms_eps; ha.arch = ctx->rope_arch; ha.att_mul = ctx->att_mul; ha.seqv = seq; ha.posv = pos; ha.seq_stride = ctx->kv_seq_stride;
         ha.group = bd_group;
         if (fuse_q) { ha.xq_out = p->XQ; ha.xs_out = p->XS; ha.xq_slots = bd_tslots(n); }
-        attn_head_dispatch(hs, [&](auto kern) { hipLaunchKernelGGL(kern, dim3(H / bd_group, n), dim3(256), attn_head_smem(hs, bd_group), s, ha); });
+        if (bd_group > 1) attn_head_dispatch<512>(hs, [&](auto kern) { hipLaunchKernelGGL(kern, dim3(H / bd_group, n), dim3(512), attn_head_smem(hs, bd_group), s, ha); });
+        else attn_head_dispatch<256>(hs, [&](auto kern) { hipLaunchKernelGGL(kern, dim3(H, n), dim3(256), attn_head_smem(hs, 1), s, ha); });
         return fuse_q;
     }
     hipLaunchKernelGGL(pf_rope_kv_kernel, dim3(H + KVH, n), dim3(64), 0, s, ra);
