@@ -736,8 +736,8 @@ int32_t gl3_create(const gl3_model_desc* desc, gl3_ctx** out) {
     TRYHIP((allow_big_lds<PRO_QUANT, EPI_RESID>()));
     TRYHIP((allow_big_lds<PRO_RMS, EPI_SWIGLU>()));
     {
-        // one launch per layer for positions < AF_MAXN (attn_head_kernel); head_size 256 does not fit its K / V tiles in LDS
-        ctx->fused_attn_ok = d.head_size % 4 == 0 && attn_head_smem(d.head_size) <= 150 * 1024 && !env_flag("GL3_NO_FUSED_ATTN", false);
+        // one launch per layer for positions < AF_MAXN (attn_head_kernel); heads of more than 128 do not fit its K / V tiles in LDS
+        ctx->fused_attn_ok = attn_head_built(d.head_size) && !env_flag("GL3_NO_FUSED_ATTN", false);
         if (ctx->fused_attn_ok) {
             hipError_t ae = hipSuccess;
             attn_head_dispatch<256>(d.head_size, [&](auto kern) { ae = hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024 - 256); });

@@ -950,19 +950,20 @@ __host__ __device__ inline size_t attn_head_smem(int hs, int group = 1) {
     return ((size_t)group * hs + (size_t)AF_MAXN * (hs + 4) + (size_t)AF_MAXN * hs + (size_t)group * AF_MAXN + hs + 16) * 4;
 }
 
-// HS: head size as a compile-time constant (64 / 128: LDS row strides become immediate offsets and the index arithmetic folds), 0 = a.hs
+// HS: head size (gl3_create takes multiples of 32; more than 128 do not fit): LDS row strides are immediate offsets, the index arithmetic folds and the loop over the head's quads is
+// unrolled around its reads ahead.  (One token behind 20 / 60 / 126, us: 32 heads of 96 with the size read at run time and every quad when it is
+// used 7.9 / 9.5 / 12.5, one quad ahead 6.9 / 8.6 / 11.4, like this 5.7 / 6.5 / 8.4; 32 heads of 32 6.3 / 7.2 / 9.0, 6.1 / 7.0 / 8.8, 4.8 / 5.4 / 6.6.)
 // NT: 256 threads for one query head, 512 for a group: its (head, position) and (head, column) pairs then take one pass each instead of two, and the chip has one workgroup per CU anyway
 // (LDS).  Bound: strictly ordered chains (scores head_size terms, sums and outputs `positions` terms), so their operands are read from LDS a group of four quads ahead.
 // 32 sequences x 8 groups of four heads of 128 behind 117 positions: 20.2 us on 256 threads with reads one quad ahead, 16.3 like this.
 template <int HS, int NT>
 static __global__ __launch_bounds__(NT, 1) void attn_head_kernel(const AttnArgs a) {
     extern __shared__ __attribute__((aligned(16))) float sm[];
-    const int hs = HS > 0 ? HS : a.hs, kvmul = a.n_heads / a.n_kv_heads, half = hs >> 1, pitch = hs + 4, q4 = hs >> 2;
-    // float4 index -> (row, column quad) of a K / V tile: shift / mask for the power-of-two head sizes, division otherwise
-    // (head_size 96: Phi-3-mini / Phi-3.5-mini, forwardJavaPhi3 with headSize = dim / heads)
-    const int q4sh = (q4 & (q4 - 1)) == 0 ? __ffs(q4) - 1 : -1;
-    auto row_of = [&](int i) { return q4sh >= 0 ? i >> q4sh : i / q4; };
-    auto col_of = [&](int i, int row) { return q4sh >= 0 ? i & (q4 - 1) : i - row * q4; };
+    constexpr int hs = HS, half = hs >> 1, pitch = hs + 4, q4 = hs >> 2;
+    const int kvmul = a.n_heads / a.n_kv_heads;
+    // float4 index -> (row, column quad) of a K / V tile
+    auto row_of = [](int i) { return i / q4; };
+    auto col_of = [](int i, int row) { return i - row * q4; };
     const int G = a.group > 1 ? a.group : 1;
     float* q_s = sm;                                 // [G][hs]
     float* kt = q_s + G * hs;
@@ -984,10 +985,10 @@ static __global__ __launch_bounds__(NT, 1) void attn_head_kernel(const AttnArgs 
     ATT_STAMP(0);
     // ---- one global round trip: cached K / V rows (both in flight at once), raw q / k / v of this token, the RoPE row
     const int nk4 = pos * q4;
-    constexpr int KMAX = 4096 / NT;                  // 127 rows x 32 float4 (head_size 128)
+    constexpr int KMAX = HS * AF_MAXN / 4 / NT;      // (127 rows; of 128: 32 float4 each)
+    static_assert(HS % 32 == 0 && KMAX * NT >= (AF_MAXN - 1) * q4, "cached rows of a head in registers");
     float4 kreg[KMAX], vreg[KMAX];                   // initialised + uniform condition + clamped index: stays in VGPRs (see attn_scores_kernel)
-    const bool in_regs = nk4 <= KMAX * NT;
-    const int per = in_regs ? (nk4 + NT - 1) / NT : 0;
+    const int per = (nk4 + NT - 1) / NT;
 #pragma unroll
     for (int u = 0; u < KMAX; ++u) {
         kreg[u] = make_float4(0.f, 0.f, 0.f, 0.f);
@@ -1006,22 +1007,13 @@ static __global__ __launch_bounds__(NT, 1) void attn_head_kernel(const AttnArgs 
         krow[i] = a.bk ? qkv[a.q_dim + kvh * hs + i] + a.bk[kvh * hs + i] : qkv[a.q_dim + kvh * hs + i];
         vt[pos * hs + i] = a.bv ? qkv[a.q_dim + a.kv_dim + kvh * hs + i] + a.bv[kvh * hs + i] : qkv[a.q_dim + a.kv_dim + kvh * hs + i];
     }
-    if (in_regs) {
 #pragma unroll
-        for (int u = 0; u < KMAX; ++u) {
-            const int i = t + u * NT;
-            if (i < nk4) {
-                const int ri = row_of(i), ci = col_of(i, ri);
-                *reinterpret_cast<float4*>(kt + ri * pitch + 4 * ci) = kreg[u];
-                *reinterpret_cast<float4*>(vt + ri * hs + 4 * ci) = vreg[u];
-            }
-        }
-    } else {                                         // head_size 256: straight to LDS
-        for (int i = t; i < nk4; i += NT) {
+    for (int u = 0; u < KMAX; ++u) {
+        const int i = t + u * NT;
+        if (i < nk4) {
             const int ri = row_of(i), ci = col_of(i, ri);
-            const size_t off = (size_t)ri * a.kv_dim + kvh * hs + 4 * ci;
-            *reinterpret_cast<float4*>(kt + ri * pitch + 4 * ci) = *reinterpret_cast<const float4*>(kcache + off);
-            *reinterpret_cast<float4*>(vt + ri * hs + 4 * ci) = *reinterpret_cast<const float4*>(vcache + off);
+            *reinterpret_cast<float4*>(kt + ri * pitch + 4 * ci) = kreg[u];
+            *reinterpret_cast<float4*>(vt + ri * hs + 4 * ci) = vreg[u];
         }
     }
     __syncthreads();
@@ -1053,28 +1045,25 @@ static __global__ __launch_bounds__(NT, 1) void attn_head_kernel(const AttnArgs 
         auto use = [&](const float4& qv, const float4& kv) {
             score = score + mul_f32_scalar(qv.x, kv.x); score = score + mul_f32_scalar(qv.y, kv.y); score = score + mul_f32_scalar(qv.z, kv.z); score = score + mul_f32_scalar(qv.w, kv.w);
         };
-        if constexpr (HS > 0) {                      // (the sched_barriers keep the reads ahead, as in attn_scores_loop_kernel)
-            float4 qa[4], ka[4], qb[4], kb[4];
-            auto rd = [&](float4 (&Q)[4], float4 (&K)[4], int c) {
+        float4 qa[4], ka[4], qb[4], kb[4];           // (the sched_barriers keep the reads ahead, as in attn_scores_loop_kernel)
+        auto rd = [&](float4 (&Q)[4], float4 (&K)[4], int c) {
 #pragma unroll
-                for (int u = 0; u < 4; ++u) { Q[u] = q4p[c + u]; K[u] = k4p[c + u]; }
-            };
-            rd(qa, ka, 0);
+            for (int u = 0; u < 4; ++u) { Q[u] = q4p[c + u]; K[u] = k4p[c + u]; }
+        };
+        rd(qa, ka, 0);
 #pragma unroll
-            for (int c = 0; c < HS / 4; c += 8) {
-                rd(qb, kb, c + 4);
-                __builtin_amdgcn_sched_barrier(0);
+        for (int c = 0; c < q4; c += 8) {
+            rd(qb, kb, c + 4);
+            __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-                for (int u = 0; u < 4; ++u) use(qa[u], ka[u]);
-                __builtin_amdgcn_sched_barrier(0);
-                if (c + 8 < HS / 4) rd(qa, ka, c + 8);
-                __builtin_amdgcn_sched_barrier(0);
+            for (int u = 0; u < 4; ++u) use(qa[u], ka[u]);
+            __builtin_amdgcn_sched_barrier(0);
+            if (c + 8 < q4) rd(qa, ka, c + 8);
+            __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-                for (int u = 0; u < 4; ++u) use(qb[u], kb[u]);
-                __builtin_amdgcn_sched_barrier(0);
-            }
-        } else
-            for (int j = 0; j < q4; ++j) use(q4p[j], k4p[j]);
+            for (int u = 0; u < 4; ++u) use(qb[u], kb[u]);
+            __builtin_amdgcn_sched_barrier(0);
+        }
         sc = a.att_mul != 0.f ? score * a.att_mul : score / sqrt_hs;
         if (G > 1) e_s[g * AF_MAXN + tt] = sc;
     }
@@ -1181,11 +1170,13 @@ static __global__ __launch_bounds__(NT, 1) void attn_head_kernel(const AttnArgs 
 }
 
 // Picks the instantiation for the head size (host side).
+static inline bool attn_head_built(int hs) { return hs == 32 || hs == 64 || hs == 96 || hs == 128; }
 template <int NT, typename F>
 static inline void attn_head_dispatch(int hs, F&& f) {
     if (hs == 128) f(attn_head_kernel<128, NT>);
+    else if (hs == 96) f(attn_head_kernel<96, NT>);
     else if (hs == 64) f(attn_head_kernel<64, NT>);
-    else f(attn_head_kernel<0, NT>);
+    else f(attn_head_kernel<32, NT>);
 }
 
 // Decode attention, part 2: softmax + weighted V sum.   Grid = n_heads x hs/16, block = 256.

@@ -1,4 +1,4 @@
-"""Static-batched decode where a workgroup serves a group of query heads (attn_head_kernel on 512 threads): head sizes with kernels of their own (64, 128) and without (32, 96), groups of 2 to 8 heads,
+"""Static-batched decode where a workgroup serves a group of query heads (attn_head_kernel on 512 threads): head sizes 32, 64, 96 and 128, groups of 2 to 8 heads,
 positions around whole quads, wavefronts and the launch's last one (127); and the norm in front of the products at the widest row that stays in registers (5120), beyond it, and where the last quad
 of a thread is missing.  Yardstick: the CPU oracle, bit for bit."""
 import dataclasses
