@@ -35,9 +35,7 @@ typedef float hy_v4f __attribute__((ext_vector_type(4)));
 __device__ __forceinline__ void hy_dma16(const void* src, void* lds_wave_base) {
     __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)src, (__attribute__((address_space(3))) void*)lds_wave_base, 16, 0, 0);
 }
-// The same for W, which leaves HBM once (the row tiles that share a tile of it run side by side on one XCD).  bfloat16: past the caches.  Prompts, us, without / with: Kosusun 8B, 600 tokens 1321 / 1272,
-// 88 460 / 439, Noditar 8B 30 tokens 441 / 420, 200 650 / 654, 512 967 / 957.  float32 row tiles are smaller and more of them read a tile again: experts' tiles
-// of 32 rows alone (Kugadra 1B: 12 tokens 789 / 774, 60 852 / 831, 181 1339 / 1342; every product: 60 tokens 854 / 828, but 181 1333 / 1355, 480 1327 / 1344).
+// The same for W; ONCE: past the caches (hy_ring_once).
 template <bool ONCE>
 __device__ __forceinline__ void hy_dma16_w(const void* src, void* lds_wave_base) {
     __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)src, (__attribute__((address_space(3))) void*)lds_wave_base, 16, 0, ONCE ? 2 : 0);
@@ -106,7 +104,7 @@ __device__ __attribute__((noinline)) hy_v16f hy_tile_again(hy_v16f c, uint32_t o
 
 // WM x WN wavefronts, BM x BN results; EPI, GR and HyGroup as for hy_gemm_kernel (GR: blockIdx.y = row tile of the list, BM rows at most).
 // Grid: x = mt nt ks workgroups (row tiles x column tiles x K splits of kper) rounded up to a multiple of 8; GR: x = column tiles.
-template <typename T, int BM, int BN, int WM, int WN, int SA, int SW, int EPI, int GR = 0, int WP = 3>
+template <typename T, int BM, int BN, int WM, int WN, int SA, int SW, int EPI, int GR, int WP, bool ONCE>
 static __global__ __launch_bounds__(WM * WN * 64, sizeof(T) == 4 ? 2 : 1) void hy_gemm_ring_kernel(const T* __restrict__ A, int lda, const T* __restrict__ Wt, int ldw, int M, int N, int K,
                                                                            float* __restrict__ C, int ldc, T* __restrict__ act, int ld_act, HyGlu glu, int mt, int nt, int ks,
                                                                            int kper, HyGroup grp = HyGroup{}) {
@@ -115,7 +113,6 @@ static __global__ __launch_bounds__(WM * WN * 64, sizeof(T) == 4 ? 2 : 1) void h
     constexpr int SZA = BM * 128, SZW = BN * 128, OW = SA * SZA;
     static_assert(SW >= SA + (sizeof(T) == 2) && SA >= 2 && NPA * NW < 2 * PA + NW && TM * WM * 32 == BM && TN * WN * 32 == BN, "tile layout");
     static_assert(SA * SZA + SW * SZW <= 160 * 1024, "LDS");
-    constexpr bool ONCE = sizeof(T) == 2 || (GR && BM == 32);
     __shared__ __attribute__((aligned(1024))) uint8_t smem[SA * SZA + SW * SZW];
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), wm = wave / WN, wn = wave % WN;
     int m0, n0, z = 0;

@@ -62,9 +62,13 @@ static int32_t hy_alloc(gl3_ctx* ctx, P** p, size_t bytes) {
     HY_HIP(hipMemset(*p, 0, bytes + GL3_TAIL_PAD));
     return GL3_OK;
 }
-static int32_t hy_alloc_mat(gl3_ctx* ctx, HyMat& m, int rows, int k, int ld) {
+static int32_t hy_alloc_table(gl3_ctx* ctx, HyMat& m, int rows, int k, int ld) {
     m.rows = rows; m.k = k; m.ld = ld;
     return hy_alloc(ctx, &m.w, (size_t)rows * ld * (ctx->hy->f32 ? 4 : 2));
+}
+static int32_t hy_alloc_mat(gl3_ctx* ctx, HyMat& m, int rows, int k, int ld) {
+    ctx->hy->mat_bytes += (size_t)rows * ld * (ctx->hy->f32 ? 4 : 2);
+    return hy_alloc_table(ctx, m, rows, k, ld);
 }
 
 // ---- shapes -----------------------------------------------------------------------------------------------------------------------
@@ -247,14 +251,14 @@ int32_t gl3_hy_create(const gl3_model_desc* desc, gl3_ctx** out, std::string& er
     TRYHIP(hipStreamCreateWithFlags(&ctx->stream, hipStreamNonBlocking));
     const int W = h->W, S = h->S, mb = h->mb, V = desc->vocab, C = desc->ctx;
     const size_t es = h->f32 ? 4 : 2;
-    TRY(hy_alloc_mat(ctx, h->emb, V, W, W));
+    TRY(hy_alloc_table(ctx, h->emb, V, W, W));
     TRY(hy_alloc_mat(ctx, h->head, V, W, W));
     TRY(hy_alloc(ctx, &h->final_norm, (size_t)W * 4));
-    if (h->bg_buckets > 0) TRY(hy_alloc_mat(ctx, h->bigram, h->bg_buckets + 1, W, W));
+    if (h->bg_buckets > 0) TRY(hy_alloc_table(ctx, h->bigram, h->bg_buckets + 1, W, W));
     h->L.resize(desc->n_layers);
     size_t slot = 0;
     int max_proj = 1, max_mix = W, max_ch = 1, max_inner = 1, max_hr = 1, max_hdv = 1, max_kx = 0, max_vx = 0, max_rz = 0, max_top = 0, max_eff = 0, max_e = 0, max_poly = 0;
-    if (h->side_dim > 0) TRY(hy_alloc_mat(ctx, h->side_emb, V, desc->n_layers * h->side_dim, desc->n_layers * h->side_dim));
+    if (h->side_dim > 0) TRY(hy_alloc_table(ctx, h->side_emb, V, desc->n_layers * h->side_dim, desc->n_layers * h->side_dim));
     int max_heads = 1, max_qr = 0, max_qfull = 0;
     bool long_latent = false;
     // one mixer's share of the layer: its offsets in the fused projection row (p0 = its first row) and in mixo / o (o0 = its first
@@ -959,6 +963,18 @@ static double hy_ring_pick(bool f32, bool b16, int M, int N, int K, bool glu, bo
     return std::max(best, (double)N * K * (f32 ? 4 : 2) / 4.4e6 + 3.0);          // the weights leave HBM at 4.4 TB/s
 }
 
+// Whether the ring kernel reads its weights past the caches.  That is for weights that no cache still holds from the call before (the plan's matrices are more than the 256 MB of the last one) and
+// that one row of tiles reads, or several side by side: one that has fewer rows runs ahead, and the others read the weights from HBM again (MB fetched, through the caches / past them: 28672 x 4096
+// in bfloat16, 320 rows as 256 + 64 249 / 302; experts of 37 rows in tiles of 32, float32, 616 / 752).  Whole prompts of n tokens, us, through the caches / past them (mean of four medians of 25):
+//   bfloat16, one row of tiles or full ones: three layers of Kosusun 8B (1.7 GB) n = 16 535 / 493, 64 591 / 546, 128 702 / 660, 256 883 / 849, 512 1324 / 1308; six of Noditar 1B (0.7 GB) 16 465 / 452,
+//     128 548 / 542, 512 911 / 895; the last tile at least half full: Noditar 8B 500 949 / 939, 384 864 / 846, 200 638 / 642; a quarter full: 320 826 / 837;
+//   plans that the cache holds: two layers of Noditar 1B (238 MB) 16 155 / 161, 64 157 / 178, 128 173 / 195, 256 225 / 235, 512 313 / 314; just more than it: Kosusun 1B (338 MB) 64 239 / 238, 200 289 / 292;
+//   experts' tiles of 32 rows, three layers of Kugadra 1B (4 of 32): bfloat16 9 455 / 426, 100 559 / 532, 300 695 / 685; float32 9 768 / 750, 100 902 / 880, 140 961 / 945, 181 985 / 980, 220 1017 / 1026,
+//     260 1126 / 1171 (a second tile takes them much longer than bfloat16 ones): up to 24 rows an expert; tiles of 64: the same.
+// (float32 products of all rows: 60 tokens 854 / 828, but 181 1333 / 1355, 480 1327 / 1344.)
+constexpr size_t HY_CACHE_BYTES = (size_t)256 << 20;
+static bool hy_ring_once(const gl3_ctx* ctx, bool one_reader) { return one_reader && ctx->hy->mat_bytes > HY_CACHE_BYTES; }
+
 // The ring kernel for a product it can take in less than limit_us (true), or nothing.  parts / max_parts as for hy_gemm.
 template <typename T>
 static bool hy_gemm_ring(gl3_ctx* ctx, const T* A, int lda, const HyMat& w, int M, float* C, int ldc, bool glu, T* act, int ld_act, HyGlu gp, int* parts, int max_parts, double limit_us = 1e30) {
@@ -972,9 +988,12 @@ static bool hy_gemm_ring(gl3_ctx* ctx, const T* A, int lda, const HyMat& w, int 
     const int kper = hy_cdiv(K / BK, ks) * BK, mt = hy_cdiv(M, HY_RING_TILES[tile].bm), nt = hy_cdiv(N, HY_RING_TILES[tile].bn);
     if (parts) *parts = ks;
     const dim3 grid((unsigned)hy_cdiv(mt * nt * ks, 8) * 8);
-#define HY_RG1(BM, BN, WM, WN, SA, SW, EPI, WP)                                                                                                         \
-    hipLaunchKernelGGL((hy_gemm_ring_kernel<T, BM, BN, WM, WN, SA, SW, EPI, 0, sizeof(T) == 4 ? WP : 1>), grid, dim3((WM) * (WN) * 64), 0, ctx->stream, A, lda, (const T*)w.w, w.ld, \
-                       M, N, K, C, ldc, act, ld_act, gp, mt, nt, ks, kper)
+    const int over = M % HY_RING_TILES[tile].bm;          // rows of the last row tile
+    const bool once = sizeof(T) == 2 && hy_ring_once(ctx, mt == 1 || over == 0 || 2 * over >= HY_RING_TILES[tile].bm);
+#define HY_RG2(BM, BN, WM, WN, SA, SW, EPI, WP, ONCE)                                                                                                   \
+    hipLaunchKernelGGL((hy_gemm_ring_kernel<T, BM, BN, WM, WN, SA, SW, EPI, 0, sizeof(T) == 4 ? WP : 1, sizeof(T) == 2 && ONCE>), grid, dim3((WM) * (WN) * 64), 0, ctx->stream, A, lda, \
+                       (const T*)w.w, w.ld, M, N, K, C, ldc, act, ld_act, gp, mt, nt, ks, kper, HyGroup{})
+#define HY_RG1(BM, BN, WM, WN, SA, SW, EPI, WP) do { if (once) HY_RG2(BM, BN, WM, WN, SA, SW, EPI, WP, true); else HY_RG2(BM, BN, WM, WN, SA, SW, EPI, WP, false); } while (0)
 #define HY_RG(BM, BN, WM, WN, SA, SW, EPI)                                                                                                              \
     do {                                                                                                                                                \
         if (sizeof(T) == 4 && !w.b16) HY_RG1(BM, BN, WM, WN, SA, SW, EPI, 3); else HY_RG1(BM, BN, WM, WN, SA, SW, EPI, 1);                               \
@@ -1009,6 +1028,7 @@ static bool hy_gemm_ring(gl3_ctx* ctx, const T* A, int lda, const HyMat& w, int 
 #undef HY_RG_128x128
 #undef HY_RG
 #undef HY_RG1
+#undef HY_RG2
     return true;
 }
 
@@ -1797,13 +1817,16 @@ static void hy_gemm_grouped(gl3_ctx* ctx, const T* A, int lda, const HyMat& w, s
     constexpr int PE = 16 / (int)sizeof(T), BK = 128 / (int)sizeof(T);
     if (K % BK == 0 && lda % PE == 0 && w.ld % PE == 0 && wstride % PE == 0 && (((uintptr_t)A | (uintptr_t)Wt) & 15) == 0 && (uint64_t)N * w.ld * sizeof(T) < 0xffff0000ull) {
     // float32 tiles of 32 rows: four workgroups a CU hide each other's stages (rings of 2 + 2; 3 + 4, two a CU: 181 tokens x 4 of 32 experts, weights of one plane, 132 + 67 us, 145 + 73; with the small products in a chain of their own 121 + 64)
-#define HY_RGG1(BM, WM, EPI, WP) hipLaunchKernelGGL((hy_gemm_ring_kernel<T, BM, 128, WM, 2, sizeof(T) == 2 && BM == 32 ? 3 : 2, sizeof(T) == 2 ? 4 : BM == 32 ? 2 : 3, EPI, 1, sizeof(T) == 4 ? WP : 1>), grid, dim3(WM * 128), 0, st, A, lda, Wt, w.ld, 0, N, K, C, ldc, act, ld_act, gp, 0, 0, 1, K, grp)
+    const bool once = hy_ring_once(ctx, sizeof(T) == 2 || P <= 24 * n_sel);
+#define HY_RGG2(BM, WM, EPI, WP, ONCE) hipLaunchKernelGGL((hy_gemm_ring_kernel<T, BM, 128, WM, 2, sizeof(T) == 2 && BM == 32 ? 3 : 2, sizeof(T) == 2 ? 4 : BM == 32 ? 2 : 3, EPI, 1, sizeof(T) == 4 ? WP : 1, BM == 32 && ONCE>), grid, dim3(WM * 128), 0, st, A, lda, Wt, w.ld, 0, N, K, C, ldc, act, ld_act, gp, 0, 0, 1, K, grp)
+#define HY_RGG1(BM, WM, EPI, WP) do { if (once) HY_RGG2(BM, WM, EPI, WP, true); else HY_RGG2(BM, WM, EPI, WP, false); } while (0)
 #define HY_RGG(BM, WM, EPI) do { if (sizeof(T) == 4 && !w.b16) HY_RGG1(BM, WM, EPI, 3); else HY_RGG1(BM, WM, EPI, 1); } while (0)
 #define HY_RGG_EPI(BM, WM) do { if (glu) HY_RGG(BM, WM, HY_EPI_GLU); else if (gp.act == 2) HY_RGG(BM, WM, HY_EPI_ACTMUL); else HY_RGG(BM, WM, HY_EPI_STORE); } while (0)
         if (bm == HY_MOE_BM_FEW) HY_RGG_EPI(HY_MOE_BM_FEW, 1); else HY_RGG_EPI(HY_MOE_BM, 2);
 #undef HY_RGG_EPI
 #undef HY_RGG
 #undef HY_RGG1
+#undef HY_RGG2
         return;
     }
     if (glu) hipLaunchKernelGGL((hy_gemm_kernel<T, T, HY_MOE_BM, 128, HY_EPI_GLU, 1>), grid, dim3(256), 0, st, A, lda, Wt, w.ld, 0, N, K, C, ldc, act, ld_act, gp, K, grp);
@@ -2216,6 +2239,7 @@ int32_t gl3_hy_profile_gemm(int32_t device, int32_t f32, int32_t rows, int32_t k
         if (hipMalloc(&a, (size_t)m * k * es + GL3_TAIL_PAD) != hipSuccess) { rc = GL3_E_OOM; break; }
         if (hipMalloc((void**)&c, (size_t)HY_KSPLIT * m * rows * 4) != hipSuccess) { rc = GL3_E_OOM; break; }
         if (hipMalloc(&act, (size_t)m * rows * es) != hipSuccess) { rc = GL3_E_OOM; break; }
+        hs.mat_bytes = (size_t)copies * rows * k * es;
         hipMemset(w, 0, (size_t)copies * rows * k * es); hipMemset(a, 0, (size_t)m * k * es);
         hipEventCreate(&e0); hipEventCreate(&e1);
         auto run = [&](int it) {

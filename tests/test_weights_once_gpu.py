@@ -1,0 +1,89 @@
+"""Prompts' weights past the caches or through them (hy_ring_once, csrc/gl3_hybrid.hip): a plan whose matrices the 256 MB cache holds and the same layers in a plan that has a larger head, on either side of
+the rule's lines in rows: the residual of every row behind the last layer is the same bits (the loads differ, nothing else).  And the plan that the cache holds is the faster one: its weights are
+still there from the pass before, and reads past the cache took 10 - 17 % longer (head not wanted in either; half of that is asked for)."""
+import time
+
+import numpy as np
+import pytest
+
+import __graft_entry__ as ge
+import test_kugadra_gpu as U
+import test_noditar_gpu as N
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def hy():
+    from importlib import import_module
+    ge.load_package()
+    return import_module(ge.PKG_NAME + ".hybrid")
+
+
+def two_plans(hy, tmp_path, cfg, shapes, dtype, **kw):
+    """The layers behind a small vocabulary and behind one whose head is 300 MB (rows of zeros behind the small one's)."""
+    rng = np.random.default_rng(7)
+    small = {}
+    for name, shp in shapes(cfg).items():
+        big = len(shp) == 2 and shp[0] * shp[1] > 4096
+        small[name] = ((rng.standard_normal(shp).astype(np.float32) * (shp[-1] ** -0.5 if big else 0.1) + (0.0 if big else 1.0)).view(np.uint32) >> 16).astype(np.uint16)
+    rows = -(-(300 << 20) // (cfg["width"] * (2 if dtype == "bfloat16" else 4)))
+    out = []
+    for which in ("held", "large"):
+        w, c = dict(small), dict(cfg)
+        if which == "large":
+            c["vocab"] = rows
+            for name in ("embed", "head"):
+                if name in w:
+                    w[name] = np.concatenate([w[name], np.zeros((rows - w[name].shape[0], cfg["width"]), np.uint16)])
+        path = tmp_path / which
+        hy.save_model_dir(str(path), c, w)
+        out.append(hy.HybridPlan.from_dir(str(path), dtype=dtype, **kw))
+    return out
+
+
+def same_rows(hy, tmp_path, cfg, shapes, dtype, counts):
+    plans = two_plans(hy, tmp_path, cfg, shapes, dtype, ctx=max(counts) + 8, max_batch=max(counts), layer_taps=True)
+    toks = np.random.default_rng(3).integers(0, cfg["vocab"], max(counts)).astype(np.int32)
+    for n in counts:
+        rows = []
+        for p in plans:
+            s = p.acquire()
+            p.step(s, toks[:n], 0)
+            rows.append(p.layer_rows(len(cfg["layers"]) - 1, n).view(np.uint32))
+            p.release(s)
+        assert np.isfinite(rows[0].view(np.float32)).all() and np.array_equal(rows[0], rows[1]), n
+    for p in plans:
+        p.close()
+
+
+# widths and feed-forwards that take the tiles of 64, 128 and 256 rows, alone on a CU and two to one; 31 / 32 of 64, 63 / 64 of 128 and 127 / 128 of 256 rows in the last tile
+@pytest.mark.parametrize("width,ff", [(256, 640), (512, 7008), (1024, 14336)])
+def test_same_bits(hy, tmp_path, width, ff):
+    cfg = N.config([N.att(heads=8, kv_heads=4, dim=64, vdim=64, ff=ff)], width=width, vocab=500, streams=1)
+    same_rows(hy, tmp_path, cfg, hy.noditar_tensor_shapes, "bfloat16", [8, 9, 64, 65, 95, 96, 128, 129, 191, 192, 256, 257, 383, 384, 512])
+
+
+@pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
+def test_same_bits_of_experts(hy, tmp_path, dtype):
+    cfg = U.config([U.lig(mlp=U.moe(experts=8, top=2, ff=192, shared=128))], width=256)
+    same_rows(hy, tmp_path, cfg, hy.kugadra_tensor_shapes, dtype, [9, 33, 95, 96, 97, 191, 192])
+
+
+def test_weights_that_the_cache_holds(hy, tmp_path):
+    cfg = N.config([N.att(heads=32, kv_heads=8, dim=64, vdim=64, ff=8192)], width=2048, vocab=500, streams=1)
+    plans = two_plans(hy, tmp_path, cfg, hy.noditar_tensor_shapes, "bfloat16", ctx=72, max_batch=64)
+    toks = np.random.default_rng(3).integers(0, 500, 64).astype(np.int32)
+    slots, times = [p.acquire() for p in plans], ([], [])
+    for _ in range(30):
+        for p, s, ts in zip(plans, slots, times):
+            for i in range(6):          # (the first passes find the other plan's weights in the cache)
+                t0 = time.perf_counter()
+                p.step(s, toks, 0)
+                if i > 1:
+                    ts.append(time.perf_counter() - t0)
+    held, large = (float(np.median(t)) * 1e6 for t in times)
+    print("64 tokens, held %.1f us, past the cache %.1f" % (held, large))
+    for p in plans:
+        p.close()
+    assert held < 0.95 * large
