@@ -557,14 +557,15 @@ static __global__ __launch_bounds__(256) void hy_gemm_kernel(const T* __restrict
     }
 }
 
-// 16 bytes that are read once (weights of a few tokens' products): past the caches, which would write others out for them.  Requests, us, without / with: Kosusun 1B
-// bfloat16 (520 MB), 5 + 24 tokens 3845 / 3700, Kugadra 1B float32, 181 + 4 1394 / 1334, one token of Noditar 8B bfloat16 (one layer, 450 MB) 124 / 115; of models that the 256 MB of cache could hold (Noditar 1B,
-// one and two layers, 180 and 240 MB) 80.5 / 80.7 and 108 / 106.
+// 16 bytes that are read once (weights of a few tokens' products): past the caches, which would write others out for them.  Steps, us, through the caches / past them: three layers of Noditar 8B
+// bfloat16 (1.3 GB), one token 309 / 283, two 378 / 360, four 493 / 474; Kosusun 8B (1.7 GB) 374 / 351, 459 / 437, 616 / 588; Noditar 1B (370 MB) 153 / 145; of plans that the 256 MB cache holds: Noditar 1B
+// (238 MB) 98 / 98, layers of 768 within the runs, one layer of Noditar 1B (179 MB) 67 / 69, of Kosusun 1B 64 / 66.
 typedef uint32_t hy_u4v __attribute__((ext_vector_type(4)));
 __device__ __forceinline__ uint4 hy_ld_once(const void* p) {
     const hy_u4v v = __builtin_nontemporal_load(reinterpret_cast<const hy_u4v*>(p));
     return make_uint4(v[0], v[1], v[2], v[3]);
 }
+template <bool ONCE> __device__ __forceinline__ uint4 hy_ld_weights(const void* p) { if constexpr (ONCE) return hy_ld_once(p); else return *reinterpret_cast<const uint4*>(p); }
 // a 16-byte piece as floats
 __device__ __forceinline__ void hy_widen(const uint4& p, float* f, const bf16_t*) {
     const uint32_t u[4] = {p.x, p.y, p.z, p.w};
@@ -580,11 +581,15 @@ __device__ __forceinline__ void hy_widen(const uint4& p, float* f, const float*)
 // the wavefronts in flight for matrices with few rows.  EPI_GLU: the pair is (gate row, up row) of one feature in the block layout above.
 // Grouped form (GR = 1, mixture of experts, MT = 1): blockIdx.y = a (token, choice) pair whose expert sel[pair] picks the N rows of the
 // stacked matrix; row `pair` of A, C and act belongs to it.  A choice that is no expert (sel[pair] >= n_sel, identity) has no products.
+// GR = 2: twice as many pairs as experts or more: weights come through the caches, where the second pair finds them.  Steps of one layer, us, past the caches / through them, two (four) pairs an expert:
+// 2 of 8 of 3 x 1024 x 2048, 8 tokens, float32 128.8 / 121.4, bfloat16 101.6 / 97.3; 2 of 4, 8 tokens 178 / 170 and 117 / 111; 4 of 4, 8 tokens 169 / 155 and 120 / 107; 2 of 8 of 3 x 1792 x 4096 282.8 / 282.6
+// and 187 / 179; one pair an expert or fewer 111.6 / 113.6, 170.2 / 172.6 (float32, 2 and 4 tokens of that); two layers of Kugadra 1B, 4 of 32, 2 tokens bfloat16 205.0 / 207.8, 4 float32 315 / 319.
 // SUB: groups of four wavefronts in the workgroup, each a workgroup of its own (gl3_hy_beside_kernels.h); (bx, by): place in the grid.
 template <typename T, typename TO, int MT, int EPI, int KS, int GR, int SUB>
 __device__ __forceinline__ void hy_matvec(int bx, int by, const T* __restrict__ A, int lda, const T* __restrict__ Wt, int ldw, int M, int N, int K, float* __restrict__ C, int ldc,
                                           TO* __restrict__ act, int ld_act, const HyGlu& glu, const int* __restrict__ sel, size_t wstride, int a_div, const float* __restrict__ row_scale, int n_sel) {
     constexpr int PE = HyPiece<T>::N;
+    constexpr bool ONCE = GR != 2;
     float rs = 1.f;          // grouped: the pair's products are multiplied by row_scale[pair] (a score that scales the expert's input scales W x)
     if constexpr (GR) {
         const int pair_ = by;
@@ -623,8 +628,8 @@ __device__ __forceinline__ void hy_matvec(int bx, int by, const T* __restrict__ 
             uint4 p0[UN], p1[UN], pa[UN][MT];
 #pragma unroll
             for (int u = 0; u < UN; ++u) {
-                p0[u] = hy_ld_once(w0 + k + u * step);
-                p1[u] = hy_ld_once(w1 + k + u * step);
+                p0[u] = hy_ld_weights<ONCE>(w0 + k + u * step);
+                p1[u] = hy_ld_weights<ONCE>(w1 + k + u * step);
 #pragma unroll
                 for (int m = 0; m < MT; ++m) pa[u][m] = *reinterpret_cast<const uint4*>(A + (size_t)min(m, M - 1) * lda + k + u * step);
             }
@@ -646,8 +651,8 @@ __device__ __forceinline__ void hy_matvec(int bx, int by, const T* __restrict__ 
 #pragma unroll 2
     for (; k < kv; k += step) {
         float f0[PE], f1[PE];
-        hy_widen(hy_ld_once(w0 + k), f0, (const T*)nullptr);
-        hy_widen(hy_ld_once(w1 + k), f1, (const T*)nullptr);
+        hy_widen(hy_ld_weights<ONCE>(w0 + k), f0, (const T*)nullptr);
+        hy_widen(hy_ld_weights<ONCE>(w1 + k), f1, (const T*)nullptr);
 #pragma unroll
         for (int m = 0; m < MT; ++m) {
             if (m < M) {

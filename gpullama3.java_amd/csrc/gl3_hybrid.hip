@@ -1802,14 +1802,16 @@ static void hy_gemm_grouped(gl3_ctx* ctx, const T* A, int lda, const HyMat& w, s
         const int pairs = hy_cdiv(N, 2);
         const bool ksplit = (long)pairs * P < 8192 && K >= 1024;
         const dim3 grid(ksplit ? pairs : hy_cdiv(pairs, 4), P);
-#define HY_GMV(KS)                                                                                                                                     \
+#define HY_GMV1(KS, GR)                                                                                                                                \
     do {                                                                                                                                              \
-        if (glu) hipLaunchKernelGGL((hy_matvec_kernel<T, T, 1, HY_EPI_GLU, KS, 1>), grid, dim3(256), 0, st, A, lda, Wt, w.ld, 1, N, K, C, ldc, act, ld_act, gp, h->sel, wstride, a_div, row_scale, n_sel);   \
-        else if (gp.act == 2) hipLaunchKernelGGL((hy_matvec_kernel<T, T, 1, HY_EPI_ACTMUL, KS, 1>), grid, dim3(256), 0, st, A, lda, Wt, w.ld, 1, N, K, C, ldc, act, ld_act, gp, h->sel, wstride, a_div, row_scale, n_sel);    \
-        else hipLaunchKernelGGL((hy_matvec_kernel<T, T, 1, HY_EPI_STORE, KS, 1>), grid, dim3(256), 0, st, A, lda, Wt, w.ld, 1, N, K, C, ldc, act, ld_act, gp, h->sel, wstride, a_div, row_scale, n_sel);    \
+        if (glu) hipLaunchKernelGGL((hy_matvec_kernel<T, T, 1, HY_EPI_GLU, KS, GR>), grid, dim3(256), 0, st, A, lda, Wt, w.ld, 1, N, K, C, ldc, act, ld_act, gp, h->sel, wstride, a_div, row_scale, n_sel);   \
+        else if (gp.act == 2) hipLaunchKernelGGL((hy_matvec_kernel<T, T, 1, HY_EPI_ACTMUL, KS, GR>), grid, dim3(256), 0, st, A, lda, Wt, w.ld, 1, N, K, C, ldc, act, ld_act, gp, h->sel, wstride, a_div, row_scale, n_sel);    \
+        else hipLaunchKernelGGL((hy_matvec_kernel<T, T, 1, HY_EPI_STORE, KS, GR>), grid, dim3(256), 0, st, A, lda, Wt, w.ld, 1, N, K, C, ldc, act, ld_act, gp, h->sel, wstride, a_div, row_scale, n_sel);    \
     } while (0)
+#define HY_GMV(KS) do { if (P < 2 * n_sel) HY_GMV1(KS, 1); else HY_GMV1(KS, 2); } while (0)          // (an expert's weights are read twice on average)
         if (ksplit) HY_GMV(4); else HY_GMV(1);
 #undef HY_GMV
+#undef HY_GMV1
         return;
     }
     const HyGroup grp{h->tiles, h->ntiles, wstride};
