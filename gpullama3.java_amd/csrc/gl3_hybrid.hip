@@ -1032,12 +1032,15 @@ static bool hy_gemm_ring(gl3_ctx* ctx, const T* A, int lda, const HyMat& w, int 
     return true;
 }
 
+// Whether the four wavefronts of a dot product's workgroup share one pair of rows (long K, few pairs in the launch).  The launches that stand for others follow the same rule, so their sums are the same bits.
+static bool hy_mv_split(long pairs, int K) { return pairs < HY_SPLIT_PAIRS && K >= HY_SPLIT_K; }
+
 // ---- single tokens: residual updates that the next product makes (gl3_hy_pre_kernels.h) -------------------------------------------------
 template <typename T, int EPI>
 static void hy_pre_launch(gl3_ctx* ctx, const HyPre& p, int S, const T* Wt, int ldw, int N, float* C, T* act, int ld_act, const HyGlu& gp) {
     const int pairs = (N + 1) / 2, wgs = std::max(1, std::min(HY_PRE_WGS, pairs));
     // the split of K that hy_gemm's kernel has (below); its places are loaded one or two at a time
-    const bool ksplit = pairs < HY_SPLIT_PAIRS && p.W >= HY_SPLIT_K, two = p.W > 4 * 64 * HyPiece<T>::N;
+    const bool ksplit = hy_mv_split(pairs, p.W), two = p.W > 4 * 64 * HyPiece<T>::N;
 #define HY_PRE1(S_, KS, UN) hipLaunchKernelGGL((hy_matvec_pre_kernel<T, S_, EPI, KS, UN>), dim3(wgs), dim3(1024), 0, ctx->stream, p, Wt, ldw, N, C, act, ld_act, gp)
 #define HY_PRE(S_) do { if (!ksplit) HY_PRE1(S_, 1, 4); else if (two) HY_PRE1(S_, 4, 2); else HY_PRE1(S_, 4, 1); } while (0)
     if (S == 1) HY_PRE(1); else if (S == 2) HY_PRE(2); else HY_PRE(4);
@@ -1082,7 +1085,7 @@ static void hy_gemm(gl3_ctx* ctx, const T* A, int lda, const HyMat& w, int M, fl
     if (M > 4 && M <= 8 && sizeof(T) == 2 && hy_gemm_ring<T>(ctx, A, lda, w, M, C, ldc, glu, act, ld_act, gp, parts, max_parts, 2.1 * N * K * 2 / 5.6e6 + 3.0)) return;
     if (M <= 8) {
         const int pairs = hy_cdiv(N, 2);
-        const bool ksplit = pairs < HY_SPLIT_PAIRS && K >= HY_SPLIT_K;       // few rows: a workgroup's four wavefronts share one pair's K
+        const bool ksplit = hy_mv_split(pairs, K);
         const int wgs = ksplit ? pairs : hy_cdiv(pairs, 4);
 #define HY_MV2(MT, KS)                                                                                                                              \
     do {                                                                                                                                            \
@@ -1717,7 +1720,6 @@ static void hy_ff_up(gl3_ctx* ctx, const T* hb, HyLayer& L, int n, T* act) {
 }
 
 // ---- one token: launches side by side (gl3_hy_beside_kernels.h) -------------------------------------------------------------------------
-static bool hy_mv_split(long pairs, int K) { return pairs < HY_SPLIT_PAIRS && K >= HY_SPLIT_K; }          // (hy_gemm's and hy_gemm_grouped's rule)
 template <typename T>
 static HyMv<T> hy_mv(const T* A, int lda, const HyMat& w, float* C, T* act, int ld_act, const HyGlu& g) { return HyMv<T>{A, lda, (const T*)w.w, w.ld, w.rows, w.k, C, 0, act, ld_act, g, nullptr, 0, 1, nullptr, 0}; }
 // The mixer of a parallel block in its one-launch form and the feed-forward's gate and up rows; false: another form or position, nothing has run.  us, launches apart / like this, 16384 x 2048 in bfloat16
@@ -1760,7 +1762,7 @@ template <typename T>
 static void hy_two(gl3_ctx* ctx, const T* A0, const HyMat& w0, float* C0, const T* A1, const HyMat& w1, float* C1) {
     const int p0 = hy_cdiv(w0.rows, 2), p1 = hy_cdiv(w1.rows, 2);
     const bool ks = hy_mv_split(p0, w0.k);
-    if (ctx->hy->pre_on || ks != hy_mv_split(p1, w1.k)) {
+    if (ks != hy_mv_split(p1, w1.k)) {          // (no deferred update waits here: the layer's projection has made it)
         hy_gemm<T>(ctx, A0, w0.k, w0, 1, C0, w0.rows, false, nullptr, 0, HyGlu{});
         hy_gemm<T>(ctx, A1, w1.k, w1, 1, C1, w1.rows, false, nullptr, 0, HyGlu{});
         return;
@@ -1800,7 +1802,7 @@ static void hy_gemm_grouped(gl3_ctx* ctx, const T* A, int lda, const HyMat& w, s
     hipStream_t st = ctx->stream;
     if (few) {
         const int pairs = hy_cdiv(N, 2);
-        const bool ksplit = (long)pairs * P < 8192 && K >= 1024;
+        const bool ksplit = hy_mv_split((long)pairs * P, K);
         const dim3 grid(ksplit ? pairs : hy_cdiv(pairs, 4), P);
 #define HY_GMV1(KS, GR)                                                                                                                                \
     do {                                                                                                                                              \
