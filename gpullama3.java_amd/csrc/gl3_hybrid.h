@@ -130,6 +130,7 @@ struct gl3_hybrid_state {
     float *X = nullptr, *proj = nullptr, *y = nullptr, *conv = nullptr, *ssm_y = nullptr, *qa = nullptr, *oc = nullptr, *kx = nullptr, *vx = nullptr, *part_acc = nullptr, *part_ml = nullptr;
     float *gates = nullptr, *rowr = nullptr;     // matrix memory: a, b, e^(-m) per (token, head), [3][mb][max heads]; attention: 1 / rms of the whole q and k rows [mb][2]
     int max_heads = 1;
+    bool apart = false;        // GL3_HY_APART=1: a token's launches that share one (gl3_hy_beside_kernels.h) stay apart
     size_t mat_bytes = 0;      // matrices of products (not the tables that tokens look up)
     void *h = nullptr, *mixo = nullptr, *xw = nullptr;
     void* act1 = nullptr;      // parallel blocks, one token: the feed-forward's activation [max ff_pad], matrix type (made while mixo is)

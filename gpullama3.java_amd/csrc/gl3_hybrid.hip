@@ -229,6 +229,7 @@ int32_t gl3_hy_create(const gl3_model_desc* desc, gl3_ctx** out, std::string& er
     h->f32 = (desc->flags & GL3_FLAG_F32_COMPUTE) != 0;
     h->plain = desc->streams == 0;
     h->parallel = desc->parallel_block != 0;
+    h->apart = env_flag("GL3_HY_APART", false);
     h->resid_mul = (h->parallel && desc->residual_scale != 0.f) ? desc->residual_scale : 1.f;
     h->logit_mul = desc->logit_scale != 0.f ? desc->logit_scale : 1.f;
     h->emb_scale = desc->embedding_scale != 0.f ? desc->embedding_scale : 1.f;
@@ -1858,7 +1859,7 @@ static void hy_moe(gl3_ctx* ctx, HyLayer& L, int n) {
     const HyRoute rt{d.route_softmax, L.route_bias, d.route_renorm, d.route_scale != 0.f ? d.route_scale : 1.f, d.route_groups, d.route_keep, E, d.route_group_max};
     const HyRouteArgs ra{h->moe_z, RZ, zparts, (size_t)n * RZ, E + d.identity, top, h->sel, h->wsel, few ? h->pair_row : nullptr, (d.shared_ff > 0 && !d.shared_ungated) ? h->sgz : nullptr, rt};
     // one token: the shared expert's gate and up rows beside the choice, its down projection beside the chosen experts'
-    const bool up_beside = n == 1 && d.shared_ff > 0 && !hy_ungated(d), down_beside = n == 1 && d.shared_ff > 0 && hy_mv_split((long)hy_cdiv(W, 2) * P, L.edown.k) == hy_mv_split(hy_cdiv(W, 2), L.down.k);
+    const bool beside = n == 1 && d.shared_ff > 0 && !h->apart, up_beside = beside && !hy_ungated(d), down_beside = beside && hy_mv_split((long)hy_cdiv(W, 2) * P, L.edown.k) == hy_mv_split(hy_cdiv(W, 2), L.down.k);
     T* shared_act = (T*)h->mixo;
     if (up_beside) {
         const bool ks = hy_mv_split(L.ff_pad, W);
@@ -2017,7 +2018,7 @@ static int32_t hy_portion_plain(gl3_ctx* ctx, int seq, const int32_t* tokens, in
             if (h->taps) r.tap = h->taps + (size_t)l * lstride;
             resid_to_mixer(r, l + 1);
         };
-        const bool beside = n == 1 && h->parallel && L.d.ff > 0 && !L.d.out_norm;
+        const bool beside = n == 1 && h->parallel && L.d.ff > 0 && !L.d.out_norm && !h->apart;
         int32_t rc = beside ? hy_parallel_one<T>(ctx, L, pos0, seq) : hy_mixer<T>(ctx, L, n, pos0, seq);
         if (rc != GL3_OK) return rc;
         HyResid r = base;
