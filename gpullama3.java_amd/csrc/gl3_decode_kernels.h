@@ -553,8 +553,8 @@ __global__ __launch_bounds__(mv_threads(NPW), NPW == 4 ? 4 : 2) void matvec_q8t_
 // copy / own reads: batched prompt of 2 tokens 137 / 132, 4 137 / 135, 8 142 / 141; layer-list steps, whose embedding has 8 - 16 workgroups a token: 1 token 112 / 109,
 // 4 152 / 152, 16 143 / 152, 32 146 / 164).
 // A single step's logits go over the link from the kernel that makes them, row by row under the rest of it, where the host takes them as they are (third word of the step's record): a kernel behind
-// the captured step takes 4.6 us for 64 KB and stands some us apart from it.  Four layers, us, a kernel behind / like this: Llama 8B Q8_0, 8 tokens behind 389 2569 / 2546, Llama 1B, one token 182 / 178,
-// 8 tokens and 128256 rows of logits 1877 / 1857, F16 1889 / 1860.
+// the captured step takes 4.6 us for 64 KB and stands some us apart from it.  Steps of four layers, us, a kernel behind / like this (medians of 40 calls in turn): Llama 1B Q8_0, 32064 rows 174.1 / 173.6,
+// F16 234.4 / 230.7, 128256 rows 227.1 / 227.4, F16 310.8 / 303.2; Llama 8B Q8_0, 16032 rows 319.7 / 318.4, Q4_0 350.8 / 348.3.
 constexpr int GL3_HOST_TOKENS = 4;
 __device__ __forceinline__ int host_int(const int* p) { return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM); }
 __device__ __forceinline__ int step_token(int* dyn, const int* host) {

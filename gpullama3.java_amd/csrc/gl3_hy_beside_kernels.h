@@ -6,7 +6,8 @@
 //   * mixtures of experts with a shared expert: the choice of the experts and the shared gate / up product; the chosen experts' and the shared expert's down projections.
 // Every product keeps its own kernel's arithmetic (hy_matvec), so results are the same bits as from the launches apart.  us, apart / together: gate and up beside a mixer in hy_mixer_up (gl3_hybrid.hip);
 // output 2048 x 4096 and down 2048 x 8192 in bfloat16 5.4 + 7.7 / 10.3; choice of 4 of 32 and shared gate / up 8192 x 2048 in float32 4.4 + 13.4 / 13.7; down projections of four experts and the shared one
-// 8.1 + 8.4 / 13.8.  Requests: Kosusun 1B bfloat16, 5 + 24 tokens 4420 -> 3845, Kugadra 1B float32, 181 + 4 tokens 1424 -> 1394.
+// 8.1 + 8.4 / 13.8.  One token, medians of 30 calls in turn (GL3_HY_APART): three layers of Kosusun 768 wide bfloat16 110 / 88, 1000 x 8192 136 / 107, 1B 164 / 145, behind 640 positions 169 / 143, 8B
+// 355 / 348, behind 300 362 / 348; float32 1B 232 / 228, behind 640 243 / 235, 2048 x 16384 318 / 323, 8B 616 / 622, behind 300 625 / 621; Kugadra 1B float32 185 / 178, bfloat16 227 / 213.
 // Bound: the weights' bytes; the mixers' chains hide behind them.
 #pragma once
 #include "gl3_hy_one_kernels.h"
@@ -37,13 +38,15 @@ static __global__ __launch_bounds__(256) void hy_matvec_two_kernel(HyMv<T> p, in
 }
 
 // Gate and up rows by workgroups of sixteen wavefronts that stay: pairs wg 16 + wavefront, + 16 wgs .., a pair's next pieces on their way while the ones before are multiplied, the token's
-// row in LDS.  Every lane's chain is hy_matvec's (KS = 1).  K a multiple of a piece, at most HY_WALK_K.  (A mixer's registers leave a CU one workgroup: with hy_matvec's wavefronts of one pair, 8 KB on the way
-// and gone, 18.7 us.  A piece of either row at a time: two and four put more on the way than the mixers' loads can stand behind, whole requests 3845 us, 3960, 3925.)
-constexpr int HY_WALK_K = 4096;
+// row in LDS.  Every lane's chain is hy_matvec's (KS = 1).  K a multiple of a piece, rows of at most HY_WALK_BYTES: with longer ones hy_matvec's wavefronts of one pair have enough on their way.  One token
+// of three layers, us, one pair a wavefront / walked: bfloat16 1000 x 4128 100.0 / 95.3, 1000 x 16384 147 / 128, 2048 x 8192 147.8 / 144.9, 2048 x 16384 192 / 184, 3072 x 8192 181.7 / 177.3, 4096 x 14336
+// 347.5 / 353.7; float32 1000 x 8192 144 / 138, 1536 x 8192 174.2 / 173.6, 2048 x 8192 227.9 / 231.2, 3072 x 8192 284.9 / 289.1.  (A mixer's registers leave a CU one workgroup.  A piece of
+// either row at a time: two and four put more on the way than the mixers' loads can stand behind, whole requests 3845 us, 3960, 3925.)
+constexpr int HY_WALK_BYTES = 6 * 1024;
 template <typename T>
 __device__ __forceinline__ void hy_walk_glu(int wg, int wgs, const HyMv<T>& p) {
     constexpr int PE = HyPiece<T>::N, UN = 1, STEP = 64 * PE;
-    __shared__ __attribute__((aligned(16))) T sh[HY_WALK_K];
+    __shared__ __attribute__((aligned(16))) T sh[HY_WALK_BYTES / sizeof(T)];
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), K = p.K;
     const int pairs = p.N >> 1, first = wg * 16 + wave, stride = wgs * 16, chunks = (K + UN * STEP - 1) / (UN * STEP), todo = first < pairs ? ((pairs - 1 - first) / stride + 1) * chunks : 0;
     uint4 a[2][UN], b[2][UN];

@@ -1746,7 +1746,7 @@ static bool hy_mixer_up(gl3_ctx* ctx, const HyLayer& L, int np, int pos0, T* act
     const bool ks = hy_mv_split(pairs, h->W), wide = at && std::max(a.D, a.V) > 64, deep = me && b.s.N > 64;
     constexpr int PE = 16 / (int)sizeof(T);
     const int mixers = a.H + b.s.heads;
-    const bool walk = !ks && h->W % PE == 0 && h->W <= HY_WALK_K && L.gu.ld % PE == 0 && mixers <= 128;
+    const bool walk = !ks && h->W % PE == 0 && h->W * (int)sizeof(T) <= HY_WALK_BYTES && L.gu.ld % PE == 0 && mixers <= 128;
     const dim3 grid(mixers + (walk ? std::min(256 - mixers, hy_cdiv(pairs, 16)) : ks ? hy_cdiv(pairs, 4) : hy_cdiv(pairs, 16)));
     T *oa = at ? (T*)h->mixo + at->o0 : nullptr, *ob = me ? (T*)h->mixo + me->o0 : nullptr;
 #define HY_MU1(NI, QN, KS) hipLaunchKernelGGL((hy_mixer_up_kernel<T, NI, QN, KS>), grid, dim3(1024), 0, ctx->stream, a, oa, b, ob, f)

@@ -1,6 +1,6 @@
 """Launches of one token that share one (csrc/gl3_hy_beside_kernels.h) take every sum in the order of the launches they stand for: the same steps in a plan whose launches stay apart (GL3_HY_APART=1)
-give the same bits.  The forms of test_side_by_side_gpu.py, and the gate / up rows that walk (hy_walk_glu) with several chunks of a row and several pairs of rows per wavefront: widths of one to sixteen
-chunks, with whole and ragged last ones, feed-forwards of less than a pair per wavefront up to five, beside attention with retention and beside mLSTM, and beside more mixer workgroups than it takes (129)."""
+give the same bits.  The forms of test_side_by_side_gpu.py, and the gate / up rows that walk (hy_walk_glu) with several chunks of a row and several pairs of rows per wavefront: widths of one to six
+chunks, with whole and ragged last ones, and past the longest row that walks, feed-forwards of less than a pair per wavefront up to five, beside attention with retention and beside mLSTM, and beside more mixer workgroups than it takes (129)."""
 import os
 
 import numpy as np
@@ -57,7 +57,7 @@ WIDE = K.par(left=K.attn(heads=96, kv_heads=2, dim=8, vdim=8, rot_dims=8), right
 
 # 16 x 249 and 253 wavefronts: a pair each up to 3984 / 4048 features
 @pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
-@pytest.mark.parametrize("width,ff", [(8, 96), (256, 3968), (264, 4096), (512, 4128), (520, 12000), (1000, 8000), (1016, 4100), (1016, 7900), (2048, 8192), (2056, 8200), (4096, 8224), (4096, 20000)])
+@pytest.mark.parametrize("width,ff", [(8, 96), (256, 3968), (264, 4096), (512, 4128), (520, 12000), (1000, 8000), (1016, 4100), (1016, 7900), (1536, 8192), (1540, 8200), (2048, 8192), (2056, 8200), (2048, 20000), (3072, 8200), (3080, 8192), (4096, 8224)])
 def test_rows_that_walk(hy, tmp_path, width, ff, dtype):
     cfg = K.config([K.par(ff=ff), K.mls(ff=ff)], width=width, vocab=600)          # (random_model_dir: matrices of fewer than 4096 entries are constant)
     hy.random_model_dir(str(tmp_path), cfg, seed=width + ff)
