@@ -387,7 +387,7 @@ enum { HY_EPI_STORE = 0, HY_EPI_GLU = 1, HY_EPI_ACTMUL = 2 };
 struct HyGlu { float limit, alpha, shift; const void* mul_table; const int* mul_rows; int mul_ld, mul_col0; int act; float cap; float* host; };      // act 1: gelu_tanh(g) u; 2: relu(u)^2, no gate; cap: plain products of a few tokens become cap tanh(. / cap)
 // One token's plain results of two rows.  glu.host (one token's logits): they also go over the link to page-locked memory, from the kernel that makes them.
 // One token, us, a copy behind it / like this (medians of 30 calls in turn): Kosusun 1B 3000 rows 135.3 / 133.9, 12000 142.4 / 141.1, 32000 158.5 / 155.8, Noditar 8B, 32000 219.2 / 215.4, Kugadra 1B float32,
-// 128256 331.0 / 327.7; nowhere slower.
+// 128256 331.0 / 327.7; where it is not the faster way: hy_row_leaves.
 __device__ __forceinline__ void hy_put2(float* C, int r0, bool has1, float s0, float s1, const HyGlu& glu) {
     if (glu.cap > 0.f) { s0 = glu.cap * tanhf(s0 / glu.cap); s1 = glu.cap * tanhf(s1 / glu.cap); }
     C[r0] = s0;

@@ -141,7 +141,7 @@ struct gl3_hybrid_state {
     hipEvent_t rec_ev[2] = {}; bool rec_busy[2] = {};                // ends of the portions that read them
     void use_record(int r, int mb_) { h_dyn = h_rec + (size_t)r * (4 + want_cap + mb_); h_want = h_dyn + 4; h_tokens = h_want + want_cap; }
     float* h_logits = nullptr;                                       // pinned [want_cap][vocab]
-    float* leave = nullptr;                                          // one wanted row: where the head's kernel also writes it (h_logits)
+    float* leave = nullptr;                                          // one wanted row: where the head's kernel also writes it (h_logits; null: a copy behind it)
     size_t part_rows = 0;
     int last_n = 0;
     int y_first = 1;           // of these, the first mixer's (two normed mixers side by side)

@@ -1062,10 +1062,14 @@ static void hy_pre_flush(gl3_ctx* ctx) {
 // 32000 x 2048 (262 MB) 82.9 / 83.2, 24000 x 4096 (393 MB) 113.7 / 115.2, 32000 x 4096 (524 MB) 136 / 140, 131072 x 4096 (2.1 GB) 403 / 430; gate and up of 36864 x 2048 to 36864 x 4096 within 3 us.
 constexpr size_t HY_PRE_BYTES = (size_t)384 << 20;
 template <typename T>
+static bool hy_pre_takes(const gl3_hybrid_state* h, const T* A, const HyMat& w, int M, const HyGlu& gp) {
+    constexpr int PE = 16 / (int)sizeof(T);
+    return h->pre_on && M == 1 && (const void*)A == h->pre.h_out && w.k == h->pre.W && (size_t)w.rows * w.ld * sizeof(T) <= HY_PRE_BYTES && w.ld % PE == 0 && ((uintptr_t)w.w & 15) == 0 && !gp.mul_table;
+}
+template <typename T>
 static bool hy_pre_gemm(gl3_ctx* ctx, const T* A, const HyMat& w, int M, float* C, bool glu, T* act, int ld_act, const HyGlu& gp) {
     gl3_hybrid_state* h = ctx->hy;
-    constexpr int PE = 16 / (int)sizeof(T);
-    if (M != 1 || (const void*)A != h->pre.h_out || w.k != h->pre.W || (size_t)w.rows * w.ld * sizeof(T) > HY_PRE_BYTES || w.ld % PE || ((uintptr_t)w.w & 15) || gp.mul_table) { hy_pre_flush<T>(ctx); return false; }
+    if (!hy_pre_takes<T>(h, A, w, M, gp)) { hy_pre_flush<T>(ctx); return false; }
     h->pre_on = false;
     if (glu) hy_pre_launch<T, HY_EPI_GLU>(ctx, h->pre, h->pre_streams, (const T*)w.w, w.ld, w.rows, nullptr, act, ld_act, gp);
     else if (gp.act == 2) hy_pre_launch<T, HY_EPI_ACTMUL>(ctx, h->pre, h->pre_streams, (const T*)w.w, w.ld, w.rows, nullptr, act, ld_act, gp);
@@ -1906,15 +1910,28 @@ static void hy_moe(gl3_ctx* ctx, HyLayer& L, int n) {
 
 // logits of the nw rows listed in h->want: final norm of the gathered rows (normed: the last sublayer's update has left it in h->xw), the head's product, the
 // optional cap * tanh(. / cap) (a few rows: in the product)
+// One row leaves for the host from the head's kernel (h->leave; null: a copy behind it).  The product behind a deferred update writes rows in a row (gl3_hy_pre_kernels.h), and that is the faster way with every
+// head measured (widths 512 - 4096, 1000 - 128256 rows: 1 - 5 us a token, at worst equal).  A dot product's workgroup writes 8 bytes a pair of rows: that is
+// faster while pairs come slowly, one to a wavefront (us a token, a copy / leaving: width 512 float32, 17000 rows 113.1 / 111.9, 32000 118.2 / 117.5, 64000 136.4 / 137.1, 128256 163 / 168; 1000 bfloat16, 128256 185 /
+// 189, float32 212.5 / 211.9; 2048 float32, 24000 144.3 / 142.3, 128256 289.7 / 287.4; 4096 bfloat16, 32000 168.4 / 166.0, 128256 301 / 294), not where a whole workgroup makes a pair (2048 bfloat16, 1000 rows
+// 110.5 / 109.0, 4000 113.5 / 114.6, 12000 119.8 / 123.5, 16382 123.0 / 128.3; 4096 float32, 12000 168.5 / 171, 16382 180.4 / 184.4).
 template <typename T>
-static void hy_logits(gl3_ctx* ctx, int nw, bool normed = false) {          // one row: to h->leave too where that is set
+static bool hy_row_leaves(const gl3_hybrid_state* h, const T* xw, const HyGlu& g) {
+    if (hy_pre_takes<T>(h, xw, h->head, 1, g)) return true;
+    return hy_mv_split(hy_cdiv(h->head.rows, 2), h->head.k) ? h->head.rows <= 2048 : h->head.rows <= 32768 || h->head.k * (int)sizeof(T) >= 4096;
+}
+template <typename T>
+static void hy_logits(gl3_ctx* ctx, int nw, bool normed = false) {          // one row: to h->leave too, or h->leave goes
     gl3_hybrid_state* h = ctx->hy;
     T* xw = (T*)h->xw;
     if (!normed) hy_streams<T>(ctx, nw, h->X, h->W, h->S, (size_t)h->mb * h->W, (const float*)nullptr, 1, 0, (const float*)nullptr, (const float*)nullptr,
                   h->ones, h->final_norm, ctx->d.rms_eps, xw, (float*)nullptr, h->want);
     HyGlu g{};
     if (nw <= 4) g.cap = h->softcap;
-    if (nw == 1) g.host = h->leave;
+    if (nw == 1) {
+        if (!hy_row_leaves<T>(h, xw, g)) h->leave = nullptr;
+        g.host = h->leave;
+    }
     hy_gemm<T>(ctx, xw, h->W, h->head, nw, h->logits, ctx->d.vocab, false, nullptr, 0, g);
     if (h->softcap > 0.f && nw > 4) {
         const size_t cnt = (size_t)nw * ctx->d.vocab;
@@ -2173,7 +2190,7 @@ int32_t gl3_hy_step(gl3_ctx* ctx, int32_t seq, const int32_t* tokens, int32_t n,
             }
             if (r != GL3_OK) return r;
             h->last_tok[seq] = tokens[off + pn - 1];
-            if (g > 1 && logits_out) {
+            if (g > 0 && logits_out && !h->leave) {
                 launch_to_host(ctx, h->logits, h->h_logits, (size_t)g * V);
                 HY_HIP(hipGetLastError());
             }
