@@ -438,9 +438,16 @@ static void launch_attention(gl3_ctx* ctx, int l, int which /* 0 both, 1 scores,
         hipLaunchKernelGGL(attn_softmax_pv_kernel, dim3(ctx->heads_l * (d.head_size / PV_COLS)), dim3(256), sm2, ctx->stream, aa);
 }
 
+// The logits' kernel can write the host's copy itself (one rank, not the row-per-lane kernels).  It does where results come no faster than the link takes them, up to 65536 rows or with long ones.  Steps of two
+// layers, us, a kernel behind / written by itself (medians of 40 calls in turn): Q8_0, 512 columns, 32064 rows 96.9 / 95.6, 65536 109.2 / 108.9, 102400 123.6 / 125.6, 152064 142.0 / 145.9; 1024: 65536 111.5 / 110.9,
+// 152064 141.9 / 145.6; 2048: 65536 128.3 / 128.2, 152064 178.3 / 179.4, 256000 233.7 / 237.0; 2560: 152064 194.6 / 194.5; Q4_0, 512: 32064 125.4 / 125.8, 65536 160 / 164, 152064 237 / 249;
+// 1024: 65536 127.8 / 127.1, 152064 162.8 / 164.2; 2048: 152064 199.9 / 199.2; F16, 512: 65536 137.5 / 135.5, 152064 169.9 / 173.0; 1024: 152064 168.2 / 166.8.
+static bool logits_leave(const gl3_ctx* ctx) {
+    const Q8Mat& w = ctx->wcls;
+    const int long_row = w.fmt == GL3_TYPE_F16 ? 1024 : w.fmt == GL3_TYPE_Q4_0 ? 2048 : 2560;
+    return ctx->d.tp_size <= 1 && (w.fmt == GL3_TYPE_Q8_0 || w.vl) && (ctx->d.vocab <= 65536 || w.k >= long_row);
+}
 // amode: attn_mode(position) — the host knows the position of the step
-// The logits' kernel can write the host's copy itself (one rank, not the row-per-lane kernels).
-static bool logits_leave(const gl3_ctx* ctx) { return ctx->d.tp_size <= 1 && (ctx->wcls.fmt == GL3_TYPE_Q8_0 || ctx->wcls.vl); }
 static int32_t enqueue_decode(gl3_ctx* ctx, bool want_logits, gl3_kernel_times* kt, int amode) {
     const gl3_model_desc& d = ctx->d;
     hipStream_t s = ctx->stream;
