@@ -968,7 +968,8 @@ static double hy_ring_pick(bool f32, bool b16, int M, int N, int K, bool glu, bo
 // that one row of tiles reads, or several side by side: one that has fewer rows runs ahead, and the others read the weights from HBM again (MB fetched, through the caches / past them: 28672 x 4096
 // in bfloat16, 320 rows as 256 + 64 249 / 302; experts of 37 rows in tiles of 32, float32, 616 / 752).  Whole prompts of n tokens, us, through the caches / past them (mean of four medians of 25):
 //   bfloat16, one row of tiles or full ones: three layers of Kosusun 8B (1.7 GB) n = 16 535 / 493, 64 591 / 546, 128 702 / 660, 256 883 / 849, 512 1324 / 1308; six of Noditar 1B (0.7 GB) 16 465 / 452,
-//     128 548 / 542, 512 911 / 895; the last tile at least half full: Noditar 8B 500 949 / 939, 384 864 / 846, 200 638 / 642; a quarter full: 320 826 / 837;
+//     128 548 / 542, 512 911 / 895; the last tile at least a third full: Noditar 8B 500 949 / 939, 384 864 / 846, 350 868 / 858, 200 638 / 642; Kosusun 8B 94 452 / 442 (94 rows
+//     as 64 + 30 of 10240 x 4096), 88 446 / 437, 220 580 / 580; less than that: Noditar 8B 320 (256 + 64) 826 / 837, Kosusun 8B 280 762 / 773, 150 549 / 563;
 //   plans that the cache holds: two layers of Noditar 1B (238 MB) 16 155 / 161, 64 157 / 178, 128 173 / 195, 256 225 / 235, 512 313 / 314; just more than it: Kosusun 1B (338 MB) 64 239 / 238, 200 289 / 292;
 //   experts' tiles of 32 rows, three layers of Kugadra 1B (4 of 32): bfloat16 9 455 / 426, 100 559 / 532, 300 695 / 685; float32 9 768 / 750, 100 902 / 880, 140 961 / 945, 181 985 / 980, 220 1017 / 1026,
 //     260 1126 / 1171 (a second tile takes them much longer than bfloat16 ones): up to 24 rows an expert; tiles of 64: the same.
@@ -990,7 +991,7 @@ static bool hy_gemm_ring(gl3_ctx* ctx, const T* A, int lda, const HyMat& w, int 
     if (parts) *parts = ks;
     const dim3 grid((unsigned)hy_cdiv(mt * nt * ks, 8) * 8);
     const int over = M % HY_RING_TILES[tile].bm;          // rows of the last row tile
-    const bool once = sizeof(T) == 2 && hy_ring_once(ctx, mt == 1 || over == 0 || 2 * over >= HY_RING_TILES[tile].bm);
+    const bool once = sizeof(T) == 2 && hy_ring_once(ctx, mt == 1 || over == 0 || 3 * over >= HY_RING_TILES[tile].bm);
 #define HY_RG2(BM, BN, WM, WN, SA, SW, EPI, WP, ONCE)                                                                                                   \
     hipLaunchKernelGGL((hy_gemm_ring_kernel<T, BM, BN, WM, WN, SA, SW, EPI, 0, sizeof(T) == 4 ? WP : 1, sizeof(T) == 2 && ONCE>), grid, dim3((WM) * (WN) * 64), 0, ctx->stream, A, lda, \
                        (const T*)w.w, w.ld, M, N, K, C, ldc, act, ld_act, gp, mt, nt, ks, kper, HyGroup{})

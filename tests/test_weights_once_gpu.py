@@ -57,11 +57,11 @@ def same_rows(hy, tmp_path, cfg, shapes, dtype, counts):
         p.close()
 
 
-# widths and feed-forwards that take the tiles of 64, 128 and 256 rows, alone on a CU and two to one; 31 / 32 of 64, 63 / 64 of 128 and 127 / 128 of 256 rows in the last tile
+# widths and feed-forwards that take the tiles of 64, 128 and 256 rows, alone on a CU and two to one; 21 / 22 and 31 / 32 of 64, 42 / 43 and 63 / 64 of 128 and 85 / 86 and 127 / 128 of 256 rows in the last tile
 @pytest.mark.parametrize("width,ff", [(256, 640), (512, 7008), (1024, 14336)])
 def test_same_bits(hy, tmp_path, width, ff):
     cfg = N.config([N.att(heads=8, kv_heads=4, dim=64, vdim=64, ff=ff)], width=width, vocab=500, streams=1)
-    same_rows(hy, tmp_path, cfg, hy.noditar_tensor_shapes, "bfloat16", [8, 9, 64, 65, 95, 96, 128, 129, 191, 192, 256, 257, 383, 384, 512])
+    same_rows(hy, tmp_path, cfg, hy.noditar_tensor_shapes, "bfloat16", [8, 9, 64, 65, 85, 86, 95, 96, 128, 129, 170, 171, 191, 192, 256, 257, 341, 342, 383, 384, 512])
 
 
 @pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
