@@ -23,18 +23,18 @@ struct HyMv {                  // one token's product, as hy_matvec takes it
     HyGlu glu;
     const int* sel; size_t wstride; int a_div; const float* row_scale; int n_sel;          // grouped
 };
-template <typename T, int EPI, int KS, int GR, int SUB>
+template <typename T, int EPI, int KS, int GR, int SUB, bool ONCE>
 __device__ __forceinline__ void hy_matvec(int bx, int by, const HyMv<T>& p) {
-    hy_matvec<T, T, 1, EPI, KS, GR, SUB>(bx, by, p.A, p.lda, p.W, p.ldw, 1, p.N, p.K, p.C, p.ldc, p.act, p.ld_act, p.glu, p.sel, p.wstride, p.a_div, p.row_scale, p.n_sel);
+    hy_matvec<T, T, 1, EPI, KS, GR, SUB, ONCE>(bx, by, p.A, p.lda, p.W, p.ldw, 1, p.N, p.K, p.C, p.ldc, p.act, p.ld_act, p.glu, p.sel, p.wstride, p.a_div, p.row_scale, p.n_sel);
 }
 
 // Two products: workgroups 0 .. wp - 1 make p, the others q (GR: gx workgroups per pair).
-template <typename T, int KS, int GR>
+template <typename T, int KS, int GR, bool ONCE>
 static __global__ __launch_bounds__(256) void hy_matvec_two_kernel(HyMv<T> p, int wp, HyMv<T> q, int gx) {
     const int b = blockIdx.x;
-    if (b < wp) { hy_matvec<T, HY_EPI_STORE, KS, 0, 1>(b, 0, p); return; }
-    if constexpr (GR) hy_matvec<T, HY_EPI_STORE, KS, 1, 1>((b - wp) % gx, (b - wp) / gx, q);
-    else hy_matvec<T, HY_EPI_STORE, KS, 0, 1>(b - wp, 0, q);
+    if (b < wp) { hy_matvec<T, HY_EPI_STORE, KS, 0, 1, ONCE>(b, 0, p); return; }
+    if constexpr (GR) hy_matvec<T, HY_EPI_STORE, KS, 1, 1, ONCE>((b - wp) % gx, (b - wp) / gx, q);
+    else hy_matvec<T, HY_EPI_STORE, KS, 0, 1, ONCE>(b - wp, 0, q);
 }
 
 // Gate and up rows by workgroups of sixteen wavefronts that stay: pairs wg 16 + wavefront, + 16 wgs .., a pair's next pieces on their way while the ones before are multiplied, the token's
@@ -43,7 +43,7 @@ static __global__ __launch_bounds__(256) void hy_matvec_two_kernel(HyMv<T> p, in
 // 347.5 / 353.7; float32 1000 x 8192 144 / 138, 1536 x 8192 174.2 / 173.6, 2048 x 8192 227.9 / 231.2, 3072 x 8192 284.9 / 289.1.  (A mixer's registers leave a CU one workgroup.  A piece of
 // either row at a time: two and four put more on the way than the mixers' loads can stand behind, whole requests 3845 us, 3960, 3925.)
 constexpr int HY_WALK_BYTES = 6 * 1024;
-template <typename T>
+template <typename T, bool ONCE>
 __device__ __forceinline__ void hy_walk_glu(int wg, int wgs, const HyMv<T>& p) {
     constexpr int PE = HyPiece<T>::N, UN = 1, STEP = 64 * PE;
     __shared__ __attribute__((aligned(16))) T sh[HY_WALK_BYTES / sizeof(T)];
@@ -56,8 +56,8 @@ __device__ __forceinline__ void hy_walk_glu(int wg, int wgs, const HyMv<T>& p) {
 #pragma unroll
         for (int u = 0; u < UN; ++u) {
             const int ku = min(k + u * STEP, K - PE);
-            a[set][u] = hy_ld_once(w0 + ku);
-            b[set][u] = hy_ld_once(w1 + ku);
+            a[set][u] = hy_ld_weights<ONCE>(w0 + ku);
+            b[set][u] = hy_ld_weights<ONCE>(w1 + ku);
         }
     };
     const uint4 row = *reinterpret_cast<const uint4*>(p.A + min(tid * PE, K - PE));          // first: the weights' answers come in order behind it
@@ -97,19 +97,19 @@ __device__ __forceinline__ void hy_walk_glu(int wg, int wgs, const HyMv<T>& p) {
 }
 
 // A mixer (attention, a matrix memory or both: gl3_hy_one_kernels.h) in the first workgroups, gate and up rows of the feed-forward in the others, sixteen wavefronts each.
-template <typename T, int NI, int QN, int KS>          // KS = 0: hy_walk_glu
+template <typename T, int NI, int QN, int KS, bool ONCE>          // KS = 0: hy_walk_glu
 static __global__ __launch_bounds__(1024) void hy_mixer_up_kernel(HyAttnOne a, T* __restrict__ out_a, HyScanOut b, T* __restrict__ out_b, HyMv<T> f) {
     const int w = blockIdx.x, mixers = a.H + b.s.heads;
     if (w < a.H) hy_attn_one<T, NI>(a, out_a, w);
     else if (w < mixers) hy_scan_out<T, QN>(b, out_b, w - a.H);
-    else if constexpr (KS == 0) hy_walk_glu<T>(w - mixers, (int)gridDim.x - mixers, f);
-    else hy_matvec<T, HY_EPI_GLU, KS, 0, 4>(w - mixers, 0, f);
+    else if constexpr (KS == 0) hy_walk_glu<T, ONCE>(w - mixers, (int)gridDim.x - mixers, f);
+    else hy_matvec<T, HY_EPI_GLU, KS, 0, 4, ONCE>(w - mixers, 0, f);
 }
 
 // The token's choice of experts in workgroup 0, gate and up rows of the shared expert in the others.
 struct HyRouteArgs { const float* z; int ldz, parts; size_t pstride; int E, top; int* sel; float* wgt; int* pair_row; float* extra_out; HyRoute rt; };
-template <typename T, int PER, int KS>
+template <typename T, int PER, int KS, bool ONCE>
 static __global__ __launch_bounds__(256) void hy_route_up_kernel(HyRouteArgs r, HyMv<T> f) {
-    if (blockIdx.x > 0) { hy_matvec<T, HY_EPI_GLU, KS, 0, 1>((int)blockIdx.x - 1, 0, f); return; }
+    if (blockIdx.x > 0) { hy_matvec<T, HY_EPI_GLU, KS, 0, 1, ONCE>((int)blockIdx.x - 1, 0, f); return; }
     if (threadIdx.x < 64) hy_route<PER>(0, r.z, r.ldz, r.parts, r.pstride, r.E, r.top, r.sel, r.wgt, r.pair_row, r.extra_out, r.rt);
 }

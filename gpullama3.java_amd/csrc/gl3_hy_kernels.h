@@ -557,9 +557,9 @@ static __global__ __launch_bounds__(256) void hy_gemm_kernel(const T* __restrict
     }
 }
 
-// 16 bytes that are read once (weights of a few tokens' products): past the caches, which would write others out for them.  Steps, us, through the caches / past them: three layers of Noditar 8B
+// 16 bytes that are read once (weights of a few tokens' products, where the plan's matrices are more than the 256 MB cache: hy_past_caches): past the caches, which would write others out for them.  Steps, us, through the caches / past them: three layers of Noditar 8B
 // bfloat16 (1.3 GB), one token 309 / 283, two 378 / 360, four 493 / 474; Kosusun 8B (1.7 GB) 374 / 351, 459 / 437, 616 / 588; Noditar 1B (370 MB) 153 / 145; of plans that the 256 MB cache holds: Noditar 1B
-// (238 MB) 98 / 98, layers of 768 within the runs, one layer of Noditar 1B (179 MB) 67 / 69, of Kosusun 1B 64 / 66.
+// (238 MB) 98 / 98, one layer of it (179 MB) 67 / 69, of Kosusun 1B 64 / 66, and a prompt's products find less behind such steps: prompts of 64 and one token 263 / 274, of 122 288 / 296, one layer and two tokens 249 / 267; generation from 4 tokens on, one layer, 1177 / 1210.
 typedef uint32_t hy_u4v __attribute__((ext_vector_type(4)));
 __device__ __forceinline__ uint4 hy_ld_once(const void* p) {
     const hy_u4v v = __builtin_nontemporal_load(reinterpret_cast<const hy_u4v*>(p));
@@ -581,15 +581,14 @@ __device__ __forceinline__ void hy_widen(const uint4& p, float* f, const float*)
 // the wavefronts in flight for matrices with few rows.  EPI_GLU: the pair is (gate row, up row) of one feature in the block layout above.
 // Grouped form (GR = 1, mixture of experts, MT = 1): blockIdx.y = a (token, choice) pair whose expert sel[pair] picks the N rows of the
 // stacked matrix; row `pair` of A, C and act belongs to it.  A choice that is no expert (sel[pair] >= n_sel, identity) has no products.
-// GR = 2: twice as many pairs as experts or more: weights come through the caches, where the second pair finds them.  Steps of one layer, us, past the caches / through them, two (four) pairs an expert:
+// ONCE: weights past the caches (hy_past_caches, and experts of fewer pairs than twice their number; with more of them they come through the caches, where the second pair finds them).  Steps of one layer, us, past the caches / through them, two (four) pairs an expert:
 // 2 of 8 of 3 x 1024 x 2048, 8 tokens, float32 128.8 / 121.4, bfloat16 101.6 / 97.3; 2 of 4, 8 tokens 178 / 170 and 117 / 111; 4 of 4, 8 tokens 169 / 155 and 120 / 107; 2 of 8 of 3 x 1792 x 4096 282.8 / 282.6
 // and 187 / 179; one pair an expert or fewer 111.6 / 113.6, 170.2 / 172.6 (float32, 2 and 4 tokens of that); two layers of Kugadra 1B, 4 of 32, 2 tokens bfloat16 205.0 / 207.8, 4 float32 315 / 319.
 // SUB: groups of four wavefronts in the workgroup, each a workgroup of its own (gl3_hy_beside_kernels.h); (bx, by): place in the grid.
-template <typename T, typename TO, int MT, int EPI, int KS, int GR, int SUB>
+template <typename T, typename TO, int MT, int EPI, int KS, int GR, int SUB, bool ONCE>
 __device__ __forceinline__ void hy_matvec(int bx, int by, const T* __restrict__ A, int lda, const T* __restrict__ Wt, int ldw, int M, int N, int K, float* __restrict__ C, int ldc,
                                           TO* __restrict__ act, int ld_act, const HyGlu& glu, const int* __restrict__ sel, size_t wstride, int a_div, const float* __restrict__ row_scale, int n_sel) {
     constexpr int PE = HyPiece<T>::N;
-    constexpr bool ONCE = GR != 2;
     float rs = 1.f;          // grouped: the pair's products are multiplied by row_scale[pair] (a score that scales the expert's input scales W x)
     if constexpr (GR) {
         const int pair_ = by;
@@ -704,12 +703,12 @@ __device__ __forceinline__ void hy_matvec(int bx, int by, const T* __restrict__ 
         }
     }
 }
-template <typename T, typename TO, int MT, int EPI, int KS, int GR = 0>
+template <typename T, typename TO, int MT, int EPI, int KS, int GR, bool ONCE>
 static __global__ __launch_bounds__(256) void hy_matvec_kernel(const T* __restrict__ A, int lda, const T* __restrict__ Wt, int ldw, int M, int N, int K,
                                                                float* __restrict__ C, int ldc, TO* __restrict__ act, int ld_act, HyGlu glu,
                                                                const int* __restrict__ sel = nullptr, size_t wstride = 0, int a_div = 1,
                                                                const float* __restrict__ row_scale = nullptr, int n_sel = 0) {
-    hy_matvec<T, TO, MT, EPI, KS, GR, 1>(blockIdx.x, blockIdx.y, A, lda, Wt, ldw, M, N, K, C, ldc, act, ld_act, glu, sel, wstride, a_div, row_scale, n_sel);
+    hy_matvec<T, TO, MT, EPI, KS, GR, 1, ONCE>(blockIdx.x, blockIdx.y, A, lda, Wt, ldw, M, N, K, C, ldc, act, ld_act, glu, sel, wstride, a_div, row_scale, n_sel);
 }
 
 // ---- attention: cache writers ---------------------------------------------------------------------------------------------------

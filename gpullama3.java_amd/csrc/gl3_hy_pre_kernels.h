@@ -28,7 +28,7 @@ __device__ __forceinline__ float hy_wave_sum_vec(float v) {
 }
 
 // UN: a wavefront's places of the walk that are loaded together
-template <typename T, int S, int EPI, int KS, int UN>
+template <typename T, int S, int EPI, int KS, int UN, bool ONCE>
 static __global__ __launch_bounds__(1024) void hy_matvec_pre_kernel(HyPre p, const T* __restrict__ Wt, int ldw, int N, float* __restrict__ C, T* __restrict__ act, int ld_act, HyGlu glu) {
     constexpr int PE = HyPiece<T>::N, STEP = KS * 64 * PE;
     __shared__ __attribute__((aligned(16))) T sh[4096];
@@ -46,8 +46,8 @@ static __global__ __launch_bounds__(1024) void hy_matvec_pre_kernel(HyPre p, con
 #pragma unroll
         for (int u = 0; u < UN; ++u) {
             const int ku = min(k + u * STEP, K - PE);
-            a[set][u] = hy_ld_once(w0 + ku);
-            b[set][u] = hy_ld_once(w1 + ku);
+            a[set][u] = hy_ld_weights<ONCE>(w0 + ku);
+            b[set][u] = hy_ld_weights<ONCE>(w1 + ku);
         }
     };
     const int w = 4 * tid;

@@ -15,6 +15,7 @@
 #include <algorithm>
 #include <cmath>
 #include <cstring>
+#include <type_traits>
 
 #include "gl3_hybrid.h"
 #include "gl3_decode_kernels.h"      // argmax_kernel
@@ -975,7 +976,9 @@ static double hy_ring_pick(bool f32, bool b16, int M, int N, int K, bool glu, bo
 //     260 1126 / 1171 (a second tile takes them much longer than bfloat16 ones): up to 24 rows an expert; tiles of 64: the same.
 // (float32 products of all rows: 60 tokens 854 / 828, but 181 1333 / 1355, 480 1327 / 1344.)
 constexpr size_t HY_CACHE_BYTES = (size_t)256 << 20;
-static bool hy_ring_once(const gl3_ctx* ctx, bool one_reader) { return one_reader && ctx->hy->mat_bytes > HY_CACHE_BYTES; }
+static bool hy_past_caches(const gl3_ctx* ctx) { return ctx->hy->mat_bytes > HY_CACHE_BYTES; }
+static bool hy_ring_once(const gl3_ctx* ctx, bool one_reader) { return one_reader && hy_past_caches(ctx); }
+template <typename F> static void hy_with_once(bool once, F&& f) { if (once) f(std::true_type{}); else f(std::false_type{}); }
 
 // The ring kernel for a product it can take in less than limit_us (true), or nothing.  parts / max_parts as for hy_gemm.
 template <typename T>
@@ -1043,9 +1046,9 @@ static void hy_pre_launch(gl3_ctx* ctx, const HyPre& p, int S, const T* Wt, int 
     const int pairs = (N + 1) / 2, wgs = std::max(1, std::min(HY_PRE_WGS, pairs));
     // the split of K that hy_gemm's kernel has (below); its places are loaded one or two at a time
     const bool ksplit = hy_mv_split(pairs, p.W), two = p.W > 4 * 64 * HyPiece<T>::N;
-#define HY_PRE1(S_, KS, UN) hipLaunchKernelGGL((hy_matvec_pre_kernel<T, S_, EPI, KS, UN>), dim3(wgs), dim3(1024), 0, ctx->stream, p, Wt, ldw, N, C, act, ld_act, gp)
+#define HY_PRE1(S_, KS, UN) hipLaunchKernelGGL((hy_matvec_pre_kernel<T, S_, EPI, KS, UN, decltype(once)::value>), dim3(wgs), dim3(1024), 0, ctx->stream, p, Wt, ldw, N, C, act, ld_act, gp)
 #define HY_PRE(S_) do { if (!ksplit) HY_PRE1(S_, 1, 4); else if (two) HY_PRE1(S_, 4, 2); else HY_PRE1(S_, 4, 1); } while (0)
-    if (S == 1) HY_PRE(1); else if (S == 2) HY_PRE(2); else HY_PRE(4);
+    hy_with_once(hy_past_caches(ctx), [&](auto once) { if (S == 1) HY_PRE(1); else if (S == 2) HY_PRE(2); else HY_PRE(4); });
 #undef HY_PRE
 #undef HY_PRE1
 }
@@ -1095,12 +1098,12 @@ static void hy_gemm(gl3_ctx* ctx, const T* A, int lda, const HyMat& w, int M, fl
         const int wgs = ksplit ? pairs : hy_cdiv(pairs, 4);
 #define HY_MV2(MT, KS)                                                                                                                              \
     do {                                                                                                                                            \
-        if (glu) hipLaunchKernelGGL((hy_matvec_kernel<T, T, MT, HY_EPI_GLU, KS>), dim3(wgs), dim3(256), 0, st, A, lda, Wt, w.ld, M, N, K, C, ldc, act, ld_act, gp);   \
-        else if (gp.mul_table || gp.act == 2) hipLaunchKernelGGL((hy_matvec_kernel<T, T, MT, HY_EPI_ACTMUL, KS>), dim3(wgs), dim3(256), 0, st, A, lda, Wt, w.ld, M, N, K, C, ldc, act, ld_act, gp);   \
-        else hipLaunchKernelGGL((hy_matvec_kernel<T, T, MT, HY_EPI_STORE, KS>), dim3(wgs), dim3(256), 0, st, A, lda, Wt, w.ld, M, N, K, C, ldc, act, ld_act, gp);    \
+        if (glu) hipLaunchKernelGGL((hy_matvec_kernel<T, T, MT, HY_EPI_GLU, KS, 0, decltype(once)::value>), dim3(wgs), dim3(256), 0, st, A, lda, Wt, w.ld, M, N, K, C, ldc, act, ld_act, gp);   \
+        else if (gp.mul_table || gp.act == 2) hipLaunchKernelGGL((hy_matvec_kernel<T, T, MT, HY_EPI_ACTMUL, KS, 0, decltype(once)::value>), dim3(wgs), dim3(256), 0, st, A, lda, Wt, w.ld, M, N, K, C, ldc, act, ld_act, gp);   \
+        else hipLaunchKernelGGL((hy_matvec_kernel<T, T, MT, HY_EPI_STORE, KS, 0, decltype(once)::value>), dim3(wgs), dim3(256), 0, st, A, lda, Wt, w.ld, M, N, K, C, ldc, act, ld_act, gp);    \
     } while (0)
 #define HY_MV(MT) do { if (ksplit) HY_MV2(MT, 4); else HY_MV2(MT, 1); } while (0)
-        if (M == 1) HY_MV(1); else if (M == 2) HY_MV(2); else if (M <= 4) HY_MV(4); else HY_MV(8);
+        hy_with_once(hy_past_caches(ctx), [&](auto once) { if (M == 1) HY_MV(1); else if (M == 2) HY_MV(2); else if (M <= 4) HY_MV(4); else HY_MV(8); });
 #undef HY_MV2
 #undef HY_MV
         return;
@@ -1754,10 +1757,12 @@ static bool hy_mixer_up(gl3_ctx* ctx, const HyLayer& L, int np, int pos0, T* act
     const bool walk = !ks && h->W % PE == 0 && h->W * (int)sizeof(T) <= HY_WALK_BYTES && L.gu.ld % PE == 0 && mixers <= 128;
     const dim3 grid(mixers + (walk ? std::min(256 - mixers, hy_cdiv(pairs, 16)) : ks ? hy_cdiv(pairs, 4) : hy_cdiv(pairs, 16)));
     T *oa = at ? (T*)h->mixo + at->o0 : nullptr, *ob = me ? (T*)h->mixo + me->o0 : nullptr;
-#define HY_MU1(NI, QN, KS) hipLaunchKernelGGL((hy_mixer_up_kernel<T, NI, QN, KS>), grid, dim3(1024), 0, ctx->stream, a, oa, b, ob, f)
+#define HY_MU1(NI, QN, KS) hipLaunchKernelGGL((hy_mixer_up_kernel<T, NI, QN, KS, decltype(once)::value>), grid, dim3(1024), 0, ctx->stream, a, oa, b, ob, f)
 #define HY_MU(NI, QN) do { if (walk) HY_MU1(NI, QN, 0); else if (ks) HY_MU1(NI, QN, 4); else HY_MU1(NI, QN, 1); } while (0)
-    if (wide) { if (deep) HY_MU(2, 8); else HY_MU(2, 4); }
-    else { if (deep) HY_MU(1, 8); else HY_MU(1, 4); }
+    hy_with_once(hy_past_caches(ctx), [&](auto once) {
+        if (wide) { if (deep) HY_MU(2, 8); else HY_MU(2, 4); }
+        else { if (deep) HY_MU(1, 8); else HY_MU(1, 4); }
+    });
 #undef HY_MU
 #undef HY_MU1
     if (at) hy_pool(ctx, *at, 1, pos0);
@@ -1775,8 +1780,10 @@ static void hy_two(gl3_ctx* ctx, const T* A0, const HyMat& w0, float* C0, const 
     }
     const int g0 = ks ? p0 : hy_cdiv(p0, 4), g1 = ks ? p1 : hy_cdiv(p1, 4);
     const HyMv<T> m0 = hy_mv<T>(A0, w0.k, w0, C0, nullptr, 0, HyGlu{}), m1 = hy_mv<T>(A1, w1.k, w1, C1, nullptr, 0, HyGlu{});
-    if (ks) hipLaunchKernelGGL((hy_matvec_two_kernel<T, 4, 0>), dim3(g0 + g1), dim3(256), 0, ctx->stream, m0, g0, m1, g1);
-    else hipLaunchKernelGGL((hy_matvec_two_kernel<T, 1, 0>), dim3(g0 + g1), dim3(256), 0, ctx->stream, m0, g0, m1, g1);
+    hy_with_once(hy_past_caches(ctx), [&](auto once) {
+        if (ks) hipLaunchKernelGGL((hy_matvec_two_kernel<T, 4, 0, decltype(once)::value>), dim3(g0 + g1), dim3(256), 0, ctx->stream, m0, g0, m1, g1);
+        else hipLaunchKernelGGL((hy_matvec_two_kernel<T, 1, 0, decltype(once)::value>), dim3(g0 + g1), dim3(256), 0, ctx->stream, m0, g0, m1, g1);
+    });
 }
 // A layer of a parallel block for one token (dense feed-forward): h->y holds the mixer's output and the feed-forward's, two parts.
 template <typename T>
@@ -1810,16 +1817,14 @@ static void hy_gemm_grouped(gl3_ctx* ctx, const T* A, int lda, const HyMat& w, s
         const int pairs = hy_cdiv(N, 2);
         const bool ksplit = hy_mv_split((long)pairs * P, K);
         const dim3 grid(ksplit ? pairs : hy_cdiv(pairs, 4), P);
-#define HY_GMV1(KS, GR)                                                                                                                                \
+#define HY_GMV(KS)                                                                                                                                     \
     do {                                                                                                                                              \
-        if (glu) hipLaunchKernelGGL((hy_matvec_kernel<T, T, 1, HY_EPI_GLU, KS, GR>), grid, dim3(256), 0, st, A, lda, Wt, w.ld, 1, N, K, C, ldc, act, ld_act, gp, h->sel, wstride, a_div, row_scale, n_sel);   \
-        else if (gp.act == 2) hipLaunchKernelGGL((hy_matvec_kernel<T, T, 1, HY_EPI_ACTMUL, KS, GR>), grid, dim3(256), 0, st, A, lda, Wt, w.ld, 1, N, K, C, ldc, act, ld_act, gp, h->sel, wstride, a_div, row_scale, n_sel);    \
-        else hipLaunchKernelGGL((hy_matvec_kernel<T, T, 1, HY_EPI_STORE, KS, GR>), grid, dim3(256), 0, st, A, lda, Wt, w.ld, 1, N, K, C, ldc, act, ld_act, gp, h->sel, wstride, a_div, row_scale, n_sel);    \
+        if (glu) hipLaunchKernelGGL((hy_matvec_kernel<T, T, 1, HY_EPI_GLU, KS, 1, decltype(once)::value>), grid, dim3(256), 0, st, A, lda, Wt, w.ld, 1, N, K, C, ldc, act, ld_act, gp, h->sel, wstride, a_div, row_scale, n_sel);   \
+        else if (gp.act == 2) hipLaunchKernelGGL((hy_matvec_kernel<T, T, 1, HY_EPI_ACTMUL, KS, 1, decltype(once)::value>), grid, dim3(256), 0, st, A, lda, Wt, w.ld, 1, N, K, C, ldc, act, ld_act, gp, h->sel, wstride, a_div, row_scale, n_sel);    \
+        else hipLaunchKernelGGL((hy_matvec_kernel<T, T, 1, HY_EPI_STORE, KS, 1, decltype(once)::value>), grid, dim3(256), 0, st, A, lda, Wt, w.ld, 1, N, K, C, ldc, act, ld_act, gp, h->sel, wstride, a_div, row_scale, n_sel);    \
     } while (0)
-#define HY_GMV(KS) do { if (P < 2 * n_sel) HY_GMV1(KS, 1); else HY_GMV1(KS, 2); } while (0)          // (an expert's weights are read twice on average)
-        if (ksplit) HY_GMV(4); else HY_GMV(1);
+        hy_with_once(hy_past_caches(ctx) && P < 2 * n_sel, [&](auto once) { if (ksplit) HY_GMV(4); else HY_GMV(1); });          // (from there on an expert's weights are read twice on average)
 #undef HY_GMV
-#undef HY_GMV1
         return;
     }
     const HyGroup grp{h->tiles, h->ntiles, wstride};
@@ -1870,8 +1875,8 @@ static void hy_moe(gl3_ctx* ctx, HyLayer& L, int n) {
         const bool ks = hy_mv_split(L.ff_pad, W);
         const HyMv<T> f = hy_mv<T>(hb, W, L.gu, nullptr, shared_act, L.ff_pad, hy_ff_glu(L));
         const dim3 grid(1 + (ks ? L.ff_pad : hy_cdiv(L.ff_pad, 4)));
-#define HY_RU(PER) do { if (ks) hipLaunchKernelGGL((hy_route_up_kernel<T, PER, 4>), grid, dim3(256), 0, st, ra, f); else hipLaunchKernelGGL((hy_route_up_kernel<T, PER, 1>), grid, dim3(256), 0, st, ra, f); } while (0)
-        if (RZ <= 64) HY_RU(1); else if (RZ <= 256) HY_RU(4); else HY_RU(HY_RT_PER);
+#define HY_RU(PER) do { if (ks) hipLaunchKernelGGL((hy_route_up_kernel<T, PER, 4, decltype(once)::value>), grid, dim3(256), 0, st, ra, f); else hipLaunchKernelGGL((hy_route_up_kernel<T, PER, 1, decltype(once)::value>), grid, dim3(256), 0, st, ra, f); } while (0)
+        hy_with_once(hy_past_caches(ctx), [&](auto once) { if (RZ <= 64) HY_RU(1); else if (RZ <= 256) HY_RU(4); else HY_RU(HY_RT_PER); });
 #undef HY_RU
     } else {
 #define HY_RT(PER) hipLaunchKernelGGL((hy_route_kernel<PER>), dim3(n), dim3(64), 0, st, ra.z, ra.ldz, ra.parts, ra.pstride, ra.E, ra.top, ra.sel, ra.wgt, ra.pair_row, ra.extra_out, rt)
@@ -1900,8 +1905,10 @@ static void hy_moe(gl3_ctx* ctx, HyLayer& L, int n) {
         HyMv<T> e = hy_mv<T>((const T*)h->eact, L.eff_pad, one_down, h->eout, nullptr, 0, HyGlu{});
         e.ldc = W; e.sel = h->sel; e.wstride = (size_t)W * L.edown.ld; e.n_sel = E;
         const HyMv<T> s = hy_mv<T>(shared_act, L.ff_pad, L.down, h->y, nullptr, 0, HyGlu{});
-        if (ks) hipLaunchKernelGGL((hy_matvec_two_kernel<T, 4, 1>), dim3(gx * (1 + P)), dim3(256), 0, st, s, gx, e, gx);
-        else hipLaunchKernelGGL((hy_matvec_two_kernel<T, 1, 1>), dim3(gx * (1 + P)), dim3(256), 0, st, s, gx, e, gx);
+        hy_with_once(hy_past_caches(ctx), [&](auto once) {
+            if (ks) hipLaunchKernelGGL((hy_matvec_two_kernel<T, 4, 1, decltype(once)::value>), dim3(gx * (1 + P)), dim3(256), 0, st, s, gx, e, gx);
+            else hipLaunchKernelGGL((hy_matvec_two_kernel<T, 1, 1, decltype(once)::value>), dim3(gx * (1 + P)), dim3(256), 0, st, s, gx, e, gx);
+        });
         h->y_parts = 1;
         return;
     }
